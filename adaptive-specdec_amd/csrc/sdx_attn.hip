@@ -28,7 +28,14 @@
 // Q operands stay in registers; V is stored transposed in LDS so both MFMA
 // operands of P V are pairs of 8-byte reads. A row that fits one chunk writes its
 // output directly; otherwise each chunk writes (O unnormalised, max, sum) in
-// fp32 and a second kernel merges the chunks of the row.
+// fp32, and the chunk of the row that finishes last merges it.
+//
+// A batch that leaves the chip short of whole 1024-token chunks runs without the
+// plan (DIRECT): the workgroups derive a finer split from the rows' lengths, and
+// a second kernel merges with a workgroup per query row. One row of 8 KV heads
+// and about 12,000 keys: 31 us, against 525 us when chunks of 64 tokens were
+// planned by one thread and 230 partials of 20 query rows merged by one workgroup
+// per KV head; 2 rows of 16,384-32,768 keys 54 us, from 445.
 // The kernels are bound by the KV bytes streamed (about 22 flop per byte),
 // not by MFMA.
 #include "sdx_launch.hpp"
@@ -299,8 +306,68 @@ __device__ __forceinline__ void va_merge(const AttnArgs& a, int64_t b, int kvh, 
   }
 }
 
-// D: head dim, 64 or 128.
-template <int D>
+// ---- launches without a plan, for batches that leave the chip short of work with
+// whole 1024-token chunks. Every wave derives the same split from the rows'
+// lengths: the chunk size that gives about VA_SLOTS workgroups (the workgroups
+// that fit the chip at once: a row split finer pays a workgroup's set-up and its
+// partials again, split coarser it leaves CUs idle), at least a.chunk (which
+// bounds the partials the workspace holds), then the chunk of slot `unit` by a
+// scan over the rows.
+constexpr int VA_SLOTS = 768;  // 3 workgroups on each of 256 CUs
+struct VaSlot {
+  int64_t b, q0, qb, kvl;  // b = -1: no chunk in this slot
+  int c, chunk;
+};
+struct VaShape {  // one row per lane
+  int64_t q0 = 0, qb = 0, kvl = 0;
+  bool ok;  // a row the launch serves
+  __device__ __forceinline__ VaShape(const AttnArgs& a, int64_t b) : ok(va_row(a, b, q0, qb, kvl)) {}
+  __device__ __forceinline__ uint64_t keys() const { return ok && qb > 0 ? (uint64_t)kvl : 0ull; }
+};
+// first: rows 0 .. 63, lane by lane
+__device__ __forceinline__ int va_direct_chunk(const AttnArgs& a, const VaShape& first) {
+  if (!a.dyn) return a.chunk;
+  uint64_t total = wave_sum_u64(first.keys());  // keys of the rows served
+  for (int64_t b0 = kWave; b0 < a.batch; b0 += kWave)
+    total += wave_sum_u64(VaShape(a, b0 + (threadIdx.x & (kWave - 1))).keys());
+  // total / chunk whole chunks and about half a chunk more per row fill the slots
+  const uint64_t nh = (uint64_t)a.hkv * (uint64_t)a.nrb, half = (uint64_t)a.batch * nh / 2;
+  const uint64_t room = VA_SLOTS - min(half, (uint64_t)(3 * VA_SLOTS / 4));
+  const uint64_t ch = (total * nh / room + 63) / 64 * 64;
+  return (int)min((uint64_t)VA_CHMAX, max((uint64_t)a.chunk, ch));
+}
+__device__ __forceinline__ VaSlot va_direct_slot(const AttnArgs& a, int64_t unit, bool report) {
+  const int lane = threadIdx.x & (kWave - 1);
+  VaShape sh(a, lane);
+  VaSlot s;
+  s.b = -1;
+  s.chunk = va_direct_chunk(a, sh);
+  int64_t before = 0;  // chunks of the rows before b0
+  for (int64_t b0 = 0; b0 < a.batch; b0 += kWave) {
+    const int64_t b = b0 + lane;
+    if (b0 > 0) sh = VaShape(a, b);
+    if (report && unit == 0 && !sh.ok && b < a.batch && a.error) *a.error = 1;
+    const uint32_t nch = (uint32_t)((sh.keys() + s.chunk - 1) / s.chunk);
+    const uint32_t incl = wave_incl_scan_u32(nch, lane);
+    const int64_t first = before + incl - nch;
+    const uint64_t hit = __ballot(nch > 0 && unit >= first && unit < first + nch);
+    if (hit) {  // uniform
+      const int src = __ffsll((unsigned long long)hit) - 1;
+      s.b = b0 + src;
+      s.q0 = __shfl((long long)sh.q0, src, kWave);
+      s.qb = __shfl((long long)sh.qb, src, kWave);
+      s.kvl = __shfl((long long)sh.kvl, src, kWave);
+      s.c = (int)(unit - __shfl((long long)first, src, kWave));
+      if (!report || unit != 0) break;  // slot 0 goes on to look at every row
+    }
+    before += rdlane(incl, kWave - 1);
+  }
+  return s;
+}
+
+// D: head dim, 64 or 128. DIRECT: no plan; the workgroup finds its chunk itself, and
+// the chunk partials are plain stores for verify_attn_merge_kernel.
+template <int D, bool DIRECT>
 __global__ void __launch_bounds__(VA_NT) __attribute__((amdgpu_waves_per_eu(3)))
 verify_attn_kernel(AttnArgs a) {
   static_assert(D == 64 || D == 128, "head dims of 64 or 128");
@@ -323,23 +390,33 @@ verify_attn_kernel(AttnArgs a) {
   const int kvh = hx % a.hkv, rb = hx / a.hkv;
   const int64_t unit = 8 * grp + rem % 8;
   if (unit >= a.nunits) return;
-  const AttnUnit un = a.units[unit];
-  if (un.b < 0) return;  // uniform: no chunk in this slot
-  const int64_t b = un.b, q0 = un.q0, qb = un.qb, kvl = un.kvl;
-  const int c = un.c, n = un.n;
+  int64_t b, q0, qb, kvl;
+  int c, n, chunk = a.chunk;
+  if constexpr (DIRECT) {
+    const VaSlot sl = va_direct_slot(a, unit, hx == 0);
+    if (sl.b < 0) return;  // uniform: no chunk in this slot
+    chunk = sl.chunk;
+    b = sl.b, c = sl.c, q0 = sl.q0, qb = sl.qb, kvl = sl.kvl;
+    n = (int)min(kvl - (int64_t)c * chunk, (int64_t)chunk);
+  } else {
+    const AttnUnit un = a.units[unit];
+    if (un.b < 0) return;  // uniform: no chunk in this slot
+    b = un.b, q0 = un.q0, qb = un.qb, kvl = un.kvl;
+    c = un.c, n = un.n;
+  }
   // the KV head's query rows of the row (qb positions x group heads), and this
   // workgroup's block of them: rows rofs .. rofs + M - 1
   const int Mt = (int)qb * a.group, rofs = VA_MAXM * rb;
   if (rofs >= Mt) return;  // uniform: the row has fewer row blocks
   const int M = min(Mt - rofs, VA_MAXM);
-  const int64_t c0 = (int64_t)c * a.chunk;
+  const int64_t c0 = (int64_t)c * chunk;
   const int64_t p0 = c0 / a.bs;  // first page of the chunk
   const int np = (int)((c0 + n - 1) / a.bs - p0 + 1);
   // the chunk's page ids go to LDS (in the V tile's space, unused yet)
   int32_t* sPage = reinterpret_cast<int32_t*>(&sVt[0][0]);
   for (int i = tid; i < np; i += VA_NT) sPage[i] = a.block_table[b * a.max_blocks + p0 + i];
   const int64_t base = kvl - qb;
-  const bool whole = kvl <= a.chunk;  // the row is one chunk: write the output directly
+  const bool whole = kvl <= chunk;  // the row is one chunk: write the output directly
   // row i = j * group + g is query head kvh * group + g of position j; local row
   // il of the block is row rofs + il
   if (tid < M) {
@@ -545,18 +622,26 @@ verify_attn_kernel(AttnArgs a) {
       if (i < M) {
         float* po = a.part_o + (part + i) * D;
 #pragma unroll
-        for (int jj = 0; jj < OJ; ++jj) va_st_f32(po + jj * 16 + lc, o[jj][r]);
-        if (lc == 0) va_st_f2(a.part_ml + (part + i) * 2, m_run[r], l_run[r]);
+        for (int jj = 0; jj < OJ; ++jj) {
+          if constexpr (DIRECT) po[jj * 16 + lc] = o[jj][r];
+          else va_st_f32(po + jj * 16 + lc, o[jj][r]);
+        }
+        if (lc == 0) {
+          if constexpr (DIRECT)
+            *reinterpret_cast<float2*>(a.part_ml + (part + i) * 2) = make_float2(m_run[r], l_run[r]);
+          else va_st_f2(a.part_ml + (part + i) * 2, m_run[r], l_run[r]);
+        }
       }
     }
   }
+  if constexpr (DIRECT) return;  // the next kernel merges
   // the workgroup's stores are done before it counts in on the (row, KV head):
   // the one that counts in last merges the row's chunks
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // gfx9 encoding: vmcnt(0)
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __syncthreads();
-  const int nch = (int)((kvl + a.chunk - 1) / a.chunk);
+  const int nch = (int)((kvl + chunk - 1) / chunk);
   const int nrbr = (Mt + VA_MAXM - 1) / VA_MAXM;  // the row's blocks of query rows
   uint32_t* const flag = reinterpret_cast<uint32_t*>(&sRow[0]);  // row offsets no longer needed
   if (tid == 0)
@@ -570,28 +655,123 @@ verify_attn_kernel(AttnArgs a) {
               reinterpret_cast<float*>(&sVt[0][0]), (int)(sizeof(sK) / sizeof(float)));
 }
 
-int attn_chunk_tokens(int64_t batch, int32_t hkv, int64_t max_tokens, int32_t chunk) {
+// Merge of the chunk partials of one query row of (row b, KV head kvh), after a
+// DIRECT launch: blockIdx.x = (b * hkv + kvh) * max_m + i. VA_NT / (D / 4) slices of
+// the workgroup each take every SL-th chunk (float4 of D per thread), then add up
+// through LDS. Bound by the latency of two dependent load rounds, so a row's
+// query rows go to workgroups of their own.
+template <int D>
+__global__ void __launch_bounds__(VA_NT) verify_attn_merge_kernel(AttnArgs a) {
+  constexpr int DL = D / 4, SL = VA_NT / DL;
+  __shared__ float4 sAcc[SL][DL];
+  __shared__ float sDen[SL], sMax[VA_NW];
+  const int tid = threadIdx.x;
+  const int64_t bh = blockIdx.x / a.max_m;
+  const int i = (int)(blockIdx.x % a.max_m);
+  const int64_t b = bh / a.hkv;
+  const int kvh = (int)(bh % a.hkv);
+  int64_t q0, qb, kvl;
+  if (!va_row(a, b, q0, qb, kvl)) return;             // uniform
+  const int chunk = va_direct_chunk(a, VaShape(a, threadIdx.x & (kWave - 1)));
+  if (i >= (int)qb * a.group || kvl <= chunk) return;  // uniform: nothing to merge
+  const int nch = (int)((kvl + chunk - 1) / chunk);
+  const int64_t p0 = bh * a.nchunk * a.max_m + i;  // chunk c's part: p0 + c * max_m
+  const float2* const ml = reinterpret_cast<const float2*>(a.part_ml);
+  float mx = -INFINITY;
+  for (int c = tid; c < nch; c += VA_NT) mx = fmaxf(mx, ml[p0 + (int64_t)c * a.max_m].x);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+  if ((tid & (kWave - 1)) == 0) sMax[tid / kWave] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(sMax[0], sMax[1]), fmaxf(sMax[2], sMax[3]));
+  static_assert(VA_NW == 4, "four wave maxima");
+  const int d4 = tid % DL, sl = tid / DL;
+  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float den = 0.0f;
+#pragma unroll 4
+  for (int c = sl; c < nch; c += SL) {
+    const int64_t p = p0 + (int64_t)c * a.max_m;
+    const float2 w = ml[p];
+    const float4 v = *reinterpret_cast<const float4*>(a.part_o + p * D + d4 * 4);
+    // m = -inf: the chunk holds none of the row's visible keys
+    const float f = w.x == -INFINITY ? 0.0f : exp2f(w.x - mx);
+    den += f * w.y;
+    acc.x += f * v.x;
+    acc.y += f * v.y;
+    acc.z += f * v.z;
+    acc.w += f * v.w;
+  }
+  sAcc[sl][d4] = acc;
+  if (d4 == 0) sDen[sl] = den;
+  __syncthreads();
+  if (sl != 0) return;
+#pragma unroll
+  for (int k = 1; k < SL; ++k) {
+    const float4 v = sAcc[k][d4];
+    acc.x += v.x;
+    acc.y += v.y;
+    acc.z += v.z;
+    acc.w += v.w;
+  }
+  den = 0.0f;
+#pragma unroll
+  for (int k = 0; k < SL; ++k) den += sDen[k];
+  const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+  uint16_t* dst = a.out + ((q0 + i / a.group) * a.hq + kvh * a.group + i % a.group) * D + d4 * 4;
+  const uint32_t lo = (uint32_t)va_bf16(acc.x * inv) | ((uint32_t)va_bf16(acc.y * inv) << 16);
+  const uint32_t hi = (uint32_t)va_bf16(acc.z * inv) | ((uint32_t)va_bf16(acc.w * inv) << 16);
+  *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
+}
+
+// Chunk slots with whole 1024-token chunks below which a call runs without a plan.
+// Measured on both sides (us per call, plan | direct; 32 / 8 heads of 128, contexts
+// up to 8,192 unless said): 512 slots (8 rows) 56 | 49, 1,024 (16 rows) 95 | 99,
+// 2,048 (32 rows) 165 | 177, 8,192 (128 rows) 502 | 584.
+constexpr int64_t VA_DIRECT_SLOTS = 1024;
+
+// Tokens per chunk (the least of a direct launch, which may take more: see
+// va_direct_chunk) and whether the call runs without a plan.
+int attn_chunk_tokens(int64_t batch, int32_t hkv, int64_t nrb, int64_t max_tokens, int32_t chunk,
+                      bool* direct) {
+  auto slots = [&](int64_t ch) { return batch * hkv * nrb * ((max_tokens + ch - 1) / ch); };
+  *direct = slots(VA_CHMAX) < VA_DIRECT_SLOTS;
   if (chunk > 0) return chunk;
-  // smallest chunk count that still leaves about 8 workgroups per CU of work
   int ch = VA_CHMAX;
+  if (*direct) {
+    // Rows of one chunk need no merge launch (about 4 us, as long as four more tiles
+    // take); else at most twice the resident workgroups if every row were as long as
+    // the table allows.
+    if (max_tokens <= 6 * VA_TOK) return 6 * VA_TOK;
+    ch = 4 * VA_TOK;
+    while (ch < VA_CHMAX && slots(ch) > 2 * VA_SLOTS) ch += 2 * VA_TOK;
+    return ch;
+  }
+  // smallest chunk count that still leaves about 8 workgroups per CU of work
   while (ch > 2 * VA_TOK && batch * hkv * ((max_tokens + ch - 1) / ch) < 8 * 256) ch /= 2;
   return ch;
 }
 
 template <int D>
 static hipError_t launch_attn_d(const AttnArgs& a, hipStream_t s) {
-  if (a.nchunk > 1 && !a.arrive) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(verify_attn_kernel<D>,
-                     dim3((unsigned)((a.nunits + 7) / 8 * 8 * a.hkv * a.nrb)),
+  const dim3 grid((unsigned)((a.nunits + 7) / 8 * 8 * a.hkv * a.nrb));
+  if (!a.direct) {
+    if (a.nchunk > 1 && !a.arrive) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(verify_attn_plan_kernel, dim3(1), dim3(VA_PLAN_NT), 0, s, a);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    hipLaunchKernelGGL((verify_attn_kernel<D, false>), grid, dim3(VA_NT), 0, s, a);
+    return hipGetLastError();
+  }
+  if (a.nchunk > 1 && !a.part_o) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((verify_attn_kernel<D, true>), grid, dim3(VA_NT), 0, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.nchunk <= 1) return e;
+  hipLaunchKernelGGL(verify_attn_merge_kernel<D>, dim3((unsigned)(a.batch * a.hkv * a.max_m)),
                      dim3(VA_NT), 0, s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_verify_attn(const AttnArgs& a, int64_t batch, hipStream_t s) {
+hipError_t launch_verify_attn(const AttnArgs& a, hipStream_t s) {
   if (a.d != 64 && a.d != 128) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(verify_attn_plan_kernel, dim3(1), dim3(VA_PLAN_NT), 0, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   return a.d == 64 ? launch_attn_d<64>(a, s) : launch_attn_d<128>(a, s);
 }
 

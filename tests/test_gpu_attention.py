@@ -220,3 +220,45 @@ def test_verify_attention_bench_shape_sampled_rows():
         got = out[int(cu[b]):int(cu[b + 1])].float().cpu().numpy()
         bad = np.abs(got - ref) > 2e-2 + 2e-2 * np.abs(ref)
         assert not bad.any(), (b, np.abs(got - ref).max())
+
+
+@pytest.mark.parametrize("B,ctx_lo,ctx_hi,hq,hkv,d,k_max,chunk", [
+    # without a plan (fewer than 1,024 chunk slots): the workgroups find their chunks
+    (1, 180, 184, 8, 2, 128, 4, 0),       # one chunk of up to 192 keys, no merge
+    (1, 186, 420, 32, 8, 128, 4, 0),      # just past it: several chunks and the merge
+    (1, 9000, 9000, 32, 8, 128, 4, 0),    # one long row over the whole chip
+    (2, 5000, 5000, 4, 1, 64, 2, 0),      # 256 query heads x chunks of 16 threads per row
+    (70, 1, 900, 2, 1, 128, 3, 0),        # rows past the first wave of 64
+    (127, 1, 700, 8, 8, 64, 2, 0),        # the most rows of a launch without a plan
+    (130, 1, 300, 4, 2, 128, 3, 64),      # a chunk size of the caller's
+    # with a plan (1,024 slots or more): merged by the last chunk of a row
+    (128, 1, 300, 32, 8, 128, 5, 64),     # rows of one and of several chunks
+    (128, 1, 900, 16, 8, 64, 5, 128),
+    (130, 1, 100, 64, 8, 128, 8, 0),      # rows of one chunk, two blocks of query rows
+])
+def test_verify_attention_with_and_without_a_plan(B, ctx_lo, ctx_hi, hq, hkv, d, k_max, chunk):
+    """Both sides of the rule that decides whether a call runs without a plan, with
+    rows of one chunk and of several, the caller's chunk size and the library's."""
+    inp = attn_inputs(B, seed=B * 17 + ctx_hi, device=DEV, ctx_lo=ctx_lo, ctx_hi=ctx_hi, hq=hq,
+                      hkv=hkv, d=d, k_max=k_max, alpha_lo=0.6, alpha_hi=0.95)
+    _check(inp, hq, hkv, chunk_tokens=chunk)
+
+
+@pytest.mark.parametrize("B", [3, 130])
+def test_verify_attention_skips_rows_it_cannot_serve(B):
+    """A row whose length exceeds its block table sets the error word and keeps its
+    output; every other row is served (one-wave and several-wave row scans)."""
+    inp = attn_inputs(B, seed=B, device=DEV, ctx_lo=20, ctx_hi=400, hq=4, hkv=1, k_max=4)
+    kv = inp["kv_len"].clone()
+    kv[B - 1] = inp["block_table"].shape[1] * 16 + 1
+    err = torch.zeros(1, dtype=torch.int32, device=DEV)
+    args = (inp["q"], inp["cu_q"], inp["k_pool"], inp["v_pool"], inp["block_table"])
+    good = verify_attention_paged(*args, inp["kv_len"], inp["max_q"]).float()
+    out = torch.full_like(inp["q"], 7.0)
+    verify_attention_paged(*args, kv, inp["max_q"], out=out, error=err)
+    torch.cuda.synchronize()
+    last = int(inp["cu_q"][B - 1])
+    assert int(err.item()) == 1
+    assert bool((out[last:] == 7.0).all())
+    # the split follows the keys that are served, so only bf16 rounding may differ
+    assert torch.allclose(out[:last].float(), good[:last], atol=1e-2, rtol=1e-2)
