@@ -89,6 +89,18 @@ int row_stats16(int dtype, const sdx::RowStatArgs& a, int64_t rows, hipStream_t 
   return hip_status(sdx::launch_rowstat16(dtype, a, rows, s), "rowstat16");
 }
 
+// Threshold statistics (sdx_thr.hip) of ntgt target and ndrf draft rows, without the
+// scratch and the outputs.
+sdx::ThrArgs thr_args(const void* target, const void* draft, int64_t ntgt, int64_t ndrf, int64_t ld,
+                      int64_t V, float T, float top_p, int32_t top_k, const Switches& sw) {
+  sdx::ThrArgs a = {};
+  a.base[0] = target; a.nrows[0] = ntgt; a.ld[0] = ld;
+  a.base[1] = draft; a.nrows[1] = ndrf; a.ld[1] = ld;
+  a.V = V; a.T = T; a.top_p = top_p; a.top_k = top_k;
+  a.use_p = sw.use_p; a.use_k = sw.use_k;
+  return a;
+}
+
 int check_vocab(int dtype, int64_t V) {
   if (V < 1) return fail(SDX_EINVAL, "vocab must be >= 1");
   if (dtype == SDX_F32 && V > sdx::kF32MaxVocab)
@@ -143,12 +155,27 @@ int sdx_to_probs(const void* logits, int dtype, int64_t rows, int64_t vocab, int
   const Switches sw = switches(temperature, top_p, top_k, vocab);
   Carve c{(uint8_t*)workspace};
   if (dtype == SDX_F32) {
-    // the large-vocabulary kernel keeps per-element intermediates in the output
-    // rows between its passes, so the output may not overlap the logits
+    // rows above kF32SortVocab keep their scratch in the output rows until the output
+    // pass, so the output may not overlap the logits
     const uintptr_t l0 = (uintptr_t)logits, l1 = l0 + (uintptr_t)(((rows - 1) * ld + vocab) * 4);
     const uintptr_t p0 = (uintptr_t)probs, p1 = p0 + (uintptr_t)(((rows - 1) * ld_out + vocab) * 4);
     if (l0 < p1 && p0 < l1)
       return fail(SDX_EINVAL, "sdx_to_probs: probs overlap the fp32 logits");
+    if (vocab > sdx::kF32SortVocab) {
+      if (sw.greedy) {
+        int64_t* am = c.take<int64_t>(rows);
+        const bool vec = aligned16(logits) && ld % 4 == 0;
+        if (int e = hip_status(sdx::launch_argmax(dtype, logits, rows, vocab, ld, vec, am, s),
+                               "argmax"))
+          return e;
+        return hip_status(sdx::launch_onehot(am, rows, vocab, probs, ld_out, s), "onehot");
+      }
+      sdx::ThrArgs a = thr_args(logits, logits, rows, 0, ld, vocab, temperature, top_p, top_k, sw);
+      a.stats = c.take<sdx::RowStat>(rows);
+      a.scratch = probs; a.scratch_stride = ld_out * 4; a.scratch_bytes = vocab * 4;
+      if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
+      return hip_status(sdx::launch_thr_output(dtype, a, rows, probs, ld_out, s), "thr_output");
+    }
     sdx::F32Args a = {};
     a.base[0] = (const float*)logits; a.nrows[0] = rows; a.ld[0] = ld;
     a.base[1] = a.base[0]; a.nrows[1] = 0; a.ld[1] = ld;
@@ -529,7 +556,17 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
                       "greedy_accept");
   }
   if (!draft_logits) return fail(SDX_EINVAL, "sdx_verify: draft_logits required when T > 0");
-  if (dtype == SDX_F32) {
+  const bool thr = dtype == SDX_F32 && vocab > sdx::kF32SortVocab;
+  if (thr) {
+    // the rows' dense space serves as scratch: the draw evaluates what it needs
+    sdx::ThrArgs a = thr_args(target_logits, draft_logits, ntgt, ndrf, vocab, vocab, temperature,
+                              top_p, top_k, sw);
+    a.ids = draft_ids; a.k = k; a.tgt_idx = tgt_idx;
+    a.stats = st;
+    a.zero = counters; a.nzero = batch;
+    a.scratch = dn; a.scratch_stride = a.scratch_bytes = vocab * 4;
+    if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
+  } else if (dtype == SDX_F32) {
     sdx::F32Args a = {};
     a.base[0] = (const float*)target_logits; a.nrows[0] = ntgt; a.ld[0] = vocab;
     a.base[1] = (const float*)draft_logits; a.nrows[1] = ndrf; a.ld[1] = vocab;
@@ -601,6 +638,15 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
   if (stats_only) return SDX_OK;
   sdx::AcceptArgs aa{st,    batch, k,         u_accept, u_final, active, jobs,
                      n_acc, flags, draft_ids, cu_k,     bad,     ntgt};
+  if (thr) {
+    sdx::ThrDrawArgs d = {};
+    d.acc = aa;
+    d.base[0] = target_logits; d.base[1] = draft_logits; d.nrows0 = ntgt;
+    d.ld[0] = d.ld[1] = vocab;
+    d.V = vocab; d.T = temperature;
+    d.recs = (uint64_t*)recs; d.counters = counters; d.y = y;
+    return hip_status(sdx::launch_thr_draw(dtype, d, batch, s), "thr_draw");
+  }
   if (dtype == SDX_F32) {
     sdx::RowSourceF32 src{dn, vocab, dn, vocab, rows, (vocab % 4) == 0};
     return hip_status(sdx::launch_draw_probs(src, &aa, jobs, batch, vocab, recs,
@@ -760,6 +806,25 @@ int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, 
     if (int r = hip_status(sdx::launch_argmax(dtype, logits, batch, vocab, ld, vec, x, s), "argmax"))
       return r;
     e.greedy = true;
+    return hip_status(sdx::launch_draft_epilogue(e, s), "draft_epilogue");
+  }
+  if (dtype == SDX_F32 && vocab > sdx::kF32SortVocab) {
+    sdx::ThrArgs a = thr_args(logits, logits, batch, 0, ld, vocab, temperature, top_p, top_k, sw);
+    a.stats = st;
+    a.zero = counters; a.nzero = batch;
+    a.scratch = dn; a.scratch_stride = a.scratch_bytes = vocab * 4;
+    if (int r = hip_status(sdx::launch_thr_stats(dtype, a, batch, s), "thr_stats")) return r;
+    sdx::ThrDrawArgs d = {};  // k = 0: the bonus draw of each row on u
+    d.acc = sdx::AcceptArgs{st,      batch,   0,       u,       u,       nullptr, jobs,
+                            nullptr, nullptr, nullptr, nullptr, nullptr, batch};
+    d.base[0] = d.base[1] = logits; d.nrows0 = batch;
+    d.ld[0] = d.ld[1] = ld;
+    d.V = vocab; d.T = temperature;
+    d.recs = (uint64_t*)recs; d.counters = counters; d.y = x;
+    d.qx = (float*)jobs;  // one value per row, for the epilogue
+    if (int r = hip_status(sdx::launch_thr_draw(dtype, d, batch, s), "thr_draw")) return r;
+    e.probs = d.qx;
+    e.ldp = 0;
     return hip_status(sdx::launch_draft_epilogue(e, s), "draft_epilogue");
   }
   if (dtype == SDX_F32) {

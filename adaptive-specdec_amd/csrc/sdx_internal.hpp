@@ -24,8 +24,10 @@ enum RowFlag : uint32_t {
                              // set by the rank kernel from its member rank
   kRowBadWs = 1u << 6,       // split row whose workspace header was not initialised
                              // (sdx_workspace_init): statistics not computed
-  kRowGatherTie = 1u << 7    // the gathered (drafted) token is a member of the row's
+  kRowGatherTie = 1u << 7,   // the gathered (drafted) token is a member of the row's
                              // partially kept boundary tie group
+  kRowNoMass = 1u << 8       // no finite maximum (every logit -inf, or a +inf): probabilities
+                             // are 0 / 0 (threshold rows, sdx_thr.hip)
 };
 
 // 64 bytes per row. Keys in [glo, ghi] form the tie group that straddles the

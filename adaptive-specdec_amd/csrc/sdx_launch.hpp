@@ -203,6 +203,9 @@ hipError_t launch_workspace_rearm(void* ws, hipStream_t s);
 // sdx_rank.hip: pgather of drafted tokens inside a partial tie group (after rowstream)
 hipError_t launch_rank_bf16(const RowStatArgs& a, int64_t rows, hipStream_t s);
 // sdx_f32.hip
+// fp32 rows up to here are sorted whole in LDS (to_probs_f32_kernel); longer ones take
+// the threshold statistics of sdx_thr.hip
+constexpr int64_t kF32SortVocab = 8192;
 // Largest vocabularies of 16-bit rows. bf16 rows stream through the histogram
 // kernel, whose normaliser queues a bin as (bin << 18 | count): counts, so the
 // vocabulary, stay below 2^18 (the largest multiple of 8 below it, as rows are
@@ -214,6 +217,53 @@ constexpr int64_t kF32MaxVocab = 262144;
 // tie-group bit words per fp32 row: one bit per id, whole 64-id wave rounds
 inline int64_t f32_tie_words(int64_t V) { return (V + 63) / 64 * 2; }
 hipError_t launch_to_probs_f32(const F32Args& a, int64_t rows, hipStream_t s);
+// sdx_thr.hip: row statistics as a threshold (see sdx_thr.hpp) and what reads them
+constexpr int kThrMaxParts = 32;    // workgroups per row
+constexpr int kThrBuckets = 1024;   // steps of m - s
+constexpr int kThrList = 2048;      // region elements listed
+constexpr int kThrRec = 1024;       // ids per draw record
+constexpr int64_t kThrCtlBytes = 1024;
+// scratch per row (with room to align its start)
+constexpr int64_t kThrScratchMin = 64 + kThrCtlBytes + kThrList * 8 + kThrBuckets * 12;
+struct ThrArgs {
+  const void* base[2];  // group 0: target rows, group 1: draft rows
+  int64_t nrows[2];
+  int64_t ld[2];
+  int64_t V;
+  const int64_t* ids;  // as in RowStatArgs
+  int32_t k;
+  const int64_t* tgt_idx;
+  float T, top_p;
+  int32_t top_k, use_p, use_k;
+  RowStat* stats;
+  uint32_t* zero;  // words [0, nzero) cleared (by row `row`'s workgroups: word `row`), or null
+  int64_t nzero;
+  void* scratch;   // row r's at r * scratch_stride bytes, no initial contents
+  int64_t scratch_stride;
+  int64_t scratch_bytes;  // bytes of it that a row may use (at least kThrScratchMin)
+  // set by launch_thr_stats: workgroups per row and their elements, in the histogram
+  // pass and in the passes that only compare
+  int32_t nparts, nlight;
+  int64_t plen, llen;
+};
+hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s);
+// to_probs rows; the scratch may lie in `out` (it is read no more)
+hipError_t launch_thr_output(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+                             hipStream_t s);
+struct ThrDrawArgs {
+  AcceptArgs acc;  // acc.k = 0: a draw from each row (a draft step)
+  const void* base[2];
+  int64_t nrows0;
+  int64_t ld[2];
+  int64_t V;
+  float T;
+  uint64_t* recs;      // [jobs, nrec, 2] masses of p and of the residual
+  uint32_t* counters;  // [jobs], zero on entry
+  int64_t* y;
+  float* qx;           // [jobs] the drawn id's probability, or null
+  int32_t nrec, nblk;  // set by launch_thr_draw
+};
+hipError_t launch_thr_draw(int dtype, ThrDrawArgs a, int64_t jobs, hipStream_t s);
 // sdx_sample.hip
 // Draw: chunk records and the per-job select in one launch (with the accept
 // chain when `acc` is given: jobs are then written by the kernel). Without

@@ -1,0 +1,1049 @@
+// to_probs statistics and outputs of rows whose values cannot be enumerated (fp32
+// logits, specdec/sampling.py:34-67), several workgroups per row.
+//
+// The transform of a row reduces to one record: its final probability is
+//   p(id) = exp_det(s - m) / zf,  s = fl32(x / T)
+//   kept  = p > vf, or p == vf and id <= idcut      (p / totf where kept, else 0)
+// because the reference keeps a prefix of the order (p descending, id ascending).
+// The record takes four kernels over `nparts` workgroups per row and one small one:
+//   1. thr_max_kernel      the row's maximum (and minimum) logit per part;
+//   2. thr_hist_kernel     the exact normaliser (96-bit fixed point per thread), and
+//                          masses (and, for top-k, counts) of the elements in NB
+//                          equal steps of m - s. The part that finishes last
+//                          finds the region: the steps that can
+//                          hold the boundary element, with a margin of 1e-6 of the
+//                          mass on each side (what rounding to p, to fixed point and
+//                          to fp32 cumulative sums can move is below 4e-7). As an
+//                          interval of p [plo, phi] it holds whole tie groups;
+//   3. thr_collect_kernel  count and exact mass of the elements above the region,
+//                          and a list (p, id) of the region's;
+//   4. thr_resolve_kernel  one workgroup per row sorts the list and walks it with the
+//                          reference's test. A region with more than kThrList
+//                          elements (a large tie group) is refined over the row
+//                          itself, ten bits of p at a time;
+// then thr_output_kernel writes to_probs rows, and thr_draw_kernel is the verify's
+// accept chain and draw, which evaluates p where it needs it: a verify writes no
+// probabilities.
+//
+// What bounds it: the instructions of the exp of pass 2, which every element needs
+// (about 50 per element: the reference division by T as two FMA steps from 1 / T,
+// the float64 reduction, nine multiply-adds, and the fixed-point value formed from
+// the mantissa and the exponent by one shift); the other passes compare a logit
+// with a threshold and evaluate only the few elements above it, compacted to full
+// waves. Splitting a row over workgroups keeps the chip full from a few rows on.
+// Measured on fp32 rows of 151,936 (one workgroup of 1024 threads per row before, with
+// seven IEEE divisions per element and dense probabilities for the draw): verify of 8
+// batch rows at k = 4 (72 rows, top-k 50) 285 -> 67 us (kernels 11 + 29 + 11 + 5 and
+// the draw 13), to_probs of 256 rows 378 -> 206 us (50 + 62 + 33 + 8 + 59: the first
+// pass also pays for the write-back of the call before, the last moves 5.3 TB/s).
+#include "sdx_thr.hpp"
+
+namespace sdx {
+
+constexpr int TH_NT = 256;
+constexpr int TH_NW = TH_NT / kWave;
+constexpr int TH_NB = kThrBuckets;
+constexpr int TH_BPT = TH_NB / TH_NT;  // buckets per thread
+
+// ---- loads: 16 bytes per lane and step, the elements before the row's first 16-byte
+// boundary with part 0, those after the last whole vector with the last part
+template <class E>
+struct ThrVec {
+  static constexpr int N = 16 / (int)sizeof(E);
+};
+__device__ __forceinline__ float thr_f(float x) { return x; }
+__device__ __forceinline__ float thr_f(uint16_t c) { return decode16<SDX_F16>(c); }
+
+// Streams part `part` of the row through f(id, x, valid), every element exactly once:
+// every lane of a wave makes every call (valid: the lane has an element), so f may
+// vote. UN vectors per thread are in flight.
+template <class E, int UN, class F>
+__device__ __forceinline__ void thr_stream(const E* __restrict__ row, int64_t V, int part,
+                                           int nparts, int64_t plen, F&& f) {
+  constexpr int N = ThrVec<E>::N;
+  const int tid = threadIdx.x;
+  int64_t head = (int64_t)(((16u - ((uint32_t)(uintptr_t)row & 15u)) & 15u) / sizeof(E));
+  if (head > V) head = V;
+  const int64_t nv = (V - head) / N;  // whole vectors of the row
+  const int64_t v0 = (int64_t)part * (plen / N);
+  const int64_t v1 = part == nparts - 1 ? nv : min(nv, v0 + plen / N);
+  if (part == 0 && tid < kWave) {  // wave 0: fewer than 64 elements
+    const bool ok = tid < head;
+    f((int64_t)tid, ok ? thr_f(row[tid]) : 0.0f, ok);
+  }
+  if (part == nparts - 1 && tid < kWave) {
+    const int64_t i = head + nv * N + tid;
+    const bool ok = i < V;
+    f(i, ok ? thr_f(row[i]) : 0.0f, ok);
+  }
+  const uint4* __restrict__ x4 = reinterpret_cast<const uint4*>(row + head);
+  for (int64_t b = v0; b < v1; b += (int64_t)UN * TH_NT) {  // uniform
+    uint4 w[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int64_t j = b + (int64_t)u * TH_NT + tid;
+      w[u] = j < v1 ? x4[j] : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      if (b + (int64_t)u * TH_NT + (tid & ~(kWave - 1)) >= v1) break;  // uniform per wave
+      const int64_t j = b + (int64_t)u * TH_NT + tid;
+      const bool ok = j < v1;
+      const int64_t i = head + j * N;
+      const uint32_t q[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        float x;
+        if constexpr (sizeof(E) == 4) x = __uint_as_float(q[e]);
+        else x = thr_f((uint16_t)(q[e >> 1] >> (16 * (e & 1))));
+        f(i + e, x, ok);
+      }
+    }
+  }
+}
+
+template <class E>
+__device__ __forceinline__ const E* thr_row(const ThrArgs& a, int64_t row) {
+  const int g = row < a.nrows[0] ? 0 : 1;
+  const int64_t r = g ? row - a.nrows[0] : row;
+  return reinterpret_cast<const E*>(a.base[g]) + r * a.ld[g];
+}
+__device__ __forceinline__ int64_t thr_gid(const ThrArgs& a, int64_t row) {
+  const int g = row < a.nrows[0] ? 0 : 1;
+  return draft_id_of_row(a.ids, a.tgt_idx, a.k, a.nrows[1], g, g ? row - a.nrows[0] : row);
+}
+// the row's scratch: ThrCtl, the list, then the masses and the counts
+__device__ __forceinline__ ThrCtl* thr_ctl(const ThrArgs& a, int64_t row) {
+  const uintptr_t p = (uintptr_t)a.scratch + (uintptr_t)row * (uintptr_t)a.scratch_stride;
+  return reinterpret_cast<ThrCtl*>((p + 63) & ~(uintptr_t)63);
+}
+__device__ __forceinline__ uint64_t* thr_list(ThrCtl* c) {
+  return reinterpret_cast<uint64_t*>(c + 1);
+}
+__device__ __forceinline__ uint64_t* thr_mass(ThrCtl* c) { return thr_list(c) + kThrList; }
+__device__ __forceinline__ uint32_t* thr_cnt(ThrCtl* c) {
+  return reinterpret_cast<uint32_t*>(thr_mass(c) + TH_NB);
+}
+
+// ---------------------------------------------------------------- 1. maximum
+template <class E>
+__global__ void __launch_bounds__(TH_NT) thr_max_kernel(ThrArgs a) {
+  __shared__ float sMx[TH_NW], sMn[TH_NW];
+  const int64_t row = blockIdx.x / a.nlight;
+  const int part = (int)(blockIdx.x % a.nlight);
+  const int tid = threadIdx.x;
+  ThrCtl* const c = thr_ctl(a, row);
+  if (part == 0 && tid == 0) {
+    c->tick = 0u; c->nlist = 0u; c->cnt_above = 0u; c->mass_above = 0ull;
+    c->z[0] = c->z[1] = c->z[2] = 0ull;
+    if (row < a.nzero) a.zero[row] = 0u;
+  }
+  if (a.nparts > 1)  // the row's histogram, a share per part
+    for (int b = part * TH_NT + tid; b < TH_NB; b += a.nlight * TH_NT) {
+      thr_mass(c)[b] = 0ull;
+      thr_cnt(c)[b] = 0u;
+    }
+  float mx = -INFINITY, mn = INFINITY;
+  thr_stream<E, 8>(thr_row<E>(a, row), a.V, part, a.nlight, a.llen,
+                   [&](int64_t, float x, bool ok) {
+                     mx = ok ? fmaxf(mx, x) : mx;
+                     mn = ok && x > -INFINITY ? fminf(mn, x) : mn;
+                   });
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+    mn = fminf(mn, __shfl_xor(mn, o, kWave));
+  }
+  if ((tid & (kWave - 1)) == 0) { sMx[tid / kWave] = mx; sMn[tid / kWave] = mn; }
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < TH_NW; ++w) { mx = fmaxf(mx, sMx[w]); mn = fminf(mn, sMn[w]); }
+    c->pmax[part] = mx;
+    c->pmin[part] = mn;
+  }
+}
+
+// ---------------------------------------------------------------- 2. normaliser, region
+// fixed62(exp_det(d)) for d <= 0 (and 0 for NaN): exp_det's steps, then the value
+// mant * 2^(k + 39) as a right shift of mant << 39 (k is in [-63, 0] after the clamp at
+// -43.5, below which the value is 0). Equal to the two functions over every fp32 d.
+__device__ __forceinline__ uint64_t thr_exp62(float d) {
+#pragma clang fp contract(off)
+  const double dd = (double)fmaxf(d, -43.5f);
+  const double kf = floor(dd * 0x1.71547652b82fep+0);
+  const float r = fmaxf((float)(dd - kf * 0x1.62e42fefa39efp-1), 0.0f);
+  float p = 0x1.71de3ap-19f;  // 1/9!
+  p = p * r + 0x1.a01a02p-16f;
+  p = p * r + 0x1.a01a02p-13f;
+  p = p * r + 0x1.6c16c2p-10f;
+  p = p * r + 0x1.111112p-7f;
+  p = p * r + 0x1.555556p-5f;
+  p = p * r + 0x1.555556p-3f;
+  p = p * r + 0x1p-1f;
+  p = p * r + 1.0f;
+  p = p * r + 1.0f;
+  p = fminf(p, 2.0f);
+  const uint32_t mant = __float_as_uint(p) - 0x3F000000u;  // p in [1, 2]: 24-bit mantissa
+  return ((uint64_t)(mant << 7) << 32) >> (uint32_t)(-(int)kf);
+}
+
+// How s = x / T is formed: T == 1; two Newton steps on x * (1 / T) with FMAs, which
+// round correctly where no step under- or overflows (the first leaves the quotient
+// within an ulp, the second is Markstein's); or the division itself.
+enum ThrDiv { kDivOne, kDivFma, kDivIeee };
+template <int DIV>
+__device__ __forceinline__ float thr_div(float x, float T, float rT) {
+  if constexpr (DIV == kDivOne) return x;
+  if constexpr (DIV == kDivIeee) return x / T;
+  const float q0 = x * rT;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-T, q0, x), rT, q0);
+  return __builtin_fmaf(__builtin_fmaf(-T, q1, x), rT, q1);
+}
+
+struct ThrHistLds {
+  uint64_t mass[TH_NB];
+  uint32_t cnt[TH_NB];
+  uint64_t s64[TH_NW];
+  uint64_t zl[TH_NW];
+  uint32_t zh[TH_NW];
+  int32_t last, b0, b1, bk;
+};
+
+__device__ __forceinline__ uint64_t thr_excl_u64(uint64_t v, uint64_t* s) {
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const uint64_t incl = wave_incl_scan_u64(v, lane);
+  __syncthreads();
+  if (lane == kWave - 1) s[w] = incl;
+  __syncthreads();
+  uint64_t off = 0;
+  for (int i = 0; i < TH_NW; ++i) off += i < w ? s[i] : 0ull;
+  return off + incl - v;
+}
+
+template <class E, int DIV, bool CNT>
+__device__ __forceinline__ void thr_hist_pass(const ThrArgs& a, ThrHistLds& L, const E* row,
+                                              int part, float m, float scale, uint64_t& zlo,
+                                              uint32_t& zhi) {
+  const float T = a.T, rT = 1.0f / a.T;
+  thr_stream<E, 4>(row, a.V, part, a.nparts, a.plen, [&](int64_t, float x, bool ok) {
+    const float d = ok ? thr_div<DIV>(x, T, rT) - m : -INFINITY;
+    const int b = (int)fminf(-d * scale, (float)(TH_NB - 1));  // NaN: the last step
+    const uint64_t f = thr_exp62(d);
+    zlo += f;
+    zhi += zlo < f ? 1u : 0u;
+    if (CNT && ok) atomicAdd(&L.cnt[b], 1u);
+    // 2^-44 units: sums of 2^18 elements fit 64 bits
+    if (f >> 18) atomicAdd((unsigned long long*)&L.mass[b], (unsigned long long)(f >> 18));
+  });
+}
+
+template <class E>
+__global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
+  __shared__ ThrHistLds L;
+  const int64_t row = blockIdx.x / a.nparts;
+  const int part = (int)(blockIdx.x % a.nparts);
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  ThrCtl* const c = thr_ctl(a, row);
+  const E* const x = thr_row<E>(a, row);
+  for (int b = tid; b < TH_NB; b += TH_NT) { L.mass[b] = 0ull; L.cnt[b] = 0u; }
+  float xmx = lane < a.nlight ? c->pmax[lane] : -INFINITY;
+  float xmn = lane < a.nlight ? c->pmin[lane] : INFINITY;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    xmx = fmaxf(xmx, __shfl_xor(xmx, o, kWave));
+    xmn = fminf(xmn, __shfl_xor(xmn, o, kWave));
+  }
+  const float T = a.T;
+  const float m = xmx / T;  // the division is monotone: the maximum of fl32(x / T)
+  // steps of 2^-e, e >= 5: the row's range (at most 32) over at most TH_NB steps
+  const float range = fminf(m - xmn / T, 32.0f);  // NaN (no finite logit): 32
+  float scale = TH_NB / 32.0f;
+  while (scale < 0x1p20f && range * (2.0f * scale) <= (float)(TH_NB - 2)) scale *= 2.0f;
+  const float axm = fabsf(xmx);
+  const int div = T == 1.0f ? kDivOne
+                  : (T >= 0x1p-20f && T <= 0x1p20f && axm <= 0x1p100f &&
+                     (axm >= 0x1p-90f || axm == 0.0f))
+                      ? kDivFma
+                      : kDivIeee;
+  __syncthreads();
+  uint64_t zlo = 0;
+  uint32_t zhi = 0;
+  if (a.use_k) {
+    if (div == kDivOne) thr_hist_pass<E, kDivOne, true>(a, L, x, part, m, scale, zlo, zhi);
+    else if (div == kDivFma) thr_hist_pass<E, kDivFma, true>(a, L, x, part, m, scale, zlo, zhi);
+    else thr_hist_pass<E, kDivIeee, true>(a, L, x, part, m, scale, zlo, zhi);
+  } else {
+    if (div == kDivOne) thr_hist_pass<E, kDivOne, false>(a, L, x, part, m, scale, zlo, zhi);
+    else if (div == kDivFma) thr_hist_pass<E, kDivFma, false>(a, L, x, part, m, scale, zlo, zhi);
+    else thr_hist_pass<E, kDivIeee, false>(a, L, x, part, m, scale, zlo, zhi);
+  }
+  U128 z = wave_sum_u128(U128{zlo, (uint64_t)zhi});
+  if (lane == 0) { L.zl[wv] = z.lo; L.zh[wv] = (uint32_t)z.hi; }
+  __syncthreads();  // and the histogram is complete
+  z = U128{0, 0};
+  for (int w = 0; w < TH_NW; ++w) z = u128_add(z, U128{L.zl[w], L.zh[w]});
+  if (a.nparts > 1) {
+    // The row's sums by device-coherent atomics, step tid + 256 i per thread (a wave's
+    // land in a few lines): nothing waits for them but the ticket. The part that
+    // finishes last then reads one histogram; adding the parts' up there instead, four
+    // in flight, took 8 to 10 us of dependent loads that miss the L2 at 15 parts.
+    uint64_t* const gm = thr_mass(c);
+    uint32_t* const gc = thr_cnt(c);
+#pragma unroll
+    for (int i = 0; i < TH_BPT; ++i) {
+      const int b = tid + i * TH_NT;
+      const uint64_t v = L.mass[b];
+      if (v)
+        __hip_atomic_fetch_add(gm + b, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (a.use_k && L.cnt[b])
+        __hip_atomic_fetch_add(gc + b, L.cnt[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (tid < 3)  // 32-bit limbs in 64-bit words
+      __hip_atomic_fetch_add(&c->z[tid], tid == 2 ? z.hi : tid == 1 ? z.lo >> 32 : z.lo & 0xFFFFFFFFu,
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // gfx9 encoding: vmcnt(0)
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();
+    if (tid == 0)
+      L.last = __hip_atomic_fetch_add(&c->tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+               (uint32_t)(a.nparts - 1);
+    __syncthreads();
+    if (!L.last) return;  // uniform
+    uint64_t tm[TH_BPT];
+    uint32_t tc[TH_BPT];
+#pragma unroll
+    for (int i = 0; i < TH_BPT; ++i) {
+      tm[i] = __hip_atomic_load(gm + tid + i * TH_NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      tc[i] = a.use_k ? __hip_atomic_load(gc + tid + i * TH_NT, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT)
+                      : 0u;
+    }
+    const uint64_t z0 = __hip_atomic_load(&c->z[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t z1 = __hip_atomic_load(&c->z[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t z2 = __hip_atomic_load(&c->z[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    z = u128_add(u128_add(U128{z0, 0}, U128{z1 << 32, z1 >> 32}), U128{0, z2});
+#pragma unroll
+    for (int i = 0; i < TH_BPT; ++i) {
+      L.mass[tid + i * TH_NT] = tm[i];
+      L.cnt[tid + i * TH_NT] = tc[i];
+    }
+    __syncthreads();
+  }
+  uint64_t mass[TH_BPT];
+  uint32_t cnt[TH_BPT];
+#pragma unroll
+  for (int i = 0; i < TH_BPT; ++i) {
+    mass[i] = L.mass[tid * TH_BPT + i];
+    cnt[i] = L.cnt[tid * TH_BPT + i];
+  }
+  // ---- the region, step indexes [b0, b1] (0 at the maximum)
+  const float zf = rn32_u128(z);
+  if (tid == 0) { L.b0 = TH_NB - 1; L.b1 = TH_NB - 1; L.bk = TH_NB - 1; }
+  uint64_t sm = 0, sc = 0;
+#pragma unroll
+  for (int i = 0; i < TH_BPT; ++i) { sm += mass[i]; sc += cnt[i]; }
+  uint64_t rm = thr_excl_u64(sm, L.s64);
+  uint64_t rc = a.use_k ? thr_excl_u64(sc, L.s64) : 0ull;
+  __syncthreads();
+  const double zu = ((double)z.hi * 0x1p64 + (double)z.lo) * 0x1p-18;
+  const double tlo = ((double)a.top_p - 1e-6) * zu, thi = ((double)a.top_p + 1e-6) * zu;
+#pragma unroll
+  for (int i = 0; i < TH_BPT; ++i) {
+    const uint64_t nm = rm + mass[i], nc = rc + cnt[i];
+    const int b = tid * TH_BPT + i;
+    // the first step whose running mass (count) reaches a bound: one writer each, as
+    // the running sums grow (the step before has not reached it)
+    if ((double)nm >= tlo && !(b > 0 && (double)rm >= tlo)) L.b0 = b;
+    if ((double)nm >= thi && !(b > 0 && (double)rm >= thi)) L.b1 = b;
+    if (a.use_k && nc >= (uint64_t)a.top_k && rc < (uint64_t)a.top_k) L.bk = b;
+    rm = nm;
+    rc = nc;
+  }
+  __syncthreads();
+  if (tid != 0) return;
+  int b0 = L.b0, b1 = L.b1;
+  bool use_k = a.use_k, use_p = a.use_p;
+  if (use_k && !use_p) {
+    b0 = b1 = L.bk;
+  } else if (use_k) {
+    if (b1 < L.bk) use_k = false;  // the nucleus ends above the k-th largest
+    else { b0 = min(b0, L.bk); b1 = L.bk; }
+  }
+  const float inv = 1.0f / scale;  // a power of two
+  float phi = -1.0f, plo = 0x1p-149f, dlo = -104.0f;  // no filter: everything is above
+  if (use_k || use_p) {
+    // edges of the steps: p at m - s = b0 / scale and (b1 + 1) / scale
+    phi = b0 == 0 ? 2.0f : exp_det(-(float)b0 * inv) / zf;
+    if (b1 < TH_NB - 1) {
+      dlo = -(float)(b1 + 1) * inv;
+      plo = fmaxf(exp_det(dlo) / zf, 0x1p-149f);
+    }
+  }
+  // no logit below xcut has p >= plo: p drops by more than its rounding within 1e-5
+  // of s, and the fp32 rounding of (m + dlo) T is within 1e-6 of its terms
+  float xcut = ((m + dlo) - (4e-6f * (fabsf(m) + fabsf(dlo)) + 2e-5f)) * T;
+  xcut -= 4e-6f * fabsf(xcut);
+  if (!(fabsf(xcut) < INFINITY)) xcut = -INFINITY;
+  c->m = m;
+  c->zf = zf;
+  c->phi = phi;
+  c->plo = plo;
+  c->xcut = xcut;
+  c->use_k = use_k ? 1 : 0;
+  c->use_p = use_p ? 1 : 0;
+}
+
+// ---------------------------------------------------------------- 3. collect
+// Per wave: ids that pass the threshold are compacted into LDS and evaluated 64 at a
+// time by full waves.
+struct ThrQueue {
+  float x[2 * kWave];
+  uint32_t id[2 * kWave];
+};
+__device__ __forceinline__ void thr_lds_sync() {  // within one wave
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_wave_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+// Appends the lanes' (x, id) with `take`; full waves go through g(x, id, true).
+template <class G>
+__device__ __forceinline__ void thr_push(ThrQueue& q, uint32_t& n, float x, uint32_t id, bool take,
+                                         G&& g) {
+  const uint64_t bm = __ballot(take);
+  if (bm == 0) return;  // uniform
+  const int lane = threadIdx.x & (kWave - 1);
+  if (take) {
+    const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+    q.x[at] = x;
+    q.id[at] = id;
+  }
+  n += (uint32_t)__popcll(bm);
+  if (n < kWave) return;  // uniform
+  thr_lds_sync();
+  const float gx = q.x[lane];
+  const uint32_t gi = q.id[lane];
+  const float tx = q.x[kWave + lane];  // the rest moves to the front
+  const uint32_t ti = q.id[kWave + lane];
+  thr_lds_sync();
+  n -= kWave;
+  if ((uint32_t)lane < n) { q.x[lane] = tx; q.id[lane] = ti; }
+  thr_lds_sync();
+  g(gx, gi, true);
+}
+template <class G>
+__device__ __forceinline__ void thr_drain(ThrQueue& q, uint32_t& n, G&& g) {
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  if (n == 0) return;  // uniform
+  thr_lds_sync();
+  const bool ok = lane < n;
+  g(ok ? q.x[lane] : -INFINITY, ok ? q.id[lane] : 0u, ok);
+  n = 0;
+}
+
+template <class E>
+__global__ void __launch_bounds__(TH_NT) thr_collect_kernel(ThrArgs a) {
+  __shared__ ThrQueue sq[TH_NW];
+  const int64_t row = blockIdx.x / a.nlight;
+  const int part = (int)(blockIdx.x % a.nlight);
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  ThrCtl* const c = thr_ctl(a, row);
+  const float m = c->m, zf = c->zf, phi = c->phi, plo = c->plo, xcut = c->xcut, T = a.T;
+  uint64_t* const list = thr_list(c);
+  uint64_t mass = 0;
+  uint32_t cnt = 0;
+  auto eval = [&](float x, uint32_t id, bool ok) {
+    const float p = ok ? exp_det_sel(x / T - m) / zf : 0.0f;
+    const bool above = ok && p > phi;
+    mass += above ? fixed62(p) : 0ull;
+    cnt += above ? 1u : 0u;
+    const bool in = ok && !above && p >= plo;
+    const uint64_t bm = __ballot(in);
+    if (bm == 0) return;  // uniform
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(&c->nlist, (uint32_t)__popcll(bm));
+    at = rdlane(at, 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+    if (in && at < (uint32_t)kThrList)
+      list[at] = ((uint64_t)(~__float_as_uint(p)) << 32) | id;  // ascending: p down, id up
+  };
+  uint32_t n = 0;
+  thr_stream<E, 8>(thr_row<E>(a, row), a.V, part, a.nlight, a.llen,
+                   [&](int64_t i, float x, bool ok) {
+                     thr_push(sq[wv], n, x, (uint32_t)i, ok && x >= xcut, eval);
+                   });
+  thr_drain(sq[wv], n, eval);
+  mass = wave_sum_u64(mass);
+  cnt = wave_sum_u32(cnt);
+  if (lane == 0 && cnt) {
+    atomicAdd((unsigned long long*)&c->mass_above, (unsigned long long)mass);
+    atomicAdd(&c->cnt_above, cnt);
+  }
+}
+
+// ---------------------------------------------------------------- 4. resolve
+struct ThrResLds {
+  uint64_t e[kThrList];  // the list; the refinement's masses
+  uint64_t t[TH_NT];     // a list of up to TH_NT entries, sorted
+  uint32_t cnt[TH_NB], low[TH_NB];
+  uint64_t s64[TH_NW];
+  uint32_t first, idcut;
+  uint64_t sum, base;
+  uint32_t nbase, bin;
+};
+static_assert(kThrList >= TH_NB, "the refinement's masses use the list's space");
+
+// p's bits at the boundary by ten bits a pass over the row (bits of p <= 1 are below
+// 2^30): the bin in which the count from the top first reaches top_k (COUNT), or whose
+// last element first fails the nucleus test, then its own bins, down to one value.
+// Returns false when no bin does. base / nbase: mass and count above the value.
+template <class E, bool COUNT>
+__device__ __forceinline__ bool thr_refine(const ThrArgs& a, ThrResLds& L, const E* x,
+                                           const ThrCtl* c, float kth, uint32_t* value,
+                                           uint64_t* base, uint64_t* nbase, uint32_t* count) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const float m = c->m, zf = c->zf, xcut = c->xcut, T = a.T;
+  uint32_t hi = 0;  // the chosen leading bits
+  uint64_t S = 0, NB = 0;
+  for (int sh = 20; sh >= 0; sh -= 10) {
+    __syncthreads();
+    for (int b = tid; b < TH_NB; b += TH_NT) { L.e[b] = 0ull; L.cnt[b] = 0u; L.low[b] = ~0u; }
+    if (tid == 0) L.first = ~0u;
+    __syncthreads();
+    thr_stream<E, 4>(x, a.V, 0, 1, a.plen, [&](int64_t, float xv, bool ok) {
+      if (!(ok && xv >= xcut)) return;
+      const float p = exp_det(xv / T - m) / zf;
+      if (!(p > 0.0f) || p < kth) return;
+      const uint32_t bits = __float_as_uint(p);
+      if (sh < 20 && (bits >> (sh + 10)) != hi) return;
+      const uint32_t b = (uint32_t)(TH_NB - 1) - ((bits >> sh) & (uint32_t)(TH_NB - 1));
+      atomicAdd((unsigned long long*)&L.e[b], (unsigned long long)fixed62(p));
+      atomicAdd(&L.cnt[b], 1u);
+      atomicMin(&L.low[b], bits);
+    });
+    __syncthreads();
+    uint64_t sm = 0, sc = 0;
+#pragma unroll
+    for (int i = 0; i < TH_BPT; ++i) { sm += L.e[tid * TH_BPT + i]; sc += L.cnt[tid * TH_BPT + i]; }
+    const uint64_t m0 = S + thr_excl_u64(sm, L.s64), c0 = NB + thr_excl_u64(sc, L.s64);
+    uint64_t rm = m0, rc = c0;
+    uint32_t mine = ~0u;
+    uint64_t bm = 0, bc = 0;
+    for (int i = 0; i < TH_BPT; ++i) {
+      const int b = tid * TH_BPT + i;
+      const uint32_t n = L.cnt[b];
+      if (n == 0) continue;
+      const uint64_t nm = rm + L.e[b], nc = rc + n;
+      const bool hit = COUNT ? nc >= (uint64_t)a.top_k
+                             : !((rn32_u64(nm) - __uint_as_float(L.low[b])) < a.top_p);
+      if (hit) { mine = (uint32_t)b; bm = rm; bc = rc; break; }
+      rm = nm;
+      rc = nc;
+    }
+    const uint64_t vote = __ballot(mine != ~0u);
+    if (vote && lane == __ffsll((unsigned long long)vote) - 1) atomicMin(&L.first, mine);
+    __syncthreads();
+    const uint32_t f = L.first;
+    if (f == ~0u) {  // uniform: none (the first pass only, as a chosen bin holds a hit)
+      __syncthreads();
+      *base = 0;
+      return false;
+    }
+    if (mine == f) { L.base = bm; L.nbase = (uint32_t)bc; L.bin = L.cnt[f]; }
+    __syncthreads();
+    S = L.base;
+    NB = L.nbase;
+    *count = L.bin;
+    hi = (hi << 10) | ((uint32_t)(TH_NB - 1) - f);
+  }
+  *value = hi;
+  *base = S;
+  *nbase = NB;
+  return true;
+}
+
+template <class E>
+__global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
+  __shared__ ThrResLds L;
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  const ThrCtl* const c = thr_ctl(a, row);
+  const E* const x = thr_row<E>(a, row);
+  const float m = c->m, zf = c->zf, T = a.T, tp = a.top_p;
+  const uint32_t n = c->nlist;
+  const bool use_k = c->use_k != 0, use_p = c->use_p != 0;
+  const uint64_t above = c->mass_above;
+  const uint64_t nabove = c->cnt_above;
+  // kept = p > vf, or p == vf and id <= idcut
+  float vf = -1.0f;
+  uint32_t idcut = 0xFFFFFFFFu;
+  bool partial = false;
+  uint64_t tot = above;
+  if (n > (uint32_t)kThrList) {  // uniform
+    float kth = 0.0f;
+    uint32_t v, gc;
+    uint64_t S, N;
+    if (use_k && thr_refine<E, true>(a, L, x, c, 0.0f, &v, &S, &N, &gc)) kth = __uint_as_float(v);
+    uint64_t r0 = 0;
+    if (use_p && thr_refine<E, false>(a, L, x, c, kth, &v, &S, &N, &gc)) {
+      // members kept: a prefix (the first element of the row is always kept)
+      vf = __uint_as_float(v);
+      const uint64_t P = fixed62(vf);
+      uint64_t lo = 0, hi = gc;
+      while (lo < hi) {  // every wave the same search, 64 candidates a step
+        const uint64_t step = (hi - lo + kWave - 1) / kWave;
+        const uint64_t cand = lo + (uint64_t)lane * step;
+        const bool keep = cand < hi &&
+                          (((rn32_u64(S + (cand + 1) * P) - vf) < tp) || (N + cand == 0));
+        const int nk = __popcll(__ballot(keep));
+        if (nk == 0) break;
+        const uint64_t lastk = lo + (uint64_t)(nk - 1) * step;
+        lo = lastk + 1;
+        hi = min(hi, lastk + step);
+      }
+      r0 = lo;
+      tot = S + r0 * P;
+      partial = r0 > 0 && r0 < gc;
+      if (r0 == 0) {
+        // no member is kept, and no id is -1: everything above vf is
+        vf = __uint_as_float(v + 1u);
+      } else if (partial) {  // the id of the r0-th member
+        uint64_t seen = 0;
+        if (tid == 0) L.idcut = 0u;
+        for (int64_t i0 = 0; i0 < a.V; i0 += TH_NT) {  // uniform
+          const int64_t i = i0 + tid;
+          const bool mem = i < a.V && exp_det(thr_f(x[i]) / T - m) / zf == vf;
+          const uint64_t bm = __ballot(mem);
+          __syncthreads();
+          if (lane == 0) L.s64[wv] = (uint64_t)__popcll(bm);
+          __syncthreads();
+          uint64_t off = seen, all = 0;
+          for (int w = 0; w < TH_NW; ++w) { off += w < wv ? L.s64[w] : 0ull; all += L.s64[w]; }
+          if (mem && off + (uint64_t)__popcll(bm & ((1ull << lane) - 1ull)) == r0 - 1)
+            L.idcut = (uint32_t)i;
+          seen += all;
+          if (seen >= r0) break;  // uniform
+        }
+        __syncthreads();
+        idcut = L.idcut;
+      }
+    } else {  // everything that top-k keeps
+      vf = kth > 0.0f ? kth : -1.0f;
+      uint64_t s = 0;
+      thr_stream<E, 4>(x, a.V, 0, 1, a.plen, [&](int64_t, float xv, bool ok) {
+        const float p = ok ? exp_det_sel(xv / T - m) / zf : 0.0f;
+        s += p >= kth ? fixed62(p) : 0ull;
+      });
+      s = wave_sum_u64(s);
+      __syncthreads();
+      if (lane == 0) L.s64[wv] = s;
+      __syncthreads();
+      tot = 0;
+      for (int w = 0; w < TH_NW; ++w) tot += L.s64[w];
+    }
+  } else if (use_k || use_p) {
+    const uint64_t* const list = reinterpret_cast<const uint64_t*>(c + 1);
+    const uint64_t* e = L.e;
+    if (n <= (uint32_t)TH_NT) {  // sort by counting the smaller entries
+      const uint64_t k0 = (uint32_t)tid < n ? list[tid] : ~0ull;
+      L.e[tid] = k0;
+      __syncthreads();
+      if ((uint32_t)tid < n) {
+        uint32_t r = 0;
+        for (uint32_t i = 0; i < n; ++i) r += L.e[i] < k0 ? 1u : 0u;
+        L.t[r] = k0;
+      }
+      __syncthreads();
+      e = L.t;
+    } else {
+      uint32_t S = TH_NT;
+      while (S < n) S <<= 1;
+      for (uint32_t i = tid; i < S; i += TH_NT) L.e[i] = i < n ? list[i] : ~0ull;
+      __syncthreads();
+      for (uint32_t size = 2; size <= S; size <<= 1)
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+          for (uint32_t i = tid; i < S; i += TH_NT) {
+            const uint32_t j = i ^ stride;
+            if (j > i) {
+              const bool up = (i & size) == 0;
+              const uint64_t ai = L.e[i], aj = L.e[j];
+              if ((ai > aj) == up) { L.e[i] = aj; L.e[j] = ai; }
+            }
+          }
+          __syncthreads();
+        }
+    }
+    auto pof = [&](uint32_t i) { return __uint_as_float(~(uint32_t)(e[i] >> 32)); };
+    // the k-th largest p (0: not among the positive ones, nothing is zeroed)
+    float kth = 0.0f;
+    if (use_k && (uint64_t)a.top_k > nabove && (uint64_t)a.top_k - nabove <= n)
+      kth = pof((uint32_t)((uint64_t)a.top_k - nabove) - 1u);
+    if (tid == 0) { L.first = n; L.sum = 0ull; }
+    // entries PER * tid ..: their masses, then the first that fails
+    const uint32_t per = (n + TH_NT - 1) / TH_NT;
+    const uint32_t i0 = min(n, (uint32_t)tid * per), i1 = min(n, i0 + per);
+    uint64_t s = 0;
+    for (uint32_t i = i0; i < i1; ++i) s += fixed62(pof(i));
+    const uint64_t ex = above + thr_excl_u64(s, L.s64);
+    uint64_t run = ex;
+    uint32_t mine = n;
+    uint64_t kept = 0;
+    for (uint32_t i = i0; i < i1; ++i) {
+      const float p = pof(i);
+      const uint64_t nr = run + fixed62(p);
+      bool keep = !(p < kth);
+      if (use_p) keep = keep && (((rn32_u64(nr) - p) < tp) || (nabove + i == 0));
+      if (!keep) { mine = i; break; }
+      run = nr;
+    }
+    kept = run - ex;
+    __syncthreads();
+    if (mine < n) atomicMin(&L.first, mine);
+    __syncthreads();
+    const uint32_t f = L.first;  // entries [0, f) are kept
+    if (i0 < f) atomicAdd((unsigned long long*)&L.sum, (unsigned long long)kept);
+    __syncthreads();
+    tot = above + L.sum;
+    if (f == 0) {
+      vf = __uint_as_float(__float_as_uint(c->phi) + 1u);  // everything above the region
+    } else {
+      vf = pof(f - 1);
+      partial = f < n && pof(f) == vf && !(vf < kth);
+      if (partial) idcut = (uint32_t)e[f - 1];
+    }
+  }
+  if (tid != 0) return;
+  const float totf = fmaxf(rn32_u64(tot), 1e-12f);
+  const bool bad = !(zf > 0.0f);  // no finite maximum: every probability is 0 / 0
+  ThrRow r;
+  r.m = m; r.zf = zf; r.totf = totf; r.vf = vf; r.idcut = idcut;
+  r.xcut = c->xcut;
+  RowStat st = {};
+  float pg = 0.0f;
+  bool gtie = false;
+  const int64_t gid = thr_gid(a, row);
+  if (gid >= 0 && gid < a.V) {
+    const float xg = thr_f(x[gid]);
+    pg = bad ? __builtin_nanf("") : thr_prob(r, xg, (uint32_t)gid, T);
+    gtie = partial && exp_det(xg / T - m) / zf == vf;
+  }
+  st.m = m; st.zf = zf; st.totf = totf; st.mass = tot;
+  st.pgather = pg;
+  st.kmax = (int32_t)__float_as_uint(vf);
+  st.klo = (int32_t)idcut;
+  st.glo = 1; st.ghi = 0;
+  st.rstar = partial ? 1 : 0;
+  st.gcount = partial ? 2 : 0;
+  st.ntbl = (int32_t)__float_as_uint(r.xcut);
+  st.argmax = -1;
+  st.flags = (gtie ? (uint32_t)kRowGatherTie : 0u) | (bad ? (uint32_t)kRowNoMass : 0u);
+  a.stats[row] = st;
+}
+
+// ---------------------------------------------------------------- to_probs output
+// Wave by wave: zeros first, 16 bytes a lane, then the kept elements, compacted and
+// evaluated by full waves, over them (the wave waits for its zeros).
+constexpr int TH_OUT = 8192;  // ids per workgroup
+
+template <class E>
+__global__ void __launch_bounds__(TH_NT) thr_output_kernel(ThrArgs a, float* out, int64_t ld_out,
+                                                           int nchunk) {
+  constexpr int N = ThrVec<E>::N;
+  constexpr int UN = TH_OUT / (TH_NT * N);
+  __shared__ ThrQueue sq[TH_NW];
+  const int64_t row = blockIdx.x / nchunk;
+  const int ch = (int)(blockIdx.x % nchunk);
+  const int tid = threadIdx.x, wv = tid / kWave;
+  const E* const x = thr_row<E>(a, row);
+  float* const o = out + row * ld_out;
+  const ThrRow r = thr_load_row(a.stats[row]);
+  const bool bad = (a.stats[row].flags & kRowNoMass) != 0;
+  const float T = a.T;
+  int64_t head = (int64_t)(((16u - ((uint32_t)(uintptr_t)x & 15u)) & 15u) / sizeof(E));
+  if (head > a.V) head = a.V;
+  const int64_t nv = (a.V - head) / N;
+  const int64_t v0 = (int64_t)ch * (TH_OUT / N), v1 = min(nv, v0 + TH_OUT / N);
+  const uint4* const x4 = reinterpret_cast<const uint4*>(x + head);
+  uint4 w[UN];
+#pragma unroll
+  for (int u = 0; u < UN; ++u) {
+    const int64_t j = v0 + (int64_t)u * TH_NT + tid;
+    w[u] = j < v1 ? x4[j] : make_uint4(0, 0, 0, 0);
+  }
+  const float fill = bad ? __builtin_nanf("") : 0.0f;
+  const bool vec = ((uintptr_t)(o + head) & 15u) == 0;  // uniform
+  auto one = [&](int64_t i) {  // the row's ends, one element a lane
+    o[i] = bad ? fill : thr_prob(r, thr_f(x[i]), (uint32_t)i, T);
+  };
+  if (ch == 0 && tid < head) one(tid);
+  if (ch == nchunk - 1 && head + nv * N + tid < a.V) one(head + nv * N + tid);
+#pragma unroll
+  for (int u = 0; u < UN; ++u) {
+    const int64_t j = v0 + (int64_t)u * TH_NT + tid;
+    if (j >= v1) continue;
+    float* const d = o + head + j * N;
+    if (vec) {
+#pragma unroll
+      for (int q = 0; q < N / 4; ++q)
+        reinterpret_cast<float4*>(d)[q] = make_float4(fill, fill, fill, fill);
+    } else {
+#pragma unroll
+      for (int e = 0; e < N; ++e) d[e] = fill;
+    }
+  }
+  if (bad) return;  // uniform
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // gfx9 encoding: vmcnt(0)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  auto put = [&](float xv, uint32_t id, bool ok) {
+    const float p = thr_prob(r, xv, id, T);
+    if (ok && p != 0.0f) o[id] = p;
+  };
+  uint32_t n = 0;
+#pragma unroll
+  for (int u = 0; u < UN; ++u) {
+    const int64_t j = v0 + (int64_t)u * TH_NT + tid;
+    const bool ok = j < v1;
+    const int64_t i = head + j * N;
+    const uint32_t q[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      float xv;
+      if constexpr (sizeof(E) == 4) xv = __uint_as_float(q[e]);
+      else xv = thr_f((uint16_t)(q[e >> 1] >> (16 * (e & 1))));
+      thr_push(sq[wv], n, xv, (uint32_t)(i + e), ok && xv >= r.xcut, put);
+    }
+  }
+  thr_drain(sq[wv], n, put);
+}
+
+// ---------------------------------------------------------------- draw
+// The verify's accept chain and draw (or, with acc.k = 0, a draft step's draw): a wave
+// per record of kThrRec ids reduces it to its p and residual masses, which need only
+// the ids where p is kept; the workgroup that completes a batch row's records adds
+// them up, picks the one that holds floor(u * total) and walks its ids. Members of a
+// boundary tie group are decided by their ids, so nothing depends on earlier records.
+struct ThrDrawLds {
+  ThrQueue q[TH_NW];
+  SampleJob job;
+  uint32_t fl;
+  int32_t last;
+  uint64_t s64[TH_NW], t64[TH_NW];
+  int64_t pick, found;
+  uint64_t at;
+};
+constexpr int TH_RV = kThrRec / TH_NT;  // ids per thread of the walk (4)
+static_assert(TH_RV * TH_NT == kThrRec, "the walk takes a record with the workgroup");
+
+template <class E>
+__global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
+  __shared__ ThrDrawLds S;
+  const int64_t j = blockIdx.x / a.nblk;
+  const int bi = (int)(blockIdx.x % a.nblk);
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  if (tid < kWave) {
+    SampleJob jb;
+    uint32_t fl;
+    const int64_t n = accept_chain_wave(a.acc, j, &jb, &fl);
+    if (lane == 0) {
+      if (bi == 0 && a.acc.n_acc) a.acc.n_acc[j] = n;
+      S.job = jb;
+      S.fl = fl;
+      S.pick = -1;
+      S.found = -1;
+    }
+  }
+  __syncthreads();
+  const SampleJob job = S.job;
+  const bool hasq = job.qrow >= 0;
+  auto rowp = [&](int64_t row) {
+    const int g = row < a.nrows0 ? 0 : 1;
+    return reinterpret_cast<const E*>(a.base[g]) + (g ? row - a.nrows0 : row) * a.ld[g];
+  };
+  const E* const xp = rowp(job.prow);
+  const E* const xq = hasq ? rowp(job.qrow) : xp;
+  const RowStat sp = a.acc.stats[job.prow];
+  const RowStat sq = a.acc.stats[hasq ? job.qrow : job.prow];
+  const ThrRow rp = thr_load_row(sp), rq = thr_load_row(sq);
+  const float T = a.T;
+  const int64_t V = a.V;
+  // ---- records
+  const int rec = bi * TH_NW + wv;
+  uint64_t mp = 0, mr = 0;
+  if (rec < a.nrec) {  // uniform per wave
+    const int64_t r0 = (int64_t)rec * kThrRec;
+    constexpr int RN = kThrRec / kWave;
+    float x[RN];
+#pragma unroll
+    for (int u = 0; u < RN; ++u) {
+      const int64_t i = r0 + u * kWave + lane;
+      x[u] = i < V ? thr_f(xp[i]) : -INFINITY;
+    }
+    auto add = [&](float xv, uint32_t id, bool ok) {
+      const float qx = hasq && ok ? thr_f(xq[id]) : 0.0f;
+      const float p = ok ? thr_prob(rp, xv, id, T) : 0.0f;
+      const float q = hasq && ok ? thr_prob(rq, qx, id, T) : 0.0f;
+      mp += fixed62(p);
+      mr += hasq ? fixed62(fmaxf(p - q, 0.0f)) : 0ull;
+    };
+    uint32_t n = 0;
+#pragma unroll
+    for (int u = 0; u < RN; ++u) {
+      const int64_t i = r0 + u * kWave + lane;
+      thr_push(S.q[wv], n, x[u], (uint32_t)i, i < V && x[u] >= rp.xcut, add);
+    }
+    thr_drain(S.q[wv], n, add);
+    mp = wave_sum_u64(mp);
+    mr = wave_sum_u64(mr);
+    if (lane == 0) {
+      uint64_t* const d = a.recs + 2 * (j * a.nrec + rec);
+      __hip_atomic_store(d, mp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(d + 1, mr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  // ---- the workgroup whose count completes the records goes on (stores done first)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // gfx9 encoding: vmcnt(0)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __syncthreads();
+  if (tid == 0)
+    S.last = __hip_atomic_fetch_add(&a.counters[j], 1u, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(a.nblk - 1);
+  __syncthreads();
+  if (!S.last) return;  // uniform
+  static_assert(kF32MaxVocab <= (int64_t)TH_NT * kThrRec, "one record per thread");
+  mp = mr = 0;
+  if (tid < a.nrec) {
+    const uint64_t* const d = a.recs + 2 * (j * a.nrec + tid);
+    mp = __hip_atomic_load(d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    mr = __hip_atomic_load(d + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const uint64_t ip = wave_incl_scan_u64(mp, lane), ir = wave_incl_scan_u64(mr, lane);
+  if (lane == kWave - 1) { S.s64[wv] = ip; S.t64[wv] = ir; }
+  __syncthreads();
+  uint64_t ep = ip - mp, er = ir - mr, totp = 0, totr = 0;
+  for (int w = 0; w < TH_NW; ++w) {
+    ep += w < wv ? S.s64[w] : 0ull;
+    er += w < wv ? S.t64[w] : 0ull;
+    totp += S.s64[w];
+    totr += S.t64[w];
+  }
+  const bool use_r = hasq && rn32_u64(totr) > 1e-9f;  // sampling.py:85-88
+  const uint64_t tot = use_r ? totr : totp, e0 = use_r ? er : ep, mine = use_r ? mr : mp;
+  const uint64_t t = uniform_threshold(job.u, tot);
+  if (tot > 0 && e0 <= t && t - e0 < mine) {  // exactly one thread
+    S.pick = tid;
+    S.at = e0;
+  }
+  __syncthreads();
+  const int64_t pick = S.pick;
+  float pw = 0.0f;  // p of this thread's ids, the found one's kept
+  if (pick >= 0) {  // uniform
+    const int64_t i0 = pick * kThrRec + (int64_t)tid * TH_RV;
+    uint64_t w[TH_RV], sum = 0;
+    float pv[TH_RV];
+#pragma unroll
+    for (int u = 0; u < TH_RV; ++u) {
+      const int64_t i = i0 + u;
+      float p = 0.0f, q = 0.0f;
+      if (i < V) {
+        p = thr_prob(rp, thr_f(xp[i]), (uint32_t)i, T);
+        if (use_r) q = thr_prob(rq, thr_f(xq[i]), (uint32_t)i, T);
+      }
+      pv[u] = p;
+      w[u] = fixed62(use_r ? fmaxf(p - q, 0.0f) : p);
+      sum += w[u];
+    }
+    const uint64_t st = S.at + thr_excl_u64(sum, S.s64);
+    if (st <= t && t - st < sum) {  // exactly one thread
+      uint64_t acc = st;
+      int64_t f = -1;
+#pragma unroll
+      for (int u = 0; u < TH_RV; ++u) {
+        acc += w[u];
+        if (f < 0 && acc > t) { f = i0 + u; pw = pv[u]; }
+      }
+      S.found = f;
+      if (a.qx) a.qx[j] = pw;
+    }
+    __syncthreads();
+  }
+  if (tid != 0) return;
+  const int64_t y = S.found;
+  a.y[j] = y;
+  if (a.qx && y < 0) a.qx[j] = 0.0f;
+  if (a.acc.flags) {
+    uint32_t fl = S.fl;
+    auto tie = [&](const ThrRow& r, const RowStat& st, const E* x) {
+      return st.rstar > 0 && st.rstar < st.gcount &&
+             exp_det(thr_f(x[y]) / T - r.m) / r.zf == r.vf;
+    };
+    if (y >= 0 && (tie(rp, sp, xp) || (use_r && tie(rq, sq, xq)))) fl |= SDX_FLAG_TIE_ORDER;
+    a.acc.flags[j] = (uint8_t)fl;
+  }
+}
+
+// ---------------------------------------------------------------- launches
+
+// Parts per row: about four workgroups per CU over the call, parts of at least 4,096
+// elements (below that a part's histogram costs more than its stream), and no more
+// than the first pass has words for.
+static int thr_parts(int64_t rows, int64_t V) {
+  const int64_t want = (1024 + rows - 1) / rows;
+  int64_t p = want < V / 4096 ? want : V / 4096;
+  if (p > kThrMaxParts) p = kThrMaxParts;
+  return (int)(p < 1 ? 1 : p);
+}
+
+
+// Of the passes that only compare: as many workgroups as the chip holds waves for.
+static int thr_light_parts(int64_t rows, int64_t V) {
+  const int64_t want = (2048 + rows - 1) / rows, most = V / 4096;
+  const int64_t p = want < most ? want : most;
+  return (int)(p < 1 ? 1 : p > kThrMaxParts ? kThrMaxParts : p);
+}
+
+template <class E>
+static hipError_t thr_stats(const ThrArgs& a, int64_t rows, hipStream_t s) {
+  const dim3 grid((unsigned)(rows * a.nparts)), light((unsigned)(rows * a.nlight));
+  hipLaunchKernelGGL(thr_max_kernel<E>, light, dim3(TH_NT), 0, s, a);
+  hipLaunchKernelGGL(thr_hist_kernel<E>, grid, dim3(TH_NT), 0, s, a);
+  hipLaunchKernelGGL(thr_collect_kernel<E>, light, dim3(TH_NT), 0, s, a);
+  hipLaunchKernelGGL(thr_resolve_kernel<E>, dim3((unsigned)rows), dim3(TH_NT), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s) {
+  if (!a.scratch || a.scratch_bytes < kThrScratchMin || a.scratch_stride < a.scratch_bytes || !a.stats || a.V > kF32MaxVocab)
+    return hipErrorInvalidValue;
+  a.nparts = thr_parts(rows, a.V);
+  const int64_t per = (a.V + a.nparts - 1) / a.nparts;
+  a.plen = (per + 7) / 8 * 8;  // whole vectors of either element size
+  a.nlight = thr_light_parts(rows, a.V);
+  const int64_t lper = (a.V + a.nlight - 1) / a.nlight;
+  a.llen = (lper + 7) / 8 * 8;
+  return dtype == SDX_F32 ? thr_stats<float>(a, rows, s) : thr_stats<uint16_t>(a, rows, s);
+}
+
+hipError_t launch_thr_output(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+                             hipStream_t s) {
+  const int nchunk = (int)((a.V + TH_OUT - 1) / TH_OUT);
+  const dim3 grid((unsigned)(rows * nchunk));
+  if (dtype == SDX_F32)
+    hipLaunchKernelGGL(thr_output_kernel<float>, grid, dim3(TH_NT), 0, s, a, out, ld_out, nchunk);
+  else
+    hipLaunchKernelGGL(thr_output_kernel<uint16_t>, grid, dim3(TH_NT), 0, s, a, out, ld_out, nchunk);
+  return hipGetLastError();
+}
+
+hipError_t launch_thr_draw(int dtype, ThrDrawArgs a, int64_t jobs, hipStream_t s) {
+  a.nrec = (int32_t)((a.V + kThrRec - 1) / kThrRec);
+  a.nblk = (a.nrec + TH_NW - 1) / TH_NW;
+  const dim3 grid((unsigned)(jobs * a.nblk));
+  if (dtype == SDX_F32) hipLaunchKernelGGL(thr_draw_kernel<float>, grid, dim3(TH_NT), 0, s, a);
+  else hipLaunchKernelGGL(thr_draw_kernel<uint16_t>, grid, dim3(TH_NT), 0, s, a);
+  return hipGetLastError();
+}
+
+}  // namespace sdx

@@ -1,0 +1,138 @@
+"""Rows that take the threshold statistics (csrc/sdx_thr.hip) against the oracle, bit
+for bit: every shape of row at which the region, its list, the refinement over the
+row or the compaction can go wrong, at vocabularies on the edges of the parts and
+records, and rows that do not start 16-byte aligned."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import sampling as O
+from specdec import _lib
+from specdec import sampling as S
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _rows(V, seed, dtype=np.float32):
+    """Rows [n, V]: spread, narrow and nearly equal logits, tie groups from a few
+    members to the whole row (past the list of 2,048, so the row is refined), rows of
+    -inf but one or a tenth, and extremes of the range."""
+    rng = np.random.RandomState(seed)
+    masked = rng.randn(V) * 3
+    masked[rng.rand(V) < 0.9] = -np.inf
+    one = np.full(V, -np.inf)
+    one[V // 2] = 1.0
+    peak = rng.randn(V) * 2
+    peak[7] = 60.0
+    half = rng.randn(V) * 2
+    half[: V // 2] = 1.25
+    rows = [rng.randn(V) * 3, rng.randn(V) * 0.3, rng.randn(V) * 0.01, np.zeros(V),
+            np.where(np.arange(V) % 3 == 0, 2.0, -1.0), np.round(rng.randn(V) * 12) / 4,
+            np.round(rng.randn(V) * 2) / 4, masked, one, np.linspace(-40, 10, V),
+            rng.randn(V) * 30, peak, half,
+            torch.tensor(rng.randn(V) * 3).bfloat16().float().numpy()]
+    if dtype == np.float32:
+        rows += [rng.randn(V) * 1e-30, -np.abs(rng.randn(V)) * 1e30]
+    return np.stack(rows).astype(dtype)
+
+
+TRANSFORMS = [(1.0, 1.0, 0), (0.8, 0.95, 0), (0.7, 0.9, 50), (1.0, 0.5, 0), (1.3, 1.0, 20),
+              (0.6, 0.999999, 0), (1.0, 0.99999994, 0), (2.0, 0.95, 3000), (0.9, 0.3, 5000),
+              (1e-3, 0.9, 0), (4e6, 0.9, 0)]
+
+
+def _same(got, ref):
+    bad = np.argwhere(got.view(np.uint32) != ref.view(np.uint32))
+    assert bad.size == 0, f"{len(bad)} elements differ, first at {bad[0]}"
+
+
+# 8193: the shortest row, one part; 12291: three parts' worth of 4,096 and 3 ids more;
+# 33000: several parts
+@pytest.mark.parametrize("V", [8193, 12291, 33000])
+@pytest.mark.parametrize("T,tp,tk", TRANSFORMS)
+def test_to_probs_rows(V, T, tp, tk):
+    x = _rows(V, V)
+    got = S.to_probs(torch.tensor(x, device=DEV), T, tp, tk).cpu().numpy()
+    _same(got, O.to_probs(x, T, tp, tk))
+
+
+def test_top_k_of_all_but_one():
+    x = _rows(9000, 1)
+    got = S.to_probs(torch.tensor(x, device=DEV), 1.0, 1.0, 8999).cpu().numpy()
+    _same(got, O.to_probs(x, 1.0, 1.0, 8999))
+
+
+@pytest.mark.parametrize("off,ld,ldo", [(0, 9001, 9003), (1, 9002, 9001), (3, 9004, 9007)])
+def test_to_probs_rows_at_any_alignment(off, ld, ldo):
+    """C ABI rows of logits and probabilities at every 16-byte phase, with strides that
+    put them out of phase with each other."""
+    V, L = 9001, _lib.lib()
+    x = _rows(V, 5)
+    n = x.shape[0]
+    buf = torch.zeros(off + n * ld, device=DEV)
+    buf[off:].view(n, ld)[:, :V].copy_(torch.tensor(x))
+    out = torch.full((n * ldo + 4,), -1.0, device=DEV)
+    ws = _lib.workspace(L.sdx_to_probs_workspace(n, V, _lib.F32), DEV, prepare=False)
+    rc = L.sdx_to_probs(ctypes.c_void_p(buf.data_ptr() + 4 * off), _lib.F32, n, V, ld, 0.8, 0.95, 0,
+                        ctypes.c_void_p(out.data_ptr()), ldo, _lib.ptr(ws), ws.numel(),
+                        _lib.stream_of(out))
+    _lib.check(rc, "to_probs")
+    got = out[: n * ldo].view(n, ldo)[:, :V].cpu().numpy()
+    _same(np.ascontiguousarray(got), O.to_probs(x, 0.8, 0.95, 0))
+    # nothing past the last row is touched
+    assert bool((out[(n - 1) * ldo + V:] == -1.0).all())
+
+
+def _verify_case(B, k, V, dtype, seed):
+    """Logits of the row shapes above (without those whose p is 0 / 0 in every target),
+    drafted ids from the likely ones and from tie groups."""
+    rng = np.random.RandomState(seed)
+    base = _rows(V, seed, np.float16 if dtype == torch.float16 else np.float32)[:14]
+    pick = rng.randint(0, 14, size=(B, k + 1))
+    tgt = base[pick].astype(np.float32)
+    drf = tgt[:, :k] + np.where(rng.rand(B, k, 1) < 0.5, 0.0,
+                                np.round(rng.randn(B, k, V)) / 4).astype(np.float32)
+    t = torch.tensor(tgt).to(dtype)
+    d = torch.tensor(drf).to(dtype)
+    ids = rng.randint(0, V, size=(B, k))
+    top = np.argsort(-d.float().numpy(), axis=-1, kind="stable")[..., :40]
+    near = np.take_along_axis(top, rng.randint(0, 40, size=(B, k, 1)), -1)[..., 0]
+    ids = np.where(rng.rand(B, k) < 0.8, near, ids)
+    return (t, d, torch.tensor(ids), torch.tensor(rng.rand(B, k).astype(np.float32)),
+            torch.tensor(rng.rand(B).astype(np.float32)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("V,T,tp,tk", [(8200, 0.8, 0.95, 0), (9217, 1.0, 0.7, 0),
+                                       (33000, 0.7, 0.9, 50), (16384, 1.0, 1.0, 0)])
+def test_verify_rows(dtype, V, T, tp, tk):
+    B, k = 12, 3
+    t, d, ids, ua, uf = _verify_case(B, k, V, dtype, V)
+    n, y, f = S.rejection_sample(t.to(DEV), d.to(DEV), ids.to(DEV), ua.to(DEV), uf.to(DEV),
+                                 temperature=T, top_p=tp, top_k=tk)
+    rn, ry, rf = O.rejection_sample(t.float().numpy(), d.float().numpy(), ids.numpy(), ua.numpy(),
+                                    uf.numpy(), T, tp, tk)
+    assert np.array_equal(n.cpu().numpy(), rn)
+    assert np.array_equal(y.cpu().numpy(), ry)
+    assert np.array_equal(f.cpu().numpy(), rf)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("V,T,tp,tk", [(8200, 0.8, 0.95, 0), (33000, 1.0, 0.7, 300)])
+def test_draft_step_rows(dtype, V, T, tp, tk):
+    """The draw of every row and the drawn id's probability; a row of -inf but one id
+    draws it."""
+    x = _rows(V, V + 1, np.float16 if dtype == torch.float16 else np.float32)[:14]
+    lg = torch.tensor(x).to(dtype)
+    u = torch.rand(14, generator=torch.Generator().manual_seed(V))
+    conf = torch.full((14,), 0.5, device=DEV)
+    xd, qx, _ = S.draft_step(lg.to(DEV), u.to(DEV), T, tp, tk, conf=conf)
+    q = O.to_probs(lg.float().numpy(), T, tp, tk)
+    ref = O.sample_from_probs(q, u.numpy())
+    assert np.array_equal(xd.cpu().numpy(), ref)
+    rq = q[np.arange(14), ref]
+    assert np.array_equal(qx.cpu().numpy(), rq)
+    assert np.array_equal(conf.cpu().numpy(), np.float32(0.5) * rq)
