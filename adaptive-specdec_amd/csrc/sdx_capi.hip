@@ -196,6 +196,19 @@ int sdx_to_probs(const void* logits, int dtype, int64_t rows, int64_t vocab, int
   }
   sdx::RowStat* st; float* tb; float* dn; sdx::SampleJob* jb; sdx::ChunkRec* rc; uint32_t* ct;
   transform_ws(c, rows, vocab, dtype, 0, &st, &tb, &dn, &jb, &rc, &ct);
+  if (dtype == SDX_F16 && vocab > sdx::kF32SortVocab) {
+    // the scratch lies in the output rows, as for fp32 (rows that overlap the logits
+    // take the register-resident kernel)
+    const uintptr_t l0 = (uintptr_t)logits, l1 = l0 + (uintptr_t)(((rows - 1) * ld + vocab) * 2);
+    const uintptr_t p0 = (uintptr_t)probs, p1 = p0 + (uintptr_t)(((rows - 1) * ld_out + vocab) * 4);
+    if (!(l0 < p1 && p0 < l1)) {
+      sdx::ThrArgs a = thr_args(logits, logits, rows, 0, ld, vocab, temperature, top_p, top_k, sw);
+      a.stats = st;
+      a.scratch = probs; a.scratch_stride = ld_out * 4; a.scratch_bytes = vocab * 4;
+      if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
+      return hip_status(sdx::launch_thr_output(dtype, a, rows, probs, ld_out, s), "thr_output");
+    }
+  }
   int64_t chunk;
   int nchunk;
   chunking(vocab, &chunk, &nchunk);
@@ -412,6 +425,13 @@ static size_t verify_ws_bytes(int64_t batch, int64_t ntgt, int64_t ndrf, int64_t
   return c.used;
 }
 
+// fp16 rows take the threshold statistics where the workspace holds their scratch
+// behind the pieces of the register-resident kernel (the sizes the queries return do;
+// sdx_verify_noalloc's fixed array may not).
+static size_t thr16_bytes(int64_t rows, int dtype) {
+  return dtype == SDX_F16 ? align256((size_t)rows * sdx::kThrScratchMin) : 0;
+}
+
 // The fused verify kernel (row statistics and draw in one launch) serves bf16
 // logits, at one k or per-row k (2 k_max + 1 <= 64, batch <= 1024);
 // SDX_VERIFY_FUSED=0 in the environment selects the two-launch path instead.
@@ -424,12 +444,14 @@ static bool fused_enabled() {
 }
 
 size_t sdx_verify_workspace(int64_t batch, int32_t k, int64_t vocab, int dtype) {
-  return verify_ws_bytes(batch, batch * ((int64_t)k + 1), batch * (int64_t)k, vocab, dtype, false);
+  return verify_ws_bytes(batch, batch * ((int64_t)k + 1), batch * (int64_t)k, vocab, dtype, false) +
+         thr16_bytes(batch * (2 * (int64_t)k + 1), dtype);
 }
 
 size_t sdx_verify_ragged_workspace(int64_t batch, int64_t target_rows, int64_t vocab, int dtype) {
   if (batch < 0 || target_rows < batch) return 0;
-  return verify_ws_bytes(batch, target_rows, target_rows - batch, vocab, dtype, true);
+  return verify_ws_bytes(batch, target_rows, target_rows - batch, vocab, dtype, true) +
+         thr16_bytes(2 * target_rows - batch, dtype);
 }
 
 static int verify_impl(const void* target_logits, const void* draft_logits, int dtype,
@@ -556,15 +578,24 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
                       "greedy_accept");
   }
   if (!draft_logits) return fail(SDX_EINVAL, "sdx_verify: draft_logits required when T > 0");
-  const bool thr = dtype == SDX_F32 && vocab > sdx::kF32SortVocab;
+  const bool thr16 = dtype == SDX_F16 && workspace_bytes >= need + thr16_bytes(rows, dtype);
+  const bool thr = thr16 || (dtype == SDX_F32 && vocab > sdx::kF32SortVocab);
+  if (dtype != SDX_F32 &&
+      (!aligned16(target_logits) || !aligned16(draft_logits) || (vocab % 8) != 0))
+    return fail(SDX_EINVAL,
+                "sdx_verify: 16-bit logits must be 16-byte aligned with vocab %% 8 == 0");
   if (thr) {
-    // the rows' dense space serves as scratch: the draw evaluates what it needs
+    // fp32: the rows' dense space serves as scratch (the draw evaluates what it needs)
     sdx::ThrArgs a = thr_args(target_logits, draft_logits, ntgt, ndrf, vocab, vocab, temperature,
                               top_p, top_k, sw);
     a.ids = draft_ids; a.k = k; a.tgt_idx = tgt_idx;
     a.stats = st;
     a.zero = counters; a.nzero = batch;
     a.scratch = dn; a.scratch_stride = a.scratch_bytes = vocab * 4;
+    if (thr16) {
+      a.scratch = c.take<uint8_t>(thr16_bytes(rows, dtype));
+      a.scratch_stride = a.scratch_bytes = sdx::kThrScratchMin;
+    }
     if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
   } else if (dtype == SDX_F32) {
     sdx::F32Args a = {};
@@ -579,9 +610,6 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
     a.tie_ld = sdx::f32_tie_words(vocab);
     if (int e = hip_status(sdx::launch_to_probs_f32(a, rows, s), "to_probs_f32")) return e;
   } else {
-    if (!aligned16(target_logits) || !aligned16(draft_logits) || (vocab % 8) != 0)
-      return fail(SDX_EINVAL,
-                  "sdx_verify: 16-bit logits must be 16-byte aligned with vocab %% 8 == 0");
     sdx::RowStatArgs a = {};
     a.base[0] = (const uint16_t*)target_logits; a.nrows[0] = ntgt; a.ld[0] = vocab;
     a.base[1] = (const uint16_t*)draft_logits; a.nrows[1] = ndrf; a.ld[1] = vocab;
@@ -772,7 +800,7 @@ static size_t draft_ws_x_offset(int64_t batch, int64_t vocab, int dtype) {
 
 size_t sdx_draft_step_workspace(int64_t batch, int64_t vocab, int dtype) {
   if (batch < 0 || vocab < 1 || !dtype_ok(dtype)) return 0;
-  return draft_ws_bytes(batch, vocab, dtype);
+  return draft_ws_bytes(batch, vocab, dtype) + thr16_bytes(batch, dtype);
 }
 
 int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, int64_t ld,
@@ -808,11 +836,19 @@ int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, 
     e.greedy = true;
     return hip_status(sdx::launch_draft_epilogue(e, s), "draft_epilogue");
   }
-  if (dtype == SDX_F32 && vocab > sdx::kF32SortVocab) {
+  if (dtype != SDX_F32 && (!aligned16(logits) || (ld % 8) != 0 || (vocab % 8) != 0))
+    return fail(SDX_EINVAL,
+                "sdx_draft_step: 16-bit rows must start 16-byte aligned, ld %% 8 == 0, vocab %% 8 == 0");
+  const bool thr16 = dtype == SDX_F16 && workspace_bytes >= need + thr16_bytes(batch, dtype);
+  if (thr16 || (dtype == SDX_F32 && vocab > sdx::kF32SortVocab)) {
     sdx::ThrArgs a = thr_args(logits, logits, batch, 0, ld, vocab, temperature, top_p, top_k, sw);
     a.stats = st;
     a.zero = counters; a.nzero = batch;
     a.scratch = dn; a.scratch_stride = a.scratch_bytes = vocab * 4;
+    if (thr16) {
+      a.scratch = (uint8_t*)workspace + need;
+      a.scratch_stride = a.scratch_bytes = sdx::kThrScratchMin;
+    }
     if (int r = hip_status(sdx::launch_thr_stats(dtype, a, batch, s), "thr_stats")) return r;
     sdx::ThrDrawArgs d = {};  // k = 0: the bonus draw of each row on u
     d.acc = sdx::AcceptArgs{st,      batch,   0,       u,       u,       nullptr, jobs,
@@ -848,9 +884,6 @@ int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, 
     e.ldp = vocab;
     return hip_status(sdx::launch_draft_epilogue(e, s), "draft_epilogue");
   }
-  if (!aligned16(logits) || (ld % 8) != 0 || (vocab % 8) != 0)
-    return fail(SDX_EINVAL,
-                "sdx_draft_step: 16-bit rows must start 16-byte aligned, ld %% 8 == 0, vocab %% 8 == 0");
   sdx::RowStatArgs a = {};
   a.base[0] = (const uint16_t*)logits; a.nrows[0] = batch; a.ld[0] = ld;
   a.base[1] = a.base[0]; a.nrows[1] = 0; a.ld[1] = ld;

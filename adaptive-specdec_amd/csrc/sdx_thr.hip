@@ -1,5 +1,5 @@
-// to_probs statistics and outputs of rows whose values cannot be enumerated (fp32
-// logits, specdec/sampling.py:34-67), several workgroups per row.
+// to_probs statistics and outputs of rows whose values are too many to count one by
+// one (fp32 and fp16 logits, specdec/sampling.py:34-67), several workgroups per row.
 //
 // The transform of a row reduces to one record: its final probability is
 //   p(id) = exp_det(s - m) / zf,  s = fl32(x / T)
@@ -35,7 +35,10 @@
 // seven IEEE divisions per element and dense probabilities for the draw): verify of 8
 // batch rows at k = 4 (72 rows, top-k 50) 285 -> 67 us (kernels 11 + 29 + 11 + 5 and
 // the draw 13), to_probs of 256 rows 378 -> 206 us (50 + 62 + 33 + 8 + 59: the first
-// pass also pays for the write-back of the call before, the last moves 5.3 TB/s).
+// pass also pays for the write-back of the call before, the last moves 5.3 TB/s). On
+// fp16 rows (one workgroup of 1024 threads and a histogram of 36,864 values per row
+// before): verify of 16 batch rows at k = 4, V = 131,072 144 -> 98 us, of 64 at V =
+// 4,096 100 -> 38 us, of one at 1,024 42 -> 31 us; to_probs of 64 x 131,072 132 -> 65 us.
 #include "sdx_thr.hpp"
 
 namespace sdx {
@@ -144,10 +147,13 @@ __global__ void __launch_bounds__(TH_NT) thr_max_kernel(ThrArgs a) {
       thr_cnt(c)[b] = 0u;
     }
   float mx = -INFINITY, mn = INFINITY;
+  bool nf = false;  // fp16: a +inf or a NaN of positive sign (fp32 rows report neither)
   thr_stream<E, 8>(thr_row<E>(a, row), a.V, part, a.nlight, a.llen,
                    [&](int64_t, float x, bool ok) {
                      mx = ok ? fmaxf(mx, x) : mx;
                      mn = ok && x > -INFINITY ? fminf(mn, x) : mn;
+                     if constexpr (sizeof(E) == 2)
+                       nf |= ok && (int32_t)__float_as_uint(x) >= 0x7F800000;
                    });
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -155,11 +161,12 @@ __global__ void __launch_bounds__(TH_NT) thr_max_kernel(ThrArgs a) {
     mn = fminf(mn, __shfl_xor(mn, o, kWave));
   }
   if ((tid & (kWave - 1)) == 0) { sMx[tid / kWave] = mx; sMn[tid / kWave] = mn; }
-  __syncthreads();
+  const int any = __syncthreads_or(nf);
   if (tid == 0) {
     for (int w = 1; w < TH_NW; ++w) { mx = fmaxf(mx, sMx[w]); mn = fminf(mn, sMn[w]); }
     c->pmax[part] = mx;
     c->pmin[part] = mn;
+    c->pnf[part] = any ? 1u : 0u;
   }
 }
 
@@ -713,6 +720,7 @@ __global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
       if (partial) idcut = (uint32_t)e[f - 1];
     }
   }
+  const bool nonfinite = __ballot(lane < a.nlight && c->pnf[lane < a.nlight ? lane : 0] != 0) != 0;
   if (tid != 0) return;
   const float totf = fmaxf(rn32_u64(tot), 1e-12f);
   const bool bad = !(zf > 0.0f);  // no finite maximum: every probability is 0 / 0
@@ -737,7 +745,8 @@ __global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
   st.gcount = partial ? 2 : 0;
   st.ntbl = (int32_t)__float_as_uint(r.xcut);
   st.argmax = -1;
-  st.flags = (gtie ? (uint32_t)kRowGatherTie : 0u) | (bad ? (uint32_t)kRowNoMass : 0u);
+  st.flags = (gtie ? (uint32_t)kRowGatherTie : 0u) | (bad ? (uint32_t)kRowNoMass : 0u) |
+             (nonfinite ? (uint32_t)kRowNonfinite : 0u);
   a.stats[row] = st;
 }
 

@@ -1,5 +1,4 @@
-// Threshold records of rows whose values cannot be enumerated: what
-// sdx_thr.hip's kernels share.
+// Threshold records of fp32 and fp16 rows: what sdx_thr.hip's kernels share.
 #pragma once
 
 #include "sdx_draw16.hpp"
@@ -40,6 +39,7 @@ struct ThrCtl {
   float m, zf, phi, plo, xcut;
   uint64_t mass_above;
   float pmax[kThrMaxParts], pmin[kThrMaxParts];
+  uint32_t pnf[kThrMaxParts];  // fp16: the part holds a +inf or +NaN
   uint64_t z[3];  // the normaliser's 32-bit limbs
 };
 static_assert(sizeof(ThrCtl) % 8 == 0 && sizeof(ThrCtl) <= kThrCtlBytes, "ThrCtl layout");

@@ -59,6 +59,14 @@ def test_to_probs_rows(V, T, tp, tk):
     _same(got, O.to_probs(x, T, tp, tk))
 
 
+@pytest.mark.parametrize("V", [8200, 33000])
+@pytest.mark.parametrize("T,tp,tk", [t for t in TRANSFORMS if t[0] > 1e-2])
+def test_to_probs_fp16_rows(V, T, tp, tk):
+    x = _rows(V, V, np.float16)
+    got = S.to_probs(torch.tensor(x, device=DEV), T, tp, tk).cpu().numpy()
+    _same(got, O.to_probs(x.astype(np.float32), T, tp, tk))
+
+
 def test_top_k_of_all_but_one():
     x = _rows(9000, 1)
     got = S.to_probs(torch.tensor(x, device=DEV), 1.0, 1.0, 8999).cpu().numpy()
@@ -105,9 +113,10 @@ def _verify_case(B, k, V, dtype, seed):
             torch.tensor(rng.rand(B).astype(np.float32)))
 
 
-@pytest.mark.parametrize("dtype", [torch.float32])
-@pytest.mark.parametrize("V,T,tp,tk", [(8200, 0.8, 0.95, 0), (9217, 1.0, 0.7, 0),
-                                       (33000, 0.7, 0.9, 50), (16384, 1.0, 1.0, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("V,T,tp,tk", [(40, 1.0, 0.9, 5), (1000, 0.8, 0.95, 0), (8200, 0.8, 0.95, 0),
+                                       (9217, 1.0, 0.7, 0), (33000, 0.7, 0.9, 50),
+                                       (16384, 1.0, 1.0, 0)])
 def test_verify_rows(dtype, V, T, tp, tk):
     B, k = 12, 3
     t, d, ids, ua, uf = _verify_case(B, k, V, dtype, V)
@@ -120,7 +129,7 @@ def test_verify_rows(dtype, V, T, tp, tk):
     assert np.array_equal(f.cpu().numpy(), rf)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("V,T,tp,tk", [(8200, 0.8, 0.95, 0), (33000, 1.0, 0.7, 300)])
 def test_draft_step_rows(dtype, V, T, tp, tk):
     """The draw of every row and the drawn id's probability; a row of -inf but one id
@@ -136,3 +145,30 @@ def test_draft_step_rows(dtype, V, T, tp, tk):
     rq = q[np.arange(14), ref]
     assert np.array_equal(qx.cpu().numpy(), rq)
     assert np.array_equal(conf.cpu().numpy(), np.float32(0.5) * rq)
+
+
+def test_fp16_verify_without_room_for_the_scratch():
+    """A workspace of the register-resident kernel's size (sdx_verify_noalloc's array for
+    many rows) still serves fp16 rows, with the same results where a row's values fit that
+    kernel's window (it flags the others); a +inf logit flags its row in both."""
+    L, B, k, V = _lib.lib(), 6, 2, 9000
+    t, d, ids, ua, uf = (x.to(DEV) for x in _verify_case(B, k, V, torch.float16, 3))
+    t[4, 1, 17] = float("inf")
+    full = L.sdx_verify_workspace(B, k, V, _lib.F16)
+    scratch = 64 + 1024 + 2048 * 8 + 1024 * 12  # per row
+    small = full - (B * (2 * k + 1) * scratch + 255) // 256 * 256
+    res = []
+    for n in (full, small):
+        ws = _lib.workspace(n, DEV)
+        out = [torch.empty(B, dtype=x, device=DEV) for x in (torch.int64, torch.int64, torch.uint8)]
+        rc = L.sdx_verify(_lib.ptr(t), _lib.ptr(d), _lib.F16, B, k, V, _lib.ptr(ids), _lib.ptr(ua),
+                          _lib.ptr(uf), None, 0.8, 0.9, 0, *[_lib.ptr(o) for o in out],
+                          _lib.ptr(ws), small if n == small else ws.numel(), _lib.stream_of(t))
+        _lib.check(rc, "verify")
+        res.append([o.cpu().numpy() for o in out])
+    fine = (np.arange(B) != 4) & (res[1][2] & S.FLAG_UNSUPPORTED == 0)
+    assert fine.sum() >= 2
+    for a, b in zip(*res):
+        assert np.array_equal(a[fine], b[fine])
+    assert not (res[0][2] & S.FLAG_UNSUPPORTED).any()
+    assert res[0][2][4] & S.FLAG_NONFINITE and res[1][2][4] & S.FLAG_NONFINITE
