@@ -33,12 +33,16 @@
 // waves. Splitting a row over workgroups keeps the chip full from a few rows on.
 // Measured on fp32 rows of 151,936 (one workgroup of 1024 threads per row before, with
 // seven IEEE divisions per element and dense probabilities for the draw): verify of 8
-// batch rows at k = 4 (72 rows, top-k 50) 285 -> 67 us (kernels 11 + 29 + 11 + 5 and
-// the draw 13), to_probs of 256 rows 378 -> 206 us (50 + 62 + 33 + 8 + 59: the first
-// pass also pays for the write-back of the call before, the last moves 5.3 TB/s). On
+// batch rows at k = 4 (72 rows, top-k 50) 285 -> 63 us (kernels 12 + 27 + 11 + 6 and
+// the draw 11), to_probs of 256 rows 378 -> 198 us (52 + 56 + 31 + 9 + 53: the first
+// pass also pays for the write-back of the call before, the last moves 5.9 TB/s). On
 // fp16 rows (one workgroup of 1024 threads and a histogram of 36,864 values per row
-// before): verify of 16 batch rows at k = 4, V = 131,072 144 -> 98 us, of 64 at V =
+// before): verify of 16 batch rows at k = 4, V = 131,072 144 -> 86 us, of 64 at V =
 // 4,096 100 -> 38 us, of one at 1,024 42 -> 31 us; to_probs of 64 x 131,072 132 -> 65 us.
+// The compare passes keep the evaluation in one place of their code (a loop over a
+// queue in LDS): unrolled into every element's place, 16 to 64 copies, the collect
+// pass of the fp16 verify took 20 us instead of 17 and its draw 22 instead of 20. The
+// queues stay small enough for eight workgroups per CU (twice the queue: 20 us).
 #include "sdx_thr.hpp"
 
 namespace sdx {
@@ -59,10 +63,12 @@ __device__ __forceinline__ float thr_f(uint16_t c) { return decode16<SDX_F16>(c)
 
 // Streams part `part` of the row through f(id, x, valid), every element exactly once:
 // every lane of a wave makes every call (valid: the lane has an element), so f may
-// vote. UN vectors per thread are in flight.
-template <class E, int UN, class F>
+// vote. UN vectors per thread are in flight; after them, g() runs once (code that
+// would otherwise stand once per element: in copies, its first passes wait for the
+// instruction cache).
+template <class E, int UN, class F, class G>
 __device__ __forceinline__ void thr_stream(const E* __restrict__ row, int64_t V, int part,
-                                           int nparts, int64_t plen, F&& f) {
+                                           int nparts, int64_t plen, F&& f, G&& g) {
   constexpr int N = ThrVec<E>::N;
   const int tid = threadIdx.x;
   int64_t head = (int64_t)(((16u - ((uint32_t)(uintptr_t)row & 15u)) & 15u) / sizeof(E));
@@ -70,17 +76,15 @@ __device__ __forceinline__ void thr_stream(const E* __restrict__ row, int64_t V,
   const int64_t nv = (V - head) / N;  // whole vectors of the row
   const int64_t v0 = (int64_t)part * (plen / N);
   const int64_t v1 = part == nparts - 1 ? nv : min(nv, v0 + plen / N);
-  if (part == 0 && tid < kWave) {  // wave 0: fewer than 64 elements
-    const bool ok = tid < head;
-    f((int64_t)tid, ok ? thr_f(row[tid]) : 0.0f, ok);
-  }
-  if (part == nparts - 1 && tid < kWave) {
-    const int64_t i = head + nv * N + tid;
-    const bool ok = i < V;
+  // the ends, by wave 0: fewer than eight elements each (lanes 0 .. and 32 ..)
+  if (tid < kWave && (part == 0 || part == nparts - 1)) {
+    const int64_t i = tid < 32 ? tid : head + nv * N + (tid - 32);
+    const bool ok = tid < 32 ? part == 0 && i < head : part == nparts - 1 && i < V;
     f(i, ok ? thr_f(row[i]) : 0.0f, ok);
   }
   const uint4* __restrict__ x4 = reinterpret_cast<const uint4*>(row + head);
-  for (int64_t b = v0; b < v1; b += (int64_t)UN * TH_NT) {  // uniform
+  // uniform; at least once, for the ends
+  for (int64_t b = v0; b == v0 || b < v1; b += (int64_t)UN * TH_NT) {
     uint4 w[UN];
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
@@ -102,7 +106,13 @@ __device__ __forceinline__ void thr_stream(const E* __restrict__ row, int64_t V,
         f(i + e, x, ok);
       }
     }
+    g();
   }
+}
+template <class E, int UN, class F>
+__device__ __forceinline__ void thr_stream(const E* __restrict__ row, int64_t V, int part,
+                                           int nparts, int64_t plen, F&& f) {
+  thr_stream<E, UN>(row, V, part, nparts, plen, f, [] {});
 }
 
 template <class E>
@@ -129,6 +139,46 @@ __device__ __forceinline__ uint32_t* thr_cnt(ThrCtl* c) {
 }
 
 // ---------------------------------------------------------------- 1. maximum
+// fp16 codes two at a time: as signed keys in value order (negative codes with their
+// low 15 bits flipped), maximum and minimum with packed 16-bit operations; -inf (and
+// NaNs of negative sign) wrap around above every finite key for the minimum.
+__device__ __forceinline__ void thr_max16(const ThrArgs& a, const uint16_t* row, int part,
+                                          float& mx, float& mn, bool& nf) {
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  typedef unsigned short u2 __attribute__((ext_vector_type(2)));
+  constexpr short kLow = -31744;  // key of the least finite value
+  s2 hi = {-32768, -32768};
+  u2 lo = {0xFFFF, 0xFFFF};
+  const int tid = threadIdx.x;
+  const int64_t nv = a.V / 8;  // rows start 16-byte aligned, V is a multiple of 8
+  const int64_t v0 = (int64_t)part * (a.llen / 8);
+  const int64_t v1 = part == a.nlight - 1 ? nv : min(nv, v0 + a.llen / 8);
+  const uint4* const x4 = reinterpret_cast<const uint4*>(row);
+  constexpr int UN = 4;
+  for (int64_t b = v0 + tid; b < v1; b += (int64_t)UN * TH_NT) {
+    uint4 w[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) w[u] = x4[min(b + (int64_t)u * TH_NT, v1 - 1)];  // again: harmless
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const uint32_t q[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const s2 c = __builtin_bit_cast(s2, q[e]);
+        const s2 k = c ^ ((c >> 15) & (s2){0x7FFF, 0x7FFF});
+        hi = __builtin_elementwise_max(hi, k);
+        lo = __builtin_elementwise_min(lo, __builtin_bit_cast(u2, (s2)(k - (s2){kLow, kLow})));
+      }
+    }
+  }
+  const int h = max((int)hi[0], (int)hi[1]);
+  const int l = min((int)lo[0], (int)lo[1]);
+  auto val = [](int k) { return thr_f((uint16_t)(k < 0 ? k ^ 0x7FFF : k)); };
+  nf = h >= 0x7C00;
+  mx = nf ? INFINITY : val(h);
+  mn = l <= 0x7C00 - 1 - kLow ? val(l + kLow) : INFINITY;
+}
+
 template <class E>
 __global__ void __launch_bounds__(TH_NT) thr_max_kernel(ThrArgs a) {
   __shared__ float sMx[TH_NW], sMn[TH_NW];
@@ -137,7 +187,7 @@ __global__ void __launch_bounds__(TH_NT) thr_max_kernel(ThrArgs a) {
   const int tid = threadIdx.x;
   ThrCtl* const c = thr_ctl(a, row);
   if (part == 0 && tid == 0) {
-    c->tick = 0u; c->nlist = 0u; c->cnt_above = 0u; c->mass_above = 0ull;
+    c->tick = 0u; c->nlist = 0u;
     c->z[0] = c->z[1] = c->z[2] = 0ull;
     if (row < a.nzero) a.zero[row] = 0u;
   }
@@ -148,13 +198,13 @@ __global__ void __launch_bounds__(TH_NT) thr_max_kernel(ThrArgs a) {
     }
   float mx = -INFINITY, mn = INFINITY;
   bool nf = false;  // fp16: a +inf or a NaN of positive sign (fp32 rows report neither)
-  thr_stream<E, 8>(thr_row<E>(a, row), a.V, part, a.nlight, a.llen,
-                   [&](int64_t, float x, bool ok) {
-                     mx = ok ? fmaxf(mx, x) : mx;
-                     mn = ok && x > -INFINITY ? fminf(mn, x) : mn;
-                     if constexpr (sizeof(E) == 2)
-                       nf |= ok && (int32_t)__float_as_uint(x) >= 0x7F800000;
-                   });
+  if constexpr (sizeof(E) == 2) thr_max16(a, thr_row<E>(a, row), part, mx, mn, nf);
+  else
+    thr_stream<E, 8>(thr_row<E>(a, row), a.V, part, a.nlight, a.llen,
+                     [&](int64_t, float x, bool ok) {
+                       mx = ok ? fmaxf(mx, x) : mx;
+                       mn = ok && x > -INFINITY ? fminf(mn, x) : mn;
+                     });
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
@@ -234,7 +284,9 @@ __device__ __forceinline__ void thr_hist_pass(const ThrArgs& a, ThrHistLds& L, c
   const float T = a.T, rT = 1.0f / a.T;
   thr_stream<E, 4>(row, a.V, part, a.nparts, a.plen, [&](int64_t, float x, bool ok) {
     const float d = ok ? thr_div<DIV>(x, T, rT) - m : -INFINITY;
-    const int b = (int)fminf(-d * scale, (float)(TH_NB - 1));  // NaN: the last step
+    // NaN (-inf logits through the FMA steps): the last step; d > 0 never, and
+    // v_cvt_u32_f32 would take it to 0
+    const uint32_t b = (uint32_t)fminf(-d * scale, (float)(TH_NB - 1));
     const uint64_t f = thr_exp62(d);
     zlo += f;
     zhi += zlo < f ? 1u : 0u;
@@ -403,58 +455,55 @@ __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
 
 // ---------------------------------------------------------------- 3. collect
 // Per wave: ids that pass the threshold are compacted into LDS and evaluated 64 at a
-// time by full waves.
+// time by full waves, in one place of the code.
+template <int N>
 struct ThrQueue {
-  float x[2 * kWave];
-  uint32_t id[2 * kWave];
+  uint2 e[kWave - 1 + N * kWave];  // bits of x, id
 };
 __device__ __forceinline__ void thr_lds_sync() {  // within one wave
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_wave_barrier();
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
-// Appends the lanes' (x, id) with `take`; full waves go through g(x, id, true).
-template <class G>
-__device__ __forceinline__ void thr_push(ThrQueue& q, uint32_t& n, float x, uint32_t id, bool take,
-                                         G&& g) {
+// Appends the lanes' (x, id) with `take`.
+template <int N>
+__device__ __forceinline__ void thr_push(ThrQueue<N>& q, uint32_t& n, float x, uint32_t id,
+                                         bool take) {
   const uint64_t bm = __ballot(take);
   if (bm == 0) return;  // uniform
-  const int lane = threadIdx.x & (kWave - 1);
   if (take) {
     const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
-    q.x[at] = x;
-    q.id[at] = id;
+    q.e[at] = make_uint2(__float_as_uint(x), id);
   }
   n += (uint32_t)__popcll(bm);
-  if (n < kWave) return;  // uniform
-  thr_lds_sync();
-  const float gx = q.x[lane];
-  const uint32_t gi = q.id[lane];
-  const float tx = q.x[kWave + lane];  // the rest moves to the front
-  const uint32_t ti = q.id[kWave + lane];
-  thr_lds_sync();
-  n -= kWave;
-  if ((uint32_t)lane < n) { q.x[lane] = tx; q.id[lane] = ti; }
-  thr_lds_sync();
-  g(gx, gi, true);
 }
-template <class G>
-__device__ __forceinline__ void thr_drain(ThrQueue& q, uint32_t& n, G&& g) {
+// g(x, id, ok) for the queue's last 64 entries while it holds at least 64, or any with
+// `all`; fewer than 64 are left, so N more pushes fit.
+template <int N, class G>
+__device__ __forceinline__ void thr_drain(ThrQueue<N>& q, uint32_t& n, bool all, G&& g) {
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  if (n == 0) return;  // uniform
-  thr_lds_sync();
-  const bool ok = lane < n;
-  g(ok ? q.x[lane] : -INFINITY, ok ? q.id[lane] : 0u, ok);
-  n = 0;
+#pragma nounroll
+  while (n >= (uint32_t)kWave || (all && n > 0)) {  // uniform
+    thr_lds_sync();
+    const uint32_t c = min(n, (uint32_t)kWave);
+    n -= c;
+    const bool ok = lane < c;
+    const uint2 e = ok ? q.e[n + lane] : make_uint2(0xFF800000u, 0u);  // -inf
+    thr_lds_sync();  // read before the next pushes
+    g(__uint_as_float(e.x), e.y, ok);
+  }
 }
 
 template <class E>
 __global__ void __launch_bounds__(TH_NT) thr_collect_kernel(ThrArgs a) {
-  __shared__ ThrQueue sq[TH_NW];
+  constexpr int UN = 8 / ThrVec<E>::N;  // 8 elements a lane between two drains
+  __shared__ ThrQueue<UN * ThrVec<E>::N + 1> sq[TH_NW];  // and the row's ends
+  __shared__ uint32_t s_cnt[TH_NW];
+  __shared__ uint64_t s_mass[TH_NW];
   const int64_t row = blockIdx.x / a.nlight;
   const int part = (int)(blockIdx.x % a.nlight);
-  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
   ThrCtl* const c = thr_ctl(a, row);
   const float m = c->m, zf = c->zf, phi = c->phi, plo = c->plo, xcut = c->xcut, T = a.T;
   uint64_t* const list = thr_list(c);
@@ -476,30 +525,33 @@ __global__ void __launch_bounds__(TH_NT) thr_collect_kernel(ThrArgs a) {
       list[at] = ((uint64_t)(~__float_as_uint(p)) << 32) | id;  // ascending: p down, id up
   };
   uint32_t n = 0;
-  thr_stream<E, 8>(thr_row<E>(a, row), a.V, part, a.nlight, a.llen,
-                   [&](int64_t i, float x, bool ok) {
-                     thr_push(sq[wv], n, x, (uint32_t)i, ok && x >= xcut, eval);
-                   });
-  thr_drain(sq[wv], n, eval);
+  thr_stream<E, UN>(
+      thr_row<E>(a, row), a.V, part, a.nlight, a.llen,
+      [&](int64_t i, float x, bool ok) { thr_push(sq[wv], n, x, (uint32_t)i, ok && x >= xcut); },
+      [&] { thr_drain(sq[wv], n, false, eval); });
+  thr_drain(sq[wv], n, true, eval);
   mass = wave_sum_u64(mass);
   cnt = wave_sum_u32(cnt);
-  if (lane == 0 && cnt) {
-    atomicAdd((unsigned long long*)&c->mass_above, (unsigned long long)mass);
-    atomicAdd(&c->cnt_above, cnt);
-  }
+  if (lane == 0) { s_mass[wv] = mass; s_cnt[wv] = cnt; }
+  __syncthreads();
+  if (tid != 0) return;
+  for (int w = 1; w < TH_NW; ++w) { mass += s_mass[w]; cnt += s_cnt[w]; }
+  c->pmass[part] = mass;
+  c->pcnt[part] = cnt;
 }
 
 // ---------------------------------------------------------------- 4. resolve
+constexpr int kThrCount = 2 * TH_NT;  // lists up to here are sorted by counting
 struct ThrResLds {
   uint64_t e[kThrList];  // the list; the refinement's masses
-  uint64_t t[TH_NT];     // a list of up to TH_NT entries, sorted
+  uint64_t t[kThrCount];  // a list of up to kThrCount entries, sorted
   uint32_t cnt[TH_NB], low[TH_NB];
   uint64_t s64[TH_NW];
   uint32_t first, idcut;
   uint64_t sum, base;
   uint32_t nbase, bin;
 };
-static_assert(kThrList >= TH_NB, "the refinement's masses use the list's space");
+static_assert(kThrList >= kThrCount && kThrList >= TH_NB, "the refinement's masses use the list's space");
 
 // p's bits at the boundary by ten bits a pass over the row (bits of p <= 1 are below
 // 2^30): the bin in which the count from the top first reaches top_k (COUNT), or whose
@@ -580,8 +632,8 @@ __global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
   const float m = c->m, zf = c->zf, T = a.T, tp = a.top_p;
   const uint32_t n = c->nlist;
   const bool use_k = c->use_k != 0, use_p = c->use_p != 0;
-  const uint64_t above = c->mass_above;
-  const uint64_t nabove = c->cnt_above;
+  const uint64_t above = wave_sum_u64(lane < a.nlight ? c->pmass[lane] : 0ull);
+  const uint64_t nabove = wave_sum_u32(lane < a.nlight ? c->pcnt[lane] : 0u);
   // kept = p > vf, or p == vf and id <= idcut
   float vf = -1.0f;
   uint32_t idcut = 0xFFFFFFFFu;
@@ -652,14 +704,27 @@ __global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
   } else if (use_k || use_p) {
     const uint64_t* const list = reinterpret_cast<const uint64_t*>(c + 1);
     const uint64_t* e = L.e;
-    if (n <= (uint32_t)TH_NT) {  // sort by counting the smaller entries
+    if (n <= (uint32_t)kThrCount) {  // sort by counting the smaller entries
       const uint64_t k0 = (uint32_t)tid < n ? list[tid] : ~0ull;
+      const uint64_t k1 = (uint32_t)tid + TH_NT < n ? list[tid + TH_NT] : ~0ull;
       L.e[tid] = k0;
+      L.e[tid + TH_NT] = k1;
       __syncthreads();
       if ((uint32_t)tid < n) {
-        uint32_t r = 0;
-        for (uint32_t i = 0; i < n; ++i) r += L.e[i] < k0 ? 1u : 0u;
-        L.t[r] = k0;
+        uint32_t r0 = 0, r1 = 0;
+        // entries past n are ~0: never smaller (kThrCount is a multiple of 16)
+        for (uint32_t i = 0; i < n; i += 16) {
+          uint64_t v[16];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) v[u] = L.e[i + u];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) {
+            r0 += v[u] < k0 ? 1u : 0u;
+            r1 += v[u] < k1 ? 1u : 0u;
+          }
+        }
+        L.t[r0] = k0;
+        if ((uint32_t)tid + TH_NT < n) L.t[r1] = k1;
       }
       __syncthreads();
       e = L.t;
@@ -753,14 +818,15 @@ __global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
 // ---------------------------------------------------------------- to_probs output
 // Wave by wave: zeros first, 16 bytes a lane, then the kept elements, compacted and
 // evaluated by full waves, over them (the wave waits for its zeros).
-constexpr int TH_OUT = 8192;  // ids per workgroup
+constexpr int TH_OUT = 8192;  // ids per workgroup: 32 a thread
 
 template <class E>
 __global__ void __launch_bounds__(TH_NT) thr_output_kernel(ThrArgs a, float* out, int64_t ld_out,
                                                            int nchunk) {
   constexpr int N = ThrVec<E>::N;
   constexpr int UN = TH_OUT / (TH_NT * N);
-  __shared__ ThrQueue sq[TH_NW];
+  constexpr int GR = 16 / N;  // vectors between two drains
+  __shared__ ThrQueue<GR * N> sq[TH_NW];
   const int64_t row = blockIdx.x / nchunk;
   const int ch = (int)(blockIdx.x % nchunk);
   const int tid = threadIdx.x, wv = tid / kWave;
@@ -810,21 +876,34 @@ __global__ void __launch_bounds__(TH_NT) thr_output_kernel(ThrArgs a, float* out
     if (ok && p != 0.0f) o[id] = p;
   };
   uint32_t n = 0;
+#pragma nounroll
+  for (int g = 0; g < UN / GR; ++g) {
 #pragma unroll
-  for (int u = 0; u < UN; ++u) {
-    const int64_t j = v0 + (int64_t)u * TH_NT + tid;
-    const bool ok = j < v1;
-    const int64_t i = head + j * N;
-    const uint32_t q[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+    for (int u = 0; u < GR; ++u) {
+      // group g's vectors by selects: an index known at run time would put w in memory
+      uint4 wu = w[u];
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
-      float xv;
-      if constexpr (sizeof(E) == 4) xv = __uint_as_float(q[e]);
-      else xv = thr_f((uint16_t)(q[e >> 1] >> (16 * (e & 1))));
-      thr_push(sq[wv], n, xv, (uint32_t)(i + e), ok && xv >= r.xcut, put);
+      for (int h = 1; h < UN / GR; ++h) {
+        const uint4 y = w[h * GR + u];
+        wu.x = g == h ? y.x : wu.x;
+        wu.y = g == h ? y.y : wu.y;
+        wu.z = g == h ? y.z : wu.z;
+        wu.w = g == h ? y.w : wu.w;
+      }
+      const int64_t j = v0 + (int64_t)(g * GR + u) * TH_NT + tid;
+      const bool ok = j < v1;
+      const int64_t i = head + j * N;
+      const uint32_t q[4] = {wu.x, wu.y, wu.z, wu.w};
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        float xv;
+        if constexpr (sizeof(E) == 4) xv = __uint_as_float(q[e]);
+        else xv = thr_f((uint16_t)(q[e >> 1] >> (16 * (e & 1))));
+        thr_push(sq[wv], n, xv, (uint32_t)(i + e), ok && xv >= r.xcut);
+      }
     }
+    thr_drain(sq[wv], n, g == UN / GR - 1, put);
   }
-  thr_drain(sq[wv], n, put);
 }
 
 // ---------------------------------------------------------------- draw
@@ -834,7 +913,8 @@ __global__ void __launch_bounds__(TH_NT) thr_output_kernel(ThrArgs a, float* out
 // them up, picks the one that holds floor(u * total) and walks its ids. Members of a
 // boundary tie group are decided by their ids, so nothing depends on earlier records.
 struct ThrDrawLds {
-  ThrQueue q[TH_NW];
+  ThrQueue<kThrRec / kWave> q[TH_NW];
+  RowStat st[2];
   SampleJob job;
   uint32_t fl;
   int32_t last;
@@ -854,7 +934,17 @@ __global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
   if (tid < kWave) {
     SampleJob jb;
     uint32_t fl;
-    const int64_t n = accept_chain_wave(a.acc, j, &jb, &fl);
+    int64_t n;
+    if (a.acc.k <= 31) {  // uniform: the 2k + 1 rows' records at once, one per lane
+      // (no row here is left for the chain to rank, so the row source is not read)
+      n = chain16_wave<SDX_F16, false>(a.acc, Eval16<SDX_F16>{}, j, &jb, &fl, S.st);
+    } else {
+      n = accept_chain_wave(a.acc, j, &jb, &fl);
+      if (lane == 0) {
+        S.st[0] = a.acc.stats[jb.prow];
+        S.st[1] = a.acc.stats[jb.qrow >= 0 ? jb.qrow : jb.prow];
+      }
+    }
     if (lane == 0) {
       if (bi == 0 && a.acc.n_acc) a.acc.n_acc[j] = n;
       S.job = jb;
@@ -872,8 +962,8 @@ __global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
   };
   const E* const xp = rowp(job.prow);
   const E* const xq = hasq ? rowp(job.qrow) : xp;
-  const RowStat sp = a.acc.stats[job.prow];
-  const RowStat sq = a.acc.stats[hasq ? job.qrow : job.prow];
+  const RowStat sp = S.st[0];
+  const RowStat sq = S.st[hasq ? 1 : 0];
   const ThrRow rp = thr_load_row(sp), rq = thr_load_row(sq);
   const float T = a.T;
   const int64_t V = a.V;
@@ -900,9 +990,9 @@ __global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
 #pragma unroll
     for (int u = 0; u < RN; ++u) {
       const int64_t i = r0 + u * kWave + lane;
-      thr_push(S.q[wv], n, x[u], (uint32_t)i, i < V && x[u] >= rp.xcut, add);
+      thr_push(S.q[wv], n, x[u], (uint32_t)i, i < V && x[u] >= rp.xcut);
     }
-    thr_drain(S.q[wv], n, add);
+    thr_drain(S.q[wv], n, true, add);
     mp = wave_sum_u64(mp);
     mr = wave_sum_u64(mr);
     if (lane == 0) {

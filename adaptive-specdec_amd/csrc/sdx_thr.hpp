@@ -34,10 +34,10 @@ __device__ __forceinline__ float thr_prob(const ThrRow& r, float x, uint32_t id,
 struct ThrCtl {
   uint32_t tick;       // parts whose sums are in (cleared by the first kernel)
   uint32_t nlist;      // region elements found
-  uint32_t cnt_above;  // elements above the region
   int32_t use_k, use_p;  // filters that the region has to decide
   float m, zf, phi, plo, xcut;
-  uint64_t mass_above;
+  uint64_t pmass[kThrMaxParts];  // per part: mass and count of the elements above the region
+  uint32_t pcnt[kThrMaxParts];
   float pmax[kThrMaxParts], pmin[kThrMaxParts];
   uint32_t pnf[kThrMaxParts];  // fp16: the part holds a +inf or +NaN
   uint64_t z[3];  // the normaliser's 32-bit limbs
