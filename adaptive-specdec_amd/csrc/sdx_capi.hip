@@ -273,12 +273,8 @@ int sdx_sample_probs(const float* probs, int64_t rows, int64_t vocab, int64_t ld
 
 // ------------------------------------------------------------------ residual_probs
 size_t sdx_residual_probs_workspace(int64_t rows, int64_t vocab) {
-  int64_t rec_ids;
-  int nrec;
-  sdx::draw_layout(vocab, &rec_ids, &nrec);
   Carve c{nullptr};
-  c.take<sdx::SampleJob>(rows);
-  c.take<sdx::ChunkRec>((size_t)rows * nrec);
+  c.take<uint64_t>((size_t)rows * sdx::dense_nrec(vocab) * 2);  // record masses
   return c.used;
 }
 
@@ -291,23 +287,12 @@ int sdx_residual_probs(const float* p, const float* q, int64_t rows, int64_t voc
   const size_t need = sdx_residual_probs_workspace(rows, vocab);
   if (!workspace || workspace_bytes < need)
     return fail(SDX_EWORKSPACE, "sdx_residual_probs: workspace %zu < %zu", workspace_bytes, need);
-  hipStream_t s = (hipStream_t)stream;
-  int64_t rec_ids;
-  int nrec;
-  sdx::draw_layout(vocab, &rec_ids, &nrec);
   Carve c{(uint8_t*)workspace};
-  sdx::SampleJob* jobs = c.take<sdx::SampleJob>(rows);
-  sdx::ChunkRec* recs = c.take<sdx::ChunkRec>((size_t)rows * nrec);
-  hipLaunchKernelGGL(sdx_jobs_from_u, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, jobs,
-                     (const float*)nullptr, rows, rows, (uint32_t*)nullptr);
-  if (int e = hip_status(hipGetLastError(), "jobs")) return e;
-  const bool vec = aligned16(p) && aligned16(q) && (ld % 4) == 0;
-  sdx::RowSourceF32 src{p, ld, q, ld, rows, vec};
-  if (int e = hip_status(sdx::launch_chunk_mass_probs(src, jobs, rows, vocab, recs, s),
-                         "chunk_mass"))
-    return e;
-  sdx::ResidualNormArgs a{p, q, ld, vocab, rec_ids, nrec, recs, out, ld_out};
-  return hip_status(sdx::launch_residual_norm(a, rows, s), "residual_norm");
+  sdx::ResidualArgs a = {};
+  a.p = p; a.q = q; a.ld = ld; a.rows = rows; a.V = vocab;
+  a.mass = c.take<uint64_t>((size_t)rows * sdx::dense_nrec(vocab) * 2);
+  a.out = out; a.ld_out = ld_out;
+  return hip_status(sdx::launch_residual(a, (hipStream_t)stream), "residual");
 }
 
 // ------------------------------------------------------------------ gather_prob

@@ -150,17 +150,19 @@ inline void draw_layout(int64_t V, int64_t* rec_ids, int* nrec) {
   *nrec = (int)((V + *rec_ids - 1) / *rec_ids);
 }
 
-struct ResidualNormArgs {
+struct ResidualArgs {
   const float* p;
   const float* q;
   int64_t ld;
+  int64_t rows;
   int64_t V;
-  int64_t rec_ids;
-  int32_t nrec;
-  const ChunkRec* recs;  // draw records of the rows (one job per row)
+  uint64_t* mass;  // [rows, dense_nrec(V), 2] masses of p and of the residual per record
   float* out;
   int64_t ld_out;
+  int32_t nrec, nchunk;  // set by launch_residual
+  bool same;
 };
+constexpr int kResIds = 4096;  // ids per workgroup of the output
 
 // sdx_rowstat.hip
 int rowstat16_nslot(int64_t V);
@@ -278,8 +280,6 @@ hipError_t launch_draw16(int fmt, const RowSource16& src, const RowStat* stats,
 hipError_t launch_draw_probs(const RowSourceF32& src, const AcceptArgs* acc, SampleJob* jobs,
                              int64_t njobs, int64_t V, ChunkRec* recs, uint32_t* counters,
                              int64_t* y, hipStream_t s, const uint32_t* tie_bits = nullptr);
-hipError_t launch_chunk_mass_probs(const RowSourceF32& src, SampleJob* jobs, int64_t njobs,
-                                   int64_t V, ChunkRec* recs, hipStream_t s);
 // to_probs output of 16-bit rows: ids per chunk (one workgroup each).
 constexpr int64_t kMatChunk = 16384;
 
@@ -293,7 +293,7 @@ struct DenseArgs {
   int64_t rows;
   int64_t V;
   int32_t nrec;
-  bool vec;        // p 16-byte aligned and ld % 4 == 0
+  bool vec;        // p 16-byte aligned and ld % 4 == 0 (the walk's loads)
   uint64_t* mass;  // [rows, nrec]
   const float* u;  // [rows]
   int64_t* y;      // [rows]
@@ -305,7 +305,7 @@ hipError_t launch_materialize16(int fmt, const RowSource16& src, const RowStat* 
                                 const float* tables, float T, int64_t rows, int64_t V,
                                 int64_t chunk, int nchunk, uint32_t* counts, float* out,
                                 int64_t ld_out, hipStream_t s);
-hipError_t launch_residual_norm(const ResidualNormArgs& a, int64_t rows, hipStream_t s);
+hipError_t launch_residual(ResidualArgs a, hipStream_t s);
 hipError_t launch_gather(const float* probs, int64_t rows, int64_t V, int64_t ld,
                          const int64_t* ids, float* out, hipStream_t s);
 // sdx_greedy.hip

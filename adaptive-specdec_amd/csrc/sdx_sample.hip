@@ -878,6 +878,45 @@ constexpr int kDenseNT = 256;
 
 __device__ __forceinline__ uint64_t dense_w(float v) { return v > 0.0f ? fixed62(v) : 0ull; }
 
+// Ids [x0, x1) of a row (at most kDenseRec) by one wave through f(id, p, q), 16-byte
+// loads from the first 16-byte boundary on (eight per row and lane in flight), the few
+// ids before it and after the last whole vector one per lane. q (null: none) lies at
+// the same 16-byte phase as p when `same`, else both go one id per lane.
+template <class F>
+__device__ __forceinline__ void dense_record(const float* __restrict__ p,
+                                             const float* __restrict__ q, bool same, int64_t x0,
+                                             int64_t x1, F&& f) {
+  const int lane = threadIdx.x & (kWave - 1);
+  if (!same) {  // uniform
+    for (int64_t i = x0 + lane; i < x1; i += kWave) f(i, p[i], q ? q[i] : 0.0f);
+    return;
+  }
+  const int64_t h = min(x1 - x0, (int64_t)(((16u - ((uint32_t)(uintptr_t)(p + x0) & 15u)) & 15u) >> 2));
+  const int64_t nv = (x1 - x0 - h) >> 2, t0 = x0 + h + 4 * nv;
+  if (lane < h) f(x0 + lane, p[x0 + lane], q ? q[x0 + lane] : 0.0f);
+  if (t0 + lane < x1) f(t0 + lane, p[t0 + lane], q ? q[t0 + lane] : 0.0f);
+  const float4* const p4 = reinterpret_cast<const float4*>(p + x0 + h);
+  const float4* const q4 = reinterpret_cast<const float4*>(q + x0 + h);
+  constexpr int N = kDenseRec / (4 * kWave);
+  float4 v[N], w[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int64_t j = i * kWave + lane;
+    v[i] = j < nv ? p4[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    w[i] = q && j < nv ? q4[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int64_t j = i * kWave + lane;
+    if (j >= nv) continue;
+    const int64_t id = x0 + h + 4 * j;
+    f(id, v[i].x, w[i].x);
+    f(id + 1, v[i].y, w[i].y);
+    f(id + 2, v[i].z, w[i].z);
+    f(id + 3, v[i].w, w[i].w);
+  }
+}
+
 __global__ void __launch_bounds__(kDenseNT) dense_mass_kernel(DenseArgs a) {
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t g = (int64_t)blockIdx.x * (kDenseNT / kWave) + threadIdx.x / kWave;
@@ -885,19 +924,9 @@ __global__ void __launch_bounds__(kDenseNT) dense_mass_kernel(DenseArgs a) {
   const int64_t row = g / a.nrec;
   const int64_t x0 = (g % a.nrec) * kDenseRec;
   const int64_t x1 = min(a.V, x0 + kDenseRec);
-  const float* src = a.p + row * a.ld;
   uint64_t s = 0;
-  if (a.vec && x1 - x0 == kDenseRec) {
-    float4 v[kDenseRec / (4 * kWave)];
-#pragma unroll
-    for (int i = 0; i < kDenseRec / (4 * kWave); ++i)
-      v[i] = *reinterpret_cast<const float4*>(src + x0 + ((int64_t)i * kWave + lane) * 4);
-#pragma unroll
-    for (int i = 0; i < kDenseRec / (4 * kWave); ++i)
-      s += dense_w(v[i].x) + dense_w(v[i].y) + dense_w(v[i].z) + dense_w(v[i].w);
-  } else {
-    for (int64_t i = x0 + lane; i < x1; i += kWave) s += dense_w(src[i]);
-  }
+  dense_record(a.p + row * a.ld, nullptr, true, x0, x1,
+               [&](int64_t, float p, float) { s += dense_w(p); });
   s = wave_sum_u64(s);
   if (lane == 0) a.mass[g] = s;
 }
@@ -975,16 +1004,39 @@ __global__ void __launch_bounds__(kDenseNT) dense_pick_kernel(DenseArgs a) {
 
 // ---------------------------------------------------------------- residual_probs output
 
-__global__ void __launch_bounds__(SM_NT) residual_norm_kernel(ResidualNormArgs a) {
+// Two launches, bound by the bytes of p, q and the output (16-byte accesses at any row
+// alignment): each wave sums one record's exact masses of p and of (p - q)_+, over the
+// ids with p > 0; then each workgroup adds up its row's records and writes kResIds ids.
+// 64 rows of 50,257: 12 + 9 us, against 13 + 17 us with the draw kernel's records and
+// one id per thread, and two padding copies of 8.6 us for rows not 16-byte aligned.
+__global__ void __launch_bounds__(kDenseNT) residual_mass_kernel(ResidualArgs a) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t g = (int64_t)blockIdx.x * (kDenseNT / kWave) + threadIdx.x / kWave;
+  if (g >= a.rows * a.nrec) return;  // whole waves
+  const int64_t row = g / a.nrec;
+  const int64_t x0 = (g % a.nrec) * kDenseRec;
+  const int64_t x1 = min(a.V, x0 + kDenseRec);
+  uint64_t mp = 0, mr = 0;
+  dense_record(a.p + row * a.ld, a.q + row * a.ld, a.same, x0, x1, [&](int64_t, float p, float q) {
+    mp += dense_w(p);
+    mr += p > 0.0f ? fixed62(fmaxf(p - q, 0.0f)) : 0ull;
+  });
+  mp = wave_sum_u64(mp);
+  mr = wave_sum_u64(mr);
+  if (lane == 0) {
+    a.mass[2 * g] = mp;
+    a.mass[2 * g + 1] = mr;
+  }
+}
+
+__global__ void __launch_bounds__(kDenseNT) residual_norm_kernel(ResidualArgs a) {
   __shared__ uint64_t s64[SM_NW];
-  const int64_t row = (int64_t)blockIdx.x / a.nrec;
-  const int64_t cidx = (int64_t)blockIdx.x % a.nrec;
-  // dense fp32 rows have no tie groups: residual mass is r0, p mass p2
+  const int64_t row = (int64_t)blockIdx.x / a.nchunk;
+  const int64_t c0 = ((int64_t)blockIdx.x % a.nchunk) * kResIds;
   uint64_t r = 0, p = 0;
-  for (int c = threadIdx.x; c < a.nrec; c += SM_NT) {
-    const ChunkRec rec = load_rec(a.recs + row * a.nrec + c);
-    r += rec.r0;
-    p += rec.p2;
+  for (int c = threadIdx.x; c < a.nrec; c += kDenseNT) {
+    p += a.mass[2 * (row * a.nrec + c)];
+    r += a.mass[2 * (row * a.nrec + c) + 1];
   }
   uint64_t totR, totP;
   block_excl_u64(r, s64, &totR);
@@ -992,14 +1044,42 @@ __global__ void __launch_bounds__(SM_NT) residual_norm_kernel(ResidualNormArgs a
   const float fr = rn32_u64(totR);
   const bool use_r = fr > 1e-9f;
   const float tot = fmaxf(use_r ? fr : rn32_u64(totP), 1e-12f);
-  const int64_t c0 = cidx * a.rec_ids;
-  const int64_t c1 = min(a.V, c0 + a.rec_ids);
-  const float* pp = a.p + row * a.ld;
-  const float* qq = a.q + row * a.ld;
-  float* o = a.out + row * a.ld_out;
-  for (int64_t idx = c0 + threadIdx.x; idx < c1; idx += SM_NT) {
-    const float v = use_r ? fmaxf(pp[idx] - qq[idx], 0.0f) : pp[idx];
-    o[idx] = v / tot;
+  const float* const pp = a.p + row * a.ld;
+  const float* const qq = a.q + row * a.ld;
+  float* const o = a.out + row * a.ld_out;
+  auto val = [&](float x, float y) { return (use_r ? fmaxf(x - y, 0.0f) : x) / tot; };
+  // each wave its part of the ids, as records; the output goes 16 bytes at a time where
+  // it lies at p's phase too
+  const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  constexpr int kSub = kResIds / SM_NW;
+  const int64_t x0 = c0 + (int64_t)w * kSub, x1 = min(a.V, x0 + kSub);
+  if (x0 >= x1) return;
+  const bool vec = a.same && (((uintptr_t)(pp + x0) ^ (uintptr_t)(o + x0)) & 15u) == 0;  // uniform
+  if (!vec) {
+    for (int64_t i = x0 + lane; i < x1; i += kWave) o[i] = val(pp[i], qq[i]);
+    return;
+  }
+  const int64_t h = min(x1 - x0, (int64_t)(((16u - ((uint32_t)(uintptr_t)(pp + x0) & 15u)) & 15u) >> 2));
+  const int64_t nv = (x1 - x0 - h) >> 2, t0 = x0 + h + 4 * nv;
+  if (lane < h) o[x0 + lane] = val(pp[x0 + lane], qq[x0 + lane]);
+  if (t0 + lane < x1) o[t0 + lane] = val(pp[t0 + lane], qq[t0 + lane]);
+  const float4* const p4 = reinterpret_cast<const float4*>(pp + x0 + h);
+  const float4* const q4 = reinterpret_cast<const float4*>(qq + x0 + h);
+  float4* const o4 = reinterpret_cast<float4*>(o + x0 + h);
+  constexpr int N = kSub / (4 * kWave);
+  float4 v[N], y[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int64_t j = i * kWave + lane;
+    v[i] = j < nv ? p4[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    y[i] = j < nv ? q4[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int64_t j = i * kWave + lane;
+    if (j < nv)
+      o4[j] = make_float4(val(v[i].x, y[i].x), val(v[i].y, y[i].y), val(v[i].z, y[i].z),
+                          val(v[i].w, y[i].w));
   }
 }
 
@@ -1095,12 +1175,6 @@ hipError_t launch_draw_probs(const RowSourceF32& src, const AcceptArgs* acc, Sam
   return launch_draw(ev, acc, jobs, njobs, V, recs, counters, y, s);
 }
 
-hipError_t launch_chunk_mass_probs(const RowSourceF32& src, SampleJob* jobs, int64_t njobs,
-                                   int64_t V, ChunkRec* recs, hipStream_t s) {
-  EvalProb ev{src.base, src.ld, src.base2, src.ld2, src.split, src.vec, nullptr, 0};
-  return launch_draw(ev, nullptr, jobs, njobs, V, recs, nullptr, nullptr, s);
-}
-
 // The look-back bound: kMatWaitTicks, or a smaller bound from SDX_PROBS_WAIT_TICKS
 // (read at every launch; tests set 0 so that a chunk whose earlier chunks have not
 // all published at its first poll gives up, while every kernel exits normally).
@@ -1145,8 +1219,17 @@ hipError_t launch_sample_dense(const DenseArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_residual_norm(const ResidualNormArgs& a, int64_t rows, hipStream_t s) {
-  hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)(a.nrec * rows)), dim3(SM_NT), 0, s, a);
+hipError_t launch_residual(ResidualArgs a, hipStream_t s) {
+  a.nrec = dense_nrec(a.V);
+  a.nchunk = (int32_t)((a.V + kResIds - 1) / kResIds);
+  // rows of p and q at one 16-byte phase (their strides are equal)
+  a.same = (((uintptr_t)a.p ^ (uintptr_t)a.q) & 15u) == 0;
+  const int64_t waves = a.rows * a.nrec;
+  const int64_t wpb = kDenseNT / kWave;
+  hipLaunchKernelGGL(residual_mass_kernel, dim3((unsigned)((waves + wpb - 1) / wpb)),
+                     dim3(kDenseNT), 0, s, a);
+  hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)(a.nchunk * a.rows)), dim3(kDenseNT), 0,
+                     s, a);
   return hipGetLastError();
 }
 

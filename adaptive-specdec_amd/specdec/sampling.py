@@ -46,19 +46,22 @@ def _switch_args(temperature, top_p, top_k):
 
 
 def _kernel_rows(x):
-    """[rows, V] in a layout the row kernels accept: fp32/bf16/fp16, rows
-    starting 16-byte aligned with a stride that is a multiple of 8 (16-bit) or
-    4 (fp32) elements. Returns (tensor, ld)."""
+    """[rows, V] in a layout the row kernels accept: fp32 rows (the kernels find each
+    row's alignment), or bf16/fp16 rows starting 16-byte aligned with a stride that
+    is a multiple of 8 elements. Returns (tensor, ld)."""
     if x.dtype not in (torch.float32, torch.bfloat16, torch.float16):
         x = x.float()                      # sampling.py:42 upcasts anything else
     x = _lib.widen_f16(x)
     V = x.shape[-1]
-    mult = 4 if x.dtype == torch.float32 else 8
-    if x.is_contiguous() and V % mult == 0 and x.data_ptr() % 16 == 0:
+    f32 = x.dtype == torch.float32
+    mult = 4 if f32 else 8
+    if x.is_contiguous() and (f32 or (V % mult == 0 and x.data_ptr() % 16 == 0)):
         return x, V
     if (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) >= V and x.stride(0) % mult == 0
             and V % mult == 0 and x.data_ptr() % 16 == 0):
         return x, x.stride(0)              # rows of a wider buffer, read in place
+    if f32:
+        return x.contiguous(), V
     ld = (V + mult - 1) // mult * mult
     buf = torch.empty((x.shape[0], ld), dtype=x.dtype, device=x.device)
     buf[:, :V].copy_(x)

@@ -608,3 +608,47 @@ def test_tie_order_flags_ragged():
     assert np.array_equal(y.cpu().numpy(), ry)
     assert np.array_equal(f.cpu().numpy(), rf)
     assert ((rf & O.FLAG_TIE_ORDER) != 0).any()
+
+
+@pytest.mark.parametrize("rows,V,off,ld", [
+    (3, 1, 0, 1), (5, 2047, 0, 2047), (4, 2051, 1, 2053), (3, 4097, 3, 4100), (2, 12289, 2, 12289),
+])
+def test_residual_and_sample_rows_at_any_alignment(rows, V, off, ld):
+    """residual_probs and sample_from_probs on rows at every 16-byte phase, at the edges
+    of the records (2,048 ids) and of the output's chunks (4,096), p and q in and out of
+    phase; rows whose residual is empty; through the C ABI for the strides."""
+    import ctypes
+
+    from specdec import _lib
+    L = _lib.lib()
+    g = torch.Generator(device=DEV).manual_seed(V)
+    p = torch.rand((rows, V), generator=g, device=DEV)
+    q = torch.rand((rows, V), generator=g, device=DEV)
+    p[torch.rand((rows, V), generator=g, device=DEV) < 0.5] = 0
+    p[:, 0] = 0.25
+    p /= p.sum(-1, keepdim=True)
+    q /= q.sum(-1, keepdim=True)
+    q[rows - 1] = p[rows - 1]                              # degenerate: p itself
+    u = torch.rand(rows, generator=g, device=DEV)
+
+    def strided(t, o):
+        buf = torch.zeros(o + rows * ld + 8, device=DEV)
+        buf[o:o + rows * ld].view(rows, ld)[:, :V].copy_(t)
+        return buf, ctypes.c_void_p(buf.data_ptr() + 4 * o)
+
+    for oq, oo in ((off, off), (off + 1, off), (off, off + 2)):
+        (pb, pp), (qb, qp) = strided(p, off), strided(q, oq)
+        out = torch.full((oo + rows * ld + 8,), -1.0, device=DEV)
+        ws = _lib.workspace(L.sdx_residual_probs_workspace(rows, V), DEV, prepare=False)
+        _lib.check(L.sdx_residual_probs(pp, qp, rows, V, ld,
+                                        ctypes.c_void_p(out.data_ptr() + 4 * oo), ld, _lib.ptr(ws),
+                                        ws.numel(), _lib.stream_of(out)), "residual")
+        got = out[oo:oo + rows * ld].view(rows, ld)
+        ref = O.residual_probs(_np(p), _np(q))
+        assert np.array_equal(_np(got[:, :V]).view(np.uint32), ref.view(np.uint32))
+        assert bool((got[:, V:] == -1.0).all()) and bool((out[:oo] == -1.0).all())
+        ids = torch.empty(rows, dtype=torch.int64, device=DEV)
+        ws = _lib.workspace(L.sdx_sample_probs_workspace(rows, V), DEV, prepare=False)
+        _lib.check(L.sdx_sample_probs(pp, rows, V, ld, _lib.ptr(u), _lib.ptr(ids), _lib.ptr(ws),
+                                      ws.numel(), _lib.stream_of(ids)), "sample")
+        assert np.array_equal(ids.cpu().numpy(), O.sample_from_probs(_np(p), _np(u)))
