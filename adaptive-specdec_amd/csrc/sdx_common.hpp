@@ -112,6 +112,41 @@ __device__ __forceinline__ uint64_t fixed62(float x) {
   return sh >= 0 ? up : (sh <= -64 ? 0ull : dn);
 }
 
+// exp_det(d) as p * 2^k (p in [1, 2], exp_det's polynomial), d clamped at -105; the two
+// values below take it from there without forming one from the other's bits.
+struct ExpParts {
+  float p;
+  int k;
+};
+__device__ __forceinline__ ExpParts exp_det_parts(float d) {
+#pragma clang fp contract(off)
+  const double dd = (double)fmaxf(d, -105.0f);
+  const double kf = floor(dd * 0x1.71547652b82fep+0);
+  const float r = fmaxf((float)(dd - kf * 0x1.62e42fefa39efp-1), 0.0f);
+  float p = 0x1.71de3ap-19f;  // 1/9!, as in exp_det_core
+  p = p * r + 0x1.a01a02p-16f;
+  p = p * r + 0x1.a01a02p-13f;
+  p = p * r + 0x1.6c16c2p-10f;
+  p = p * r + 0x1.111112p-7f;
+  p = p * r + 0x1.555556p-5f;
+  p = p * r + 0x1.555556p-3f;
+  p = p * r + 0x1p-1f;
+  p = p * r + 1.0f;
+  p = p * r + 1.0f;
+  return ExpParts{fminf(p, 2.0f), (int)kf};
+}
+// exp_det(d): v_ldexp_f32 rounds a subnormal result once, as exp_det does.
+__device__ __forceinline__ float exp_det_of_parts(const ExpParts& x, float d) {
+  return d >= -104.0f ? ldexpf(x.p, x.k) : 0.0f;
+}
+// fixed62(exp_det(d)): the 24-bit mantissa shifted by the exponent, mant << 39 >> -k;
+// 0 below d = -43.5 (e^-43.5 < 2^-62, and k >= -63 above it) and for NaN.
+__device__ __forceinline__ uint64_t fixed62_of_parts(const ExpParts& x, float d) {
+  const uint32_t mant = __float_as_uint(x.p) - 0x3F000000u;
+  const uint64_t f = ((uint64_t)(mant << 7) << 32) >> ((uint32_t)(-x.k) & 63u);
+  return d >= -43.5f ? f : 0ull;
+}
+
 // i * 2^-62 rounded once to fp32 (nearest, ties to even).
 __device__ __forceinline__ float rn32_u64(uint64_t i) {
   if (i == 0) return 0.0f;

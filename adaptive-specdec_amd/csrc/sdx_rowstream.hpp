@@ -779,11 +779,12 @@ __device__ __forceinline__ int64_t rowstream_body(const RowStatArgs& a, SkLdsT<N
     auto zterm2 = [&](uint32_t e0, uint32_t e1) {
       const uint32_t c0 = e0 & 0x3FFFFu, c1 = e1 & 0x3FFFFu;
       const int b0 = (int)(e0 >> 18), b1 = (int)(e1 >> 18);
-      const float x0 = exp_det_sel(sk_d(bm.key_rep_sel(b0), invT, m));
-      const float x1 = exp_det_sel(sk_d(bm.key_rep_sel(b1), invT, m));
-      if (c0 != 0 && bmax - b0 < SK_ETOP) L.etop[bmax - b0] = x0;
-      if (c1 != 0 && bmax - b1 < SK_ETOP) L.etop[bmax - b1] = x1;
-      const uint64_t f0 = fixed62(x0), f1 = fixed62(x1);
+      const float d0 = sk_d(bm.key_rep_sel(b0), invT, m);
+      const float d1 = sk_d(bm.key_rep_sel(b1), invT, m);
+      const ExpParts x0 = exp_det_parts(d0), x1 = exp_det_parts(d1);
+      if (c0 != 0 && bmax - b0 < SK_ETOP) L.etop[bmax - b0] = exp_det_of_parts(x0, d0);
+      if (c1 != 0 && bmax - b1 < SK_ETOP) L.etop[bmax - b1] = exp_det_of_parts(x1, d1);
+      const uint64_t f0 = fixed62_of_parts(x0, d0), f1 = fixed62_of_parts(x1, d1);
       slo += (uint64_t)c0 * (uint32_t)f0 + (uint64_t)c1 * (uint32_t)f1;
       shi += (uint64_t)c0 * (uint32_t)(f0 >> 32) + (uint64_t)c1 * (uint32_t)(f1 >> 32);
     };
