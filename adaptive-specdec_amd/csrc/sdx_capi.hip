@@ -73,7 +73,8 @@ size_t transform_ws(Carve& c, int64_t rows, int64_t V, int dtype, int64_t njobs,
   sdx::draw_layout(V, &rec_ids, &nrec);
   *stats = c.take<sdx::RowStat>(rows);
   *tables = dtype == SDX_F32 ? nullptr : c.take<float>((size_t)rows * sdx::kTbl);
-  *dense = dtype == SDX_F32 ? c.take<float>((size_t)rows * V) : nullptr;
+  // fp32: the threshold statistics' scratch (rows above kThrSmall), a row each
+  *dense = dtype == SDX_F32 && V > sdx::kThrSmall ? c.take<float>((size_t)rows * V) : nullptr;
   *jobs = njobs ? c.take<sdx::SampleJob>(njobs) : nullptr;
   *recs = njobs ? c.take<sdx::ChunkRec>((size_t)njobs * nrec) : nullptr;
   *counters = njobs ? c.take<uint32_t>((size_t)njobs) : nullptr;
@@ -99,6 +100,20 @@ sdx::ThrArgs thr_args(const void* target, const void* draft, int64_t ntgt, int64
   a.V = V; a.T = T; a.top_p = top_p; a.top_k = top_k;
   a.use_p = sw.use_p; a.use_k = sw.use_k;
   return a;
+}
+
+// to_probs through the threshold statistics; longer rows keep their scratch in the
+// output rows, which may not overlap the logits.
+int thr_to_probs(int dtype, const void* logits, int64_t rows, int64_t V, int64_t ld, float T,
+                 float top_p, int32_t top_k, const Switches& sw, sdx::RowStat* stats, float* probs,
+                 int64_t ld_out, hipStream_t s) {
+  sdx::ThrArgs a = thr_args(logits, logits, rows, 0, ld, V, T, top_p, top_k, sw);
+  if (V <= sdx::kThrSmall)
+    return hip_status(sdx::launch_thr_small(dtype, a, rows, probs, ld_out, s), "thr_small");
+  a.stats = stats;
+  a.scratch = probs; a.scratch_stride = ld_out * 4; a.scratch_bytes = V * 4;
+  if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
+  return hip_status(sdx::launch_thr_output(dtype, a, rows, probs, ld_out, s), "thr_output");
 }
 
 int check_vocab(int dtype, int64_t V) {
@@ -155,36 +170,22 @@ int sdx_to_probs(const void* logits, int dtype, int64_t rows, int64_t vocab, int
   const Switches sw = switches(temperature, top_p, top_k, vocab);
   Carve c{(uint8_t*)workspace};
   if (dtype == SDX_F32) {
-    // rows above kF32SortVocab keep their scratch in the output rows until the output
+    // rows above kThrSmall keep their scratch in the output rows until the output
     // pass, so the output may not overlap the logits
     const uintptr_t l0 = (uintptr_t)logits, l1 = l0 + (uintptr_t)(((rows - 1) * ld + vocab) * 4);
     const uintptr_t p0 = (uintptr_t)probs, p1 = p0 + (uintptr_t)(((rows - 1) * ld_out + vocab) * 4);
     if (l0 < p1 && p0 < l1)
       return fail(SDX_EINVAL, "sdx_to_probs: probs overlap the fp32 logits");
-    if (vocab > sdx::kF32SortVocab) {
-      if (sw.greedy) {
-        int64_t* am = c.take<int64_t>(rows);
-        const bool vec = aligned16(logits) && ld % 4 == 0;
-        if (int e = hip_status(sdx::launch_argmax(dtype, logits, rows, vocab, ld, vec, am, s),
-                               "argmax"))
-          return e;
-        return hip_status(sdx::launch_onehot(am, rows, vocab, probs, ld_out, s), "onehot");
-      }
-      sdx::ThrArgs a = thr_args(logits, logits, rows, 0, ld, vocab, temperature, top_p, top_k, sw);
-      a.stats = c.take<sdx::RowStat>(rows);
-      a.scratch = probs; a.scratch_stride = ld_out * 4; a.scratch_bytes = vocab * 4;
-      if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
-      return hip_status(sdx::launch_thr_output(dtype, a, rows, probs, ld_out, s), "thr_output");
+    if (sw.greedy) {
+      int64_t* am = c.take<int64_t>(rows);
+      const bool vec = aligned16(logits) && ld % 4 == 0;
+      if (int e = hip_status(sdx::launch_argmax(dtype, logits, rows, vocab, ld, vec, am, s),
+                             "argmax"))
+        return e;
+      return hip_status(sdx::launch_onehot(am, rows, vocab, probs, ld_out, s), "onehot");
     }
-    sdx::F32Args a = {};
-    a.base[0] = (const float*)logits; a.nrows[0] = rows; a.ld[0] = ld;
-    a.base[1] = a.base[0]; a.nrows[1] = 0; a.ld[1] = ld;
-    a.V = vocab; a.ids = nullptr; a.k = 0;
-    a.T = temperature; a.top_p = top_p; a.top_k = top_k;
-    a.use_p = sw.use_p; a.use_k = sw.use_k; a.greedy = sw.greedy;
-    a.out = probs; a.ld_out = ld_out;
-    a.stats = c.take<sdx::RowStat>(rows);
-    return hip_status(sdx::launch_to_probs_f32(a, rows, s), "to_probs_f32");
+    return thr_to_probs(dtype, logits, rows, vocab, ld, temperature, top_p, top_k, sw,
+                        c.take<sdx::RowStat>(rows), probs, ld_out, s);
   }
   if (!aligned16(logits) || (ld % 8) != 0)
     return fail(SDX_EINVAL, "sdx_to_probs: 16-bit rows must start 16-byte aligned (ld %% 8 == 0)");
@@ -196,18 +197,13 @@ int sdx_to_probs(const void* logits, int dtype, int64_t rows, int64_t vocab, int
   }
   sdx::RowStat* st; float* tb; float* dn; sdx::SampleJob* jb; sdx::ChunkRec* rc; uint32_t* ct;
   transform_ws(c, rows, vocab, dtype, 0, &st, &tb, &dn, &jb, &rc, &ct);
-  if (dtype == SDX_F16 && vocab > sdx::kF32SortVocab) {
-    // the scratch lies in the output rows, as for fp32 (rows that overlap the logits
-    // take the register-resident kernel)
+  if (dtype == SDX_F16) {
+    // rows that overlap the logits take the register-resident kernel
     const uintptr_t l0 = (uintptr_t)logits, l1 = l0 + (uintptr_t)(((rows - 1) * ld + vocab) * 2);
     const uintptr_t p0 = (uintptr_t)probs, p1 = p0 + (uintptr_t)(((rows - 1) * ld_out + vocab) * 4);
-    if (!(l0 < p1 && p0 < l1)) {
-      sdx::ThrArgs a = thr_args(logits, logits, rows, 0, ld, vocab, temperature, top_p, top_k, sw);
-      a.stats = st;
-      a.scratch = probs; a.scratch_stride = ld_out * 4; a.scratch_bytes = vocab * 4;
-      if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
-      return hip_status(sdx::launch_thr_output(dtype, a, rows, probs, ld_out, s), "thr_output");
-    }
+    if (!(l0 < p1 && p0 < l1))
+      return thr_to_probs(dtype, logits, rows, vocab, ld, temperature, top_p, top_k, sw, st, probs,
+                          ld_out, s);
   }
   int64_t chunk;
   int nchunk;
@@ -406,15 +402,15 @@ static size_t verify_ws_bytes(int64_t batch, int64_t ntgt, int64_t ndrf, int64_t
     c.take<int32_t>(rows);  // the rows in batch-row order (fused kernel)
     c.take<int32_t>(rows);  // each row's batch row
   }
-  if (dtype == SDX_F32) c.take<uint32_t>((size_t)rows * sdx::f32_tie_words(vocab));  // tie bits
   return c.used;
 }
 
 // fp16 rows take the threshold statistics where the workspace holds their scratch
 // behind the pieces of the register-resident kernel (the sizes the queries return do;
 // sdx_verify_noalloc's fixed array may not).
-static size_t thr16_bytes(int64_t rows, int dtype) {
-  return dtype == SDX_F16 ? align256((size_t)rows * sdx::kThrScratchMin) : 0;
+static size_t thr16_bytes(int64_t rows, int64_t vocab, int dtype) {
+  return dtype == SDX_F16 && vocab > sdx::kThrSmall ? align256((size_t)rows * sdx::kThrScratchMin)
+                                                    : 0;
 }
 
 // The fused verify kernel (row statistics and draw in one launch) serves bf16
@@ -430,13 +426,13 @@ static bool fused_enabled() {
 
 size_t sdx_verify_workspace(int64_t batch, int32_t k, int64_t vocab, int dtype) {
   return verify_ws_bytes(batch, batch * ((int64_t)k + 1), batch * (int64_t)k, vocab, dtype, false) +
-         thr16_bytes(batch * (2 * (int64_t)k + 1), dtype);
+         thr16_bytes(batch * (2 * (int64_t)k + 1), vocab, dtype);
 }
 
 size_t sdx_verify_ragged_workspace(int64_t batch, int64_t target_rows, int64_t vocab, int dtype) {
   if (batch < 0 || target_rows < batch) return 0;
   return verify_ws_bytes(batch, target_rows, target_rows - batch, vocab, dtype, true) +
-         thr16_bytes(2 * target_rows - batch, dtype);
+         thr16_bytes(2 * target_rows - batch, vocab, dtype);
 }
 
 static int verify_impl(const void* target_logits, const void* draft_logits, int dtype,
@@ -549,8 +545,6 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
                            "ragged_rows"))
       return e;
   }
-  uint32_t* tie_bits =
-      dtype == SDX_F32 ? c.take<uint32_t>((size_t)rows * sdx::f32_tie_words(vocab)) : nullptr;
 
   if (sw.greedy) {
     // one-hot p: only the target argmax matters (see sdx_verify_greedy)
@@ -563,8 +557,8 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
                       "greedy_accept");
   }
   if (!draft_logits) return fail(SDX_EINVAL, "sdx_verify: draft_logits required when T > 0");
-  const bool thr16 = dtype == SDX_F16 && workspace_bytes >= need + thr16_bytes(rows, dtype);
-  const bool thr = thr16 || (dtype == SDX_F32 && vocab > sdx::kF32SortVocab);
+  const bool thr16 = dtype == SDX_F16 && workspace_bytes >= need + thr16_bytes(rows, vocab, dtype);
+  const bool thr = thr16 || dtype == SDX_F32;
   if (dtype != SDX_F32 &&
       (!aligned16(target_logits) || !aligned16(draft_logits) || (vocab % 8) != 0))
     return fail(SDX_EINVAL,
@@ -578,22 +572,10 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
     a.zero = counters; a.nzero = batch;
     a.scratch = dn; a.scratch_stride = a.scratch_bytes = vocab * 4;
     if (thr16) {
-      a.scratch = c.take<uint8_t>(thr16_bytes(rows, dtype));
+      a.scratch = c.take<uint8_t>(thr16_bytes(rows, vocab, dtype));
       a.scratch_stride = a.scratch_bytes = sdx::kThrScratchMin;
     }
     if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;
-  } else if (dtype == SDX_F32) {
-    sdx::F32Args a = {};
-    a.base[0] = (const float*)target_logits; a.nrows[0] = ntgt; a.ld[0] = vocab;
-    a.base[1] = (const float*)draft_logits; a.nrows[1] = ndrf; a.ld[1] = vocab;
-    a.V = vocab; a.ids = draft_ids; a.k = k; a.tgt_idx = tgt_idx;
-    a.T = temperature; a.top_p = top_p; a.top_k = top_k;
-    a.use_p = sw.use_p; a.use_k = sw.use_k; a.greedy = 0;
-    a.out = dn; a.ld_out = vocab; a.stats = st;
-    a.zero = counters; a.nzero = batch;
-    a.tie_bits = tie_bits;
-    a.tie_ld = sdx::f32_tie_words(vocab);
-    if (int e = hip_status(sdx::launch_to_probs_f32(a, rows, s), "to_probs_f32")) return e;
   } else {
     sdx::RowStatArgs a = {};
     a.base[0] = (const uint16_t*)target_logits; a.nrows[0] = ntgt; a.ld[0] = vocab;
@@ -659,12 +641,6 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
     d.V = vocab; d.T = temperature;
     d.recs = (uint64_t*)recs; d.counters = counters; d.y = y;
     return hip_status(sdx::launch_thr_draw(dtype, d, batch, s), "thr_draw");
-  }
-  if (dtype == SDX_F32) {
-    sdx::RowSourceF32 src{dn, vocab, dn, vocab, rows, (vocab % 4) == 0};
-    return hip_status(sdx::launch_draw_probs(src, &aa, jobs, batch, vocab, recs,
-                                             counters, y, s, tie_bits),
-                      "draw_probs");
   }
   sdx::RowSource16 src{(const uint16_t*)target_logits, vocab, (const uint16_t*)draft_logits, vocab,
                        ntgt, true};
@@ -785,7 +761,7 @@ static size_t draft_ws_x_offset(int64_t batch, int64_t vocab, int dtype) {
 
 size_t sdx_draft_step_workspace(int64_t batch, int64_t vocab, int dtype) {
   if (batch < 0 || vocab < 1 || !dtype_ok(dtype)) return 0;
-  return draft_ws_bytes(batch, vocab, dtype) + thr16_bytes(batch, dtype);
+  return draft_ws_bytes(batch, vocab, dtype) + thr16_bytes(batch, vocab, dtype);
 }
 
 int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, int64_t ld,
@@ -824,8 +800,8 @@ int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, 
   if (dtype != SDX_F32 && (!aligned16(logits) || (ld % 8) != 0 || (vocab % 8) != 0))
     return fail(SDX_EINVAL,
                 "sdx_draft_step: 16-bit rows must start 16-byte aligned, ld %% 8 == 0, vocab %% 8 == 0");
-  const bool thr16 = dtype == SDX_F16 && workspace_bytes >= need + thr16_bytes(batch, dtype);
-  if (thr16 || (dtype == SDX_F32 && vocab > sdx::kF32SortVocab)) {
+  const bool thr16 = dtype == SDX_F16 && workspace_bytes >= need + thr16_bytes(batch, vocab, dtype);
+  if (thr16 || dtype == SDX_F32) {
     sdx::ThrArgs a = thr_args(logits, logits, batch, 0, ld, vocab, temperature, top_p, top_k, sw);
     a.stats = st;
     a.zero = counters; a.nzero = batch;
@@ -846,27 +822,6 @@ int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, 
     if (int r = hip_status(sdx::launch_thr_draw(dtype, d, batch, s), "thr_draw")) return r;
     e.probs = d.qx;
     e.ldp = 0;
-    return hip_status(sdx::launch_draft_epilogue(e, s), "draft_epilogue");
-  }
-  if (dtype == SDX_F32) {
-    hipLaunchKernelGGL(sdx_jobs_from_u, dim3((unsigned)((batch + 255) / 256)), dim3(256), 0, s,
-                       jobs, u, batch, (int64_t)-1, counters);
-    if (int r = hip_status(hipGetLastError(), "jobs")) return r;
-    sdx::F32Args a = {};
-    a.base[0] = (const float*)logits; a.nrows[0] = batch; a.ld[0] = ld;
-    a.base[1] = a.base[0]; a.nrows[1] = 0; a.ld[1] = ld;
-    a.V = vocab; a.ids = nullptr; a.k = 0;
-    a.T = temperature; a.top_p = top_p; a.top_k = top_k;
-    a.use_p = sw.use_p; a.use_k = sw.use_k; a.greedy = 0;
-    a.out = dn; a.ld_out = vocab; a.stats = st;
-    if (int r = hip_status(sdx::launch_to_probs_f32(a, batch, s), "to_probs_f32")) return r;
-    sdx::RowSourceF32 src{dn, vocab, dn, vocab, batch, (vocab % 4) == 0};
-    if (int r = hip_status(sdx::launch_draw_probs(src, nullptr, jobs, batch, vocab, recs, counters,
-                                                  x, s),
-                           "draw_probs"))
-      return r;
-    e.probs = dn;
-    e.ldp = vocab;
     return hip_status(sdx::launch_draft_epilogue(e, s), "draft_epilogue");
   }
   sdx::RowStatArgs a = {};

@@ -115,13 +115,5 @@ struct RowSource16 {
   int64_t split;
   bool vec;  // every row start is 16-byte aligned
 };
-struct RowSourceF32 {
-  const float* base;
-  int64_t ld;
-  const float* base2;
-  int64_t ld2;
-  int64_t split;
-  bool vec;
-};
 
 }  // namespace sdx

@@ -62,26 +62,6 @@ struct RowStatArgs {
   const int32_t* jm_order;  // ... or, at per-row k, in this order (block's q -> row)
 };
 
-struct F32Args {
-  const float* base[2];
-  int64_t nrows[2];
-  int64_t ld[2];
-  int64_t V;
-  const int64_t* ids;
-  int32_t k;
-  const int64_t* tgt_idx;  // per-row k: target row -> index into ids (-1: bonus), or null
-  float T, top_p;
-  int32_t top_k, use_p, use_k, greedy;
-  float* out;  // dense probabilities [rows, ld_out]
-  int64_t ld_out;
-  RowStat* stats;  // may be null
-  uint32_t* zero;  // words [0, nzero) cleared (block `row` clears word `row`), or null
-  int64_t nzero;
-  int64_t tie_ld;      // words per row of tie_bits (f32_tie_words(V))
-  uint32_t* tie_bits;  // [rows, tie_ld]: members of the row's partially kept
-                       // boundary tie group, one bit per id (null: not written)
-};
-
 // One final draw: weights from row `prow` (and `qrow` for a residual).
 struct SampleJob {
   int64_t prow;     // row whose probabilities are p
@@ -204,10 +184,6 @@ hipError_t launch_workspace_init(void* ws, size_t bytes, hipStream_t s);
 hipError_t launch_workspace_rearm(void* ws, hipStream_t s);
 // sdx_rank.hip: pgather of drafted tokens inside a partial tie group (after rowstream)
 hipError_t launch_rank_bf16(const RowStatArgs& a, int64_t rows, hipStream_t s);
-// sdx_f32.hip
-// fp32 rows up to here are sorted whole in LDS (to_probs_f32_kernel); longer ones take
-// the threshold statistics of sdx_thr.hip
-constexpr int64_t kF32SortVocab = 8192;
 // Largest vocabularies of 16-bit rows. bf16 rows stream through the histogram
 // kernel, whose normaliser queues a bin as (bin << 18 | count): counts, so the
 // vocabulary, stay below 2^18 (the largest multiple of 8 below it, as rows are
@@ -216,14 +192,12 @@ constexpr int64_t kF32SortVocab = 8192;
 constexpr int64_t kMaxVocabBf16 = (1 << 18) - 8;
 constexpr int64_t kMaxVocabF16 = 16 * 20 * 512;
 constexpr int64_t kF32MaxVocab = 262144;
-// tie-group bit words per fp32 row: one bit per id, whole 64-id wave rounds
-inline int64_t f32_tie_words(int64_t V) { return (V + 63) / 64 * 2; }
-hipError_t launch_to_probs_f32(const F32Args& a, int64_t rows, hipStream_t s);
 // sdx_thr.hip: row statistics as a threshold (see sdx_thr.hpp) and what reads them
 constexpr int kThrMaxParts = 32;    // workgroups per row
 constexpr int kThrBuckets = 1024;   // steps of m - s
 constexpr int kThrList = 2048;      // region elements listed
 constexpr int kThrRec = 1024;       // ids per draw record
+constexpr int64_t kThrSmall = 8192; // rows up to here take one workgroup and no scratch
 constexpr int64_t kThrCtlBytes = 1024;
 // scratch per row (with room to align its start)
 constexpr int64_t kThrScratchMin = 64 + kThrCtlBytes + kThrList * 8 + kThrBuckets * 12;
@@ -248,7 +222,12 @@ struct ThrArgs {
   int32_t nparts, nlight;
   int64_t plen, llen;
 };
+// (rows of at most kThrSmall elements need no scratch)
 hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s);
+// rows of at most kThrSmall elements: statistics (a.stats) and to_probs rows (out), each
+// where not null
+hipError_t launch_thr_small(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+                            hipStream_t s);
 // to_probs rows; the scratch may lie in `out` (it is read no more)
 hipError_t launch_thr_output(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
                              hipStream_t s);
@@ -271,15 +250,12 @@ hipError_t launch_thr_draw(int dtype, ThrDrawArgs a, int64_t jobs, hipStream_t s
 // chain when `acc` is given: jobs are then written by the kernel). Without
 // `acc`, `jobs` must hold the draws already.
 // `counters` ([njobs] words) must be zero on entry: the kernel launched just
-// before the draw clears them (RowStatArgs / F32Args `zero`).
+// before the draw clears them (RowStatArgs `zero`).
 // `recs` holds njobs * nrec records (draw_layout).
 hipError_t launch_draw16(int fmt, const RowSource16& src, const RowStat* stats,
                          const float* tables, float T, const AcceptArgs* acc, SampleJob* jobs,
                          int64_t njobs, int64_t V, ChunkRec* recs, uint32_t* counters, int64_t* y,
                          hipStream_t s);
-hipError_t launch_draw_probs(const RowSourceF32& src, const AcceptArgs* acc, SampleJob* jobs,
-                             int64_t njobs, int64_t V, ChunkRec* recs, uint32_t* counters,
-                             int64_t* y, hipStream_t s, const uint32_t* tie_bits = nullptr);
 // to_probs output of 16-bit rows: ids per chunk (one workgroup each).
 constexpr int64_t kMatChunk = 16384;
 

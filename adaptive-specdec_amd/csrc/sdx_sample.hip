@@ -29,68 +29,6 @@ namespace sdx {
 
 
 
-struct EvalProb {
-  static constexpr bool kGroups = false;
-  static constexpr int kFmt = SDX_F32;
-  static constexpr int kLdsTbl = 1;
-  struct Raw {
-    float4 a, b;
-  };
-  const float* base;
-  int64_t ld;
-  const float* base2;
-  int64_t ld2;
-  int64_t split;
-  bool vec;
-  const uint32_t* tie_bits;  // per row bits_ld words: members of a partial
-                             // boundary tie group (null: no membership known)
-  int64_t bits_ld;
-  struct Row {
-    const float* ptr;
-    float vg;
-    const uint32_t* bits;
-  };
-  __device__ void stage(int64_t, float*) const {}
-  __device__ void bind(Row& r, int64_t row, const float*) const {
-    r.ptr = row < split ? base + row * ld : base2 + (row - split) * ld2;
-    r.vg = 0.0f;
-    r.bits = tie_bits ? tie_bits + row * bits_ld : nullptr;
-  }
-  __device__ static int32_t rstar(const Row&) { return 0; }
-  __device__ static bool in_tie_group(const Row& r, int64_t id) {
-    return r.bits && ((r.bits[id >> 5] >> (id & 31)) & 1u) != 0;
-  }
-  __device__ Raw fetch(const Row& r, int64_t idx, int64_t lim) const {
-    Raw x;
-    if (vec && idx + 8 <= lim) {
-      x.a = *reinterpret_cast<const float4*>(r.ptr + idx);
-      x.b = *reinterpret_cast<const float4*>(r.ptr + idx + 4);
-    } else {
-      float v[8];
-#pragma unroll
-      for (int t = 0; t < 8; ++t) v[t] = idx + t < lim ? r.ptr[idx + t] : 0.0f;
-      x.a = make_float4(v[0], v[1], v[2], v[3]);
-      x.b = make_float4(v[4], v[5], v[6], v[7]);
-    }
-    return x;
-  }
-  __device__ uint32_t eval(const Row&, int64_t idx, int64_t lim, const Raw& x, float v[8]) const {
-    v[0] = x.a.x; v[1] = x.a.y; v[2] = x.a.z; v[3] = x.a.w;
-    v[4] = x.b.x; v[5] = x.b.y; v[6] = x.b.z; v[7] = x.b.w;
-    uint32_t live = 0;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      if (idx + t >= lim) v[t] = 0.0f;
-      live |= (v[t] > 0.0f ? 1u : 0u) << (8 + t);
-    }
-    return live;  // no tie groups; bits 8..15: nonzero probabilities
-  }
-  __device__ uint32_t load8(const Row& r, int64_t idx, int64_t lim, float v[8]) const {
-    return eval(r, idx, lim, fetch(r, idx, lim), v) & 0xFFu;
-  }
-};
-
-
 // One wave walks ids [i0, i1) in id order, the member ranks at i0 being
 // (bp, bq), and returns the mass (residual when use_r, else p). With `find`
 // (base <= t), the lane holding the first id whose prefix mass, counted from
@@ -1166,13 +1104,6 @@ hipError_t launch_draw_rows16(int fmt, const RowSource16& src, const RowStat* st
   return launch_draw(Eval16<SDX_F16>{src.base, src.ld, src.base2, src.ld2, src.split, stats,
                                       tables, T},
                      nullptr, jobs, njobs, V, recs, counters, y, s);
-}
-
-hipError_t launch_draw_probs(const RowSourceF32& src, const AcceptArgs* acc, SampleJob* jobs,
-                             int64_t njobs, int64_t V, ChunkRec* recs, uint32_t* counters,
-                             int64_t* y, hipStream_t s, const uint32_t* tie_bits) {
-  EvalProb ev{src.base, src.ld, src.base2, src.ld2, src.split, src.vec, tie_bits, f32_tie_words(V)};
-  return launch_draw(ev, acc, jobs, njobs, V, recs, counters, y, s);
 }
 
 // The look-back bound: kMatWaitTicks, or a smaller bound from SDX_PROBS_WAIT_TICKS

@@ -257,6 +257,83 @@ __device__ __forceinline__ float thr_div(float x, float T, float rT) {
   return __builtin_fmaf(__builtin_fmaf(-T, q1, x), rT, q1);
 }
 
+__device__ __forceinline__ ThrDiv thr_div_kind(float T, float xmax) {
+  const float a = fabsf(xmax);
+  if (T == 1.0f) return kDivOne;
+  return T >= 0x1p-20f && T <= 0x1p20f && a <= 0x1p100f && (a >= 0x1p-90f || a == 0.0f) ? kDivFma
+                                                                                       : kDivIeee;
+}
+// Steps of m - s per unit, 2^e with e >= 5: the row's range (at most 32) over at most
+// TH_NB steps.
+__device__ __forceinline__ float thr_scale(float m, float xmn, float T) {
+  const float range = fminf(m - xmn / T, 32.0f);  // NaN (no finite logit): 32
+  float scale = TH_NB / 32.0f;
+  while (scale < 0x1p20f && range * (2.0f * scale) <= (float)(TH_NB - 2)) scale *= 2.0f;
+  return scale;
+}
+// One element of the histogram pass.
+template <int DIV, bool CNT>
+__device__ __forceinline__ void thr_hist_one(float x, bool ok, float T, float rT, float m,
+                                             float scale, uint64_t* mass, uint32_t* cnt,
+                                             uint64_t& zlo, uint32_t& zhi) {
+  const float d = ok ? thr_div<DIV>(x, T, rT) - m : -INFINITY;
+  // NaN (-inf logits through the FMA steps): the last step; d > 0 never, and
+  // v_cvt_u32_f32 would take it to 0
+  const uint32_t b = (uint32_t)fminf(-d * scale, (float)(TH_NB - 1));
+  const uint64_t f = thr_exp62(d);
+  zlo += f;
+  zhi += zlo < f ? 1u : 0u;
+  if (CNT && ok) atomicAdd(&cnt[b], 1u);
+  // 2^-44 units: sums of 2^18 elements fit 64 bits
+  if (f >> 18) atomicAdd((unsigned long long*)&mass[b], (unsigned long long)(f >> 18));
+}
+// What a region of steps [b0, b1] (and the step bk of the k-th largest) decides.
+struct ThrCut {
+  float phi, plo, xcut;
+  bool use_k, use_p;
+};
+__device__ __forceinline__ ThrCut thr_cut(const ThrArgs& a, float m, float zf, float scale, int b0,
+                                          int b1, int bk) {
+  ThrCut c;
+  c.use_k = a.use_k;
+  c.use_p = a.use_p;
+  if (c.use_k && !c.use_p) {
+    b0 = b1 = bk;
+  } else if (c.use_k) {
+    if (b1 < bk) c.use_k = false;  // the nucleus ends above the k-th largest
+    else { b0 = min(b0, bk); b1 = bk; }
+  }
+  const float inv = 1.0f / scale;  // a power of two
+  c.phi = -1.0f;                   // no filter: everything is above
+  c.plo = 0x1p-149f;
+  float dlo = -104.0f;
+  if (c.use_k || c.use_p) {
+    // edges of the steps: p at m - s = b0 / scale and (b1 + 1) / scale
+    c.phi = b0 == 0 ? 2.0f : exp_det(-(float)b0 * inv) / zf;
+    if (b1 < TH_NB - 1) {
+      dlo = -(float)(b1 + 1) * inv;
+      c.plo = fmaxf(exp_det(dlo) / zf, 0x1p-149f);
+    }
+  }
+  // no logit below xcut has p >= plo: p drops by more than its rounding within 1e-5
+  // of s, and the fp32 rounding of (m + dlo) T is within 1e-6 of its terms
+  c.xcut = ((m + dlo) - (4e-6f * (fabsf(m) + fabsf(dlo)) + 2e-5f)) * a.T;
+  c.xcut -= 4e-6f * fabsf(c.xcut);
+  if (!(fabsf(c.xcut) < INFINITY)) c.xcut = -INFINITY;
+  return c;
+}
+// The region's steps from running sums: this step's mass (and count) between rm and nm
+// (rc and nc) of the row's, zu the row's normaliser in the masses' units. One writer
+// each, as the running sums grow (the step before has not reached the bound).
+__device__ __forceinline__ void thr_mark(const ThrArgs& a, int b, uint64_t rm, uint64_t nm,
+                                         uint64_t rc, uint64_t nc, double zu, int32_t* b0,
+                                         int32_t* b1, int32_t* bk) {
+  const double tlo = ((double)a.top_p - 1e-6) * zu, thi = ((double)a.top_p + 1e-6) * zu;
+  if ((double)nm >= tlo && !(b > 0 && (double)rm >= tlo)) *b0 = b;
+  if ((double)nm >= thi && !(b > 0 && (double)rm >= thi)) *b1 = b;
+  if (a.use_k && nc >= (uint64_t)a.top_k && rc < (uint64_t)a.top_k) *bk = b;
+}
+
 struct ThrHistLds {
   uint64_t mass[TH_NB];
   uint32_t cnt[TH_NB];
@@ -266,6 +343,8 @@ struct ThrHistLds {
   int32_t last, b0, b1, bk;
 };
 
+// Exclusive scan over a workgroup of NW waves; `s` holds NW words.
+template <int NW = TH_NW>
 __device__ __forceinline__ uint64_t thr_excl_u64(uint64_t v, uint64_t* s) {
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   const uint64_t incl = wave_incl_scan_u64(v, lane);
@@ -273,7 +352,7 @@ __device__ __forceinline__ uint64_t thr_excl_u64(uint64_t v, uint64_t* s) {
   if (lane == kWave - 1) s[w] = incl;
   __syncthreads();
   uint64_t off = 0;
-  for (int i = 0; i < TH_NW; ++i) off += i < w ? s[i] : 0ull;
+  for (int i = 0; i < NW; ++i) off += i < w ? s[i] : 0ull;
   return off + incl - v;
 }
 
@@ -283,16 +362,7 @@ __device__ __forceinline__ void thr_hist_pass(const ThrArgs& a, ThrHistLds& L, c
                                               uint32_t& zhi) {
   const float T = a.T, rT = 1.0f / a.T;
   thr_stream<E, 4>(row, a.V, part, a.nparts, a.plen, [&](int64_t, float x, bool ok) {
-    const float d = ok ? thr_div<DIV>(x, T, rT) - m : -INFINITY;
-    // NaN (-inf logits through the FMA steps): the last step; d > 0 never, and
-    // v_cvt_u32_f32 would take it to 0
-    const uint32_t b = (uint32_t)fminf(-d * scale, (float)(TH_NB - 1));
-    const uint64_t f = thr_exp62(d);
-    zlo += f;
-    zhi += zlo < f ? 1u : 0u;
-    if (CNT && ok) atomicAdd(&L.cnt[b], 1u);
-    // 2^-44 units: sums of 2^18 elements fit 64 bits
-    if (f >> 18) atomicAdd((unsigned long long*)&L.mass[b], (unsigned long long)(f >> 18));
+    thr_hist_one<DIV, CNT>(x, ok, T, rT, m, scale, L.mass, L.cnt, zlo, zhi);
   });
 }
 
@@ -314,16 +384,8 @@ __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
   }
   const float T = a.T;
   const float m = xmx / T;  // the division is monotone: the maximum of fl32(x / T)
-  // steps of 2^-e, e >= 5: the row's range (at most 32) over at most TH_NB steps
-  const float range = fminf(m - xmn / T, 32.0f);  // NaN (no finite logit): 32
-  float scale = TH_NB / 32.0f;
-  while (scale < 0x1p20f && range * (2.0f * scale) <= (float)(TH_NB - 2)) scale *= 2.0f;
-  const float axm = fabsf(xmx);
-  const int div = T == 1.0f ? kDivOne
-                  : (T >= 0x1p-20f && T <= 0x1p20f && axm <= 0x1p100f &&
-                     (axm >= 0x1p-90f || axm == 0.0f))
-                      ? kDivFma
-                      : kDivIeee;
+  const float scale = thr_scale(m, xmn, T);
+  const ThrDiv div = thr_div_kind(T, xmx);
   __syncthreads();
   uint64_t zlo = 0;
   uint32_t zhi = 0;
@@ -406,51 +468,23 @@ __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
   uint64_t rc = a.use_k ? thr_excl_u64(sc, L.s64) : 0ull;
   __syncthreads();
   const double zu = ((double)z.hi * 0x1p64 + (double)z.lo) * 0x1p-18;
-  const double tlo = ((double)a.top_p - 1e-6) * zu, thi = ((double)a.top_p + 1e-6) * zu;
 #pragma unroll
   for (int i = 0; i < TH_BPT; ++i) {
     const uint64_t nm = rm + mass[i], nc = rc + cnt[i];
-    const int b = tid * TH_BPT + i;
-    // the first step whose running mass (count) reaches a bound: one writer each, as
-    // the running sums grow (the step before has not reached it)
-    if ((double)nm >= tlo && !(b > 0 && (double)rm >= tlo)) L.b0 = b;
-    if ((double)nm >= thi && !(b > 0 && (double)rm >= thi)) L.b1 = b;
-    if (a.use_k && nc >= (uint64_t)a.top_k && rc < (uint64_t)a.top_k) L.bk = b;
+    thr_mark(a, tid * TH_BPT + i, rm, nm, rc, nc, zu, &L.b0, &L.b1, &L.bk);
     rm = nm;
     rc = nc;
   }
   __syncthreads();
   if (tid != 0) return;
-  int b0 = L.b0, b1 = L.b1;
-  bool use_k = a.use_k, use_p = a.use_p;
-  if (use_k && !use_p) {
-    b0 = b1 = L.bk;
-  } else if (use_k) {
-    if (b1 < L.bk) use_k = false;  // the nucleus ends above the k-th largest
-    else { b0 = min(b0, L.bk); b1 = L.bk; }
-  }
-  const float inv = 1.0f / scale;  // a power of two
-  float phi = -1.0f, plo = 0x1p-149f, dlo = -104.0f;  // no filter: everything is above
-  if (use_k || use_p) {
-    // edges of the steps: p at m - s = b0 / scale and (b1 + 1) / scale
-    phi = b0 == 0 ? 2.0f : exp_det(-(float)b0 * inv) / zf;
-    if (b1 < TH_NB - 1) {
-      dlo = -(float)(b1 + 1) * inv;
-      plo = fmaxf(exp_det(dlo) / zf, 0x1p-149f);
-    }
-  }
-  // no logit below xcut has p >= plo: p drops by more than its rounding within 1e-5
-  // of s, and the fp32 rounding of (m + dlo) T is within 1e-6 of its terms
-  float xcut = ((m + dlo) - (4e-6f * (fabsf(m) + fabsf(dlo)) + 2e-5f)) * T;
-  xcut -= 4e-6f * fabsf(xcut);
-  if (!(fabsf(xcut) < INFINITY)) xcut = -INFINITY;
+  const ThrCut t = thr_cut(a, m, zf, scale, L.b0, L.b1, L.bk);
   c->m = m;
   c->zf = zf;
-  c->phi = phi;
-  c->plo = plo;
-  c->xcut = xcut;
-  c->use_k = use_k ? 1 : 0;
-  c->use_p = use_p ? 1 : 0;
+  c->phi = t.phi;
+  c->plo = t.plo;
+  c->xcut = t.xcut;
+  c->use_k = t.use_k ? 1 : 0;
+  c->use_p = t.use_p ? 1 : 0;
 }
 
 // ---------------------------------------------------------------- 3. collect
@@ -541,14 +575,143 @@ __global__ void __launch_bounds__(TH_NT) thr_collect_kernel(ThrArgs a) {
 }
 
 // ---------------------------------------------------------------- 4. resolve
+// kept = p > vf, or p == vf and id <= idcut; partial: the group of vf keeps a part of
+// its members; tot: the kept mass.
+struct ThrEnd {
+  float vf = -1.0f;
+  uint32_t idcut = 0xFFFFFFFFu;
+  bool partial = false;
+  uint64_t tot = 0;
+};
+struct ThrWalkLds {
+  uint32_t first;
+  uint64_t sum;
+};
+// The list's entries (e[0, n), any order, ~0 from there to NC or the next power of two)
+// sorted ascending: up to NC of them by counting the smaller entries (into t), else in
+// place. Returns where they are.
+template <int NT, int NC>
+__device__ __forceinline__ const uint64_t* thr_sort(uint64_t* e, uint64_t* t, uint32_t n) {
+  const uint32_t tid = threadIdx.x;
+  static_assert(NC == NT || NC == 2 * NT, "one or two entries per thread");
+  if (n <= (uint32_t)NC) {  // uniform
+    const uint64_t k0 = tid < n ? e[tid] : ~0ull;
+    const uint64_t k1 = NC > NT && tid + NT < n ? e[tid + NT] : ~0ull;
+    if (tid < n) {
+      uint32_t r0 = 0, r1 = 0;
+      for (uint32_t i = 0; i < n; i += 16) {  // ~0 past n: never smaller
+        uint64_t v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = e[i + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          r0 += v[u] < k0 ? 1u : 0u;
+          if (NC > NT) r1 += v[u] < k1 ? 1u : 0u;
+        }
+      }
+      t[r0] = k0;
+      if (NC > NT && tid + NT < n) t[r1] = k1;
+    }
+    __syncthreads();
+    return t;
+  }
+  uint32_t S = NT;
+  while (S < n) S <<= 1;
+  for (uint32_t size = 2; size <= S; size <<= 1)
+    for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+      for (uint32_t i = tid; i < S; i += NT) {
+        const uint32_t j = i ^ stride;
+        if (j > i) {
+          const bool up = (i & size) == 0;
+          const uint64_t ai = e[i], aj = e[j];
+          if ((ai > aj) == up) { e[i] = aj; e[j] = ai; }
+        }
+      }
+      __syncthreads();
+    }
+  return e;
+}
+// The reference's walk over the sorted region: `above` and `nabove` are the mass and
+// count of the elements above it, phi its upper edge.
+template <int NT>
+__device__ __forceinline__ ThrEnd thr_walk(const ThrArgs& a, const uint64_t* e, uint32_t n,
+                                           bool use_k, bool use_p, uint64_t above, uint64_t nabove,
+                                           float phi, ThrWalkLds& L, uint64_t* s64) {
+  const uint32_t tid = threadIdx.x;
+  ThrEnd r;
+  auto pof = [&](uint32_t i) { return __uint_as_float(~(uint32_t)(e[i] >> 32)); };
+  // the k-th largest p (0: not among the positive ones, nothing is zeroed)
+  float kth = 0.0f;
+  if (use_k && (uint64_t)a.top_k > nabove && (uint64_t)a.top_k - nabove <= n)
+    kth = pof((uint32_t)((uint64_t)a.top_k - nabove) - 1u);
+  if (tid == 0) { L.first = n; L.sum = 0ull; }
+  // entries per * tid ..: their masses, then the first that fails
+  const uint32_t per = (n + NT - 1) / NT;
+  const uint32_t i0 = min(n, tid * per), i1 = min(n, i0 + per);
+  uint64_t s = 0;
+  for (uint32_t i = i0; i < i1; ++i) s += fixed62(pof(i));
+  const uint64_t ex = above + thr_excl_u64<NT / kWave>(s, s64);
+  uint64_t run = ex;
+  uint32_t mine = n;
+  for (uint32_t i = i0; i < i1; ++i) {
+    const float p = pof(i);
+    const uint64_t nr = run + fixed62(p);
+    bool keep = !(p < kth);
+    if (use_p) keep = keep && (((rn32_u64(nr) - p) < a.top_p) || (nabove + i == 0));
+    if (!keep) { mine = i; break; }
+    run = nr;
+  }
+  __syncthreads();
+  if (mine < n) atomicMin(&L.first, mine);
+  __syncthreads();
+  const uint32_t f = L.first;  // entries [0, f) are kept
+  if (i0 < f) atomicAdd((unsigned long long*)&L.sum, (unsigned long long)(run - ex));
+  __syncthreads();
+  r.tot = above + L.sum;
+  if (f == 0) {
+    r.vf = __uint_as_float(__float_as_uint(phi) + 1u);  // everything above the region
+  } else {
+    r.vf = pof(f - 1);
+    r.partial = f < n && pof(f) == r.vf && !(r.vf < kth);
+    if (r.partial) r.idcut = (uint32_t)e[f - 1];
+  }
+  return r;
+}
+// The row's record, with the final probability of its gathered token (one thread).
+__device__ __forceinline__ RowStat thr_record(const ThrEnd& r, float m, float zf, float xcut,
+                                              int64_t gid, int64_t V, float xg, float T,
+                                              bool nonfinite) {
+  const float totf = fmaxf(rn32_u64(r.tot), 1e-12f);
+  const bool bad = !(zf > 0.0f);  // no finite maximum: every probability is 0 / 0
+  const ThrRow row{m, zf, totf, r.vf, xcut, r.idcut};
+  RowStat st = {};
+  bool gtie = false;
+  if (gid >= 0 && gid < V) {
+    st.pgather = bad ? __builtin_nanf("") : thr_prob(row, xg, (uint32_t)gid, T);
+    gtie = r.partial && exp_det(xg / T - m) / zf == r.vf;
+  }
+  st.m = m; st.zf = zf; st.totf = totf; st.mass = r.tot;
+  st.kmax = (int32_t)__float_as_uint(r.vf);
+  st.klo = (int32_t)r.idcut;
+  st.glo = 1; st.ghi = 0;
+  st.rstar = r.partial ? 1 : 0;
+  st.gcount = r.partial ? 2 : 0;
+  st.ntbl = (int32_t)__float_as_uint(xcut);
+  st.argmax = -1;
+  st.flags = (gtie ? (uint32_t)kRowGatherTie : 0u) | (bad ? (uint32_t)kRowNoMass : 0u) |
+             (nonfinite ? (uint32_t)kRowNonfinite : 0u);
+  return st;
+}
+
 constexpr int kThrCount = 2 * TH_NT;  // lists up to here are sorted by counting
 struct ThrResLds {
   uint64_t e[kThrList];  // the list; the refinement's masses
   uint64_t t[kThrCount];  // a list of up to kThrCount entries, sorted
   uint32_t cnt[TH_NB], low[TH_NB];
   uint64_t s64[TH_NW];
+  ThrWalkLds w;
   uint32_t first, idcut;
-  uint64_t sum, base;
+  uint64_t base;
   uint32_t nbase, bin;
 };
 static_assert(kThrList >= kThrCount && kThrList >= TH_NB, "the refinement's masses use the list's space");
@@ -634,11 +797,14 @@ __global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
   const bool use_k = c->use_k != 0, use_p = c->use_p != 0;
   const uint64_t above = wave_sum_u64(lane < a.nlight ? c->pmass[lane] : 0ull);
   const uint64_t nabove = wave_sum_u32(lane < a.nlight ? c->pcnt[lane] : 0u);
-  // kept = p > vf, or p == vf and id <= idcut
-  float vf = -1.0f;
-  uint32_t idcut = 0xFFFFFFFFu;
-  bool partial = false;
-  uint64_t tot = above;
+  const int64_t gid = thr_gid(a, row);
+  const float xg = gid >= 0 && gid < a.V ? thr_f(x[gid]) : 0.0f;
+  ThrEnd r;
+  float& vf = r.vf;
+  uint32_t& idcut = r.idcut;
+  bool& partial = r.partial;
+  uint64_t& tot = r.tot;
+  tot = above;
   if (n > (uint32_t)kThrList) {  // uniform
     float kth = 0.0f;
     uint32_t v, gc;
@@ -703,116 +869,202 @@ __global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
     }
   } else if (use_k || use_p) {
     const uint64_t* const list = reinterpret_cast<const uint64_t*>(c + 1);
-    const uint64_t* e = L.e;
-    if (n <= (uint32_t)kThrCount) {  // sort by counting the smaller entries
-      const uint64_t k0 = (uint32_t)tid < n ? list[tid] : ~0ull;
-      const uint64_t k1 = (uint32_t)tid + TH_NT < n ? list[tid + TH_NT] : ~0ull;
-      L.e[tid] = k0;
-      L.e[tid + TH_NT] = k1;
-      __syncthreads();
-      if ((uint32_t)tid < n) {
-        uint32_t r0 = 0, r1 = 0;
-        // entries past n are ~0: never smaller (kThrCount is a multiple of 16)
-        for (uint32_t i = 0; i < n; i += 16) {
-          uint64_t v[16];
-#pragma unroll
-          for (int u = 0; u < 16; ++u) v[u] = L.e[i + u];
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            r0 += v[u] < k0 ? 1u : 0u;
-            r1 += v[u] < k1 ? 1u : 0u;
-          }
-        }
-        L.t[r0] = k0;
-        if ((uint32_t)tid + TH_NT < n) L.t[r1] = k1;
-      }
-      __syncthreads();
-      e = L.t;
-    } else {
-      uint32_t S = TH_NT;
-      while (S < n) S <<= 1;
-      for (uint32_t i = tid; i < S; i += TH_NT) L.e[i] = i < n ? list[i] : ~0ull;
-      __syncthreads();
-      for (uint32_t size = 2; size <= S; size <<= 1)
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-          for (uint32_t i = tid; i < S; i += TH_NT) {
-            const uint32_t j = i ^ stride;
-            if (j > i) {
-              const bool up = (i & size) == 0;
-              const uint64_t ai = L.e[i], aj = L.e[j];
-              if ((ai > aj) == up) { L.e[i] = aj; L.e[j] = ai; }
-            }
-          }
-          __syncthreads();
-        }
-    }
-    auto pof = [&](uint32_t i) { return __uint_as_float(~(uint32_t)(e[i] >> 32)); };
-    // the k-th largest p (0: not among the positive ones, nothing is zeroed)
-    float kth = 0.0f;
-    if (use_k && (uint64_t)a.top_k > nabove && (uint64_t)a.top_k - nabove <= n)
-      kth = pof((uint32_t)((uint64_t)a.top_k - nabove) - 1u);
-    if (tid == 0) { L.first = n; L.sum = 0ull; }
-    // entries PER * tid ..: their masses, then the first that fails
-    const uint32_t per = (n + TH_NT - 1) / TH_NT;
-    const uint32_t i0 = min(n, (uint32_t)tid * per), i1 = min(n, i0 + per);
-    uint64_t s = 0;
-    for (uint32_t i = i0; i < i1; ++i) s += fixed62(pof(i));
-    const uint64_t ex = above + thr_excl_u64(s, L.s64);
-    uint64_t run = ex;
-    uint32_t mine = n;
-    uint64_t kept = 0;
-    for (uint32_t i = i0; i < i1; ++i) {
-      const float p = pof(i);
-      const uint64_t nr = run + fixed62(p);
-      bool keep = !(p < kth);
-      if (use_p) keep = keep && (((rn32_u64(nr) - p) < tp) || (nabove + i == 0));
-      if (!keep) { mine = i; break; }
-      run = nr;
-    }
-    kept = run - ex;
+    uint32_t S = kThrCount;
+    while (S < n) S <<= 1;
+    for (uint32_t i = tid; i < S; i += TH_NT) L.e[i] = i < n ? list[i] : ~0ull;
     __syncthreads();
-    if (mine < n) atomicMin(&L.first, mine);
-    __syncthreads();
-    const uint32_t f = L.first;  // entries [0, f) are kept
-    if (i0 < f) atomicAdd((unsigned long long*)&L.sum, (unsigned long long)kept);
-    __syncthreads();
-    tot = above + L.sum;
-    if (f == 0) {
-      vf = __uint_as_float(__float_as_uint(c->phi) + 1u);  // everything above the region
-    } else {
-      vf = pof(f - 1);
-      partial = f < n && pof(f) == vf && !(vf < kth);
-      if (partial) idcut = (uint32_t)e[f - 1];
-    }
+    r = thr_walk<TH_NT>(a, thr_sort<TH_NT, kThrCount>(L.e, L.t, n), n, use_k, use_p, above, nabove, c->phi,
+                        L.w, L.s64);
   }
   const bool nonfinite = __ballot(lane < a.nlight && c->pnf[lane < a.nlight ? lane : 0] != 0) != 0;
-  if (tid != 0) return;
-  const float totf = fmaxf(rn32_u64(tot), 1e-12f);
-  const bool bad = !(zf > 0.0f);  // no finite maximum: every probability is 0 / 0
-  ThrRow r;
-  r.m = m; r.zf = zf; r.totf = totf; r.vf = vf; r.idcut = idcut;
-  r.xcut = c->xcut;
-  RowStat st = {};
-  float pg = 0.0f;
-  bool gtie = false;
-  const int64_t gid = thr_gid(a, row);
-  if (gid >= 0 && gid < a.V) {
-    const float xg = thr_f(x[gid]);
-    pg = bad ? __builtin_nanf("") : thr_prob(r, xg, (uint32_t)gid, T);
-    gtie = partial && exp_det(xg / T - m) / zf == vf;
+  if (tid == 0) a.stats[row] = thr_record(r, m, zf, c->xcut, gid, a.V, xg, T, nonfinite);
+}
+
+// ---------------------------------------------------------------- short rows
+// Rows of at most kThrSmall elements: the same in one launch, a workgroup per row that
+// holds the row in registers (TS_PER elements a thread: 256 threads for rows of up to
+// 2,048, 512 up to 4,096, 1,024 above, so that short rows share a CU) and the whole
+// region in LDS (no refinement). With `out`, also the to_probs row. Bound by the
+// latency of its chain of block reductions. to_probs of 64 fp32 rows of 4,096: 15 us
+// against 69 us for a bitonic sort of the row in LDS, of 256 of 8,192 20 against 131 us,
+// of 20,000 of 64 143 against 1,141 us.
+constexpr int TS_PER = 8;
+template <int NT>
+struct ThrSmallLds {
+  uint64_t e[TS_PER * NT];  // the region's list
+  union {
+    struct {
+      uint64_t mass[TH_NB];
+      uint32_t cnt[TH_NB];
+    } h;
+    uint64_t t[NT];
+  };
+  uint64_t s64[NT / kWave], t64[NT / kWave];
+  uint32_t u32[NT / kWave];
+  float mx[NT / kWave], mn[NT / kWave];
+  ThrWalkLds w;
+  uint32_t n;
+  int32_t b0, b1, bk, nf;
+};
+
+template <int NT, int DIV, bool CNT>
+__device__ __forceinline__ void thr_small_hist(const ThrArgs& a, ThrSmallLds<NT>& L,
+                                               const float (&x)[TS_PER], float m, float scale,
+                                               uint64_t& zlo, uint32_t& zhi) {
+  const float T = a.T, rT = 1.0f / a.T;
+#pragma unroll
+  for (int u = 0; u < TS_PER; ++u) {
+    if (u * NT >= a.V) break;  // uniform
+    const bool ok = u * NT + (int)threadIdx.x < a.V;
+    thr_hist_one<DIV, CNT>(x[u], ok, T, rT, m, scale, L.h.mass, L.h.cnt, zlo, zhi);
   }
-  st.m = m; st.zf = zf; st.totf = totf; st.mass = tot;
-  st.pgather = pg;
-  st.kmax = (int32_t)__float_as_uint(vf);
-  st.klo = (int32_t)idcut;
-  st.glo = 1; st.ghi = 0;
-  st.rstar = partial ? 1 : 0;
-  st.gcount = partial ? 2 : 0;
-  st.ntbl = (int32_t)__float_as_uint(r.xcut);
-  st.argmax = -1;
-  st.flags = (gtie ? (uint32_t)kRowGatherTie : 0u) | (bad ? (uint32_t)kRowNoMass : 0u) |
-             (nonfinite ? (uint32_t)kRowNonfinite : 0u);
-  a.stats[row] = st;
+}
+
+template <class E, int NT>
+__global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, int64_t ld_out) {
+  constexpr int NW = NT / kWave;
+  constexpr int BPT = TH_NB / NT;  // steps per thread
+  __shared__ ThrSmallLds<NT> L;
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  const E* const xr = thr_row<E>(a, row);
+  const int V = (int)a.V;
+  const float T = a.T;
+  const int64_t gid = thr_gid(a, row);
+  float xg = 0.0f;
+  if (tid == 0) {
+    if (row < a.nzero) a.zero[row] = 0u;
+    if (gid >= 0 && gid < V) xg = thr_f(xr[gid]);
+    L.n = 0u;
+    L.b0 = L.b1 = L.bk = TH_NB - 1;
+    L.nf = 0;
+  }
+#pragma unroll
+  for (int i = 0; i < BPT; ++i) {
+    L.h.mass[tid + i * NT] = 0ull;
+    L.h.cnt[tid + i * NT] = 0u;
+  }
+  float x[TS_PER];
+  float mx = -INFINITY, mn = INFINITY;
+  bool nf = false;
+#pragma unroll
+  for (int u = 0; u < TS_PER; ++u) {
+    const int i = u * NT + tid;
+    x[u] = i < V ? thr_f(xr[i]) : -INFINITY;
+  }
+#pragma unroll
+  for (int u = 0; u < TS_PER; ++u) {
+    if (sizeof(E) == 2) nf |= (int32_t)__float_as_uint(x[u]) >= 0x7F800000;
+    mx = fmaxf(mx, x[u]);
+    mn = x[u] > -INFINITY ? fminf(mn, x[u]) : mn;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+    mn = fminf(mn, __shfl_xor(mn, o, kWave));
+  }
+  if (lane == 0) { L.mx[wv] = mx; L.mn[wv] = mn; }
+  const uint64_t nfw = __ballot(nf);
+  __syncthreads();
+  if (lane == 0 && nfw) atomicOr(&L.nf, 1);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) { mx = fmaxf(mx, L.mx[w]); mn = fminf(mn, L.mn[w]); }
+  const float m = mx / T;
+  const float scale = thr_scale(m, mn, T);
+  const ThrDiv div = thr_div_kind(T, mx);
+  uint64_t zlo = 0;
+  uint32_t zhi = 0;
+  if (a.use_k) {
+    if (div == kDivOne) thr_small_hist<NT, kDivOne, true>(a, L, x, m, scale, zlo, zhi);
+    else if (div == kDivFma) thr_small_hist<NT, kDivFma, true>(a, L, x, m, scale, zlo, zhi);
+    else thr_small_hist<NT, kDivIeee, true>(a, L, x, m, scale, zlo, zhi);
+  } else {
+    if (div == kDivOne) thr_small_hist<NT, kDivOne, false>(a, L, x, m, scale, zlo, zhi);
+    else if (div == kDivFma) thr_small_hist<NT, kDivFma, false>(a, L, x, m, scale, zlo, zhi);
+    else thr_small_hist<NT, kDivIeee, false>(a, L, x, m, scale, zlo, zhi);
+  }
+  U128 z = wave_sum_u128(U128{zlo, (uint64_t)zhi});
+  if (lane == 0) { L.s64[wv] = z.lo; L.t64[wv] = z.hi; }
+  __syncthreads();  // and the histogram is complete
+  z = U128{0, 0};
+  for (int w = 0; w < NW; ++w) z = u128_add(z, U128{L.s64[w], L.t64[w]});
+  const float zf = rn32_u128(z);
+  const bool bad = !(zf > 0.0f);
+  ThrEnd r;
+  ThrCut c;
+  {
+    uint64_t ms[BPT], ct[BPT], sm = 0, sc = 0;
+#pragma unroll
+    for (int i = 0; i < BPT; ++i) {
+      ms[i] = L.h.mass[tid * BPT + i];
+      ct[i] = L.h.cnt[tid * BPT + i];
+      sm += ms[i];
+      sc += ct[i];
+    }
+    uint64_t rm = thr_excl_u64<NW>(sm, L.s64);
+    uint64_t rc = a.use_k ? thr_excl_u64<NW>(sc, L.s64) : 0ull;
+    const double zu = ((double)z.hi * 0x1p64 + (double)z.lo) * 0x1p-18;
+#pragma unroll
+    for (int i = 0; i < BPT; ++i) {
+      thr_mark(a, tid * BPT + i, rm, rm + ms[i], rc, rc + ct[i], zu, &L.b0, &L.b1, &L.bk);
+      rm += ms[i];
+      rc += ct[i];
+    }
+    __syncthreads();
+    c = thr_cut(a, m, zf, scale, L.b0, L.b1, L.bk);
+  }
+  // p of this thread's elements; what lies above the region, and the region's list
+  float p[TS_PER];
+  uint64_t mass = 0;
+  uint32_t cnt = 0;
+#pragma unroll
+  for (int u = 0; u < TS_PER; ++u) {
+    p[u] = 0.0f;
+    if (u * NT >= V) continue;  // uniform
+    const int i = u * NT + tid;
+    const bool take = i < V && x[u] >= c.xcut;
+    if (__ballot(take)) p[u] = take ? exp_det_sel(x[u] / T - m) / zf : 0.0f;
+    const bool above = take && p[u] > c.phi;
+    mass += above ? fixed62(p[u]) : 0ull;
+    cnt += above ? 1u : 0u;
+    const bool in = take && !above && p[u] >= c.plo;
+    const uint64_t bm = __ballot(in);
+    if (bm) {  // uniform per wave
+      uint32_t at = 0;
+      if (lane == 0) at = atomicAdd(&L.n, (uint32_t)__popcll(bm));
+      at = rdlane(at, 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+      if (in) L.e[at] = ((uint64_t)(~__float_as_uint(p[u])) << 32) | (uint32_t)i;
+    }
+  }
+  mass = wave_sum_u64(mass);
+  cnt = wave_sum_u32(cnt);
+  __syncthreads();  // the scans' words are read, the list is complete
+  if (lane == 0) { L.s64[wv] = mass; L.u32[wv] = cnt; }
+  __syncthreads();
+  uint64_t above = 0, nabove = 0;
+  for (int w = 0; w < NW; ++w) { above += L.s64[w]; nabove += L.u32[w]; }
+  const uint32_t n = L.n;
+  r.tot = above;
+  if (c.use_k || c.use_p) {  // uniform
+    uint32_t S = NT;
+    while (S < n) S <<= 1;  // at most TS_PER * NT
+    for (uint32_t i = n + tid; i < S; i += NT) L.e[i] = ~0ull;
+    __syncthreads();
+    r = thr_walk<NT>(a, thr_sort<NT, NT>(L.e, L.t, n), n, c.use_k, c.use_p, above, nabove, c.phi,
+                        L.w, L.s64);
+  }
+  if (tid == 0 && a.stats)
+    a.stats[row] = thr_record(r, m, zf, c.xcut, gid, V, xg, T, L.nf != 0);
+  if (!out) return;
+  const float totf = fmaxf(rn32_u64(r.tot), 1e-12f);
+  float* const o = out + row * ld_out;
+#pragma unroll
+  for (int u = 0; u < TS_PER; ++u) {
+    const int i = u * NT + tid;
+    const bool kept = p[u] > r.vf || (p[u] == r.vf && (uint32_t)i <= r.idcut);
+    if (i < V) o[i] = bad ? __builtin_nanf("") : kept ? p[u] / totf : 0.0f;
+  }
 }
 
 // ---------------------------------------------------------------- to_probs output
@@ -1113,7 +1365,28 @@ static hipError_t thr_stats(const ThrArgs& a, int64_t rows, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <class E>
+static hipError_t thr_small(const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+                            hipStream_t s) {
+  const dim3 grid((unsigned)rows);
+  if (a.V <= TS_PER * 256)
+    hipLaunchKernelGGL((thr_small_kernel<E, 256>), grid, dim3(256), 0, s, a, out, ld_out);
+  else if (a.V <= TS_PER * 512)
+    hipLaunchKernelGGL((thr_small_kernel<E, 512>), grid, dim3(512), 0, s, a, out, ld_out);
+  else
+    hipLaunchKernelGGL((thr_small_kernel<E, 1024>), grid, dim3(1024), 0, s, a, out, ld_out);
+  return hipGetLastError();
+}
+
+hipError_t launch_thr_small(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+                            hipStream_t s) {
+  if (a.V > kThrSmall || (!a.stats && !out)) return hipErrorInvalidValue;
+  return dtype == SDX_F32 ? thr_small<float>(a, rows, out, ld_out, s)
+                          : thr_small<uint16_t>(a, rows, out, ld_out, s);
+}
+
 hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s) {
+  if (a.V <= kThrSmall) return launch_thr_small(dtype, a, rows, nullptr, 0, s);
   if (!a.scratch || a.scratch_bytes < kThrScratchMin || a.scratch_stride < a.scratch_bytes || !a.stats || a.V > kF32MaxVocab)
     return hipErrorInvalidValue;
   a.nparts = thr_parts(rows, a.V);

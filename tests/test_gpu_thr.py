@@ -49,6 +49,19 @@ def _same(got, ref):
     assert bad.size == 0, f"{len(bad)} elements differ, first at {bad[0]}"
 
 
+# one workgroup per row: a few ids, and both sides of the workgroup sizes
+@pytest.mark.parametrize("V", [9, 1000, 2048, 2049, 4096, 4097, 8192])
+@pytest.mark.parametrize("T,tp,tk", TRANSFORMS)
+def test_to_probs_short_rows(V, T, tp, tk):
+    x = _rows(V, V)
+    got = S.to_probs(torch.tensor(x, device=DEV), T, tp, tk).cpu().numpy()
+    _same(got, O.to_probs(x, T, tp, tk))
+    if V % 8 == 0 and T > 1e-2:
+        h = _rows(V, V, np.float16)
+        got = S.to_probs(torch.tensor(h, device=DEV), T, tp, tk).cpu().numpy()
+        _same(got, O.to_probs(h.astype(np.float32), T, tp, tk))
+
+
 # 8193: the shortest row, one part; 12291: three parts' worth of 4,096 and 3 ids more;
 # 33000: several parts
 @pytest.mark.parametrize("V", [8193, 12291, 33000])
