@@ -118,18 +118,37 @@ def dtype_code(t):
 def require_gpu(*tensors):
     """Every tensor must live on the ROCm device; there is no CPU path."""
     for t in tensors:
-        if t is not None and (not isinstance(t, torch.Tensor) or t.device.type != "cuda"):
+        if t is not None and (not isinstance(t, torch.Tensor) or not t.is_cuda):
             raise RuntimeError(
                 "specdec (MI355X build) runs on ROCm device tensors only; got "
                 f"{getattr(t, 'device', type(t))}")
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """The device address as an int (what c_void_p arguments take fastest)."""
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(device):
+    """The handle of the device's current stream, without building a Stream object
+    where torch offers that."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def stream_of(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return _stream(t.device)
+
+
+def as_dtype(t, dtype):
+    """t as a contiguous tensor of `dtype` (t itself where it is one)."""
+    if t.dtype is dtype and t.is_contiguous():
+        return t
+    return t.to(dtype).contiguous()
 
 
 def workspace(nbytes, device, prepare=True):
@@ -157,11 +176,11 @@ def cached_workspace(nbytes, device, kind):
     workspaces keep their header (magic word and zeroed counters) at fixed
     offsets that other entry points would overwrite. Under graph capture a new
     workspace is allocated (from the graph's pool) and not kept."""
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     prepare = kind in _PREPARED_KINDS
     if torch.cuda.is_current_stream_capturing():
         return workspace(nbytes, dev, prepare)
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream, kind)
+    key = (dev.index, _stream(dev), kind)
     ws = _WS_CACHE.get(key)
     if ws is None or ws.numel() < int(nbytes):
         ws = workspace(nbytes, dev, prepare)

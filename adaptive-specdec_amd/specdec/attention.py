@@ -52,9 +52,9 @@ def verify_attention_paged(q, cu_q, k_pool, v_pool, block_table, kv_len, max_q, 
     if not (k_pool.is_contiguous() and v_pool.is_contiguous()):
         raise ValueError("verify_attention_paged: pools must be contiguous")
     q = q.contiguous()
-    cu = cu_q.to(torch.int64).contiguous()
-    kl = kv_len.to(torch.int64).contiguous()
-    bt = block_table.to(torch.int32).contiguous()
+    cu = _lib.as_dtype(cu_q, torch.int64)
+    kl = _lib.as_dtype(kv_len, torch.int64)
+    bt = _lib.as_dtype(block_table, torch.int32)
     if out is None:
         out = torch.empty_like(q)
     if workspace is None:

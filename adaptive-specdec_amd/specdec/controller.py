@@ -76,7 +76,7 @@ class DeviceController:
         observed draft/target forward-time ratio ([1] fp32 device tensor), or None
         to keep c. Updates the state and `k` (and `cu_k`) in place on the device."""
         _lib.require_gpu(n_acc)
-        n_acc = n_acc.to(torch.int64).contiguous()
+        n_acc = _lib.as_dtype(n_acc, torch.int64)
         ku = (self.k if k_used is None else k_used.to(torch.int64)).contiguous()
         k_next = self._k_next
         rc = _lib.lib().sdx_controller_update(

@@ -223,7 +223,7 @@ class RaggedCache(_HFCache):
         mutation, which re-reads it) `advance` runs on the device, max_len is an
         upper bound and `attn_mask` is built from the device lengths."""
         _lib.require_gpu(n)
-        n = n.to(torch.int64).contiguous()
+        n = _lib.as_dtype(n, torch.int64)
         rc = _lib.lib().sdx_kv_rollback(_lib.ptr(self.lengths), self.batch_size, _lib.ptr(n),
                                         _lib.ptr(self.error), _lib.stream_of(n))
         _lib.check(rc, "RaggedCache.rollback_device")
@@ -299,7 +299,7 @@ class PagedKVCache:
         """lengths -= n (device [B] int64); all-or-nothing, `error` set if any row
         would go negative (`kvcache.py:174-190`)."""
         _lib.require_gpu(n)
-        n = n.to(torch.int64).contiguous()
+        n = _lib.as_dtype(n, torch.int64)
         rc = _lib.lib().sdx_kv_rollback(_lib.ptr(self.lengths), self.batch_size, _lib.ptr(n),
                                         _lib.ptr(self.error), _lib.stream_of(n))
         _lib.check(rc, "PagedKVCache.rollback")

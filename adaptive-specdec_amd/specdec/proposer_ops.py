@@ -40,8 +40,8 @@ def drafting_slot_mapping(block_table, positions, block_size, max_model_len,
     otherwise slot = block_table[r, pos // bs] * bs + pos % bs
     (`proposer.py:299-314`). Returns (clamped_positions, slot_mapping), int64."""
     _lib.require_gpu(block_table, positions)
-    bt = block_table.to(torch.int32).contiguous()
-    pos = positions.to(torch.int64).contiguous()
+    bt = _lib.as_dtype(block_table, torch.int32)
+    pos = _lib.as_dtype(positions, torch.int64)
     rows = pos.numel()
     clamped = torch.empty(rows, dtype=torch.int64, device=pos.device)
     slots = torch.empty(rows, dtype=torch.int64, device=pos.device)

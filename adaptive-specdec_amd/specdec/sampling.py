@@ -185,9 +185,9 @@ def rejection_sample(target_logits, draft_logits, draft_ids, u_accept, u_final, 
         dl = None if dl is None else dl.float()
     tl = tl.contiguous()
     dl = None if dl is None else dl.contiguous()
-    ids = draft_ids.to(torch.int64).contiguous()
-    ua = u_accept.to(torch.float32).contiguous()
-    uf = u_final.to(torch.float32).contiguous()
+    ids = _lib.as_dtype(draft_ids, torch.int64)
+    ua = _lib.as_dtype(u_accept, torch.float32)
+    uf = _lib.as_dtype(u_final, torch.float32)
     act = None if active is None else active.to(torch.uint8).contiguous()
     if out is None:
         n_acc = torch.empty(B, dtype=torch.int64, device=dev)
@@ -235,7 +235,7 @@ def rejection_sample_ragged(target_logits, draft_logits, draft_ids, u_accept, u_
     B = cu_k.numel() - 1
     if NT < B:
         raise ValueError(f"target_logits has {NT} rows, fewer than the {B} batch rows")
-    cu = cu_k.to(torch.int64).contiguous()
+    cu = _lib.as_dtype(cu_k, torch.int64)
     if k_max is None:
         k_max = int((cu[1:] - cu[:-1]).max().item()) if B > 0 else 1
     k_max = max(int(k_max), 1)
@@ -253,9 +253,9 @@ def rejection_sample_ragged(target_logits, draft_logits, draft_ids, u_accept, u_
     if greedy:
         dl = tl  # not read; the C ABI wants a pointer of the right type
     dl = dl.contiguous()
-    ids = draft_ids.to(torch.int64).contiguous()
-    ua = u_accept.to(torch.float32).contiguous()
-    uf = u_final.to(torch.float32).contiguous()
+    ids = _lib.as_dtype(draft_ids, torch.int64)
+    ua = _lib.as_dtype(u_accept, torch.float32)
+    uf = _lib.as_dtype(u_final, torch.float32)
     if ids.numel() != NT - B or ua.numel() != NT - B or uf.numel() != B:
         raise ValueError("draft_ids / u_accept must hold sum(k_b) entries and u_final B")
     act = None if active is None else active.to(torch.uint8).contiguous()
@@ -427,7 +427,7 @@ def draft_step(logits, u, temperature=1.0, top_p=1.0, top_k=0, conf=None, tau=No
         x, qx, stop = out
     if B == 0:
         return x, qx, stop
-    uu = None if T == 0.0 else u.to(torch.float32).contiguous()
+    uu = None if T == 0.0 else _lib.as_dtype(u, torch.float32)
     if conf is not None and (conf.dtype != torch.float32 or not conf.is_contiguous()):
         raise ValueError("conf must be a contiguous fp32 tensor (updated in place)")
     need = L.sdx_draft_step_workspace(B, V, dt)
