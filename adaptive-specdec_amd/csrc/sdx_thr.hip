@@ -263,11 +263,14 @@ __device__ __forceinline__ ThrDiv thr_div_kind(float T, float xmax) {
   return T >= 0x1p-20f && T <= 0x1p20f && a <= 0x1p100f && (a >= 0x1p-90f || a == 0.0f) ? kDivFma
                                                                                        : kDivIeee;
 }
-// Steps of m - s per unit, 2^e with e >= 5: the row's range (at most 32) over at most
-// TH_NB steps.
-__device__ __forceinline__ float thr_scale(float m, float xmn, float T) {
-  const float range = fminf(m - xmn / T, 32.0f);  // NaN (no finite logit): 32
-  float scale = TH_NB / 32.0f;
+// Steps of m - s per unit, 2^e: the row's range over at most TH_NB steps. The nucleus
+// ends within 32 of the maximum (below lies less than 2^18 e^-32 of the mass; a top_p
+// that near 1 takes the last step), the k-th largest anywhere p is above 0.
+__device__ __forceinline__ float thr_scale(float m, float xmn, float T, bool use_k) {
+  const float most = use_k ? 104.0f : 32.0f;
+  const float range = fminf(m - xmn / T, most);  // NaN (no finite logit): the most
+  float scale = use_k ? 8.0f : 32.0f;
+  static_assert(104 * 8 <= TH_NB - 2 && 32 * 32 <= TH_NB, "the widest range fits the steps");
   while (scale < 0x1p20f && range * (2.0f * scale) <= (float)(TH_NB - 2)) scale *= 2.0f;
   return scale;
 }
@@ -384,7 +387,7 @@ __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
   }
   const float T = a.T;
   const float m = xmx / T;  // the division is monotone: the maximum of fl32(x / T)
-  const float scale = thr_scale(m, xmn, T);
+  const float scale = thr_scale(m, xmn, T, a.use_k);
   const ThrDiv div = thr_div_kind(T, xmx);
   __syncthreads();
   uint64_t zlo = 0;
@@ -970,7 +973,7 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
 #pragma unroll
   for (int w = 0; w < NW; ++w) { mx = fmaxf(mx, L.mx[w]); mn = fminf(mn, L.mn[w]); }
   const float m = mx / T;
-  const float scale = thr_scale(m, mn, T);
+  const float scale = thr_scale(m, mn, T, a.use_k);
   const ThrDiv div = thr_div_kind(T, mx);
   uint64_t zlo = 0;
   uint32_t zhi = 0;
