@@ -33,12 +33,12 @@
 // waves. Splitting a row over workgroups keeps the chip full from a few rows on.
 // Measured on fp32 rows of 151,936 (one workgroup of 1024 threads per row before, with
 // seven IEEE divisions per element and dense probabilities for the draw): verify of 8
-// batch rows at k = 4 (72 rows, top-k 50) 285 -> 63 us (kernels 12 + 27 + 11 + 6 and
-// the draw 11), to_probs of 256 rows 378 -> 198 us (52 + 56 + 31 + 9 + 53: the first
+// batch rows at k = 4 (72 rows, top-k 50) 285 -> 61 us (kernels 11 + 26 + 11 + 6 and
+// the draw 11), to_probs of 256 rows 378 -> 197 us (52 + 56 + 31 + 8 + 53: the first
 // pass also pays for the write-back of the call before, the last moves 5.9 TB/s). On
 // fp16 rows (one workgroup of 1024 threads and a histogram of 36,864 values per row
-// before): verify of 16 batch rows at k = 4, V = 131,072 144 -> 86 us, of 64 at V =
-// 4,096 100 -> 38 us, of one at 1,024 42 -> 31 us; to_probs of 64 x 131,072 132 -> 65 us.
+// before): verify of 16 batch rows at k = 4, V = 131,072 144 -> 79 us (10 + 31 + 16 + 8
+// and the draw 17), of 64 at V = 32,000 161 -> 90 us; to_probs of 64 x 131,072 132 -> 65 us.
 // The compare passes keep the evaluation in one place of their code (a loop over a
 // queue in LDS): unrolled into every element's place, 16 to 64 copies, the collect
 // pass of the fp16 verify took 20 us instead of 17 and its draw 22 instead of 20. The
@@ -665,10 +665,15 @@ __device__ __forceinline__ ThrEnd thr_walk(const ThrArgs& a, const uint64_t* e, 
     run = nr;
   }
   __syncthreads();
-  if (mine < n) atomicMin(&L.first, mine);
+  // one LDS atomic per wave (a wave's lanes at one address go one after the other)
+  const uint64_t fail = __ballot(mine < n);
+  if (fail && (int)(tid & (kWave - 1)) == __ffsll((unsigned long long)fail) - 1)
+    atomicMin(&L.first, mine);  // the wave's first: entries go up with the thread
   __syncthreads();
   const uint32_t f = L.first;  // entries [0, f) are kept
-  if (i0 < f) atomicAdd((unsigned long long*)&L.sum, (unsigned long long)(run - ex));
+  const uint64_t part = wave_sum_u64(i0 < f ? run - ex : 0ull);
+  if ((tid & (kWave - 1)) == 0 && part)
+    atomicAdd((unsigned long long*)&L.sum, (unsigned long long)part);
   __syncthreads();
   r.tot = above + L.sum;
   if (f == 0) {
@@ -948,13 +953,13 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
     L.h.cnt[tid + i * NT] = 0u;
   }
   float x[TS_PER];
+  E raw[TS_PER];  // all loads first
   float mx = -INFINITY, mn = INFINITY;
   bool nf = false;
 #pragma unroll
-  for (int u = 0; u < TS_PER; ++u) {
-    const int i = u * NT + tid;
-    x[u] = i < V ? thr_f(xr[i]) : -INFINITY;
-  }
+  for (int u = 0; u < TS_PER; ++u) raw[u] = xr[min(u * NT + tid, V - 1)];
+#pragma unroll
+  for (int u = 0; u < TS_PER; ++u) x[u] = u * NT + tid < V ? thr_f(raw[u]) : -INFINITY;
 #pragma unroll
   for (int u = 0; u < TS_PER; ++u) {
     if (sizeof(E) == 2) nf |= (int32_t)__float_as_uint(x[u]) >= 0x7F800000;
@@ -1228,12 +1233,14 @@ __global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
   if (rec < a.nrec) {  // uniform per wave
     const int64_t r0 = (int64_t)rec * kThrRec;
     constexpr int RN = kThrRec / kWave;
+    // codes first, unconditionally: an element's bounds check and conversion between
+    // the loads made each wait for the one before (fp16: 5 us for the 16)
+    E raw[RN];
+#pragma unroll
+    for (int u = 0; u < RN; ++u) raw[u] = xp[min(r0 + u * kWave + lane, V - 1)];
     float x[RN];
 #pragma unroll
-    for (int u = 0; u < RN; ++u) {
-      const int64_t i = r0 + u * kWave + lane;
-      x[u] = i < V ? thr_f(xp[i]) : -INFINITY;
-    }
+    for (int u = 0; u < RN; ++u) x[u] = thr_f(raw[u]);
     auto add = [&](float xv, uint32_t id, bool ok) {
       const float qx = hasq && ok ? thr_f(xq[id]) : 0.0f;
       const float p = ok ? thr_prob(rp, xv, id, T) : 0.0f;
@@ -1297,14 +1304,17 @@ __global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
     const int64_t i0 = pick * kThrRec + (int64_t)tid * TH_RV;
     uint64_t w[TH_RV], sum = 0;
     float pv[TH_RV];
+    E pc[TH_RV], qc[TH_RV];
+#pragma unroll
+    for (int u = 0; u < TH_RV; ++u) {  // all loads first
+      pc[u] = xp[min(i0 + u, V - 1)];
+      qc[u] = xq[min(i0 + u, V - 1)];
+    }
 #pragma unroll
     for (int u = 0; u < TH_RV; ++u) {
       const int64_t i = i0 + u;
-      float p = 0.0f, q = 0.0f;
-      if (i < V) {
-        p = thr_prob(rp, thr_f(xp[i]), (uint32_t)i, T);
-        if (use_r) q = thr_prob(rq, thr_f(xq[i]), (uint32_t)i, T);
-      }
+      const float p = i < V ? thr_prob(rp, thr_f(pc[u]), (uint32_t)i, T) : 0.0f;
+      const float q = use_r && i < V ? thr_prob(rq, thr_f(qc[u]), (uint32_t)i, T) : 0.0f;
       pv[u] = p;
       w[u] = fixed62(use_r ? fmaxf(p - q, 0.0f) : p);
       sum += w[u];
