@@ -147,7 +147,7 @@ int sdx_workspace_init(void* workspace, size_t bytes, sdx_stream_t stream) {
 size_t sdx_to_probs_workspace(int64_t rows, int64_t vocab, int dtype) {
   Carve c{nullptr};
   sdx::RowStat* st; float* tb; float* dn; sdx::SampleJob* jb; sdx::ChunkRec* rc; uint32_t* ct;
-  // fp32 rows are written straight to the output: no dense scratch
+  // the threshold statistics' scratch lies in the output rows: none here
   transform_ws(c, rows, vocab, dtype == SDX_F32 ? SDX_BF16 : dtype, 0, &st, &tb, &dn, &jb, &rc, &ct);
   int64_t chunk;
   int nchunk;
@@ -564,7 +564,7 @@ static int verify_impl(const void* target_logits, const void* draft_logits, int 
     return fail(SDX_EINVAL,
                 "sdx_verify: 16-bit logits must be 16-byte aligned with vocab %% 8 == 0");
   if (thr) {
-    // fp32: the rows' dense space serves as scratch (the draw evaluates what it needs)
+    // fp32: `dn` is the scratch; fp16: appended to the workspace
     sdx::ThrArgs a = thr_args(target_logits, draft_logits, ntgt, ndrf, vocab, vocab, temperature,
                               top_p, top_k, sw);
     a.ids = draft_ids; a.k = k; a.tgt_idx = tgt_idx;
@@ -742,7 +742,7 @@ int sdx_verify_greedy(const void* target_logits, int dtype, int64_t batch, int32
 }
 
 // ------------------------------------------------------------------ draft step
-// workspace: header, the row statistics / tables (dense probabilities for fp32),
+// workspace: header, the row statistics / tables (threshold scratch for fp32),
 // the draws' jobs, records and counters, the split parts of bf16 rows
 static size_t draft_ws_bytes(int64_t batch, int64_t vocab, int dtype) {
   Carve c{nullptr};
@@ -821,7 +821,6 @@ int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, 
     d.qx = (float*)jobs;  // one value per row, for the epilogue
     if (int r = hip_status(sdx::launch_thr_draw(dtype, d, batch, s), "thr_draw")) return r;
     e.probs = d.qx;
-    e.ldp = 0;
     return hip_status(sdx::launch_draft_epilogue(e, s), "draft_epilogue");
   }
   sdx::RowStatArgs a = {};

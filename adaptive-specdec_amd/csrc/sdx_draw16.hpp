@@ -59,9 +59,7 @@ __device__ inline uint64_t block_excl_u64(uint64_t v, uint64_t* s, uint64_t* tot
 // is both, returning the group bits.
 template <int FMT>
 struct Eval16 {
-  static constexpr bool kGroups = true;
   static constexpr int kFmt = FMT;
-  static constexpr int kLdsTbl = kTbl;
   using Raw = uint4;
   const uint16_t* base;
   int64_t ld;

@@ -36,7 +36,7 @@ __global__ void __launch_bounds__(256) draft_epilogue_kernel(DraftEpiArgs a) {
       if (a.greedy) {
         p = 1.0f;
       } else if (a.probs) {
-        p = a.ldp ? a.probs[b * a.ldp + x] : a.probs[b];
+        p = a.probs[b];
       } else {
         const uint16_t* row = a.codes + b * a.ld;
         const float* tbl = a.tables + b * kTbl;

@@ -323,8 +323,7 @@ struct DraftEpiArgs {
   bool greedy;             // temperature <= 0: the drafted token has probability 1
   const uint16_t* codes;   // 16-bit rows [B, ld]
   int64_t ld;
-  const float* probs;      // fp32 path: dense probabilities [B, ldp] (else null)
-  int64_t ldp;
+  const float* probs;      // threshold rows: q(x) of each row [B], from the draw (else null)
   const RowStat* stats;
   const float* tables;
   float T;

@@ -18,8 +18,10 @@
 // Keys below the window (logits more than ~2^28 below the maximum at
 // ordinary temperatures) carry exp_det == 0 and are checked to do so.
 //
-// This kernel serves fp16 rows; bf16 rows go through the streaming kernel
-// (sdx_rowstream.hip).
+// This kernel serves the fp16 rows that sdx_thr.hip cannot: verify and draft
+// calls whose workspace has no room for its scratch (the fixed workspace of
+// the allocation-free verify) and to_probs whose output overlaps the logits.
+// bf16 rows go through the streaming kernel (sdx_rowstream.hip).
 #include "sdx_launch.hpp"
 
 namespace sdx {

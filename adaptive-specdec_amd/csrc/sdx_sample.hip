@@ -18,8 +18,9 @@
 //                (sampling.py:85-88); target floor(u * total); the record
 //                holding it; a wave scan in id order for the first id whose
 //                prefix mass exceeds it.
-// Element probabilities come from an evaluator: codes + RowStat + table for
-// 16-bit logits, or dense fp32 probability rows (which have no groups).
+// Element probabilities come from an evaluator: codes + RowStat + table of
+// 16-bit logits (Eval16). fp32 rows, and fp16 rows where the workspace holds
+// the scratch, are drawn by thr_draw_kernel (sdx_thr.hip) instead.
 #include "sdx_draw16.hpp"
 
 #include <cstdlib>
@@ -50,16 +51,13 @@ __device__ uint64_t wave_walk(const Ev& ev, const typename Ev::Row& rp, const ty
       mp = ev.load8(rp, idx, i1, p);
       if (use_r) mq = ev.load8(rq, idx, i1, q);
     }
-    uint32_t rk_p = bp, rk_q = bq;
-    if constexpr (Ev::kGroups) {  // member ranks: wave scan of packed (p count, q count)
-      const uint32_t cnt = (uint32_t)__popc(mp) | ((uint32_t)__popc(mq) << 16);
-      const uint32_t incl = wave_incl_scan_u32(cnt, lane);
-      const uint32_t tot = rdlane(incl, kWave - 1);
-      rk_p += (incl - cnt) & 0xFFFFu;
-      rk_q += (incl - cnt) >> 16;
-      bp += tot & 0xFFFFu;
-      bq += tot >> 16;
-    }
+    // member ranks: wave scan of packed (p count, q count)
+    const uint32_t cnt = (uint32_t)__popc(mp) | ((uint32_t)__popc(mq) << 16);
+    const uint32_t cincl = wave_incl_scan_u32(cnt, lane);
+    const uint32_t ctot = rdlane(cincl, kWave - 1);
+    uint32_t rk_p = bp + ((cincl - cnt) & 0xFFFFu), rk_q = bq + ((cincl - cnt) >> 16);
+    bp += ctot & 0xFFFFu;
+    bq += ctot >> 16;
     uint64_t w[8], mine = 0;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -106,15 +104,14 @@ struct DrawArgs {
   int32_t nblk;        // blocks per job
   ChunkRec* recs;      // [jobs, nrec]
   uint32_t* counters;  // [jobs], zero on entry (cleared by the kernel before)
-  int64_t* y;          // null: records only
+  int64_t* y;
 };
 
 template <class Ev>
 __global__ void __launch_bounds__(SM_NT) draw_kernel(Ev ev, DrawArgs a) {
-  __shared__ float tbl_p[Ev::kLdsTbl];
-  __shared__ float tbl_q[Ev::kLdsTbl];
+  __shared__ float tbl_p[kTbl];
+  __shared__ float tbl_q[kTbl];
   __shared__ float lst_p[SM_NW][kDrawSub];  // per-wave lists of ids with p mass
-  __shared__ float lst_q[SM_NW][kDrawSub];
   __shared__ unsigned long long acc[SM_NW][6];  // per-wave record sums (16-bit rows)
   __shared__ SampleJob s_job;
   __shared__ uint64_t s64[SM_NW];
@@ -171,177 +168,101 @@ __global__ void __launch_bounds__(SM_NT) draw_kernel(Ev ev, DrawArgs a) {
       const int64_t nround = (x_end - x_beg + kDrawSub - 1) / kDrawSub;
       const int64_t rpr = a.rec_ids / kDrawSub;  // rounds per record
       const int64_t lane_off = (int64_t)lane * 8;
-      uint64_t p2 = 0, r0 = 0, ra = 0, rb = 0, rpm = 0;
-      uint32_t np = 0, nq = 0, ndbl = 0;
-      // one round: evaluate, compact the ids that may carry p mass into this
-      // wave's LDS list (sign bits mark group members), reduce one per lane;
-      // a round that ends a record publishes it
-      auto round = [&](const typename Ev::Raw& cp, const typename Ev::Raw& cq, int64_t ro) {
-        const int64_t s0 = x_beg + ro * kDrawSub;
-        const int64_t rec = s0 / a.rec_ids;
-        const int64_t e1 = min(a.V, (rec + 1) * a.rec_ids);
-        const int64_t cur = s0 + lane_off;
-        float p[8], q[8];
-        const uint32_t ep = ev.eval(rp, cur, e1, cp, p);
-        const uint32_t mp = ep & 0xFFu, lp = (ep >> 8) & 0xFFu;
-        uint32_t mq = 0;
-        if (hasq) {
-          mq = ev.eval(rq, cur, e1, cq, q) & 0xFFu;
-        } else {
-#pragma unroll
-          for (int t = 0; t < 8; ++t) q[t] = 0.0f;
-        }
-        np += __popc(mp);
-        nq += __popc(mq);
-        const uint32_t c = __popc(lp);
-        const uint32_t incl = wave_incl_scan_u32(c, lane);
-        const uint32_t n = rdlane(incl, kWave - 1);
-        uint32_t o = incl - c;
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-          if ((lp >> t) & 1u) {
-            lst_p[w][o] = __uint_as_float(__float_as_uint(p[t]) | (((mp >> t) & 1u) << 31));
-            lst_q[w][o] = __uint_as_float(__float_as_uint(q[t]) | (((mq >> t) & 1u) << 31));
-            ++o;
-          }
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_wave_barrier();
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        for (uint32_t i = lane; i < n; i += kWave) {
-          const uint32_t bp = __float_as_uint(lst_p[w][i]), bq = __float_as_uint(lst_q[w][i]);
-          const bool ip = (bp >> 31) != 0, iq = (bq >> 31) != 0;
-          const float pv = __uint_as_float(bp & 0x7FFFFFFFu);
-          const float qv = __uint_as_float(bq & 0x7FFFFFFFu);
-          const uint64_t wr = fixed62(fmaxf(pv - qv, 0.0f));
-          const uint64_t fp = fixed62(pv);
-          p2 += ip ? 0ull : fp;
-          r0 += (!ip && !iq) ? wr : 0ull;
-          ra += (!ip && iq) ? wr : 0ull;
-          rb += (!ip && iq) ? fp : 0ull;
-          rpm += (ip && !iq) ? wr : 0ull;
-          ndbl += (ip && iq) ? 1u : 0u;
-        }
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_wave_barrier();  // list reads done before the next round's writes
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        if ((ro + 1) % rpr == 0 || ro + 1 == nround) {
-          ChunkRec rc;
-          rc.p2 = wave_sum_u64(p2);
-          rc.r0 = wave_sum_u64(r0);
-          rc.ra = wave_sum_u64(ra);
-          rc.rb = wave_sum_u64(rb);
-          rc.rp = wave_sum_u64(rpm);
-          rc.np = wave_sum_u32(np);
-          rc.nq = wave_sum_u32(nq);
-          rc.ndbl = wave_sum_u32(ndbl);
-          rc.pad = 0;
-          rc.pad2 = 0;
-          if (lane == 0) store_rec(a.recs + j * a.nrec + rec, rc);
-          p2 = r0 = ra = rb = rpm = 0;
-          np = nq = ndbl = 0;
-        }
-      };
-      // 16-bit rows, lean: keys from packed codes, group-member counts from
+      // One round: keys from packed codes, group-member counts from
       // ballots (scalar popcounts), the ids that may carry p mass (p's kept
       // keys, ~2% under a nucleus) compacted by ballot into this wave's LDS list
       // as packed (p code, q code) and evaluated one per lane, sums
       // accumulated with LDS atomics (no per-record wave reductions).
       uint32_t np_s = 0, nq_s = 0;
-      if constexpr (Ev::kGroups) {
-        if (lane < 6) acc[w][lane] = 0ull;
+      if (lane < 6) acc[w][lane] = 0ull;
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_wave_barrier();
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      auto round16 = [&](const typename Ev::Raw& cp, const typename Ev::Raw& cq, int64_t ro) {
+        const int64_t s0 = x_beg + ro * kDrawSub;
+        const int64_t rec = s0 / a.rec_ids;
+        const int64_t e1 = min(a.V, (rec + 1) * a.rec_ids);
+        const int nvalid = (int)max<int64_t>(0, min<int64_t>(8, e1 - (s0 + lane_off)));
+        const int32_t klo_p = rp.st.klo, glo_p = rp.st.glo, ghi_p = rp.st.ghi;
+        const int32_t klo_q = hasq ? rq.st.klo : 0x7FFFFFFF;
+        const int32_t glo_q = hasq ? rq.st.glo : 1, ghi_q = hasq ? rq.st.ghi : 0;
+        const uint32_t pw[4] = {cp.x, cp.y, cp.z, cp.w};
+        const uint32_t qw[4] = {cq.x, cq.y, cq.z, cq.w};
+        uint32_t kp2[4], kq2[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          kp2[i] = keys2_of_codes2(pw[i]);
+          kq2[i] = keys2_of_codes2(qw[i]);
+        }
+        uint32_t* lst = reinterpret_cast<uint32_t*>(&lst_p[w][0]);
+        uint32_t off = 0;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const int sh = 16 * (t & 1);
+          const int32_t kp = (int32_t)((kp2[t >> 1] >> sh) & 0xFFFFu);
+          const int32_t kq = (int32_t)((kq2[t >> 1] >> sh) & 0xFFFFu);
+          const bool valid = t < nvalid;
+          const bool lv = valid && kp >= klo_p;
+          const uint64_t bl = __ballot(lv);
+          np_s += (uint32_t)__popcll(__ballot(valid && kp >= glo_p && kp <= ghi_p));
+          nq_s += (uint32_t)__popcll(__ballot(valid && kq >= glo_q && kq <= ghi_q));
+          if (lv) {
+            const uint32_t pos =
+                off + __builtin_amdgcn_mbcnt_hi((uint32_t)(bl >> 32),
+                                                __builtin_amdgcn_mbcnt_lo((uint32_t)bl, 0u));
+            lst[pos] = ((pw[t >> 1] >> sh) & 0xFFFFu) | (((qw[t >> 1] >> sh) & 0xFFFFu) << 16);
+          }
+          off += (uint32_t)__popcll(bl);
+        }
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_wave_barrier();
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      }
-      auto round16 = [&](const typename Ev::Raw& cp, const typename Ev::Raw& cq, int64_t ro) {
-        if constexpr (Ev::kGroups) {
-          const int64_t s0 = x_beg + ro * kDrawSub;
-          const int64_t rec = s0 / a.rec_ids;
-          const int64_t e1 = min(a.V, (rec + 1) * a.rec_ids);
-          const int nvalid = (int)max<int64_t>(0, min<int64_t>(8, e1 - (s0 + lane_off)));
-          const int32_t klo_p = rp.st.klo, glo_p = rp.st.glo, ghi_p = rp.st.ghi;
-          const int32_t klo_q = hasq ? rq.st.klo : 0x7FFFFFFF;
-          const int32_t glo_q = hasq ? rq.st.glo : 1, ghi_q = hasq ? rq.st.ghi : 0;
-          const uint32_t pw[4] = {cp.x, cp.y, cp.z, cp.w};
-          const uint32_t qw[4] = {cq.x, cq.y, cq.z, cq.w};
-          uint32_t kp2[4], kq2[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            kp2[i] = keys2_of_codes2(pw[i]);
-            kq2[i] = keys2_of_codes2(qw[i]);
+        auto tval = [&](const RowStat& st, const float* tb, int32_t key, uint32_t code) -> float {
+          const int32_t tt = st.kmax - key;
+          if (tt < st.ntbl) return tb[tt];
+          return val16_exp<Ev::kFmt>(code, ev.T, st.m, st.zf, st.totf);
+        };
+        for (uint32_t i = lane; i < off; i += kWave) {
+          const uint32_t e = lst[i];
+          const uint32_t cpd = e & 0xFFFFu, cqd = e >> 16;
+          const int32_t kp = (int32_t)key_of_code16(cpd), kq = (int32_t)key_of_code16(cqd);
+          const bool ip = kp >= glo_p && kp <= ghi_p;
+          const bool iq = kq >= glo_q && kq <= ghi_q;
+          const float pv = ip ? rp.vg : tval(rp.st, tbl_p, kp, cpd);
+          float qv = 0.0f;
+          if (hasq) qv = iq ? rq.vg : (kq >= klo_q ? tval(rq.st, tbl_q, kq, cqd) : 0.0f);
+          const uint64_t wr = fixed62(fmaxf(pv - qv, 0.0f));
+          const uint64_t fp = fixed62(pv);
+          atomicAdd(&acc[w][0], ip ? 0ull : fp);
+          atomicAdd(&acc[w][1], (!ip && !iq) ? wr : 0ull);
+          atomicAdd(&acc[w][2], (!ip && iq) ? wr : 0ull);
+          atomicAdd(&acc[w][3], (!ip && iq) ? fp : 0ull);
+          atomicAdd(&acc[w][4], (ip && !iq) ? wr : 0ull);
+          atomicAdd(&acc[w][5], (ip && iq) ? 1ull : 0ull);
+        }
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_wave_barrier();  // list / sums settled before reuse
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if ((ro + 1) % rpr == 0 || ro + 1 == nround) {
+          if (lane == 0) {
+            ChunkRec rc;
+            rc.p2 = acc[w][0];
+            rc.r0 = acc[w][1];
+            rc.ra = acc[w][2];
+            rc.rb = acc[w][3];
+            rc.rp = acc[w][4];
+            rc.ndbl = (uint32_t)acc[w][5];
+            rc.np = np_s;
+            rc.nq = nq_s;
+            rc.pad = 0;
+            rc.pad2 = 0;
+            store_rec(a.recs + j * a.nrec + rec, rc);
+            for (int i = 0; i < 6; ++i) acc[w][i] = 0ull;
           }
-          uint32_t* lst = reinterpret_cast<uint32_t*>(&lst_p[w][0]);
-          uint32_t off = 0;
-#pragma unroll
-          for (int t = 0; t < 8; ++t) {
-            const int sh = 16 * (t & 1);
-            const int32_t kp = (int32_t)((kp2[t >> 1] >> sh) & 0xFFFFu);
-            const int32_t kq = (int32_t)((kq2[t >> 1] >> sh) & 0xFFFFu);
-            const bool valid = t < nvalid;
-            const bool lv = valid && kp >= klo_p;
-            const uint64_t bl = __ballot(lv);
-            np_s += (uint32_t)__popcll(__ballot(valid && kp >= glo_p && kp <= ghi_p));
-            nq_s += (uint32_t)__popcll(__ballot(valid && kq >= glo_q && kq <= ghi_q));
-            if (lv) {
-              const uint32_t pos =
-                  off + __builtin_amdgcn_mbcnt_hi((uint32_t)(bl >> 32),
-                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)bl, 0u));
-              lst[pos] = ((pw[t >> 1] >> sh) & 0xFFFFu) | (((qw[t >> 1] >> sh) & 0xFFFFu) << 16);
-            }
-            off += (uint32_t)__popcll(bl);
-          }
+          np_s = nq_s = 0;
           __atomic_signal_fence(__ATOMIC_SEQ_CST);
           __builtin_amdgcn_wave_barrier();
           __atomic_signal_fence(__ATOMIC_SEQ_CST);
-          auto tval = [&](const RowStat& st, const float* tb, int32_t key, uint32_t code) -> float {
-            const int32_t tt = st.kmax - key;
-            if (tt < st.ntbl) return tb[tt];
-            return val16_exp<Ev::kFmt>(code, ev.T, st.m, st.zf, st.totf);
-          };
-          for (uint32_t i = lane; i < off; i += kWave) {
-            const uint32_t e = lst[i];
-            const uint32_t cpd = e & 0xFFFFu, cqd = e >> 16;
-            const int32_t kp = (int32_t)key_of_code16(cpd), kq = (int32_t)key_of_code16(cqd);
-            const bool ip = kp >= glo_p && kp <= ghi_p;
-            const bool iq = kq >= glo_q && kq <= ghi_q;
-            const float pv = ip ? rp.vg : tval(rp.st, tbl_p, kp, cpd);
-            float qv = 0.0f;
-            if (hasq) qv = iq ? rq.vg : (kq >= klo_q ? tval(rq.st, tbl_q, kq, cqd) : 0.0f);
-            const uint64_t wr = fixed62(fmaxf(pv - qv, 0.0f));
-            const uint64_t fp = fixed62(pv);
-            atomicAdd(&acc[w][0], ip ? 0ull : fp);
-            atomicAdd(&acc[w][1], (!ip && !iq) ? wr : 0ull);
-            atomicAdd(&acc[w][2], (!ip && iq) ? wr : 0ull);
-            atomicAdd(&acc[w][3], (!ip && iq) ? fp : 0ull);
-            atomicAdd(&acc[w][4], (ip && !iq) ? wr : 0ull);
-            atomicAdd(&acc[w][5], (ip && iq) ? 1ull : 0ull);
-          }
-          __atomic_signal_fence(__ATOMIC_SEQ_CST);
-          __builtin_amdgcn_wave_barrier();  // list / sums settled before reuse
-          __atomic_signal_fence(__ATOMIC_SEQ_CST);
-          if ((ro + 1) % rpr == 0 || ro + 1 == nround) {
-            if (lane == 0) {
-              ChunkRec rc;
-              rc.p2 = acc[w][0];
-              rc.r0 = acc[w][1];
-              rc.ra = acc[w][2];
-              rc.rb = acc[w][3];
-              rc.rp = acc[w][4];
-              rc.ndbl = (uint32_t)acc[w][5];
-              rc.np = np_s;
-              rc.nq = nq_s;
-              rc.pad = 0;
-              rc.pad2 = 0;
-              store_rec(a.recs + j * a.nrec + rec, rc);
-              for (int i = 0; i < 6; ++i) acc[w][i] = 0ull;
-            }
-            np_s = nq_s = 0;
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            __builtin_amdgcn_wave_barrier();
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-          }
-        } else {
-          round(cp, cq, ro);
         }
       };
       typename Ev::Raw ap = {}, aq = {}, bp_ = {}, bq_ = {};
@@ -369,7 +290,6 @@ __global__ void __launch_bounds__(SM_NT) draw_kernel(Ev ev, DrawArgs a) {
       }
     }
   }
-  if (!a.y) return;
 
   // ---- 3. the block that completes the job's records draws. Each wave waits
   // for its record stores (vmcnt(0)) before the block's counter increment, so
