@@ -696,7 +696,9 @@ int sdx_verify_noalloc(const void* target_logits, const void* draft_logits, int 
                        uint8_t* flags, sdx_stream_t stream) {
   if (batch < 0 || k < 1 || !dtype_ok(dtype))
     return fail(SDX_EINVAL, "sdx_verify_noalloc: bad arguments");
-  const size_t need = sdx_verify_workspace(batch, k, vocab, dtype);
+  // without the fp16 scratch, which the call uses only where it fits too
+  const size_t need = verify_ws_bytes(batch, batch * ((int64_t)k + 1), batch * (int64_t)k, vocab,
+                                      dtype, false);
   if (need > kScratchBytes)
     return fail(SDX_EWORKSPACE,
                 "sdx_verify_noalloc: batch %lld, k %d, vocab %lld need %zu bytes of scratch, more "

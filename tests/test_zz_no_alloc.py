@@ -23,10 +23,10 @@ def _outs(B):
             torch.empty(B, dtype=torch.uint8, device=DEV))
 
 
-def _launch(noalloc, inp, B, k, V, T, tp, outs, ws=None):
+def _launch(noalloc, inp, B, k, V, T, tp, outs, ws=None, dt=_lib.BF16):
     L = _lib.lib()
     n, y, f = outs
-    common = (_lib.ptr(inp["target"]), _lib.ptr(inp["draft"]), _lib.BF16, B, k, V,
+    common = (_lib.ptr(inp["target"]), _lib.ptr(inp["draft"]), dt, B, k, V,
               _lib.ptr(inp["draft_ids"]), _lib.ptr(inp["u_accept"]), _lib.ptr(inp["u_final"]),
               None, ctypes.c_float(T), ctypes.c_float(tp), 0, _lib.ptr(n), _lib.ptr(y),
               _lib.ptr(f))
@@ -38,11 +38,11 @@ def _launch(noalloc, inp, B, k, V, T, tp, outs, ws=None):
     _lib.check(rc, "sdx_verify_noalloc" if noalloc else "sdx_verify")
 
 
-def _call(noalloc, inp, B, k, V, T, tp):
+def _call(noalloc, inp, B, k, V, T, tp, dt=_lib.BF16):
     outs = _outs(B)
     ws = None if noalloc else _lib.workspace(
-        _lib.lib().sdx_verify_workspace(B, k, V, _lib.BF16), DEV)
-    _launch(noalloc, inp, B, k, V, T, tp, outs, ws)
+        _lib.lib().sdx_verify_workspace(B, k, V, dt), DEV)
+    _launch(noalloc, inp, B, k, V, T, tp, outs, ws, dt)
     torch.cuda.synchronize()
     return tuple(t.cpu().numpy() for t in outs)
 
@@ -106,6 +106,21 @@ def test_noalloc_scratch_rearms_after_give_up():
     got = _call(True, inp, B, k, V, T, tp)
     for g, w, name in zip(got, want, ("n_acc", "y", "flags")):
         assert np.array_equal(g, w), f"after the give-up: {name} differs"
+
+
+@pytest.mark.parametrize("B", [16, 80])
+def test_noalloc_fp16(B):
+    """fp16 rows with and without room for the threshold scratch in the library's array:
+    80 rows at k = 4 fit the register-resident kernel's pieces only."""
+    T, tp, k, V = 0.8, 0.95, 4, 8448
+    full = _lib.lib().sdx_verify_workspace(B, k, V, _lib.F16)
+    assert (full > 24 << 20) == (B == 80)
+    inp = verify_inputs(B, k, V, seed=1000 + B, device=DEV, temperature=T, top_p=tp)
+    inp = dict(inp, target=inp["target"].half(), draft=inp["draft"].half())
+    got = _call(True, inp, B, k, V, T, tp, _lib.F16)
+    want = _call(False, inp, B, k, V, T, tp, _lib.F16)
+    for g, w, name in zip(got, want, ("n_acc", "y", "flags")):
+        assert np.array_equal(g, w), f"B={B}: {name} differs"
 
 
 def test_noalloc_rejects_requests_beyond_its_scratch():
