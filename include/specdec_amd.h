@@ -52,7 +52,8 @@ enum sdx_flag {
   SDX_FLAG_UNSUPPORTED = 4,     /* a row's probability mass spans more distinct logit values
                                    than the row kernels' histogram windows cover (only with
                                    |logit| >= 2^18 at temperatures above ~2500, or fp16 rows
-                                   spanning over 36 binades of mass): results unspecified */
+                                   spanning over 36 binades of mass where the workspace has
+                                   no room for the threshold scratch): results unspecified */
   SDX_FLAG_BAD_ROW = 8,         /* per-row k: the row offsets (cu_k) were inconsistent with
                                    k_max or the row counts; n_acc 0, y unspecified */
   SDX_FLAG_WORKSPACE = 16,      /* the verify workspace was not prepared by
@@ -90,16 +91,13 @@ int sdx_workspace_init(void* workspace, size_t bytes, sdx_stream_t stream);
  * (first index among maxima); top_p outside (0, 1) -> no nucleus; top_k <= 0
  * or >= vocab -> no top-k.
  * Vocabularies: bf16 rows up to 262,136 (2^18 - 8), fp16 up to 163,840, fp32 up
- * to 262,144 (above 8,192 the fp32 rows take a multi-pass kernel that sorts only
- * the nucleus boundary region, at most 7,168 distinct probabilities: a row whose region is
- * larger is flagged SDX_FLAG_UNSUPPORTED with NaN probabilities); larger ones
- * return SDX_EUNSUPPORTED (here and in the verify entry points) before anything
- * is launched. (The Python entry points widen longer fp16 rows to fp32, which
+ * to 262,144; larger ones return SDX_EUNSUPPORTED (here and in the verify entry
+ * points) before anything is launched. (The Python entry points widen longer fp16 rows to fp32, which
  * is exact, and call the fp32 path.) */
 
 /* to_probs (sampling.py:34-67): logits [rows, vocab] (dtype) -> probs [rows, vocab] fp32.
- * probs may not overlap fp32 logits (SDX_EINVAL): above 8,192 tokens the fp32 kernel
- * keeps each element's exp, then its probability, in the output row between passes. */
+ * probs may not overlap fp32 logits (SDX_EINVAL): above 8,192 tokens the
+ * kernels keep their scratch in the output rows until the last pass. */
 size_t sdx_to_probs_workspace(int64_t rows, int64_t vocab, int dtype);
 int sdx_to_probs(const void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
                  float temperature, float top_p, int32_t top_k,
