@@ -150,10 +150,18 @@ __device__ __forceinline__ void thr_max16(const ThrArgs& a, const uint16_t* row,
   s2 hi = {-32768, -32768};
   u2 lo = {0xFFFF, 0xFFFF};
   const int tid = threadIdx.x;
-  const int64_t nv = a.V / 8;  // rows start 16-byte aligned, V is a multiple of 8
+  const int64_t nv = a.V / 8;  // rows start 16-byte aligned
   const int64_t v0 = (int64_t)part * (a.llen / 8);
   const int64_t v1 = part == a.nlight - 1 ? nv : min(nv, v0 + a.llen / 8);
   const uint4* const x4 = reinterpret_cast<const uint4*>(row);
+  auto fold = [&](uint32_t q) {
+    const s2 c = __builtin_bit_cast(s2, q);
+    const s2 k = c ^ ((c >> 15) & (s2){0x7FFF, 0x7FFF});
+    hi = __builtin_elementwise_max(hi, k);
+    lo = __builtin_elementwise_min(lo, __builtin_bit_cast(u2, (s2)(k - (s2){kLow, kLow})));
+  };
+  // to_probs takes any V: the elements after the last whole vector
+  if (part == a.nlight - 1 && nv * 8 + tid < a.V) fold(row[nv * 8 + tid] * 0x10001u);
   constexpr int UN = 4;
   for (int64_t b = v0 + tid; b < v1; b += (int64_t)UN * TH_NT) {
     uint4 w[UN];
@@ -163,12 +171,7 @@ __device__ __forceinline__ void thr_max16(const ThrArgs& a, const uint16_t* row,
     for (int u = 0; u < UN; ++u) {
       const uint32_t q[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const s2 c = __builtin_bit_cast(s2, q[e]);
-        const s2 k = c ^ ((c >> 15) & (s2){0x7FFF, 0x7FFF});
-        hi = __builtin_elementwise_max(hi, k);
-        lo = __builtin_elementwise_min(lo, __builtin_bit_cast(u2, (s2)(k - (s2){kLow, kLow})));
-      }
+      for (int e = 0; e < 4; ++e) fold(q[e]);
     }
   }
   const int h = max((int)hi[0], (int)hi[1]);

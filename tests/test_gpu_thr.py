@@ -80,6 +80,17 @@ def test_to_probs_fp16_rows(V, T, tp, tk):
     _same(got, O.to_probs(x.astype(np.float32), T, tp, tk))
 
 
+# odd lengths, the maximum (or an infinity) among the ids after the last whole 16 bytes
+@pytest.mark.parametrize("V", [9, 1001, 8191, 8193, 8199, 33001, 50257])
+def test_to_probs_fp16_odd_rows(V):
+    x = _rows(V, V, np.float16)
+    x[:4, V - 1] = 40.0
+    x[4:8, V - 1 - V % 8 // 2] = 35.0
+    for T, tp, tk in ((0.8, 0.95, 0), (1.0, 1.0, 0), (1.0, 0.9, 50)):
+        got = S.to_probs(torch.tensor(x, device=DEV), T, tp, tk).cpu().numpy()
+        _same(got, O.to_probs(x.astype(np.float32), T, tp, tk))
+
+
 def test_top_k_of_all_but_one():
     x = _rows(9000, 1)
     got = S.to_probs(torch.tensor(x, device=DEV), 1.0, 1.0, 8999).cpu().numpy()
@@ -130,8 +141,8 @@ def _verify_case(B, k, V, dtype, seed):
 @pytest.mark.parametrize("V,T,tp,tk", [(40, 1.0, 0.9, 5), (1000, 0.8, 0.95, 0), (8200, 0.8, 0.95, 0),
                                        (9217, 1.0, 0.7, 0), (33000, 0.7, 0.9, 50),
                                        (16384, 1.0, 1.0, 0)])
-def test_verify_rows(dtype, V, T, tp, tk):
-    B, k = 12, 3
+@pytest.mark.parametrize("B,k", [(12, 3), (3, 40)])  # 40: more positions than half a wave
+def test_verify_rows(dtype, V, T, tp, tk, B, k):
     t, d, ids, ua, uf = _verify_case(B, k, V, dtype, V)
     n, y, f = S.rejection_sample(t.to(DEV), d.to(DEV), ids.to(DEV), ua.to(DEV), uf.to(DEV),
                                  temperature=T, top_p=tp, top_k=tk)
