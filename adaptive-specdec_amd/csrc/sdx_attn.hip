@@ -30,12 +30,12 @@
 // output directly; otherwise each chunk writes (O unnormalised, max, sum) in
 // fp32, and the chunk of the row that finishes last merges it.
 //
-// A batch that leaves the chip short of whole 1024-token chunks runs without the
-// plan (DIRECT): the workgroups derive a finer split from the rows' lengths, and
-// a second kernel merges with a workgroup per query row. One row of 8 KV heads
-// and about 12,000 keys: 31 us, against 525 us when chunks of 64 tokens were
-// planned by one thread and 230 partials of 20 query rows merged by one workgroup
-// per KV head; 2 rows of 16,384-32,768 keys 54 us, from 445.
+// A small batch that leaves the chip short of whole 1024-token chunks runs without the
+// plan (DIRECT): the workgroups find their chunks themselves, and a second kernel
+// merges with a workgroup per query row. Both forms add the same numbers in the same
+// order. One row of 8 KV heads and about 12,000 keys: 37 us, against 525 us when one
+// thread plans its 190 chunks of 64 tokens and a workgroup per KV head merges their
+// partials of 20 query rows; 2 rows of 16,384-32,768 keys 65 us, from 515.
 // The kernels are bound by the KV bytes streamed (about 22 flop per byte),
 // not by MFMA.
 #include "sdx_launch.hpp"
@@ -226,6 +226,10 @@ __device__ __forceinline__ float4 va_ld_f4(const float* p) {  // p 16-byte align
   return make_float4(lo.x, lo.y, hi.x, hi.y);
 }
 
+// (m, l) pairs that va_merge stages in LDS: what its tile buffers hold.
+template <int D>
+constexpr int va_merge_cap() { return VA_TOK * va_ks<D>() * (int)sizeof(uint16_t) / (int)sizeof(float); }
+
 // Merge of the chunk partials of row b, KV head kvh (a row longer than one
 // chunk) by the whole workgroup: out = sum_c w_c O_c with
 // w_c = 2^(m_c - m) / sum_c' 2^(m_c' - m) l_c' and m the row's largest m_c. The
@@ -238,7 +242,7 @@ __device__ __forceinline__ void va_merge(const AttnArgs& a, int64_t b, int kvh, 
                                          int nch, float* sW, float* sL, int cap) {
   const int64_t part0 = (b * a.hkv + kvh) * a.nchunk * a.max_m;
   const bool staged = nch * M <= cap;  // uniform
-  if (staged) {
+  if (staged) {  // verify_attn_merge_kernel keeps the order of both forms' sums
     for (int e = threadIdx.x; e < nch * M; e += VA_NT) {  // sW, sL [c * M + i] = m, l of (c, i)
       const int ch = e / M, i = e % M;
       const float2 ml = va_ld_f2(a.part_ml + (part0 + (int64_t)ch * a.max_m + i) * 2);
@@ -307,16 +311,18 @@ __device__ __forceinline__ void va_merge(const AttnArgs& a, int64_t b, int kvh, 
 }
 
 // ---- launches without a plan, for batches that leave the chip short of work with
-// whole 1024-token chunks. Every wave derives the same split from the rows'
-// lengths: the chunk size that gives about VA_SLOTS workgroups (the workgroups
-// that fit the chip at once: a row split finer pays a workgroup's set-up and its
-// partials again, split coarser it leaves CUs idle), at least a.chunk (which
-// bounds the partials the workspace holds), then the chunk of slot `unit` by a
-// scan over the rows.
+// whole 1024-token chunks. Chunks are the planned launch's (their size is a function
+// of the call's shapes), and so is the order of every sum: a row's output is the same
+// bits either way, whatever the other rows hold. A workgroup takes a span of
+// consecutive chunks of a row, one after the other, each with a partial of its own.
+// Every wave derives the same spans from the rows' lengths: the length that gives
+// about VA_SLOTS workgroups (the workgroups that fit the chip at once: a row split
+// finer pays a workgroup's set-up again, split coarser it leaves CUs idle), then the
+// span of slot `unit` by a scan over the rows.
 constexpr int VA_SLOTS = 768;  // 3 workgroups on each of 256 CUs
 struct VaSlot {
-  int64_t b, q0, qb, kvl;  // b = -1: no chunk in this slot
-  int c, chunk;
+  int64_t b, q0, qb, kvl;  // b = -1: no span in this slot
+  int c, span;             // first chunk, tokens per span (whole chunks)
 };
 struct VaShape {  // one row per lane
   int64_t q0 = 0, qb = 0, kvl = 0;
@@ -325,39 +331,38 @@ struct VaShape {  // one row per lane
   __device__ __forceinline__ uint64_t keys() const { return ok && qb > 0 ? (uint64_t)kvl : 0ull; }
 };
 // first: rows 0 .. 63, lane by lane
-__device__ __forceinline__ int va_direct_chunk(const AttnArgs& a, const VaShape& first) {
-  if (!a.dyn) return a.chunk;
+__device__ __forceinline__ int va_direct_span(const AttnArgs& a, const VaShape& first) {
   uint64_t total = wave_sum_u64(first.keys());  // keys of the rows served
   for (int64_t b0 = kWave; b0 < a.batch; b0 += kWave)
     total += wave_sum_u64(VaShape(a, b0 + (threadIdx.x & (kWave - 1))).keys());
-  // total / chunk whole chunks and about half a chunk more per row fill the slots
+  // total / span whole spans and about half a span more per row fill the slots
   const uint64_t nh = (uint64_t)a.hkv * (uint64_t)a.nrb, half = (uint64_t)a.batch * nh / 2;
   const uint64_t room = VA_SLOTS - min(half, (uint64_t)(3 * VA_SLOTS / 4));
-  const uint64_t ch = (total * nh / room + 63) / 64 * 64;
-  return (int)min((uint64_t)VA_CHMAX, max((uint64_t)a.chunk, ch));
+  const uint64_t n = (total * nh / room + a.chunk - 1) / a.chunk;
+  return a.chunk * (int)max(1ull, min((unsigned long long)(VA_CHMAX / a.chunk), (unsigned long long)n));
 }
 __device__ __forceinline__ VaSlot va_direct_slot(const AttnArgs& a, int64_t unit, bool report) {
   const int lane = threadIdx.x & (kWave - 1);
   VaShape sh(a, lane);
   VaSlot s;
   s.b = -1;
-  s.chunk = va_direct_chunk(a, sh);
-  int64_t before = 0;  // chunks of the rows before b0
+  s.span = va_direct_span(a, sh);
+  int64_t before = 0;  // spans of the rows before b0
   for (int64_t b0 = 0; b0 < a.batch; b0 += kWave) {
     const int64_t b = b0 + lane;
     if (b0 > 0) sh = VaShape(a, b);
     if (report && unit == 0 && !sh.ok && b < a.batch && a.error) *a.error = 1;
-    const uint32_t nch = (uint32_t)((sh.keys() + s.chunk - 1) / s.chunk);
-    const uint32_t incl = wave_incl_scan_u32(nch, lane);
-    const int64_t first = before + incl - nch;
-    const uint64_t hit = __ballot(nch > 0 && unit >= first && unit < first + nch);
+    const uint32_t nsp = (uint32_t)((sh.keys() + s.span - 1) / s.span);
+    const uint32_t incl = wave_incl_scan_u32(nsp, lane);
+    const int64_t first = before + incl - nsp;
+    const uint64_t hit = __ballot(nsp > 0 && unit >= first && unit < first + nsp);
     if (hit) {  // uniform
       const int src = __ffsll((unsigned long long)hit) - 1;
       s.b = b0 + src;
       s.q0 = __shfl((long long)sh.q0, src, kWave);
       s.qb = __shfl((long long)sh.qb, src, kWave);
       s.kvl = __shfl((long long)sh.kvl, src, kWave);
-      s.c = (int)(unit - __shfl((long long)first, src, kWave));
+      s.c = (int)(unit - __shfl((long long)first, src, kWave)) * (s.span / a.chunk);
       if (!report || unit != 0) break;  // slot 0 goes on to look at every row
     }
     before += rdlane(incl, kWave - 1);
@@ -365,8 +370,8 @@ __device__ __forceinline__ VaSlot va_direct_slot(const AttnArgs& a, int64_t unit
   return s;
 }
 
-// D: head dim, 64 or 128. DIRECT: no plan; the workgroup finds its chunk itself, and
-// the chunk partials are plain stores for verify_attn_merge_kernel.
+// D: head dim, 64 or 128. DIRECT: no plan; the workgroup finds its span of chunks
+// itself, and the chunk partials are plain stores for verify_attn_merge_kernel.
 template <int D, bool DIRECT>
 __global__ void __launch_bounds__(VA_NT) __attribute__((amdgpu_waves_per_eu(3)))
 verify_attn_kernel(AttnArgs a) {
@@ -391,13 +396,13 @@ verify_attn_kernel(AttnArgs a) {
   const int64_t unit = 8 * grp + rem % 8;
   if (unit >= a.nunits) return;
   int64_t b, q0, qb, kvl;
-  int c, n, chunk = a.chunk;
+  int c, n;
+  const int chunk = a.chunk;
   if constexpr (DIRECT) {
     const VaSlot sl = va_direct_slot(a, unit, hx == 0);
-    if (sl.b < 0) return;  // uniform: no chunk in this slot
-    chunk = sl.chunk;
+    if (sl.b < 0) return;  // uniform: no span in this slot
     b = sl.b, c = sl.c, q0 = sl.q0, qb = sl.qb, kvl = sl.kvl;
-    n = (int)min(kvl - (int64_t)c * chunk, (int64_t)chunk);
+    n = (int)min(kvl - (int64_t)c * chunk, (int64_t)sl.span);  // below, "the chunk" is the span
   } else {
     const AttnUnit un = a.units[unit];
     if (un.b < 0) return;  // uniform: no chunk in this slot
@@ -577,45 +582,13 @@ verify_attn_kernel(AttnArgs a) {
   uint32_t vA[8], vB[8], okA, okB;
   gather(0, kA, vA, okA);
   gather(VA_TOK, kB, vB, okB);
-  // one exit, at the bottom: both register sets are then in flight in the same
-  // order on every entry to the loop, so each stage waits for its own set only
-  // (a second tile past the chunk's end is all masked, with V zeroed)
-  for (int t0 = 0;; t0 += 2 * VA_TOK) {
-    stage(kA, vA, okA);
-    __syncthreads();
-    gather(t0 + 2 * VA_TOK, kA, vA, okA);
-    if (active) compute(t0);
-    __syncthreads();  // the tile's LDS is rewritten next
-    stage(kB, vB, okB);
-    __syncthreads();
-    gather(t0 + 3 * VA_TOK, kB, vB, okB);
-    if (active) compute(t0 + VA_TOK);
-    __syncthreads();
-    if (t0 + 2 * VA_TOK >= n) break;
-  }
-  if (bad && a.error) *a.error = 1;
-  // the row index is rebuilt here rather than kept live across the tile loop
+  // the row index is rebuilt where it is needed rather than kept live across the loop
   int lre = lr;
-  asm volatile("" : "+v"(lre));
-
-  if (whole) {  // out[q0 + j, kvh * group + g, :] = O / l
+  // a chunk's partial: O unnormalised and (max, sum) per query row, in the part of
+  // (row b, KV head, chunk cp); the block's rows from rofs
+  auto put_partial = [&](int cp) {
+    const int64_t part = ((b * a.hkv + kvh) * a.nchunk + cp) * a.max_m + rofs;
     if (!active) return;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = r0 + lre + r;
-      if (i < M) {
-        uint16_t* dst = a.out + sRow[i];
-        const float inv = l_run[r] > 0.0f ? 1.0f / l_run[r] : 0.0f;
-#pragma unroll
-        for (int jj = 0; jj < OJ; ++jj) dst[jj * 16 + lc] = va_bf16(o[jj][r] * inv);
-      }
-    }
-    return;
-  }
-  // the chunk's partial: O unnormalised and (max, sum) per query row, in the
-  // part of (row b, KV head, chunk c); the block's rows from rofs
-  const int64_t part = ((b * a.hkv + kvh) * a.nchunk + c) * a.max_m + rofs;
-  if (active) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + lre + r;
@@ -633,8 +606,58 @@ verify_attn_kernel(AttnArgs a) {
         }
       }
     }
+  };
+  // one exit, at the bottom: both register sets are then in flight in the same
+  // order on every entry to the loop, so each stage waits for its own set only
+  // (a second tile past the chunk's end is all masked, with V zeroed)
+  [[maybe_unused]] int left = chunk;  // DIRECT: tokens to the end of chunk c
+  for (int t0 = 0;; t0 += 2 * VA_TOK) {
+    stage(kA, vA, okA);
+    __syncthreads();
+    gather(t0 + 2 * VA_TOK, kA, vA, okA);
+    if (active) compute(t0);
+    __syncthreads();  // the tile's LDS is rewritten next
+    stage(kB, vB, okB);
+    __syncthreads();
+    gather(t0 + 3 * VA_TOK, kB, vB, okB);
+    if (active) compute(t0 + VA_TOK);
+    __syncthreads();
+    if constexpr (DIRECT) {  // chunks are whole steps of this loop
+      left -= 2 * VA_TOK;
+      if (!whole && (left == 0 || t0 + 2 * VA_TOK >= n)) {  // uniform
+        asm volatile("" : "+v"(lre));
+        put_partial(c++);
+        left = chunk;
+#pragma unroll
+        for (int j = 0; j < OJ; ++j) o[j] = (va_f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          m_run[r] = -INFINITY;
+          l_run[r] = 0.0f;
+        }
+      }
+    }
+    if (t0 + 2 * VA_TOK >= n) break;
+  }
+  if (bad && a.error) *a.error = 1;
+  asm volatile("" : "+v"(lre));
+
+  if (whole) {  // out[q0 + j, kvh * group + g, :] = O / l
+    if (!active) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = r0 + lre + r;
+      if (i < M) {
+        uint16_t* dst = a.out + sRow[i];
+        const float inv = l_run[r] > 0.0f ? 1.0f / l_run[r] : 0.0f;
+#pragma unroll
+        for (int jj = 0; jj < OJ; ++jj) dst[jj * 16 + lc] = va_bf16(o[jj][r] * inv);
+      }
+    }
+    return;
   }
   if constexpr (DIRECT) return;  // the next kernel merges
+  put_partial(c);
   // the workgroup's stores are done before it counts in on the (row, KV head):
   // the one that counts in last merges the row's chunks
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -651,102 +674,135 @@ verify_attn_kernel(AttnArgs a) {
   if (!*flag) return;  // uniform
   // the tile buffers hold the merge's weights
   static_assert(sizeof(sK) <= sizeof(sVt), "merge weights sized by the K tile");
+  static_assert(sizeof(sK) / sizeof(float) == va_merge_cap<D>(), "the merge kernel's staging");
   va_merge<D>(a, b, kvh, q0, Mt, nch, reinterpret_cast<float*>(&sK[0][0]),
               reinterpret_cast<float*>(&sVt[0][0]), (int)(sizeof(sK) / sizeof(float)));
 }
 
 // Merge of the chunk partials of one query row of (row b, KV head kvh), after a
-// DIRECT launch: blockIdx.x = (b * hkv + kvh) * max_m + i. VA_NT / (D / 4) slices of
-// the workgroup each take every SL-th chunk (float4 of D per thread), then add up
-// through LDS. Bound by the latency of two dependent load rounds, so a row's
-// query rows go to workgroups of their own.
-template <int D>
-__global__ void __launch_bounds__(VA_NT) verify_attn_merge_kernel(AttnArgs a) {
-  constexpr int DL = D / 4, SL = VA_NT / DL;
-  __shared__ float4 sAcc[SL][DL];
-  __shared__ float sDen[SL], sMax[VA_NW];
-  const int tid = threadIdx.x;
+// DIRECT launch: blockIdx.x = (b * hkv + kvh) * max_m + i. va_merge's sums, element for
+// element in its order (chunk by chunk; the weights normalised first where it stages
+// them, the sum last where it does not). Bound by latency: the loads of VM_UN chunks per
+// thread are issued at once (partials come from other XCDs, past the L2), the weighted
+// partials go through LDS, and a thread per output dim adds them up in order.
+constexpr int VM_UN = 16;
+template <int D, int VM_NT>
+__global__ void __launch_bounds__(VM_NT) verify_attn_merge_kernel(AttnArgs a) {
+  constexpr int DL = D / 4, SL = VM_NT / DL;  // a chunk's partial: DL threads of float4
+  constexpr int RU = 4;                       // chunks per thread and round through LDS
+  constexpr int CAP = va_merge_cap<D>();
+  __shared__ float4 sV[RU * SL][DL];
+  __shared__ __align__(16) float sL[(CAP + 15) / 16 * 16];
+  __shared__ float sMax[VM_NT / kWave], sDen;
+  const int tid = threadIdx.x, d4 = tid % DL, sl = tid / DL;
   const int64_t bh = blockIdx.x / a.max_m;
   const int i = (int)(blockIdx.x % a.max_m);
   const int64_t b = bh / a.hkv;
   const int kvh = (int)(bh % a.hkv);
   int64_t q0, qb, kvl;
-  if (!va_row(a, b, q0, qb, kvl)) return;             // uniform
-  const int chunk = va_direct_chunk(a, VaShape(a, threadIdx.x & (kWave - 1)));
-  if (i >= (int)qb * a.group || kvl <= chunk) return;  // uniform: nothing to merge
-  const int nch = (int)((kvl + chunk - 1) / chunk);
+  if (!va_row(a, b, q0, qb, kvl)) return;         // uniform
+  const int Mt = (int)qb * a.group;
+  if (i >= Mt || kvl <= a.chunk) return;          // uniform: nothing to merge
+  const int nch = (int)((kvl + a.chunk - 1) / a.chunk);
+  const bool staged = (int64_t)nch * Mt <= CAP;
   const int64_t p0 = bh * a.nchunk * a.max_m + i;  // chunk c's part: p0 + c * max_m
-  const float2* const ml = reinterpret_cast<const float2*>(a.part_ml);
+  const float2* const ml = reinterpret_cast<const float2*>(a.part_ml) + p0;
+  const float4* const po = reinterpret_cast<const float4*>(a.part_o) + p0 * DL + d4;
+  float4 v[VM_UN];  // chunks cb + u SL + sl
+  float mc[VM_UN];
+  auto load = [&](int cb) {
+#pragma unroll
+    for (int u = 0; u < VM_UN; ++u) {
+      if (cb + u * SL >= nch) break;  // uniform
+      const int64_t c = min(cb + u * SL + sl, nch - 1);
+      v[u] = po[c * a.max_m * DL];
+      mc[u] = ml[c * a.max_m].x;
+    }
+  };
+  load(0);
   float mx = -INFINITY;
-  for (int c = tid; c < nch; c += VA_NT) mx = fmaxf(mx, ml[p0 + (int64_t)c * a.max_m].x);
+  for (int c = tid; c < nch; c += VM_NT) mx = fmaxf(mx, ml[(int64_t)c * a.max_m].x);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
   if ((tid & (kWave - 1)) == 0) sMax[tid / kWave] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(sMax[0], sMax[1]), fmaxf(sMax[2], sMax[3]));
-  static_assert(VA_NW == 4, "four wave maxima");
-  const int d4 = tid % DL, sl = tid / DL;
-  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  float den = 0.0f;
-#pragma unroll 4
-  for (int c = sl; c < nch; c += SL) {
-    const int64_t p = p0 + (int64_t)c * a.max_m;
-    const float2 w = ml[p];
-    const float4 v = *reinterpret_cast<const float4*>(a.part_o + p * D + d4 * 4);
-    // m = -inf: the chunk holds none of the row's visible keys
-    const float f = w.x == -INFINITY ? 0.0f : exp2f(w.x - mx);
-    den += f * w.y;
-    acc.x += f * v.x;
-    acc.y += f * v.y;
-    acc.z += f * v.z;
-    acc.w += f * v.w;
+#pragma unroll
+  for (int w = 0; w < VM_NT / kWave; ++w) mx = fmaxf(mx, sMax[w]);
+  // m = -inf: the chunk holds none of the row's visible keys
+  auto weight = [&](float m) { return m == -INFINITY ? 0.0f : exp2f(m - mx); };
+  float den = 0.0f;  // thread 0
+  for (int cb = 0; cb < nch; cb += CAP) {  // uniform
+    const int nb = min(CAP, nch - cb);
+    for (int c = tid; c < (nb + 15) / 16 * 16; c += VM_NT) {  // zeros after the last: den stays
+      const float2 w = ml[(int64_t)(cb + min(c, nb - 1)) * a.max_m];
+      sL[c] = c < nb ? weight(w.x) * w.y : 0.0f;
+    }
+    __syncthreads();
+    if (tid == 0)
+      for (int c = 0; c < nb; c += 16) {
+        float x[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) x[u] = sL[c + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) den += x[u];
+      }
+    __syncthreads();
   }
-  sAcc[sl][d4] = acc;
-  if (d4 == 0) sDen[sl] = den;
+  if (tid == 0) sDen = den;
   __syncthreads();
-  if (sl != 0) return;
+  const float inv = sDen > 0.0f ? 1.0f / sDen : 0.0f;
+  float acc = 0.0f;  // threads below D
+  for (int cb = 0; cb < nch; cb += VM_UN * SL) {  // uniform
+    if (cb > 0) load(cb);
 #pragma unroll
-  for (int k = 1; k < SL; ++k) {
-    const float4 v = sAcc[k][d4];
-    acc.x += v.x;
-    acc.y += v.y;
-    acc.z += v.z;
-    acc.w += v.w;
+    for (int r = 0; r < VM_UN / RU; ++r) {
+      const int c0 = cb + r * RU * SL;
+      if (c0 >= nch) break;  // uniform
+#pragma unroll
+      for (int q = 0; q < RU; ++q) {
+        const int u = r * RU + q;
+        const float f = weight(mc[u]), w = staged ? f * inv : f;
+        float4 x = make_float4(w * v[u].x, w * v[u].y, w * v[u].z, w * v[u].w);
+        // such a chunk is left out where the weights are not staged
+        if (!staged && mc[u] == -INFINITY) x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        sV[q * SL + sl][d4] = x;
+      }
+      __syncthreads();
+      if (tid < D) {
+        const float* const x = reinterpret_cast<const float*>(&sV[0][0]) + tid;
+        const int nb = min(RU * SL, nch - c0);
+#pragma unroll 16
+        for (int c = 0; c < nb; ++c) acc += x[c * D];
+      }
+      __syncthreads();
+    }
   }
-  den = 0.0f;
-#pragma unroll
-  for (int k = 0; k < SL; ++k) den += sDen[k];
-  const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-  uint16_t* dst = a.out + ((q0 + i / a.group) * a.hq + kvh * a.group + i % a.group) * D + d4 * 4;
-  const uint32_t lo = (uint32_t)va_bf16(acc.x * inv) | ((uint32_t)va_bf16(acc.y * inv) << 16);
-  const uint32_t hi = (uint32_t)va_bf16(acc.z * inv) | ((uint32_t)va_bf16(acc.w * inv) << 16);
-  *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
+  if (tid >= D) return;
+  if (!staged) acc *= inv;
+  a.out[((q0 + i / a.group) * a.hq + kvh * a.group + i % a.group) * D + tid] = va_bf16(acc);
 }
 
-// Chunk slots with whole 1024-token chunks below which a call runs without a plan.
-// Measured on both sides (us per call, plan | direct; 32 / 8 heads of 128, contexts
-// up to 8,192 unless said): 512 slots (8 rows) 56 | 49, 1,024 (16 rows) 95 | 99,
-// 2,048 (32 rows) 165 | 177, 8,192 (128 rows) 502 | 584.
-constexpr int64_t VA_DIRECT_SLOTS = 1024;
+// A call runs without a plan when whole 1024-token chunks would leave the chip short
+// of work and its rows have few (row, KV head, query block) triples: the merge kernel
+// and the row scans grow with them, the plan's one workgroup with the chunks of a row.
+// Measured on both sides (us per call, plan | direct; 32 / 8 heads of 128 unless said):
+// 8 triples (1 row of 12,000 keys) 294 | 32, 64 (8 rows of 1,024-8,192) 74 | 61, 96
+// (12 rows of 4,096) 78 | 72, (24 rows of 4 / 4 heads, 2,048-4,096) 61 | 50, 120
+// (15 rows of 1,024-8,192) 83 | 91, 500 (500 rows of 4 / 1 heads, 64-512) 40 | 70.
+// With chunks of 1,024 a row's chunks are few and the plan's order of them, longest
+// first, is worth more: 8 rows of 1,024-8,192 71 | 82.
+constexpr int64_t VA_DIRECT_SLOTS = 1024, VA_DIRECT_ROWS = 96;
 
-// Tokens per chunk (the least of a direct launch, which may take more: see
-// va_direct_chunk) and whether the call runs without a plan.
-int attn_chunk_tokens(int64_t batch, int32_t hkv, int64_t nrb, int64_t max_tokens, int32_t chunk,
-                      bool* direct) {
-  auto slots = [&](int64_t ch) { return batch * hkv * nrb * ((max_tokens + ch - 1) / ch); };
-  *direct = slots(VA_CHMAX) < VA_DIRECT_SLOTS;
+bool attn_direct(int64_t batch, int32_t hkv, int64_t nrb, int64_t max_tokens, int32_t chunk) {
+  const int64_t rows = batch * hkv * nrb;
+  return rows <= VA_DIRECT_ROWS && chunk < VA_CHMAX &&
+         rows * ((max_tokens + VA_CHMAX - 1) / VA_CHMAX) < VA_DIRECT_SLOTS;
+}
+
+int attn_chunk_tokens(int64_t batch, int32_t hkv, int64_t max_tokens, int32_t chunk) {
   if (chunk > 0) return chunk;
-  int ch = VA_CHMAX;
-  if (*direct) {
-    // Rows of one chunk need no merge launch (about 4 us, as long as four more tiles
-    // take); else at most twice the resident workgroups if every row were as long as
-    // the table allows.
-    if (max_tokens <= 6 * VA_TOK) return 6 * VA_TOK;
-    ch = 4 * VA_TOK;
-    while (ch < VA_CHMAX && slots(ch) > 2 * VA_SLOTS) ch += 2 * VA_TOK;
-    return ch;
-  }
   // smallest chunk count that still leaves about 8 workgroups per CU of work
+  int ch = VA_CHMAX;
   while (ch > 2 * VA_TOK && batch * hkv * ((max_tokens + ch - 1) / ch) < 8 * 256) ch /= 2;
   return ch;
 }
@@ -765,8 +821,12 @@ static hipError_t launch_attn_d(const AttnArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((verify_attn_kernel<D, true>), grid, dim3(VA_NT), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.nchunk <= 1) return e;
-  hipLaunchKernelGGL(verify_attn_merge_kernel<D>, dim3((unsigned)(a.batch * a.hkv * a.max_m)),
-                     dim3(VA_NT), 0, s, a);
+  // as many threads as the longest row's chunks keep busy in one round of loads
+  const dim3 mgrid((unsigned)(a.batch * a.hkv * a.max_m));
+  if (a.nchunk <= VM_UN * (128 / (D / 4)))
+    hipLaunchKernelGGL((verify_attn_merge_kernel<D, 128>), mgrid, dim3(128), 0, s, a);
+  else
+    hipLaunchKernelGGL((verify_attn_merge_kernel<D, 512>), mgrid, dim3(512), 0, s, a);
   return hipGetLastError();
 }
 

@@ -991,7 +991,7 @@ int sdx_kv_append_paged(void* pool, int64_t layer_stride, int64_t side_stride, c
 // chunking of the keys shared by the workspace query and the launch
 static int attn_plan(int64_t batch, int32_t max_q, int32_t num_q_heads, int32_t num_kv_heads,
                      int32_t block_size, int64_t max_blocks, int32_t chunk_tokens, int32_t* chunk,
-                     int32_t* nchunk, bool* direct, size_t* bytes) {
+                     int32_t* nchunk, size_t* bytes) {
   if (batch < 0 || max_q < 1 || num_q_heads < 1 || num_kv_heads < 1 || block_size < 1 ||
       max_blocks < 1 || chunk_tokens < 0)
     return fail(SDX_EINVAL, "sdx_verify_attention: bad arguments");
@@ -1005,8 +1005,7 @@ static int attn_plan(int64_t batch, int32_t max_q, int32_t num_q_heads, int32_t 
     return fail(SDX_EUNSUPPORTED, "sdx_verify_attention: max_blocks * block_size >= 2^31");
   const int64_t m = (int64_t)max_q * (num_q_heads / num_kv_heads);
   const int64_t nrb = (m + 63) / 64;  // workgroups per (chunk, KV head): 64 query rows each
-  const int32_t ch =
-      sdx::attn_chunk_tokens(batch, num_kv_heads, nrb, max_tokens, chunk_tokens, direct);
+  const int32_t ch = sdx::attn_chunk_tokens(batch, num_kv_heads, max_tokens, chunk_tokens);
   const int64_t nch = (max_tokens + ch - 1) / ch;
   if (m > 0x7FFFFFFF / 64 || nch * batch * num_kv_heads * nrb > 0x7FFFFFFF)
     return fail(SDX_EUNSUPPORTED, "sdx_verify_attention: grid of %lld chunk workgroups is too large",
@@ -1026,10 +1025,9 @@ size_t sdx_verify_attention_workspace(int64_t batch, int32_t max_q, int32_t num_
                                       int32_t num_kv_heads, int32_t block_size,
                                       int64_t max_blocks, int32_t chunk_tokens) {
   int32_t ch, nch;
-  bool direct;
   size_t bytes = 0;
   if (attn_plan(batch, max_q, num_q_heads, num_kv_heads, block_size, max_blocks, chunk_tokens,
-                &ch, &nch, &direct, &bytes) != SDX_OK)
+                &ch, &nch, &bytes) != SDX_OK)
     return 0;
   return bytes;
 }
@@ -1048,10 +1046,9 @@ int sdx_verify_attention_paged(const void* q, int dtype, int64_t batch, const in
   if (dtype != SDX_BF16 || (head_dim != 64 && head_dim != 128))
     return fail(SDX_EUNSUPPORTED, "sdx_verify_attention_paged: bf16 with head_dim 64 or 128 only");
   int32_t ch = 0, nch = 0;
-  bool direct = false;
   size_t need = 0;
   const int rc = attn_plan(batch, max_q, num_q_heads, num_kv_heads, block_size, max_blocks,
-                           chunk_tokens, &ch, &nch, &direct, &need);
+                           chunk_tokens, &ch, &nch, &need);
   if (rc != SDX_OK) return rc;
   const int32_t group = num_q_heads / num_kv_heads;
   if (num_blocks * block_size * num_kv_heads >= (int64_t)0xFFFFFFFF)
@@ -1087,8 +1084,7 @@ int sdx_verify_attention_paged(const void* q, int dtype, int64_t batch, const in
   a.max_m = max_q * group;
   a.nrb = (a.max_m + 63) / 64;
   a.nunits = batch * (int64_t)nch;
-  a.direct = direct;
-  a.dyn = direct && chunk_tokens == 0;
+  a.direct = sdx::attn_direct(batch, num_kv_heads, a.nrb, max_blocks * block_size, ch);
   const size_t ubytes = ((size_t)a.nunits * sizeof(sdx::AttnUnit) + 15) & ~(size_t)15;
   a.units = (sdx::AttnUnit*)workspace;
   const int64_t nparts = batch * num_kv_heads * (int64_t)nch * a.max_m;

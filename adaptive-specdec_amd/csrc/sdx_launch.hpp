@@ -435,12 +435,11 @@ struct AttnArgs {
                             // by the plan kernel)
   int32_t nrb;              // blocks of 64 query rows per (chunk, KV head): ceil(max_m / 64)
   bool direct;              // no plan: workgroups find their chunks, a second kernel merges
-  bool dyn;                 // direct: the chunk size follows the rows' lengths (>= chunk)
 };
-// tokens per key chunk (chunk > 0: that value, else the default for the shape; nrb as
-// in AttnArgs), and whether the call runs without a plan
-int attn_chunk_tokens(int64_t batch, int32_t hkv, int64_t nrb, int64_t max_tokens, int32_t chunk,
-                      bool* direct);
+// tokens per key chunk (chunk > 0: that value, else the default for the shape)
+int attn_chunk_tokens(int64_t batch, int32_t hkv, int64_t max_tokens, int32_t chunk);
+// whether the call runs without a plan (nrb as in AttnArgs)
+bool attn_direct(int64_t batch, int32_t hkv, int64_t nrb, int64_t max_tokens, int32_t chunk);
 hipError_t launch_verify_attn(const AttnArgs& a, hipStream_t s);
 // sdx_kv.hip
 hipError_t launch_kv_advance(int64_t* lengths, int64_t batch, int64_t q, hipStream_t s);

@@ -364,12 +364,11 @@ int sdx_kv_append_paged(void* pool, int64_t layer_stride, int64_t side_stride,
  * in chunks of chunk_tokens (0: the library's default for the shape; else a
  * multiple of 64, at most 1024) handled by separate workgroups, longest chunks
  * first; rows of more than one chunk merge fp32 partials (the row's last chunk
- * to finish merges it, or, in batches too small to fill the chip with chunks of
- * 1024, a second kernel; there the default chunk size also follows the rows'
- * lengths on the device, so a row's last bits may depend on the other rows: pass
- * chunk_tokens for a split of its own). `workspace` holds the chunk list, the
- * partials and the rows' arrival counters (sdx_verify_attention_workspace bytes,
- * 16-byte aligned, no initial contents). One or two kernels are queued on `stream`. A row
+ * to finish merges it, or, in small batches, a second kernel: the same sums in
+ * the same order, so a row's output depends on the call's shapes and the row
+ * alone). `workspace` holds the chunk list, the partials and the rows' arrival
+ * counters (sdx_verify_attention_workspace bytes, 16-byte aligned, no initial
+ * contents). One or two kernels are queued on `stream`. A row
  * whose shape is out of range sets *error (nullable) and is skipped; page ids
  * outside the pool set *error and the row's output is unspecified. bf16,
  * head_dim 64 or 128. A KV head with more than 64 query rows (max_q x query heads

@@ -223,15 +223,20 @@ def test_verify_attention_bench_shape_sampled_rows():
 
 
 @pytest.mark.parametrize("B,ctx_lo,ctx_hi,hq,hkv,d,k_max,chunk", [
-    # without a plan (fewer than 1,024 chunk slots): the workgroups find their chunks
+    # without a plan (at most 96 (row, KV head) pairs, chunks of fewer than 1,024 tokens
+    # and fewer than 1,024 slots of that): the workgroups find their chunks
     (1, 180, 184, 8, 2, 128, 4, 0),       # one chunk of up to 192 keys, no merge
     (1, 186, 420, 32, 8, 128, 4, 0),      # just past it: several chunks and the merge
     (1, 9000, 9000, 32, 8, 128, 4, 0),    # one long row over the whole chip
     (2, 5000, 5000, 4, 1, 64, 2, 0),      # 256 query heads x chunks of 16 threads per row
     (70, 1, 900, 2, 1, 128, 3, 0),        # rows past the first wave of 64
-    (127, 1, 700, 8, 8, 64, 2, 0),        # the most rows of a launch without a plan
-    (130, 1, 300, 4, 2, 128, 3, 64),      # a chunk size of the caller's
-    # with a plan (1,024 slots or more): merged by the last chunk of a row
+    (96, 1, 900, 2, 1, 128, 3, 0),        # the most rows of a launch without a plan
+    (48, 1, 300, 4, 2, 128, 3, 64),       # a chunk size of the caller's
+    # with a plan: merged by the last chunk of a row
+    (97, 1, 900, 2, 1, 128, 3, 0),
+    (8, 1, 4000, 32, 8, 128, 4, 1024),
+    (127, 1, 700, 8, 8, 64, 2, 0),
+    (130, 1, 300, 4, 2, 128, 3, 64),
     (128, 1, 300, 32, 8, 128, 5, 64),     # rows of one and of several chunks
     (128, 1, 900, 16, 8, 64, 5, 128),
     (130, 1, 100, 64, 8, 128, 8, 0),      # rows of one chunk, two blocks of query rows
@@ -244,21 +249,62 @@ def test_verify_attention_with_and_without_a_plan(B, ctx_lo, ctx_hi, hq, hkv, d,
     _check(inp, hq, hkv, chunk_tokens=chunk)
 
 
-@pytest.mark.parametrize("B", [3, 130])
+@pytest.mark.parametrize("B", [3, 96, 130])
 def test_verify_attention_skips_rows_it_cannot_serve(B):
     """A row whose length exceeds its block table sets the error word and keeps its
-    output; every other row is served (one-wave and several-wave row scans)."""
+    output; every other row is served (one wave of rows, two, and a plan)."""
     inp = attn_inputs(B, seed=B, device=DEV, ctx_lo=20, ctx_hi=400, hq=4, hkv=1, k_max=4)
     kv = inp["kv_len"].clone()
     kv[B - 1] = inp["block_table"].shape[1] * 16 + 1
     err = torch.zeros(1, dtype=torch.int32, device=DEV)
     args = (inp["q"], inp["cu_q"], inp["k_pool"], inp["v_pool"], inp["block_table"])
-    good = verify_attention_paged(*args, inp["kv_len"], inp["max_q"]).float()
+    good = verify_attention_paged(*args, inp["kv_len"], inp["max_q"])
     out = torch.full_like(inp["q"], 7.0)
     verify_attention_paged(*args, kv, inp["max_q"], out=out, error=err)
     torch.cuda.synchronize()
     last = int(inp["cu_q"][B - 1])
     assert int(err.item()) == 1
     assert bool((out[last:] == 7.0).all())
-    # the split follows the keys that are served, so only bf16 rounding may differ
-    assert torch.allclose(out[:last].float(), good[:last], atol=1e-2, rtol=1e-2)
+    assert torch.equal(out[:last], good[:last])
+
+
+def _wide_table(inp, tokens):
+    """The block table widened to `tokens` tokens a row (unused entries -1)."""
+    bt = inp["block_table"]
+    wide = torch.full((bt.shape[0], tokens // 16), -1, dtype=bt.dtype, device=bt.device)
+    wide[:, :bt.shape[1]] = bt
+    return wide
+
+
+@pytest.mark.parametrize("B,ctx_lo,ctx_hi,hq,hkv,d,k_max,chunk,wide", [
+    # narrow table: no plan; wide table (1,024 slots of 1,024 tokens or more): a plan
+    (1, 4000, 4100, 32, 8, 128, 4, 64, 131072),   # weights staged in LDS
+    (2, 8000, 8192, 32, 8, 128, 8, 64, 65536),    # too many for it: formed per element
+    (3, 700, 2600, 16, 4, 64, 4, 128, 131072),    # head dim 64; chunks past the last key
+    (2, 1500, 2600, 64, 8, 128, 8, 256, 65536),   # two blocks of query rows
+    (70, 1, 900, 2, 1, 128, 3, 64, 16384),        # rows past the first wave of 64
+])
+def test_verify_attention_same_bits_with_and_without_a_plan(B, ctx_lo, ctx_hi, hq, hkv, d, k_max,
+                                                            chunk, wide):
+    """At one chunk size the two launches add the same numbers in the same order."""
+    inp = attn_inputs(B, seed=B * 19 + ctx_hi, device=DEV, ctx_lo=ctx_lo, ctx_hi=ctx_hi, hq=hq,
+                      hkv=hkv, d=d, k_max=k_max, alpha_lo=0.6, alpha_hi=0.95)
+    args = (inp["q"], inp["cu_q"], inp["k_pool"], inp["v_pool"])
+    outs = [verify_attention_paged(*args, bt, inp["kv_len"], inp["max_q"], chunk_tokens=chunk)
+            for bt in (inp["block_table"], _wide_table(inp, wide))]
+    assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("chunk", [0, 128])
+@pytest.mark.parametrize("B,ctx", [(2, 30000), (8, 6000), (12, 4000)])
+def test_verify_attention_rows_do_not_depend_on_the_others(B, ctx, chunk):
+    """A row's output is the same bits whatever the lengths of the other rows."""
+    inp = attn_inputs(B, seed=B + ctx, device=DEV, ctx_lo=ctx - 100, ctx_hi=ctx, hq=16, hkv=8,
+                      k_max=4)
+    args = (inp["q"], inp["cu_q"], inp["k_pool"], inp["v_pool"], inp["block_table"])
+    kv = inp["kv_len"].clone()
+    kv[1:] = kv[1:] // 7 + 8
+    full = verify_attention_paged(*args, inp["kv_len"], inp["max_q"], chunk_tokens=chunk)
+    part = verify_attention_paged(*args, kv, inp["max_q"], chunk_tokens=chunk)
+    n = int(inp["cu_q"][1])
+    assert torch.equal(full[:n], part[:n])
