@@ -318,11 +318,16 @@ __device__ __forceinline__ ThrCut thr_cut(const ThrArgs& a, float m, float zf, f
     c.phi = b0 == 0 ? 2.0f : exp_det(-(float)b0 * inv) / zf;
     if (b1 < TH_NB - 1) {
       dlo = -(float)(b1 + 1) * inv;
-      c.plo = fmaxf(exp_det(dlo) / zf, 0x1p-149f);
+      c.plo = exp_det(dlo) / zf;
+      // a subnormal p can be the same over a whole unit of s: every positive p then
+      if (!(c.plo >= 0x1p-126f)) {
+        c.plo = 0x1p-149f;
+        dlo = -104.0f;
+      }
     }
   }
-  // no logit below xcut has p >= plo: p drops by more than its rounding within 1e-5
-  // of s, and the fp32 rounding of (m + dlo) T is within 1e-6 of its terms
+  // no logit below xcut has p >= plo: a normal p drops by more than its rounding within
+  // 1e-5 of s, and the fp32 rounding of (m + dlo) T is within 1e-6 of its terms
   c.xcut = ((m + dlo) - (4e-6f * (fabsf(m) + fabsf(dlo)) + 2e-5f)) * a.T;
   c.xcut -= 4e-6f * fabsf(c.xcut);
   if (!(fabsf(c.xcut) < INFINITY)) c.xcut = -INFINITY;

@@ -91,6 +91,26 @@ def test_to_probs_fp16_odd_rows(V):
         _same(got, O.to_probs(x.astype(np.float32), T, tp, tk))
 
 
+@pytest.mark.parametrize("V", [1000, 4097, 9000, 33000])
+def test_top_k_among_subnormal_probabilities(V):
+    """The k-th largest probability is subnormal: its tie group spans up to a unit of the
+    logits over T, far below the group's largest logit, and all of it is kept."""
+    rng = np.random.RandomState(V)
+    x = np.full((4, V), -200.0, np.float32)
+    x[0, [10, 20, 30]] = 0.0, -103.0, -103.5
+    for r in (1, 2):  # 70 logits where p runs from normal to 0
+        x[r, rng.permutation(V)[:70]] = -rng.uniform(85.0, 104.5, 70)
+        x[r, 5] = 0.0
+    x[3] = rng.randn(V) * 3
+    ties = 0
+    for T, tp, tk in [(1.0, 1.0, k) for k in range(2, 70)] + \
+            [(t, 0.9, k) for t in (0.02, 0.03, 0.05, 0.08) for k in (20, 50, 200)]:
+        ref = O.to_probs(x, T, tp, tk)
+        ties += int(((ref > 0).sum(-1) > tk).any())
+        _same(S.to_probs(torch.tensor(x, device=DEV), T, tp, tk).cpu().numpy(), ref)
+    assert ties > 5
+
+
 def test_top_k_of_all_but_one():
     x = _rows(9000, 1)
     got = S.to_probs(torch.tensor(x, device=DEV), 1.0, 1.0, 8999).cpu().numpy()
