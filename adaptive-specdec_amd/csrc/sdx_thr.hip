@@ -45,6 +45,8 @@
 // queues stay small enough for eight workgroups per CU (twice the queue: 20 us).
 #include "sdx_thr.hpp"
 
+#include <type_traits>
+
 namespace sdx {
 
 constexpr int TH_NT = 256;
@@ -277,8 +279,12 @@ __device__ __forceinline__ float thr_scale(float m, float xmn, float T, bool use
   while (scale < 0x1p20f && range * (2.0f * scale) <= (float)(TH_NB - 2)) scale *= 2.0f;
   return scale;
 }
-// One element of the histogram pass.
-template <int DIV, bool CNT>
+// One element of the histogram pass: its mass where the filter is a nucleus, its count
+// where it is a top-k (each an LDS atomic). What lies in the last step is not counted:
+// the k-th largest is there if no other step holds it, and at low temperatures most of
+// a row is (64 lanes at one LDS address go one after the other: fp16 verify of 16 rows,
+// V = 131,072, T = 0.1, top-k 20 97 us with it, 74 without).
+template <int DIV, bool MASS, bool CNT>
 __device__ __forceinline__ void thr_hist_one(float x, bool ok, float T, float rT, float m,
                                              float scale, uint64_t* mass, uint32_t* cnt,
                                              uint64_t& zlo, uint32_t& zhi) {
@@ -289,9 +295,9 @@ __device__ __forceinline__ void thr_hist_one(float x, bool ok, float T, float rT
   const uint64_t f = thr_exp62(d);
   zlo += f;
   zhi += zlo < f ? 1u : 0u;
-  if (CNT && ok) atomicAdd(&cnt[b], 1u);
+  if (CNT && b < (uint32_t)(TH_NB - 1)) atomicAdd(&cnt[b], 1u);  // (not ok: the last step)
   // 2^-44 units: sums of 2^18 elements fit 64 bits
-  if (f >> 18) atomicAdd((unsigned long long*)&mass[b], (unsigned long long)(f >> 18));
+  if (MASS && f >> 18) atomicAdd((unsigned long long*)&mass[b], (unsigned long long)(f >> 18));
 }
 // What a region of steps [b0, b1] (and the step bk of the k-th largest) decides.
 struct ThrCut {
@@ -367,14 +373,18 @@ __device__ __forceinline__ uint64_t thr_excl_u64(uint64_t v, uint64_t* s) {
   return off + incl - v;
 }
 
-template <class E, int DIV, bool CNT>
-__device__ __forceinline__ void thr_hist_pass(const ThrArgs& a, ThrHistLds& L, const E* row,
-                                              int part, float m, float scale, uint64_t& zlo,
-                                              uint32_t& zhi) {
-  const float T = a.T, rT = 1.0f / a.T;
-  thr_stream<E, 4>(row, a.V, part, a.nparts, a.plen, [&](int64_t, float x, bool ok) {
-    thr_hist_one<DIV, CNT>(x, ok, T, rT, m, scale, L.mass, L.cnt, zlo, zhi);
-  });
+// f(DIV, MASS, CNT) as integral constants, for the row's division and the call's filters.
+template <class F>
+__device__ __forceinline__ void thr_hist_kind(const ThrArgs& a, ThrDiv div, F&& f) {
+  auto kind = [&](auto mass, auto cnt) {
+    if (div == kDivOne) f(std::integral_constant<int, kDivOne>{}, mass, cnt);
+    else if (div == kDivFma) f(std::integral_constant<int, kDivFma>{}, mass, cnt);
+    else f(std::integral_constant<int, kDivIeee>{}, mass, cnt);
+  };
+  if (a.use_p && a.use_k) kind(std::true_type{}, std::true_type{});
+  else if (a.use_p) kind(std::true_type{}, std::false_type{});
+  else if (a.use_k) kind(std::false_type{}, std::true_type{});
+  else kind(std::false_type{}, std::false_type{});
 }
 
 template <class E>
@@ -400,15 +410,13 @@ __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
   __syncthreads();
   uint64_t zlo = 0;
   uint32_t zhi = 0;
-  if (a.use_k) {
-    if (div == kDivOne) thr_hist_pass<E, kDivOne, true>(a, L, x, part, m, scale, zlo, zhi);
-    else if (div == kDivFma) thr_hist_pass<E, kDivFma, true>(a, L, x, part, m, scale, zlo, zhi);
-    else thr_hist_pass<E, kDivIeee, true>(a, L, x, part, m, scale, zlo, zhi);
-  } else {
-    if (div == kDivOne) thr_hist_pass<E, kDivOne, false>(a, L, x, part, m, scale, zlo, zhi);
-    else if (div == kDivFma) thr_hist_pass<E, kDivFma, false>(a, L, x, part, m, scale, zlo, zhi);
-    else thr_hist_pass<E, kDivIeee, false>(a, L, x, part, m, scale, zlo, zhi);
-  }
+  const float rT = 1.0f / T;
+  thr_hist_kind(a, div, [&](auto DIV, auto MASS, auto CNT) {
+    thr_stream<E, 4>(x, a.V, part, a.nparts, a.plen, [&](int64_t, float xv, bool ok) {
+      thr_hist_one<DIV.value, MASS.value, CNT.value>(xv, ok, T, rT, m, scale, L.mass, L.cnt, zlo,
+                                                     zhi);
+    });
+  });
   U128 z = wave_sum_u128(U128{zlo, (uint64_t)zhi});
   if (lane == 0) { L.zl[wv] = z.lo; L.zh[wv] = (uint32_t)z.hi; }
   __syncthreads();  // and the histogram is complete
@@ -923,19 +931,6 @@ struct ThrSmallLds {
   int32_t b0, b1, bk, nf;
 };
 
-template <int NT, int DIV, bool CNT>
-__device__ __forceinline__ void thr_small_hist(const ThrArgs& a, ThrSmallLds<NT>& L,
-                                               const float (&x)[TS_PER], float m, float scale,
-                                               uint64_t& zlo, uint32_t& zhi) {
-  const float T = a.T, rT = 1.0f / a.T;
-#pragma unroll
-  for (int u = 0; u < TS_PER; ++u) {
-    if (u * NT >= a.V) break;  // uniform
-    const bool ok = u * NT + (int)threadIdx.x < a.V;
-    thr_hist_one<DIV, CNT>(x[u], ok, T, rT, m, scale, L.h.mass, L.h.cnt, zlo, zhi);
-  }
-}
-
 template <class E, int NT>
 __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, int64_t ld_out) {
   constexpr int NW = NT / kWave;
@@ -990,15 +985,15 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
   const ThrDiv div = thr_div_kind(T, mx);
   uint64_t zlo = 0;
   uint32_t zhi = 0;
-  if (a.use_k) {
-    if (div == kDivOne) thr_small_hist<NT, kDivOne, true>(a, L, x, m, scale, zlo, zhi);
-    else if (div == kDivFma) thr_small_hist<NT, kDivFma, true>(a, L, x, m, scale, zlo, zhi);
-    else thr_small_hist<NT, kDivIeee, true>(a, L, x, m, scale, zlo, zhi);
-  } else {
-    if (div == kDivOne) thr_small_hist<NT, kDivOne, false>(a, L, x, m, scale, zlo, zhi);
-    else if (div == kDivFma) thr_small_hist<NT, kDivFma, false>(a, L, x, m, scale, zlo, zhi);
-    else thr_small_hist<NT, kDivIeee, false>(a, L, x, m, scale, zlo, zhi);
-  }
+  const float rT = 1.0f / T;
+  thr_hist_kind(a, div, [&](auto DIV, auto MASS, auto CNT) {
+#pragma unroll
+    for (int u = 0; u < TS_PER; ++u) {
+      if (u * NT >= V) break;  // uniform
+      thr_hist_one<DIV.value, MASS.value, CNT.value>(x[u], u * NT + tid < V, T, rT, m, scale,
+                                                     L.h.mass, L.h.cnt, zlo, zhi);
+    }
+  });
   U128 z = wave_sum_u128(U128{zlo, (uint64_t)zhi});
   if (lane == 0) { L.s64[wv] = z.lo; L.t64[wv] = z.hi; }
   __syncthreads();  // and the histogram is complete
