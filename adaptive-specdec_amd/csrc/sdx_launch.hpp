@@ -221,12 +221,13 @@ struct ThrArgs {
   // pass and in the passes that only compare
   int32_t nparts, nlight;
   int64_t plen, llen;
+  float dmax;  // set by the launch: steps of the histogram pass reach this far below m
 };
 // (rows of at most kThrSmall elements need no scratch)
 hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s);
 // rows of at most kThrSmall elements: statistics (a.stats) and to_probs rows (out), each
 // where not null
-hipError_t launch_thr_small(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+hipError_t launch_thr_small(int dtype, ThrArgs a, int64_t rows, float* out, int64_t ld_out,
                             hipStream_t s);
 // to_probs rows; the scratch may lie in `out` (it is read no more)
 hipError_t launch_thr_output(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,

@@ -45,6 +45,7 @@
 // queues stay small enough for eight workgroups per CU (twice the queue: 20 us).
 #include "sdx_thr.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 namespace sdx {
@@ -67,10 +68,11 @@ __device__ __forceinline__ float thr_f(uint16_t c) { return decode16<SDX_F16>(c)
 // every lane of a wave makes every call (valid: the lane has an element), so f may
 // vote. UN vectors per thread are in flight; after them, g() runs once (code that
 // would otherwise stand once per element: in copies, its first passes wait for the
-// instruction cache).
-template <class E, int UN, class F, class G>
+// instruction cache). With SKIP, whole vectors of a wave below `low` are left out.
+template <class E, int UN, bool SKIP = false, class F, class G>
 __device__ __forceinline__ void thr_stream(const E* __restrict__ row, int64_t V, int part,
-                                           int nparts, int64_t plen, F&& f, G&& g) {
+                                           int nparts, int64_t plen, F&& f, G&& g,
+                                           float low = 0.0f) {
   constexpr int N = ThrVec<E>::N;
   const int tid = threadIdx.x;
   int64_t head = (int64_t)(((16u - ((uint32_t)(uintptr_t)row & 15u)) & 15u) / sizeof(E));
@@ -100,13 +102,20 @@ __device__ __forceinline__ void thr_stream(const E* __restrict__ row, int64_t V,
       const bool ok = j < v1;
       const int64_t i = head + j * N;
       const uint32_t q[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+      float x[N];
 #pragma unroll
       for (int e = 0; e < N; ++e) {
-        float x;
-        if constexpr (sizeof(E) == 4) x = __uint_as_float(q[e]);
-        else x = thr_f((uint16_t)(q[e >> 1] >> (16 * (e & 1))));
-        f(i + e, x, ok);
+        if constexpr (sizeof(E) == 4) x[e] = __uint_as_float(q[e]);
+        else x[e] = thr_f((uint16_t)(q[e >> 1] >> (16 * (e & 1))));
       }
+      if constexpr (SKIP) {
+        float mx = x[0];
+#pragma unroll
+        for (int e = 1; e < N; ++e) mx = fmaxf(mx, x[e]);
+        if (__ballot(ok && mx >= low) == 0) continue;  // uniform
+      }
+#pragma unroll
+      for (int e = 0; e < N; ++e) f(i + e, x[e], ok);
     }
     g();
   }
@@ -268,26 +277,44 @@ __device__ __forceinline__ ThrDiv thr_div_kind(float T, float xmax) {
   return T >= 0x1p-20f && T <= 0x1p20f && a <= 0x1p100f && (a >= 0x1p-90f || a == 0.0f) ? kDivFma
                                                                                        : kDivIeee;
 }
-// Steps of m - s per unit, 2^e: the row's range over at most TH_NB steps. The nucleus
-// ends within 32 of the maximum (below lies less than 2^18 e^-32 of the mass; a top_p
-// that near 1 takes the last step), the k-th largest anywhere p is above 0.
-__device__ __forceinline__ float thr_scale(float m, float xmn, float T, bool use_k) {
-  const float most = use_k ? 104.0f : 32.0f;
-  const float range = fminf(m - xmn / T, most);  // NaN (no finite logit): the most
-  float scale = use_k ? 8.0f : 32.0f;
+// Steps of m - s per unit, 2^e: the row's range, as far as it can hold the boundary
+// (a.dmax), over at most TH_NB steps. A small top-k bounds the elements of a step, and
+// takes a quarter of them: each step that is not empty is an atomic or two per part
+// (fp32 verify of 16 rows, V = 32,000, T = 0.7, top_p 0.9, top-k 50: histogram pass
+// 20.5 us with up to all steps, 16.3 with a quarter).
+__device__ __forceinline__ float thr_scale(const ThrArgs& a, float m, float xmn) {
+  const float range = fminf(m - xmn / a.T, a.dmax);  // NaN (no finite logit): the most
   static_assert(104 * 8 <= TH_NB - 2 && 32 * 32 <= TH_NB, "the widest range fits the steps");
-  while (scale < 0x1p20f && range * (2.0f * scale) <= (float)(TH_NB - 2)) scale *= 2.0f;
-  return scale;
+  const bool few = a.use_k && a.top_k <= 1024;
+  const float steps = few ? (float)(TH_NB / 4) : (float)(TH_NB - 2);
+  const float q = fminf(steps / fmaxf(range, 0x1p-10f), 0x1p20f);
+  const float least = a.dmax > 32.0f ? 8.0f : few ? 1.0f : 32.0f;
+  return fmaxf(__uint_as_float(__float_as_uint(q) & 0x7F800000u), least);
+}
+// The first step that is left out of the histogram: the last one, or the first past
+// a.dmax.
+__device__ __forceinline__ uint32_t thr_steps(const ThrArgs& a, float scale) {
+  return (uint32_t)fminf(a.dmax * scale + 1.0f, (float)(TH_NB - 1));
+}
+// Logits below this have no part in the histogram pass: m - s is past the steps and
+// past 43.5, below which the fixed-point exp is 0.
+__device__ __forceinline__ float thr_xskip(float m, float scale, uint32_t steps, float T) {
+  const float d = fmaxf(43.5f, (float)steps / scale);
+  float x = ((m - d) - (4e-6f * (fabsf(m) + d) + 2e-5f)) * T;  // as xcut below
+  x -= 4e-6f * fabsf(x);
+  return fabsf(x) < INFINITY ? x : -INFINITY;
 }
 // One element of the histogram pass: its mass where the filter is a nucleus, its count
-// where it is a top-k (each an LDS atomic). What lies in the last step is not counted:
-// the k-th largest is there if no other step holds it, and at low temperatures most of
-// a row is (64 lanes at one LDS address go one after the other: fp16 verify of 16 rows,
-// V = 131,072, T = 0.1, top-k 20 97 us with it, 74 without).
-template <int DIV, bool MASS, bool CNT>
+// where it is a top-k (each an LDS atomic). What lies past `steps` is left out: a
+// boundary that no step holds is there, and much of a row can be, most of it at low
+// temperatures (64 lanes at one LDS address go one after the other: fp16 verify of 16
+// rows, V = 131,072, T = 0.1, top-k 20 97 us with it, 74 without).
+// `steps` is past every element (ALL) where a top-k's range holds them and T does not
+// press them together: the comparison costs such a pass 2%.
+template <int DIV, bool MASS, bool CNT, bool ALL = false>
 __device__ __forceinline__ void thr_hist_one(float x, bool ok, float T, float rT, float m,
-                                             float scale, uint64_t* mass, uint32_t* cnt,
-                                             uint64_t& zlo, uint32_t& zhi) {
+                                             float scale, uint32_t steps, uint64_t* mass,
+                                             uint32_t* cnt, uint64_t& zlo, uint32_t& zhi) {
   const float d = ok ? thr_div<DIV>(x, T, rT) - m : -INFINITY;
   // NaN (-inf logits through the FMA steps): the last step; d > 0 never, and
   // v_cvt_u32_f32 would take it to 0
@@ -295,9 +322,11 @@ __device__ __forceinline__ void thr_hist_one(float x, bool ok, float T, float rT
   const uint64_t f = thr_exp62(d);
   zlo += f;
   zhi += zlo < f ? 1u : 0u;
-  if (CNT && b < (uint32_t)(TH_NB - 1)) atomicAdd(&cnt[b], 1u);  // (not ok: the last step)
+  const bool in = ALL ? ok : b < steps;  // (not ok: never)
+  if (CNT && in) atomicAdd(&cnt[b], 1u);
   // 2^-44 units: sums of 2^18 elements fit 64 bits
-  if (MASS && f >> 18) atomicAdd((unsigned long long*)&mass[b], (unsigned long long)(f >> 18));
+  const uint64_t fm = ALL || in ? f >> 18 : 0ull;  // (not ok: f is 0)
+  if (MASS && fm) atomicAdd((unsigned long long*)&mass[b], (unsigned long long)fm);
 }
 // What a region of steps [b0, b1] (and the step bk of the k-th largest) decides.
 struct ThrCut {
@@ -387,7 +416,11 @@ __device__ __forceinline__ void thr_hist_kind(const ThrArgs& a, ThrDiv div, F&& 
   else kind(std::false_type{}, std::false_type{});
 }
 
-template <class E>
+// SKIP: whole vectors of logits that have no part in the pass are left out. They are
+// most of a row at low temperatures, but the test ends the overlap of one vector's
+// chains with the next's: fp16 verify of 16 rows, V = 131,072, top-k 20 at T = 0.1 74 ->
+// 65 us with it; fp32 verify of 16 rows, V = 32,000 at T = 0.7 44 -> 49 us.
+template <class E, bool SKIP>
 __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
   __shared__ ThrHistLds L;
   const int64_t row = blockIdx.x / a.nparts;
@@ -405,17 +438,20 @@ __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
   }
   const float T = a.T;
   const float m = xmx / T;  // the division is monotone: the maximum of fl32(x / T)
-  const float scale = thr_scale(m, xmn, T, a.use_k);
+  const float scale = thr_scale(a, m, xmn);
   const ThrDiv div = thr_div_kind(T, xmx);
   __syncthreads();
   uint64_t zlo = 0;
   uint32_t zhi = 0;
   const float rT = 1.0f / T;
+  const uint32_t steps = thr_steps(a, scale);
+  const float low = thr_xskip(m, scale, steps, T);
   thr_hist_kind(a, div, [&](auto DIV, auto MASS, auto CNT) {
-    thr_stream<E, 4>(x, a.V, part, a.nparts, a.plen, [&](int64_t, float xv, bool ok) {
-      thr_hist_one<DIV.value, MASS.value, CNT.value>(xv, ok, T, rT, m, scale, L.mass, L.cnt, zlo,
-                                                     zhi);
-    });
+    auto one = [&](int64_t, float xv, bool ok) {
+      thr_hist_one<DIV.value, MASS.value, CNT.value, CNT.value && !SKIP>(
+          xv, ok, T, rT, m, scale, steps, L.mass, L.cnt, zlo, zhi);
+    };
+    thr_stream<E, 4, SKIP>(x, a.V, part, a.nparts, a.plen, one, [] {}, low);
   });
   U128 z = wave_sum_u128(U128{zlo, (uint64_t)zhi});
   if (lane == 0) { L.zl[wv] = z.lo; L.zh[wv] = (uint32_t)z.hi; }
@@ -981,7 +1017,8 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
 #pragma unroll
   for (int w = 0; w < NW; ++w) { mx = fmaxf(mx, L.mx[w]); mn = fminf(mn, L.mn[w]); }
   const float m = mx / T;
-  const float scale = thr_scale(m, mn, T, a.use_k);
+  const float scale = thr_scale(a, m, mn);
+  const uint32_t steps = thr_steps(a, scale);
   const ThrDiv div = thr_div_kind(T, mx);
   uint64_t zlo = 0;
   uint32_t zhi = 0;
@@ -991,7 +1028,7 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
     for (int u = 0; u < TS_PER; ++u) {
       if (u * NT >= V) break;  // uniform
       thr_hist_one<DIV.value, MASS.value, CNT.value>(x[u], u * NT + tid < V, T, rT, m, scale,
-                                                     L.h.mass, L.h.cnt, zlo, zhi);
+                                                     steps, L.h.mass, L.h.cnt, zlo, zhi);
     }
   });
   U128 z = wave_sum_u128(U128{zlo, (uint64_t)zhi});
@@ -1353,6 +1390,20 @@ __global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
 
 // ---------------------------------------------------------------- launches
 
+// How far below the maximum (in s) the boundary of a row can lie. Top-k: anywhere p is
+// above 0 (104 units). A nucleus ends where less than 1 - top_p of the mass is left,
+// and D units below the maximum that is at most V e^-D of it (of at least 1): within 15
+// units for V = 151,936 and top_p 0.95, so that a row's finite mask values do not widen
+// the steps; 32 units where top_p is so near 1 that its rounding counts. With a top-k
+// too, the nucleus bounds the range only at low temperatures (see thr_hist_one).
+constexpr float TH_LOWT = 0.25f;
+static float thr_dmax(const ThrArgs& a) {
+  const double most = a.use_k ? 104.0 : 32.0;
+  const double rest = 1.0 - (double)a.top_p - 2e-6;  // the region's margin of 1e-6, and roundings
+  if (!a.use_p || rest < 2e-6 || (a.use_k && a.T > TH_LOWT)) return (float)most;
+  return (float)fmin(most, log((double)a.V) - log(rest) + 0.25);
+}
+
 // Parts per row: about four workgroups per CU over the call, parts of at least 4,096
 // elements (below that a part's histogram costs more than its stream), and no more
 // than the first pass has words for.
@@ -1375,7 +1426,8 @@ template <class E>
 static hipError_t thr_stats(const ThrArgs& a, int64_t rows, hipStream_t s) {
   const dim3 grid((unsigned)(rows * a.nparts)), light((unsigned)(rows * a.nlight));
   hipLaunchKernelGGL(thr_max_kernel<E>, light, dim3(TH_NT), 0, s, a);
-  hipLaunchKernelGGL(thr_hist_kernel<E>, grid, dim3(TH_NT), 0, s, a);
+  if (a.T <= TH_LOWT) hipLaunchKernelGGL((thr_hist_kernel<E, true>), grid, dim3(TH_NT), 0, s, a);
+  else hipLaunchKernelGGL((thr_hist_kernel<E, false>), grid, dim3(TH_NT), 0, s, a);
   hipLaunchKernelGGL(thr_collect_kernel<E>, light, dim3(TH_NT), 0, s, a);
   hipLaunchKernelGGL(thr_resolve_kernel<E>, dim3((unsigned)rows), dim3(TH_NT), 0, s, a);
   return hipGetLastError();
@@ -1394,8 +1446,9 @@ static hipError_t thr_small(const ThrArgs& a, int64_t rows, float* out, int64_t 
   return hipGetLastError();
 }
 
-hipError_t launch_thr_small(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+hipError_t launch_thr_small(int dtype, ThrArgs a, int64_t rows, float* out, int64_t ld_out,
                             hipStream_t s) {
+  a.dmax = thr_dmax(a);
   if (a.V > kThrSmall || (!a.stats && !out)) return hipErrorInvalidValue;
   return dtype == SDX_F32 ? thr_small<float>(a, rows, out, ld_out, s)
                           : thr_small<uint16_t>(a, rows, out, ld_out, s);
@@ -1405,6 +1458,7 @@ hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s) {
   if (a.V <= kThrSmall) return launch_thr_small(dtype, a, rows, nullptr, 0, s);
   if (!a.scratch || a.scratch_bytes < kThrScratchMin || a.scratch_stride < a.scratch_bytes || !a.stats || a.V > kF32MaxVocab)
     return hipErrorInvalidValue;
+  a.dmax = thr_dmax(a);
   a.nparts = thr_parts(rows, a.V);
   const int64_t per = (a.V + a.nparts - 1) / a.nparts;
   a.plen = (per + 7) / 8 * 8;  // whole vectors of either element size
