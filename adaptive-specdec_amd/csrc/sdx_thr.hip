@@ -5,7 +5,8 @@
 //   p(id) = exp_det(s - m) / zf,  s = fl32(x / T)
 //   kept  = p > vf, or p == vf and id <= idcut      (p / totf where kept, else 0)
 // because the reference keeps a prefix of the order (p descending, id ascending).
-// The record takes four kernels over `nparts` workgroups per row and one small one:
+// The record takes three kernels over several workgroups per row (nlight of them where
+// a pass only compares, nparts in the histogram pass) and one with a workgroup per row:
 //   1. thr_max_kernel      the row's maximum (and minimum) logit per part;
 //   2. thr_hist_kernel     the exact normaliser (96-bit fixed point per thread), and
 //                          masses (and, for top-k, counts) of the elements in NB
@@ -19,8 +20,8 @@
 //                          and a list (p, id) of the region's;
 //   4. thr_resolve_kernel  one workgroup per row sorts the list and walks it with the
 //                          reference's test. A region with more than kThrList
-//                          elements (a large tie group) is refined over the row
-//                          itself, ten bits of p at a time;
+//                          elements (a tie group, or a flat row) is refined over the
+//                          row itself, a thousand bins of p at a time;
 // then thr_output_kernel writes to_probs rows, and thr_draw_kernel is the verify's
 // accept chain and draw, which evaluates p where it needs it: a verify writes no
 // probabilities.
@@ -278,14 +279,14 @@ __device__ __forceinline__ ThrDiv thr_div_kind(float T, float xmax) {
                                                                                        : kDivIeee;
 }
 // Steps of m - s per unit, 2^e: the row's range, as far as it can hold the boundary
-// (a.dmax), over at most TH_NB steps. A small top-k bounds the elements of a step, and
-// takes a quarter of them: each step that is not empty is an atomic or two per part
-// (fp32 verify of 16 rows, V = 32,000, T = 0.7, top_p 0.9, top-k 50: histogram pass
+// (a.dmax), over at most TH_NB steps; a quarter of them where a nucleus bounds the range
+// and a small top-k the elements of a step: each step that is not empty is an atomic or
+// two per part (fp32 verify of 16 rows, V = 32,000, top_p 0.9, top-k 50: histogram pass
 // 20.5 us with up to all steps, 16.3 with a quarter).
 __device__ __forceinline__ float thr_scale(const ThrArgs& a, float m, float xmn) {
   const float range = fminf(m - xmn / a.T, a.dmax);  // NaN (no finite logit): the most
   static_assert(104 * 8 <= TH_NB - 2 && 32 * 32 <= TH_NB, "the widest range fits the steps");
-  const bool few = a.use_k && a.top_k <= 1024;
+  const bool few = a.use_k && a.dmax <= 32.0f && a.top_k <= 1024;
   const float steps = few ? (float)(TH_NB / 4) : (float)(TH_NB - 2);
   const float q = fminf(steps / fmaxf(range, 0x1p-10f), 0x1p20f);
   const float least = a.dmax > 32.0f ? 8.0f : few ? 1.0f : 32.0f;
@@ -763,178 +764,370 @@ __device__ __forceinline__ RowStat thr_record(const ThrEnd& r, float m, float zf
   return st;
 }
 
+// ---- refinement: a region with more elements than its list holds (a tie group, or many
+// logits within a step) is split by p's bits, TH_NB bins a pass over the row, until the
+// bin that holds the boundary fits the list or is one value.
+struct ThrSpan {
+  uint32_t lo, hi;     // bits of p: the boundary is in [lo, hi]
+  uint64_t above;      // mass and count of the elements above hi
+  uint64_t nabove;
+  uint32_t n;          // elements in [lo, hi]
+  bool use_k, use_p;   // filters that [lo, hi] has to decide
+};
+struct ThrPickLds {
+  uint32_t fk, fp;
+  uint64_t mass, count, total;
+  uint32_t n;
+};
+__device__ __forceinline__ uint32_t thr_bin_shift(const ThrSpan& r) {
+  uint32_t sh = 0;
+  while (((r.hi - r.lo) >> sh) >= (uint32_t)TH_NB) ++sh;
+  return sh;
+}
+// r narrowed to the bin (2^sh values of p each, bin 0 at r.hi; their masses, counts and
+// least bits) that holds the boundary: the first in which the count from the top
+// reaches top_k, or whose last element fails the nucleus test, whichever comes first.
+// False: none does, everything in r is kept (r.above: with its mass).
+template <int NT>
+__device__ __forceinline__ bool thr_pick(const ThrArgs& a, const uint64_t* mass,
+                                         const uint32_t* cnt, const uint32_t* low, uint32_t sh,
+                                         ThrSpan& r, ThrPickLds& L, uint64_t* s64) {
+  constexpr int BPT = TH_NB / NT;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  if (tid == 0) L.fk = L.fp = ~0u;
+  uint64_t sm = 0, sc = 0;
+#pragma unroll
+  for (int i = 0; i < BPT; ++i) { sm += mass[tid * BPT + i]; sc += cnt[tid * BPT + i]; }
+  const uint64_t m0 = r.above + thr_excl_u64<NT / kWave>(sm, s64);
+  const uint64_t c0 = r.nabove + thr_excl_u64<NT / kWave>(sc, s64);
+  uint64_t rm = m0, rc = c0;
+  uint32_t mk = ~0u, mp = ~0u;
+#pragma unroll
+  for (int i = 0; i < BPT; ++i) {
+    const int b = tid * BPT + i;
+    const uint32_t n = cnt[b];
+    rm += mass[b];
+    rc += n;
+    if (n == 0) continue;
+    if (mk == ~0u && rc >= (uint64_t)a.top_k) mk = (uint32_t)b;
+    if (mp == ~0u && !((rn32_u64(rm) - __uint_as_float(low[b])) < a.top_p)) mp = (uint32_t)b;
+  }
+  if (tid == NT - 1) L.total = rm;
+  const uint64_t vk = __ballot(mk != ~0u), vp = __ballot(mp != ~0u);  // bins go up with the lane
+  if (vk && lane == __ffsll((unsigned long long)vk) - 1) atomicMin(&L.fk, mk);
+  if (vp && lane == __ffsll((unsigned long long)vp) - 1) atomicMin(&L.fp, mp);
+  __syncthreads();
+  const uint32_t fk = r.use_k ? L.fk : ~0u, fp = r.use_p ? L.fp : ~0u, f = min(fk, fp);
+  if (f == ~0u) {  // uniform
+    r.above = L.total;
+    __syncthreads();
+    return false;
+  }
+  if ((uint32_t)tid == f / BPT) {
+    rm = m0;
+    rc = c0;
+    for (uint32_t b = (uint32_t)tid * BPT; b < f; ++b) { rm += mass[b]; rc += cnt[b]; }
+    L.mass = rm;
+    L.count = rc;
+    L.n = cnt[f];
+  }
+  __syncthreads();
+  // the filter that ends in a later bin has no say
+  r.use_k = fk == f;
+  r.use_p = fp == f;
+  r.above = L.mass;
+  r.nabove = L.count;
+  r.n = L.n;
+  r.hi -= f << sh;
+  r.lo = max(r.lo, r.hi - (1u << sh) + 1u);
+  __syncthreads();
+  return true;
+}
+// How many members of the tie group of p = v pass the nucleus test, of n below mass
+// `above` and count `nabove` (a prefix; every wave the same search, 64 candidates a step).
+__device__ __forceinline__ uint64_t thr_tie_kept(float v, uint64_t above, uint64_t nabove,
+                                                 uint64_t n, float tp) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint64_t P = fixed62(v);
+  uint64_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint64_t step = (hi - lo + kWave - 1) / kWave;
+    const uint64_t cand = lo + (uint64_t)lane * step;
+    const bool keep = cand < hi && (((rn32_u64(above + (cand + 1) * P) - v) < tp) ||
+                                    (nabove + cand == 0));  // the row's first is always kept
+    const int nk = __popcll(__ballot(keep));
+    if (nk == 0) break;
+    const uint64_t last = lo + (uint64_t)(nk - 1) * step;
+    lo = last + 1;
+    hi = min(hi, last + step);
+  }
+  return lo;
+}
+// The end at a single value of p, of which `kept` members are.
+__device__ __forceinline__ ThrEnd thr_tie_end(const ThrSpan& r, uint64_t kept) {
+  ThrEnd e;
+  e.vf = __uint_as_float(kept > 0 ? r.lo : r.lo + 1u);  // none: everything above
+  e.tot = r.above + kept * fixed62(__uint_as_float(r.lo));
+  e.partial = kept > 0 && kept < r.n;
+  return e;
+}
+// One region element's share of the bins, where `in`; lanes that hold one value (a
+// tie group) add it once.
+__device__ __forceinline__ void thr_bin_add(bool in, uint32_t bits, uint32_t hi, uint32_t sh,
+                                            uint64_t* mass, uint32_t* cnt, uint32_t* low) {
+  const uint64_t bm = __ballot(in);
+  if (bm == 0) return;  // uniform
+  const int src = __ffsll((unsigned long long)bm) - 1;
+  const uint32_t first = rdlane(bits, src);
+  const bool one = __ballot(in && bits != first) == 0;
+  if (one ? (int)(threadIdx.x & (kWave - 1)) == src : in) {
+    const uint32_t b = (hi - bits) >> sh, n = one ? (uint32_t)__popcll(bm) : 1u;
+    atomicAdd((unsigned long long*)&mass[b], (unsigned long long)(n * fixed62(__uint_as_float(bits))));
+    atomicAdd(&cnt[b], n);
+    atomicMin(&low[b], bits);
+  }
+}
+
 constexpr int kThrCount = 2 * TH_NT;  // lists up to here are sorted by counting
+template <int NT>
 struct ThrResLds {
   uint64_t e[kThrList];  // the list; the refinement's masses
-  uint64_t t[kThrCount];  // a list of up to kThrCount entries, sorted
   uint32_t cnt[TH_NB], low[TH_NB];
-  uint64_t s64[TH_NW];
+  uint64_t s64[NT / kWave];
   ThrWalkLds w;
-  uint32_t first, idcut;
-  uint64_t base;
-  uint32_t nbase, bin;
+  ThrPickLds pick;
+  uint32_t n, idcut;
+  union {
+    uint64_t t[kThrCount];  // a list of up to kThrCount entries, sorted
+    ThrQueue<4> q[NT / kWave];
+  };
 };
 static_assert(kThrList >= kThrCount && kThrList >= TH_NB, "the refinement's masses use the list's space");
 
-// p's bits at the boundary by ten bits a pass over the row (bits of p <= 1 are below
-// 2^30): the bin in which the count from the top first reaches top_k (COUNT), or whose
-// last element first fails the nucleus test, then its own bins, down to one value.
-// Returns false when no bin does. base / nbase: mass and count above the value.
-template <class E, bool COUNT>
-__device__ __forceinline__ bool thr_refine(const ThrArgs& a, ThrResLds& L, const E* x,
-                                           const ThrCtl* c, float kth, uint32_t* value,
-                                           uint64_t* base, uint64_t* nbase, uint32_t* count) {
-  const int tid = threadIdx.x, lane = tid & (kWave - 1);
-  const float m = c->m, zf = c->zf, xcut = c->xcut, T = a.T;
-  uint32_t hi = 0;  // the chosen leading bits
-  uint64_t S = 0, NB = 0;
-  for (int sh = 20; sh >= 0; sh -= 10) {
-    __syncthreads();
-    for (int b = tid; b < TH_NB; b += TH_NT) { L.e[b] = 0ull; L.cnt[b] = 0u; L.low[b] = ~0u; }
-    if (tid == 0) L.first = ~0u;
-    __syncthreads();
-    thr_stream<E, 4>(x, a.V, 0, 1, a.plen, [&](int64_t, float xv, bool ok) {
-      if (!(ok && xv >= xcut)) return;
-      const float p = exp_det(xv / T - m) / zf;
-      if (!(p > 0.0f) || p < kth) return;
-      const uint32_t bits = __float_as_uint(p);
-      if (sh < 20 && (bits >> (sh + 10)) != hi) return;
-      const uint32_t b = (uint32_t)(TH_NB - 1) - ((bits >> sh) & (uint32_t)(TH_NB - 1));
-      atomicAdd((unsigned long long*)&L.e[b], (unsigned long long)fixed62(p));
-      atomicAdd(&L.cnt[b], 1u);
-      atomicMin(&L.low[b], bits);
-    });
-    __syncthreads();
-    uint64_t sm = 0, sc = 0;
-#pragma unroll
-    for (int i = 0; i < TH_BPT; ++i) { sm += L.e[tid * TH_BPT + i]; sc += L.cnt[tid * TH_BPT + i]; }
-    const uint64_t m0 = S + thr_excl_u64(sm, L.s64), c0 = NB + thr_excl_u64(sc, L.s64);
-    uint64_t rm = m0, rc = c0;
-    uint32_t mine = ~0u;
-    uint64_t bm = 0, bc = 0;
-    for (int i = 0; i < TH_BPT; ++i) {
-      const int b = tid * TH_BPT + i;
-      const uint32_t n = L.cnt[b];
-      if (n == 0) continue;
-      const uint64_t nm = rm + L.e[b], nc = rc + n;
-      const bool hit = COUNT ? nc >= (uint64_t)a.top_k
-                             : !((rn32_u64(nm) - __uint_as_float(L.low[b])) < a.top_p);
-      if (hit) { mine = (uint32_t)b; bm = rm; bc = rc; break; }
-      rm = nm;
-      rc = nc;
+// Logits that can have p in [lo, hi] (bits): m - s = -ln(p zf), with the margins of xcut;
+// a subnormal bound does not cut.
+struct ThrWindow {
+  float lo, hi;
+  __device__ __forceinline__ ThrWindow(const ThrCtl* c, float T, uint32_t pl, uint32_t ph) {
+    const float m = c->m, lz = logf(c->zf);
+    auto at = [&](uint32_t bits, float sgn) {
+      const float d = logf(__uint_as_float(bits)) + lz;
+      const float x = ((m + d) + sgn * (4e-6f * (fabsf(m) + fabsf(d)) + 2e-5f)) * T;
+      return x + sgn * 4e-6f * fabsf(x);
+    };
+    lo = pl >= 0x00800000u ? fmaxf(at(pl, -1.0f), c->xcut) : c->xcut;
+    hi = ph >= 0x00800000u ? at(ph, 1.0f) : INFINITY;
+    if (!(fabsf(lo) < INFINITY)) lo = c->xcut;
+    if (!(fabsf(hi) < INFINITY)) hi = INFINITY;
+  }
+  __device__ __forceinline__ bool has(float x) const { return x >= lo && x <= hi; }
+};
+// p of an element, the lanes' where `ok`; a wave whose logits are all the last one's
+// (a tie group) keeps its p.
+struct ThrEval {
+  float m, zf, T, lx = __builtin_nanf(""), lp = 0.0f;
+  __device__ __forceinline__ float operator()(float x, bool ok) {
+    if (__ballot(ok && x != lx) == 0) return lp;  // uniform
+    const float p = exp_det_sel(x / T - m) / zf;
+    const uint64_t bm = __ballot(ok);
+    const int src = __ffsll((unsigned long long)bm) - 1;
+    const float x0 = __uint_as_float(rdlane(__float_as_uint(x), src));
+    if (__ballot(ok && x != x0) == 0) {
+      lx = x0;
+      lp = __uint_as_float(rdlane(__float_as_uint(p), src));
     }
-    const uint64_t vote = __ballot(mine != ~0u);
-    if (vote && lane == __ffsll((unsigned long long)vote) - 1) atomicMin(&L.first, mine);
+    return p;
+  }
+};
+// Every element of the row in the window through g(x, id, ok) by full waves of the
+// NT threads; 16 elements a lane in flight.
+template <class E, int NT, class G>
+__device__ __forceinline__ void thr_scan(const E* __restrict__ row, int64_t V, const ThrWindow& w,
+                                         ThrQueue<4>& q, G&& g) {
+  constexpr int N = ThrVec<E>::N, UN = 16 / N;
+  const int tid = threadIdx.x;
+  uint32_t n = 0;
+  int64_t head = (int64_t)(((16u - ((uint32_t)(uintptr_t)row & 15u)) & 15u) / sizeof(E));
+  if (head > V) head = V;
+  const int64_t nv = (V - head) / N;
+  if (tid < kWave) {  // the ends, as in thr_stream
+    const int64_t i = tid < 32 ? tid : head + nv * N + (tid - 32);
+    const bool ok = tid < 32 ? i < head : i < V;
+    const float x = ok ? thr_f(row[i]) : 0.0f;
+    thr_push(q, n, x, (uint32_t)i, ok && w.has(x));
+  }
+  const uint4* __restrict__ x4 = reinterpret_cast<const uint4*>(row + head);
+  for (int64_t b = 0; b < nv; b += (int64_t)UN * NT) {  // uniform
+    uint4 v[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int64_t j = b + (int64_t)u * NT + tid;
+      v[u] = j < nv ? x4[j] : make_uint4(0, 0, 0, 0);
+    }
+#pragma nounroll
+    for (int h = 0; h < 4; ++h) {  // four elements of each lane, by selects (see the output)
+      const int u = h * UN / 4;
+      uint4 y = v[0];
+#pragma unroll
+      for (int k = 1; k < UN; ++k) {
+        y.x = u == k ? v[k].x : y.x;
+        y.y = u == k ? v[k].y : y.y;
+        y.z = u == k ? v[k].z : y.z;
+        y.w = u == k ? v[k].w : y.w;
+      }
+      const int64_t j = b + (int64_t)u * NT + tid;
+      const int64_t i = head + j * N + (N > 4 ? 4 * (h & 1) : 0);
+      if constexpr (N > 4) {
+        y.x = h & 1 ? y.z : y.x;
+        y.y = h & 1 ? y.w : y.y;
+      }
+      const uint32_t c[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float x;
+        if constexpr (sizeof(E) == 4) x = __uint_as_float(c[e]);
+        else x = thr_f((uint16_t)(c[e >> 1] >> (16 * (e & 1))));
+        thr_push(q, n, x, (uint32_t)(i + e), j < nv && w.has(x));
+      }
+      thr_drain(q, n, false, g);
+    }
+  }
+  thr_drain(q, n, true, g);
+}
+// The id of member `k` (from 0, by id) of the tie group of p = v: the ids are split over
+// the waves, which count their members, then the part that holds it again.
+template <class E, int NT>
+__device__ __forceinline__ uint32_t thr_member(const ThrArgs& a, ThrResLds<NT>& L, const E* row,
+                                               const ThrWindow& w, ThrEval ev, float v, uint64_t k) {
+  constexpr int NW = NT / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  int64_t lo = 0, hi = a.V;
+  auto members = [&](float x, bool ok) {
+    const bool c = ok && w.has(x);
+    return __ballot(c) == 0 ? 0ull : __ballot(ev(x, c) == v && c);
+  };
+  while (hi - lo > kWave) {  // uniform
+    const int64_t per = ((hi - lo + NW - 1) / NW + kWave - 1) / kWave * kWave;
+    const int64_t i0 = lo + wv * per, i1 = min(hi, i0 + per);
+    uint32_t n = 0;
+    for (int64_t i = i0; i < i1; i += 8 * kWave) {
+      E c[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) c[u] = row[min(i + u * kWave + lane, hi - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        n += (uint32_t)__popcll(members(thr_f(c[u]), i + u * kWave + lane < i1));
+    }
     __syncthreads();
-    const uint32_t f = L.first;
-    if (f == ~0u) {  // uniform: none (the first pass only, as a chosen bin holds a hit)
+    if (lane == 0) L.s64[wv] = n;
+    __syncthreads();
+    int s = 0;
+    while (s < NW - 1 && k >= L.s64[s]) k -= L.s64[s++];
+    lo += s * per;
+    hi = min(hi, lo + per);
+  }
+  const bool ok = lo + lane < hi;
+  const uint64_t bm = members(ok ? thr_f(row[lo + lane]) : 0.0f, ok);
+  const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
+                                                __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+  if (wv == 0 && ((bm >> lane) & 1u) && at == (uint32_t)k) L.idcut = (uint32_t)(lo + lane);
+  __syncthreads();
+  return L.idcut;
+}
+// True: e is the end. False: r is narrowed to at most kThrList elements, which are in
+// L.e. A pass takes about 15 us at 151,936 elements: the row by one CU, compared with the
+// window, the elements in it evaluated by full waves.
+template <class E, int NT>
+__device__ __forceinline__ bool thr_refine(const ThrArgs& a, ThrResLds<NT>& L, const E* x,
+                                           const ThrCtl* c, ThrSpan& r, ThrEnd& e) {
+  const int tid = threadIdx.x, wv = tid / kWave;
+  ThrEval ev{c->m, c->zf, a.T};
+  while (true) {  // at most four rounds: [lo, hi] shrinks by TH_NB
+    const ThrWindow w(c, a.T, r.lo, r.hi);
+    __syncthreads();
+    if (r.n <= (uint32_t)kThrList) {
+      if (tid == 0) L.n = 0u;
       __syncthreads();
-      *base = 0;
+      thr_scan<E, NT>(x, a.V, w, L.q[wv], [&](float xv, uint32_t id, bool ok) {
+        const uint32_t bits = __float_as_uint(ev(xv, ok));
+        const bool in = ok && bits >= r.lo && bits <= r.hi;
+        const uint64_t bm = __ballot(in);
+        if (bm == 0) return;  // uniform
+        uint32_t at = 0;
+        if ((tid & (kWave - 1)) == 0) at = atomicAdd(&L.n, (uint32_t)__popcll(bm));
+        at = rdlane(at, 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+        if (in && at < (uint32_t)kThrList) L.e[at] = ((uint64_t)(~bits) << 32) | id;
+      });
+      __syncthreads();
       return false;
     }
-    if (mine == f) { L.base = bm; L.nbase = (uint32_t)bc; L.bin = L.cnt[f]; }
+    if (r.lo == r.hi) {
+      const float v = __uint_as_float(r.lo);
+      const uint64_t kept = r.use_p ? thr_tie_kept(v, r.above, r.nabove, r.n, a.top_p) : r.n;
+      e = thr_tie_end(r, kept);
+      if (e.partial) e.idcut = thr_member<E, NT>(a, L, x, w, ev, v, kept - 1);
+      return true;
+    }
+    for (int b = tid; b < TH_NB; b += NT) { L.e[b] = 0ull; L.cnt[b] = 0u; L.low[b] = ~0u; }
     __syncthreads();
-    S = L.base;
-    NB = L.nbase;
-    *count = L.bin;
-    hi = (hi << 10) | ((uint32_t)(TH_NB - 1) - f);
+    const uint32_t sh = thr_bin_shift(r);
+    thr_scan<E, NT>(x, a.V, w, L.q[wv], [&](float xv, uint32_t, bool ok) {
+      const uint32_t bits = __float_as_uint(ev(xv, ok));
+      thr_bin_add(ok && bits >= r.lo && bits <= r.hi, bits, r.hi, sh, L.e, L.cnt, L.low);
+    });
+    __syncthreads();
+    if (!thr_pick<NT>(a, L.e, L.cnt, L.low, sh, r, L.pick, L.s64)) {
+      e.vf = __uint_as_float(r.lo);
+      e.tot = r.above;
+      return true;
+    }
   }
-  *value = hi;
-  *base = S;
-  *nbase = NB;
-  return true;
 }
 
-template <class E>
-__global__ void __launch_bounds__(TH_NT) thr_resolve_kernel(ThrArgs a) {
-  __shared__ ThrResLds L;
+// One workgroup per row. Only a refinement uses more than the first TH_NT threads; the
+// others end at once otherwise. NT 1,024 where every row has a CU of its own (a row of
+// 131,072 equal logits, T = 0.7, top_p 0.9, top-k 50 231 us against 546 with 256), 256
+// for more rows (fp16 to_probs of 576 rows of 32,000 85 us, 89 with 1,024).
+template <class E, int NT>
+__global__ void __launch_bounds__(NT) thr_resolve_kernel(ThrArgs a) {
+  __shared__ ThrResLds<NT> L;
   const int64_t row = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const ThrCtl* const c = thr_ctl(a, row);
-  const E* const x = thr_row<E>(a, row);
-  const float m = c->m, zf = c->zf, T = a.T, tp = a.top_p;
   const uint32_t n = c->nlist;
-  const bool use_k = c->use_k != 0, use_p = c->use_p != 0;
-  const uint64_t above = wave_sum_u64(lane < a.nlight ? c->pmass[lane] : 0ull);
-  const uint64_t nabove = wave_sum_u32(lane < a.nlight ? c->pcnt[lane] : 0u);
+  if (n <= (uint32_t)kThrList && tid >= TH_NT) return;  // whole waves
+  const E* const x = thr_row<E>(a, row);
+  const float m = c->m, zf = c->zf, T = a.T;
+  ThrSpan sp;
+  sp.above = wave_sum_u64(lane < a.nlight ? c->pmass[lane] : 0ull);
+  sp.nabove = wave_sum_u32(lane < a.nlight ? c->pcnt[lane] : 0u);
+  sp.n = n;
+  sp.use_k = c->use_k != 0;
+  sp.use_p = c->use_p != 0;
   const int64_t gid = thr_gid(a, row);
   const float xg = gid >= 0 && gid < a.V ? thr_f(x[gid]) : 0.0f;
+  float phi = c->phi;
   ThrEnd r;
-  float& vf = r.vf;
-  uint32_t& idcut = r.idcut;
-  bool& partial = r.partial;
-  uint64_t& tot = r.tot;
-  tot = above;
-  if (n > (uint32_t)kThrList) {  // uniform
-    float kth = 0.0f;
-    uint32_t v, gc;
-    uint64_t S, N;
-    if (use_k && thr_refine<E, true>(a, L, x, c, 0.0f, &v, &S, &N, &gc)) kth = __uint_as_float(v);
-    uint64_t r0 = 0;
-    if (use_p && thr_refine<E, false>(a, L, x, c, kth, &v, &S, &N, &gc)) {
-      // members kept: a prefix (the first element of the row is always kept)
-      vf = __uint_as_float(v);
-      const uint64_t P = fixed62(vf);
-      uint64_t lo = 0, hi = gc;
-      while (lo < hi) {  // every wave the same search, 64 candidates a step
-        const uint64_t step = (hi - lo + kWave - 1) / kWave;
-        const uint64_t cand = lo + (uint64_t)lane * step;
-        const bool keep = cand < hi &&
-                          (((rn32_u64(S + (cand + 1) * P) - vf) < tp) || (N + cand == 0));
-        const int nk = __popcll(__ballot(keep));
-        if (nk == 0) break;
-        const uint64_t lastk = lo + (uint64_t)(nk - 1) * step;
-        lo = lastk + 1;
-        hi = min(hi, lastk + step);
-      }
-      r0 = lo;
-      tot = S + r0 * P;
-      partial = r0 > 0 && r0 < gc;
-      if (r0 == 0) {
-        // no member is kept, and no id is -1: everything above vf is
-        vf = __uint_as_float(v + 1u);
-      } else if (partial) {  // the id of the r0-th member
-        uint64_t seen = 0;
-        if (tid == 0) L.idcut = 0u;
-        for (int64_t i0 = 0; i0 < a.V; i0 += TH_NT) {  // uniform
-          const int64_t i = i0 + tid;
-          const bool mem = i < a.V && exp_det(thr_f(x[i]) / T - m) / zf == vf;
-          const uint64_t bm = __ballot(mem);
-          __syncthreads();
-          if (lane == 0) L.s64[wv] = (uint64_t)__popcll(bm);
-          __syncthreads();
-          uint64_t off = seen, all = 0;
-          for (int w = 0; w < TH_NW; ++w) { off += w < wv ? L.s64[w] : 0ull; all += L.s64[w]; }
-          if (mem && off + (uint64_t)__popcll(bm & ((1ull << lane) - 1ull)) == r0 - 1)
-            L.idcut = (uint32_t)i;
-          seen += all;
-          if (seen >= r0) break;  // uniform
-        }
-        __syncthreads();
-        idcut = L.idcut;
-      }
-    } else {  // everything that top-k keeps
-      vf = kth > 0.0f ? kth : -1.0f;
-      uint64_t s = 0;
-      thr_stream<E, 4>(x, a.V, 0, 1, a.plen, [&](int64_t, float xv, bool ok) {
-        const float p = ok ? exp_det_sel(xv / T - m) / zf : 0.0f;
-        s += p >= kth ? fixed62(p) : 0ull;
-      });
-      s = wave_sum_u64(s);
-      __syncthreads();
-      if (lane == 0) L.s64[wv] = s;
-      __syncthreads();
-      tot = 0;
-      for (int w = 0; w < TH_NW; ++w) tot += L.s64[w];
-    }
-  } else if (use_k || use_p) {
+  r.tot = sp.above;
+  bool done = !(sp.use_k || sp.use_p);
+  if (__builtin_expect(n > (uint32_t)kThrList, 0)) {  // uniform
+    sp.lo = __float_as_uint(c->plo);
+    sp.hi = __float_as_uint(fminf(phi, 1.0f));
+    done = thr_refine<E, NT>(a, L, x, c, sp, r);
+    phi = __uint_as_float(sp.hi);
+    if (tid >= TH_NT) return;  // whole waves
+  } else if (!done) {
     const uint64_t* const list = reinterpret_cast<const uint64_t*>(c + 1);
+    for (uint32_t i = tid; i < n; i += TH_NT) L.e[i] = list[i];
+  }
+  if (!done) {  // uniform
     uint32_t S = kThrCount;
-    while (S < n) S <<= 1;
-    for (uint32_t i = tid; i < S; i += TH_NT) L.e[i] = i < n ? list[i] : ~0ull;
+    while (S < sp.n) S <<= 1;
+    for (uint32_t i = sp.n + tid; i < S; i += TH_NT) L.e[i] = ~0ull;
     __syncthreads();
-    r = thr_walk<TH_NT>(a, thr_sort<TH_NT, kThrCount>(L.e, L.t, n), n, use_k, use_p, above, nabove, c->phi,
-                        L.w, L.s64);
+    r = thr_walk<TH_NT>(a, thr_sort<TH_NT, kThrCount>(L.e, L.t, sp.n), sp.n, sp.use_k, sp.use_p,
+                        sp.above, sp.nabove, phi, L.w, L.s64);
   }
   const bool nonfinite = __ballot(lane < a.nlight && c->pnf[lane < a.nlight ? lane : 0] != 0) != 0;
   if (tid == 0) a.stats[row] = thr_record(r, m, zf, c->xcut, gid, a.V, xg, T, nonfinite);
@@ -1429,7 +1622,10 @@ static hipError_t thr_stats(const ThrArgs& a, int64_t rows, hipStream_t s) {
   if (a.T <= TH_LOWT) hipLaunchKernelGGL((thr_hist_kernel<E, true>), grid, dim3(TH_NT), 0, s, a);
   else hipLaunchKernelGGL((thr_hist_kernel<E, false>), grid, dim3(TH_NT), 0, s, a);
   hipLaunchKernelGGL(thr_collect_kernel<E>, light, dim3(TH_NT), 0, s, a);
-  hipLaunchKernelGGL(thr_resolve_kernel<E>, dim3((unsigned)rows), dim3(TH_NT), 0, s, a);
+  if (rows <= 256)
+    hipLaunchKernelGGL((thr_resolve_kernel<E, 1024>), dim3((unsigned)rows), dim3(1024), 0, s, a);
+  else
+    hipLaunchKernelGGL((thr_resolve_kernel<E, 256>), dim3((unsigned)rows), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

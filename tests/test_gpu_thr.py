@@ -111,6 +111,30 @@ def test_top_k_among_subnormal_probabilities(V):
     assert ties > 5
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("V", [9001, 33000, 151936])
+def test_to_probs_refined_rows(dtype, V):
+    """Regions past the list of 2,048: flat rows whose masked ids (a finite value) widen
+    the steps, tie groups within and across them, values too near for the first bins.
+    The boundary ends in a short list, in a tie group (whole or in part) or nowhere."""
+    rng = np.random.RandomState(V)
+    x = np.stack([rng.randn(V), rng.randn(V), np.round(rng.randn(V) * 8) / 8, rng.randn(V) * 1e-3,
+                  np.where(np.arange(V) % 3 == 0, 2.0, -1.0), np.full(V, 0.5),
+                  np.where(rng.rand(V) < 0.5, 1.25, rng.randn(V))])
+    x[1:, :: V // 100] = -1e4
+    t = torch.tensor(x).to(dtype)
+    x = t.float().numpy()
+    for T, tp, tk in [(1.5, 0.9, 0), (4.0, 0.9, 0), (2.0, 1.0, 5000), (8.0, 1.0, V // 2),
+                      (3.0, 0.6, V // 4), (8.0, 0.3, V // 4), (8.0, 0.3, V // 3 + 2),
+                      (50.0, 0.5, 0), (50.0, 1.0, V - 200), (50.0, 0.999999, 0)]:
+        ref = O.to_probs(x, T, tp, tk)
+        _same(S.to_probs(t.to(DEV), T, tp, tk).cpu().numpy(), ref)
+        if V == 9001:  # more rows than CUs: smaller workgroups
+            got = S.to_probs(t.to(DEV).repeat(40, 1), T, tp, tk).view(40, *t.shape)
+            assert torch.equal(got, got[:1].expand_as(got))
+            _same(got[0].cpu().numpy(), ref)
+
+
 def test_top_k_of_all_but_one():
     x = _rows(9000, 1)
     got = S.to_probs(torch.tensor(x, device=DEV), 1.0, 1.0, 8999).cpu().numpy()
