@@ -1135,20 +1135,19 @@ __global__ void __launch_bounds__(NT) thr_resolve_kernel(ThrArgs a) {
 
 // ---------------------------------------------------------------- short rows
 // Rows of at most kThrSmall elements: the same in one launch, a workgroup per row that
-// holds the row in registers (TS_PER elements a thread: 256 threads for rows of up to
-// 2,048, 512 up to 4,096, 1,024 above, so that short rows share a CU) and the whole
-// region in LDS (no refinement). With `out`, also the to_probs row. Bound by the
-// latency of its chain of block reductions. to_probs of 64 fp32 rows of 4,096: 15 us
-// against 69 us for a bitonic sort of the row in LDS, of 256 of 8,192 20 against 131 us,
-// of 20,000 of 64 143 against 1,141 us.
-constexpr int TS_PER = 8;
+// holds the row in registers (PER elements a thread: 256 threads for rows of up to
+// 2,048, 512 up to 4,096, 1,024 above, so that short rows share a CU). A region of more
+// than a list of NT is refined as above, from the registers. With `out`, also the
+// to_probs row. Bound by the latency of its chain of block reductions. to_probs of 64
+// fp32 rows of 4,096: 15 us against 69 us for a bitonic sort of the row in LDS, of 256
+// of 8,192 20 against 131 us, of 20,000 of 64 143 against 1,141 us.
 template <int NT>
 struct ThrSmallLds {
-  uint64_t e[TS_PER * NT];  // the region's list
+  uint64_t e[NT];  // the region's list
   union {
     struct {
       uint64_t mass[TH_NB];
-      uint32_t cnt[TH_NB];
+      uint32_t cnt[TH_NB], low[TH_NB];
     } h;
     uint64_t t[NT];
   };
@@ -1156,11 +1155,86 @@ struct ThrSmallLds {
   uint32_t u32[NT / kWave];
   float mx[NT / kWave], mn[NT / kWave];
   ThrWalkLds w;
-  uint32_t n;
+  ThrPickLds pick;
+  uint32_t n, idcut;
   int32_t b0, b1, bk, nf;
 };
+// Appends the lanes' (p, id) with `in` to the list of NT, counting all.
+template <int NT>
+__device__ __forceinline__ void thr_small_list(ThrSmallLds<NT>& L, bool in, float p, uint32_t id) {
+  const uint64_t bm = __ballot(in);
+  if (bm == 0) return;  // uniform per wave
+  uint32_t at = 0;
+  if ((threadIdx.x & (kWave - 1)) == 0) at = atomicAdd(&L.n, (uint32_t)__popcll(bm));
+  at = rdlane(at, 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
+                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+  if (in && at < (uint32_t)NT) L.e[at] = ((uint64_t)(~__float_as_uint(p)) << 32) | id;
+}
+// The refinement: as thr_refine, over the p of the workgroup's elements u NT + thread
+// (0 past the row).
+template <int NT, int PER>
+__device__ __forceinline__ bool thr_small_refine(const ThrArgs& a, ThrSmallLds<NT>& L,
+                                                 const float (&p)[PER], ThrSpan& r, ThrEnd& e) {
+  constexpr int NW = NT / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  static_assert(PER * NW <= TH_NB, "the members' counts use the bins' space");
+  while (true) {  // at most four rounds: [lo, hi] shrinks by TH_NB
+    __syncthreads();
+    if (r.n <= (uint32_t)NT) {
+      if (tid == 0) L.n = 0u;
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const uint32_t bits = __float_as_uint(p[u]);
+        thr_small_list<NT>(L, bits >= r.lo && bits <= r.hi, p[u], (uint32_t)(u * NT + tid));
+      }
+      __syncthreads();
+      return false;
+    }
+    if (r.lo == r.hi) {
+      const uint64_t kept =
+          r.use_p ? thr_tie_kept(__uint_as_float(r.lo), r.above, r.nabove, r.n, a.top_p) : r.n;
+      e = thr_tie_end(r, kept);
+      if (!e.partial) return true;  // uniform
+      // the id of member kept - 1: members by (u, wave, lane)
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const uint64_t bm = __ballot(__float_as_uint(p[u]) == r.lo);
+        if (lane == 0) L.h.cnt[u * NW + wv] = (uint32_t)__popcll(bm);
+      }
+      __syncthreads();
+      uint32_t k = (uint32_t)kept - 1u, s = 0;
+      while (s < (uint32_t)(PER * NW - 1) && k >= L.h.cnt[s]) k -= L.h.cnt[s++];
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const bool mem = __float_as_uint(p[u]) == r.lo;
+        const uint64_t bm = __ballot(mem);
+        const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
+        if (s == (uint32_t)(u * NW + wv) && mem && at == k) L.idcut = (uint32_t)(u * NT + tid);
+      }
+      __syncthreads();
+      e.idcut = L.idcut;
+      return true;
+    }
+    for (int b = tid; b < TH_NB; b += NT) { L.h.mass[b] = 0ull; L.h.cnt[b] = 0u; L.h.low[b] = ~0u; }
+    __syncthreads();
+    const uint32_t sh = thr_bin_shift(r);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const uint32_t bits = __float_as_uint(p[u]);
+      thr_bin_add(bits >= r.lo && bits <= r.hi, bits, r.hi, sh, L.h.mass, L.h.cnt, L.h.low);
+    }
+    __syncthreads();
+    if (!thr_pick<NT>(a, L.h.mass, L.h.cnt, L.h.low, sh, r, L.pick, L.s64)) {
+      e.vf = __uint_as_float(r.lo);
+      e.tot = r.above;
+      return true;
+    }
+  }
+}
 
-template <class E, int NT>
+template <class E, int NT, int PER>
 __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, int64_t ld_out) {
   constexpr int NW = NT / kWave;
   constexpr int BPT = TH_NB / NT;  // steps per thread
@@ -1184,16 +1258,16 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
     L.h.mass[tid + i * NT] = 0ull;
     L.h.cnt[tid + i * NT] = 0u;
   }
-  float x[TS_PER];
-  E raw[TS_PER];  // all loads first
+  float x[PER];
+  E raw[PER];  // all loads first
   float mx = -INFINITY, mn = INFINITY;
   bool nf = false;
 #pragma unroll
-  for (int u = 0; u < TS_PER; ++u) raw[u] = xr[min(u * NT + tid, V - 1)];
+  for (int u = 0; u < PER; ++u) raw[u] = xr[min(u * NT + tid, V - 1)];
 #pragma unroll
-  for (int u = 0; u < TS_PER; ++u) x[u] = u * NT + tid < V ? thr_f(raw[u]) : -INFINITY;
+  for (int u = 0; u < PER; ++u) x[u] = u * NT + tid < V ? thr_f(raw[u]) : -INFINITY;
 #pragma unroll
-  for (int u = 0; u < TS_PER; ++u) {
+  for (int u = 0; u < PER; ++u) {
     if (sizeof(E) == 2) nf |= (int32_t)__float_as_uint(x[u]) >= 0x7F800000;
     mx = fmaxf(mx, x[u]);
     mn = x[u] > -INFINITY ? fminf(mn, x[u]) : mn;
@@ -1218,7 +1292,7 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
   const float rT = 1.0f / T;
   thr_hist_kind(a, div, [&](auto DIV, auto MASS, auto CNT) {
 #pragma unroll
-    for (int u = 0; u < TS_PER; ++u) {
+    for (int u = 0; u < PER; ++u) {
       if (u * NT >= V) break;  // uniform
       thr_hist_one<DIV.value, MASS.value, CNT.value>(x[u], u * NT + tid < V, T, rT, m, scale,
                                                      steps, L.h.mass, L.h.cnt, zlo, zhi);
@@ -1233,7 +1307,9 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
   const bool bad = !(zf > 0.0f);
   ThrEnd r;
   ThrCut c;
-  {
+  if (!a.use_k && !a.use_p) {  // uniform: everything is above
+    c = thr_cut(a, m, zf, scale, 0, 0, 0);
+  } else {
     uint64_t ms[BPT], ct[BPT], sm = 0, sc = 0;
 #pragma unroll
     for (int i = 0; i < BPT; ++i) {
@@ -1255,11 +1331,11 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
     c = thr_cut(a, m, zf, scale, L.b0, L.b1, L.bk);
   }
   // p of this thread's elements; what lies above the region, and the region's list
-  float p[TS_PER];
+  float p[PER];
   uint64_t mass = 0;
   uint32_t cnt = 0;
 #pragma unroll
-  for (int u = 0; u < TS_PER; ++u) {
+  for (int u = 0; u < PER; ++u) {
     p[u] = 0.0f;
     if (u * NT >= V) continue;  // uniform
     const int i = u * NT + tid;
@@ -1268,15 +1344,7 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
     const bool above = take && p[u] > c.phi;
     mass += above ? fixed62(p[u]) : 0ull;
     cnt += above ? 1u : 0u;
-    const bool in = take && !above && p[u] >= c.plo;
-    const uint64_t bm = __ballot(in);
-    if (bm) {  // uniform per wave
-      uint32_t at = 0;
-      if (lane == 0) at = atomicAdd(&L.n, (uint32_t)__popcll(bm));
-      at = rdlane(at, 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32),
-                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
-      if (in) L.e[at] = ((uint64_t)(~__float_as_uint(p[u])) << 32) | (uint32_t)i;
-    }
+    thr_small_list<NT>(L, take && !above && p[u] >= c.plo, p[u], (uint32_t)i);
   }
   mass = wave_sum_u64(mass);
   cnt = wave_sum_u32(cnt);
@@ -1285,15 +1353,26 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
   __syncthreads();
   uint64_t above = 0, nabove = 0;
   for (int w = 0; w < NW; ++w) { above += L.s64[w]; nabove += L.u32[w]; }
-  const uint32_t n = L.n;
+  ThrSpan sp;
+  sp.above = above;
+  sp.nabove = nabove;
+  sp.n = L.n;
+  sp.use_k = c.use_k;
+  sp.use_p = c.use_p;
   r.tot = above;
-  if (c.use_k || c.use_p) {  // uniform
-    uint32_t S = NT;
-    while (S < n) S <<= 1;  // at most TS_PER * NT
-    for (uint32_t i = n + tid; i < S; i += NT) L.e[i] = ~0ull;
+  bool done = !(c.use_k || c.use_p);
+  float phi = c.phi;
+  if (__builtin_expect(sp.n > (uint32_t)NT, 0)) {  // uniform
+    sp.lo = __float_as_uint(c.plo);
+    sp.hi = __float_as_uint(fminf(phi, 1.0f));
+    done = thr_small_refine<NT, PER>(a, L, p, sp, r);
+    phi = __uint_as_float(sp.hi);
+  }
+  if (!done) {  // uniform
+    for (uint32_t i = sp.n + tid; i < (uint32_t)NT; i += NT) L.e[i] = ~0ull;
     __syncthreads();
-    r = thr_walk<NT>(a, thr_sort<NT, NT>(L.e, L.t, n), n, c.use_k, c.use_p, above, nabove, c.phi,
-                        L.w, L.s64);
+    r = thr_walk<NT>(a, thr_sort<NT, NT>(L.e, L.t, sp.n), sp.n, sp.use_k, sp.use_p, sp.above,
+                     sp.nabove, phi, L.w, L.s64);
   }
   if (tid == 0 && a.stats)
     a.stats[row] = thr_record(r, m, zf, c.xcut, gid, V, xg, T, L.nf != 0);
@@ -1301,7 +1380,7 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
   const float totf = fmaxf(rn32_u64(r.tot), 1e-12f);
   float* const o = out + row * ld_out;
 #pragma unroll
-  for (int u = 0; u < TS_PER; ++u) {
+  for (int u = 0; u < PER; ++u) {
     const int i = u * NT + tid;
     const bool kept = p[u] > r.vf || (p[u] == r.vf && (uint32_t)i <= r.idcut);
     if (i < V) o[i] = bad ? __builtin_nanf("") : kept ? p[u] / totf : 0.0f;
@@ -1633,12 +1712,12 @@ template <class E>
 static hipError_t thr_small(const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
                             hipStream_t s) {
   const dim3 grid((unsigned)rows);
-  if (a.V <= TS_PER * 256)
-    hipLaunchKernelGGL((thr_small_kernel<E, 256>), grid, dim3(256), 0, s, a, out, ld_out);
-  else if (a.V <= TS_PER * 512)
-    hipLaunchKernelGGL((thr_small_kernel<E, 512>), grid, dim3(512), 0, s, a, out, ld_out);
+  if (a.V <= 8 * 256)
+    hipLaunchKernelGGL((thr_small_kernel<E, 256, 8>), grid, dim3(256), 0, s, a, out, ld_out);
+  else if (a.V <= 8 * 512)
+    hipLaunchKernelGGL((thr_small_kernel<E, 512, 8>), grid, dim3(512), 0, s, a, out, ld_out);
   else
-    hipLaunchKernelGGL((thr_small_kernel<E, 1024>), grid, dim3(1024), 0, s, a, out, ld_out);
+    hipLaunchKernelGGL((thr_small_kernel<E, 1024, 8>), grid, dim3(1024), 0, s, a, out, ld_out);
   return hipGetLastError();
 }
 

@@ -112,9 +112,9 @@ def test_top_k_among_subnormal_probabilities(V):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
-@pytest.mark.parametrize("V", [9001, 33000, 151936])
+@pytest.mark.parametrize("V", [1001, 2048, 4001, 8192, 9001, 33000, 151936])
 def test_to_probs_refined_rows(dtype, V):
-    """Regions past the list of 2,048: flat rows whose masked ids (a finite value) widen
+    """Regions past the list (2,048, or 256 to 1,024 in short rows): flat rows whose masked ids (a finite value) widen
     the steps, tie groups within and across them, values too near for the first bins.
     The boundary ends in a short list, in a tie group (whole or in part) or nowhere."""
     rng = np.random.RandomState(V)
