@@ -110,6 +110,8 @@ int thr_to_probs(int dtype, const void* logits, int64_t rows, int64_t V, int64_t
   sdx::ThrArgs a = thr_args(logits, logits, rows, 0, ld, V, T, top_p, top_k, sw);
   if (V <= sdx::kThrSmall)
     return hip_status(sdx::launch_thr_small(dtype, a, rows, probs, ld_out, s), "thr_small");
+  if (sdx::thr_plain(V, sw.use_k, sw.use_p))
+    return hip_status(sdx::launch_thr_plain(dtype, a, rows, probs, ld_out, s), "thr_plain");
   a.stats = stats;
   a.scratch = probs; a.scratch_stride = ld_out * 4; a.scratch_bytes = V * 4;
   if (int e = hip_status(sdx::launch_thr_stats(dtype, a, rows, s), "thr_stats")) return e;

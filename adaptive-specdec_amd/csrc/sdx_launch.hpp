@@ -229,6 +229,10 @@ hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s);
 // where not null
 hipError_t launch_thr_small(int dtype, ThrArgs a, int64_t rows, float* out, int64_t ld_out,
                             hipStream_t s);
+// to_probs rows without a filter in one launch, and whether a call takes it
+bool thr_plain(int64_t V, int use_k, int use_p);
+hipError_t launch_thr_plain(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+                            hipStream_t s);
 // to_probs rows; the scratch may lie in `out` (it is read no more)
 hipError_t launch_thr_output(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
                              hipStream_t s);

@@ -22,7 +22,8 @@
 //                          reference's test. A region with more than kThrList
 //                          elements (a tie group, or a flat row) is refined over the
 //                          row itself, a thousand bins of p at a time;
-// then thr_output_kernel writes to_probs rows, and thr_draw_kernel is the verify's
+// then thr_output_kernel writes to_probs rows (of up to 32,768 ids and without a filter
+// thr_plain_kernel alone), and thr_draw_kernel is the verify's
 // accept chain and draw, which evaluates p where it needs it: a verify writes no
 // probabilities.
 //
@@ -1387,6 +1388,121 @@ __global__ void __launch_bounds__(NT) thr_small_kernel(ThrArgs a, float* out, in
   }
 }
 
+// ---------------------------------------------------------------- rows without a filter
+// softmax alone, a workgroup per row and one launch: maximum, exact normaliser, p and its
+// exact sum (p waits in the output row), division. The row's later passes come from the
+// L2. Bound by the instructions of two exps per element. fp32 to_probs at T = 0.7, us, the
+// kernels above | this: 1 row of 8,200 38 | 13, of 32,000 39 | 33, of 40,000 39 | 42; 256
+// rows of 8,200 47 | 15, of 32,000 83 | 44; 1,024 rows of 32,000 228 | 135. fp16: 1 row of
+// 32,000 40 | 37, 256 rows 85 | 47.
+constexpr int TP_NT = 1024, TP_NW = TP_NT / kWave;
+template <class E>
+__global__ void __launch_bounds__(TP_NT) thr_plain_kernel(ThrArgs a, float* out, int64_t ld_out) {
+  constexpr int N = ThrVec<E>::N;
+  __shared__ uint64_t s64[TP_NW], t64[TP_NW];
+  __shared__ float s_mx[TP_NW];
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  const E* const x = thr_row<E>(a, row);
+  float* const o = out + row * ld_out;
+  const int64_t V = a.V;
+  int64_t head = (int64_t)(((16u - ((uint32_t)(uintptr_t)x & 15u)) & 15u) / sizeof(E));
+  if (head > V) head = V;
+  const int64_t nv = (V - head) / N;
+  // the elements before the first and after the last whole vector: one a thread
+  const int64_t ie = tid < N ? (tid < head ? tid : -1)
+                             : tid < 2 * N && head + nv * N + (tid - N) < V
+                                   ? head + nv * N + (tid - N) : -1;
+  const float xe = ie >= 0 ? thr_f(x[ie]) : 0.0f;
+  const uint4* const x4 = reinterpret_cast<const uint4*>(x + head);
+  auto elem = [](const uint4& w, int e) {
+    const uint32_t q[4] = {w.x, w.y, w.z, w.w};
+    if constexpr (sizeof(E) == 4) return __uint_as_float(q[e]);
+    else return thr_f((uint16_t)(q[e >> 1] >> (16 * (e & 1))));
+  };
+  float mx = ie >= 0 ? xe : -INFINITY;
+  for (int64_t j = tid; j < nv; j += TP_NT) {
+    const uint4 w = x4[j];
+#pragma unroll
+    for (int e = 0; e < N; ++e) mx = fmaxf(mx, elem(w, e));
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, kWave));
+  if (lane == 0) s_mx[wv] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < TP_NW; ++w) mx = fmaxf(mx, s_mx[w]);
+  const float T = a.T, m = mx / T;
+  uint64_t zlo = 0;
+  uint32_t zhi = 0;
+  auto add = [&](float v) {
+    const uint64_t f = thr_exp62(v / T - m);
+    zlo += f;
+    zhi += zlo < f ? 1u : 0u;
+  };
+  if (ie >= 0) add(xe);
+#pragma unroll 2
+  for (int64_t j = tid; j < nv; j += TP_NT) {
+    const uint4 w = x4[j];
+#pragma unroll
+    for (int e = 0; e < N; ++e) add(elem(w, e));
+  }
+  U128 z = wave_sum_u128(U128{zlo, (uint64_t)zhi});
+  if (lane == 0) { s64[wv] = z.lo; t64[wv] = z.hi; }
+  __syncthreads();
+  z = U128{0, 0};
+  for (int w = 0; w < TP_NW; ++w) z = u128_add(z, U128{s64[w], t64[w]});
+  const float zf = rn32_u128(z);
+  const bool bad = !(zf > 0.0f);  // no finite maximum: every probability is 0 / 0
+  const bool vec = ((uintptr_t)(o + head) & 15u) == 0;  // uniform
+  uint64_t mass = 0;
+  auto prob = [&](float v) {  // a NaN logit has no mass, as above
+    const float p = v == v ? exp_det_sel(v / T - m) / zf : 0.0f;
+    mass += fixed62(p);
+    return bad ? __builtin_nanf("") : p;
+  };
+  if (ie >= 0) o[ie] = prob(xe);
+#pragma unroll 2
+  for (int64_t j = tid; j < nv; j += TP_NT) {
+    const uint4 w = x4[j];
+    float* const d = o + head + j * N;
+#pragma unroll
+    for (int h = 0; h < N; h += 4) {
+      const float4 p = make_float4(prob(elem(w, h)), prob(elem(w, h + 1)), prob(elem(w, h + 2)),
+                                   prob(elem(w, h + 3)));
+      if (vec) {
+        *reinterpret_cast<float4*>(d + h) = p;
+      } else {
+        d[h] = p.x; d[h + 1] = p.y; d[h + 2] = p.z; d[h + 3] = p.w;
+      }
+    }
+  }
+  mass = wave_sum_u64(mass);
+  __syncthreads();  // the normaliser's words are read
+  if (lane == 0) s64[wv] = mass;
+  __syncthreads();
+  uint64_t tot = 0;
+  for (int w = 0; w < TP_NW; ++w) tot += s64[w];
+  const float totf = fmaxf(rn32_u64(tot), 1e-12f);
+  // a thread's own elements again
+  if (ie >= 0) o[ie] = o[ie] / totf;
+#pragma unroll 2
+  for (int64_t j = tid; j < nv; j += TP_NT) {
+    float* const d = o + head + j * N;
+#pragma unroll
+    for (int h = 0; h < N; h += 4) {
+      if (vec) {
+        float4 p = *reinterpret_cast<const float4*>(d + h);
+        p.x /= totf; p.y /= totf; p.z /= totf; p.w /= totf;
+        *reinterpret_cast<float4*>(d + h) = p;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[h + e] /= totf;
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------- to_probs output
 // Wave by wave: zeros first, 16 bytes a lane, then the kept elements, compacted and
 // evaluated by full waves, over them (the wave waits for its zeros).
@@ -1727,6 +1843,19 @@ hipError_t launch_thr_small(int dtype, ThrArgs a, int64_t rows, float* out, int6
   if (a.V > kThrSmall || (!a.stats && !out)) return hipErrorInvalidValue;
   return dtype == SDX_F32 ? thr_small<float>(a, rows, out, ld_out, s)
                           : thr_small<uint16_t>(a, rows, out, ld_out, s);
+}
+
+// Above this a row is too long for one workgroup of a call with few (see the kernel).
+bool thr_plain(int64_t V, int use_k, int use_p) { return !use_k && !use_p && V <= 32768; }
+
+hipError_t launch_thr_plain(int dtype, const ThrArgs& a, int64_t rows, float* out, int64_t ld_out,
+                            hipStream_t s) {
+  const dim3 grid((unsigned)rows);
+  if (dtype == SDX_F32)
+    hipLaunchKernelGGL(thr_plain_kernel<float>, grid, dim3(TP_NT), 0, s, a, out, ld_out);
+  else
+    hipLaunchKernelGGL(thr_plain_kernel<uint16_t>, grid, dim3(TP_NT), 0, s, a, out, ld_out);
+  return hipGetLastError();
 }
 
 hipError_t launch_thr_stats(int dtype, ThrArgs a, int64_t rows, hipStream_t s) {

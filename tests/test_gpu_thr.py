@@ -162,6 +162,36 @@ def test_to_probs_rows_at_any_alignment(off, ld, ldo):
     assert bool((out[(n - 1) * ldo + V:] == -1.0).all())
 
 
+# 8193: the shortest row of this kernel, 32768: its longest; odd fp16 lengths
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("V", [8193, 12345, 32761, 32768])
+@pytest.mark.parametrize("T", [1.0, 0.7, 0.03, 400.0])
+def test_to_probs_without_a_filter(dtype, V, T):
+    x = _rows(V, V, dtype)
+    got = S.to_probs(torch.tensor(x, device=DEV), T).cpu().numpy()
+    _same(got, O.to_probs(x.astype(np.float32), T, 1.0, 0))
+    x[0], x[1, 3] = -np.inf, np.inf  # no finite maximum: 0 / 0
+    got = S.to_probs(torch.tensor(x, device=DEV), T).cpu().numpy()
+    assert np.isnan(got[:2]).all() and not np.isnan(got[2:]).any()
+
+
+@pytest.mark.parametrize("off,ld,ldo", [(0, 9001, 9003), (1, 9002, 9001), (3, 9004, 9007)])
+def test_to_probs_without_a_filter_at_any_alignment(off, ld, ldo):
+    V, L = 9001, _lib.lib()
+    x = _rows(V, 6)
+    n = x.shape[0]
+    buf = torch.zeros(off + n * ld, device=DEV)
+    buf[off:].view(n, ld)[:, :V].copy_(torch.tensor(x))
+    out = torch.full((n * ldo + 4,), -1.0, device=DEV)
+    ws = _lib.workspace(L.sdx_to_probs_workspace(n, V, _lib.F32), DEV, prepare=False)
+    rc = L.sdx_to_probs(buf.data_ptr() + 4 * off, _lib.F32, n, V, ld, 0.8, 1.0, 0, _lib.ptr(out),
+                        ldo, _lib.ptr(ws), ws.numel(), _lib.stream_of(out))
+    _lib.check(rc, "to_probs")
+    got = out[: n * ldo].view(n, ldo)
+    _same(np.ascontiguousarray(got[:, :V].cpu().numpy()), O.to_probs(x, 0.8, 1.0, 0))
+    assert bool((got[:-1, V:] == -1.0).all()) and bool((out[(n - 1) * ldo + V:] == -1.0).all())
+
+
 def _verify_case(B, k, V, dtype, seed):
     """Logits of the row shapes above (without those whose p is 0 / 0 in every target),
     drafted ids from the likely ones and from tie groups."""
