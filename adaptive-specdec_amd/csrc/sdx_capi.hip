@@ -234,15 +234,16 @@ size_t sdx_sample_probs_workspace(int64_t rows, int64_t vocab) {
   return c.used;
 }
 
+// a draw from each row on u[row], and the draws' counters cleared
 __global__ void sdx_jobs_from_u(sdx::SampleJob* jobs, const float* u, int64_t rows,
-                                int64_t qsplit, uint32_t* counters) {
+                                uint32_t* counters) {
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= rows) return;
-  if (counters) counters[r] = 0u;
+  counters[r] = 0u;
   sdx::SampleJob j;
   j.prow = r;
-  j.qrow = qsplit >= 0 ? qsplit + r : -1;
-  j.u = u ? u[r] : 0.0f;
+  j.qrow = -1;
+  j.u = u[r];
   j.pad = 0;
   jobs[r] = j;
 }
@@ -866,7 +867,7 @@ int sdx_draft_step(const void* logits, int dtype, int64_t batch, int64_t vocab, 
   } else {
     if (int r = row_stats16(dtype, a, batch, s)) return r;
     hipLaunchKernelGGL(sdx_jobs_from_u, dim3((unsigned)((batch + 255) / 256)), dim3(256), 0, s,
-                       jobs, u, batch, (int64_t)-1, counters);
+                       jobs, u, batch, counters);
     if (int r = hip_status(hipGetLastError(), "jobs")) return r;
     if (int r = hip_status(sdx::launch_draw_rows16(dtype, src, st, tb, temperature, jobs, batch,
                                                    vocab, recs, counters, x, s),

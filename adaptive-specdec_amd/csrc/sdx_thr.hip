@@ -239,7 +239,9 @@ __global__ void __launch_bounds__(TH_NT) thr_max_kernel(ThrArgs a) {
 // ---------------------------------------------------------------- 2. normaliser, region
 // fixed62(exp_det(d)) for d <= 0 (and 0 for NaN): exp_det's steps, then the value
 // mant * 2^(k + 39) as a right shift of mant << 39 (k is in [-63, 0] after the clamp at
-// -43.5, below which the value is 0). Equal to the two functions over every fp32 d.
+// -43.5, below which the value is 0). Equal to the two functions over every fp32 d:
+// above the clamp p 2^k is normal, so exp_det does not round and fixed62 truncates the
+// same 24 bits.
 __device__ __forceinline__ uint64_t thr_exp62(float d) {
 #pragma clang fp contract(off)
   const double dd = (double)fmaxf(d, -43.5f);
