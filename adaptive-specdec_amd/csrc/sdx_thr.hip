@@ -35,12 +35,12 @@
 // waves. Splitting a row over workgroups keeps the chip full from a few rows on.
 // Measured on fp32 rows of 151,936 (one workgroup of 1024 threads per row before, with
 // seven IEEE divisions per element and dense probabilities for the draw): verify of 8
-// batch rows at k = 4 (72 rows, top-k 50) 285 -> 61 us (kernels 11 + 26 + 11 + 6 and
-// the draw 11), to_probs of 256 rows 378 -> 197 us (52 + 56 + 31 + 8 + 53: the first
-// pass also pays for the write-back of the call before, the last moves 5.9 TB/s). On
+// batch rows at k = 4 (72 rows, top-k 50) 283 -> 61 us (kernels 10 + 26 + 11 + 6 and
+// the draw 11), to_probs of 256 rows 370 -> 197 us (53 + 56 + 32 + 7 + 54: the exp pass
+// issues 54 vector instructions an element, on full SIMDs; the last moves 6.3 TB/s). On
 // fp16 rows (one workgroup of 1024 threads and a histogram of 36,864 values per row
-// before): verify of 16 batch rows at k = 4, V = 131,072 144 -> 79 us (10 + 31 + 16 + 8
-// and the draw 17), of 64 at V = 32,000 161 -> 90 us; to_probs of 64 x 131,072 132 -> 65 us.
+// before): verify of 16 batch rows at k = 4, V = 131,072 142 -> 79 us (10 + 31 + 16 + 8
+// and the draw 17), of 64 at V = 32,000 165 -> 75 us; to_probs of 64 x 131,072 132 -> 54 us.
 // The compare passes keep the evaluation in one place of their code (a loop over a
 // queue in LDS): unrolled into every element's place, 16 to 64 copies, the collect
 // pass of the fp16 verify took 20 us instead of 17 and its draw 22 instead of 20. The
@@ -1142,8 +1142,8 @@ __global__ void __launch_bounds__(NT) thr_resolve_kernel(ThrArgs a) {
 // 2,048, 512 up to 4,096, 1,024 above, so that short rows share a CU). A region of more
 // than a list of NT is refined as above, from the registers. With `out`, also the
 // to_probs row. Bound by the latency of its chain of block reductions. to_probs of 64
-// fp32 rows of 4,096: 15 us against 69 us for a bitonic sort of the row in LDS, of 256
-// of 8,192 20 against 131 us, of 20,000 of 64 143 against 1,141 us.
+// fp32 rows of 4,096: 13 us against 69 us for a bitonic sort of the row in LDS, of 256
+// of 8,192 21 against 131 us, of 20,000 of 64 148 against 1,141 us.
 template <int NT>
 struct ThrSmallLds {
   uint64_t e[NT];  // the region's list
