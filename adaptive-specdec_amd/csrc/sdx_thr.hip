@@ -1098,19 +1098,23 @@ __global__ void __launch_bounds__(NT) thr_resolve_kernel(ThrArgs a) {
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const ThrCtl* const c = thr_ctl(a, row);
+  // everything that needs no other is loaded before the first wait
   const uint32_t n = c->nlist;
-  if (n <= (uint32_t)kThrList && tid >= TH_NT) return;  // whole waves
   const E* const x = thr_row<E>(a, row);
   const float m = c->m, zf = c->zf, T = a.T;
+  const uint64_t pm = lane < a.nlight ? c->pmass[lane] : 0ull;
+  const uint32_t pc = lane < a.nlight ? c->pcnt[lane] : 0u;
+  const uint32_t pnf = lane < a.nlight ? c->pnf[lane] : 0u;
+  const int64_t gid = thr_gid(a, row);
   ThrSpan sp;
-  sp.above = wave_sum_u64(lane < a.nlight ? c->pmass[lane] : 0ull);
-  sp.nabove = wave_sum_u32(lane < a.nlight ? c->pcnt[lane] : 0u);
-  sp.n = n;
   sp.use_k = c->use_k != 0;
   sp.use_p = c->use_p != 0;
-  const int64_t gid = thr_gid(a, row);
-  const float xg = gid >= 0 && gid < a.V ? thr_f(x[gid]) : 0.0f;
   float phi = c->phi;
+  if (NT > TH_NT && n <= (uint32_t)kThrList && tid >= TH_NT) return;  // whole waves
+  const float xg = gid >= 0 && gid < a.V ? thr_f(x[gid]) : 0.0f;
+  sp.above = wave_sum_u64(pm);
+  sp.nabove = wave_sum_u32(pc);
+  sp.n = n;
   ThrEnd r;
   r.tot = sp.above;
   bool done = !(sp.use_k || sp.use_p);
@@ -1132,7 +1136,7 @@ __global__ void __launch_bounds__(NT) thr_resolve_kernel(ThrArgs a) {
     r = thr_walk<TH_NT>(a, thr_sort<TH_NT, kThrCount>(L.e, L.t, sp.n), sp.n, sp.use_k, sp.use_p,
                         sp.above, sp.nabove, phi, L.w, L.s64);
   }
-  const bool nonfinite = __ballot(lane < a.nlight && c->pnf[lane < a.nlight ? lane : 0] != 0) != 0;
+  const bool nonfinite = __ballot(pnf != 0) != 0;
   if (tid == 0) a.stats[row] = thr_record(r, m, zf, c->xcut, gid, a.V, xg, T, nonfinite);
 }
 
