@@ -35,12 +35,12 @@
 // waves. Splitting a row over workgroups keeps the chip full from a few rows on.
 // Measured on fp32 rows of 151,936 (one workgroup of 1024 threads per row before, with
 // seven IEEE divisions per element and dense probabilities for the draw): verify of 8
-// batch rows at k = 4 (72 rows, top-k 50) 283 -> 61 us (kernels 10 + 26 + 11 + 6 and
+// batch rows at k = 4 (72 rows, top-k 50) 283 -> 60 us (kernels 10 + 26 + 11 + 6 and
 // the draw 11), to_probs of 256 rows 370 -> 197 us (53 + 56 + 32 + 7 + 54: the exp pass
 // issues 54 vector instructions an element, on full SIMDs; the last moves 6.3 TB/s). On
 // fp16 rows (one workgroup of 1024 threads and a histogram of 36,864 values per row
-// before): verify of 16 batch rows at k = 4, V = 131,072 142 -> 79 us (10 + 31 + 16 + 8
-// and the draw 17), of 64 at V = 32,000 165 -> 75 us; to_probs of 64 x 131,072 132 -> 54 us.
+// before): verify of 16 batch rows at k = 4, V = 131,072 142 -> 77 us (10 + 30 + 16 + 8
+// and the draw 17), of 64 at V = 32,000 165 -> 74 us; to_probs of 64 x 131,072 132 -> 54 us.
 // The compare passes keep the evaluation in one place of their code (a loop over a
 // queue in LDS): unrolled into every element's place, 16 to 64 copies, the collect
 // pass of the fp16 verify took 20 us instead of 17 and its draw 22 instead of 20. The
@@ -313,8 +313,8 @@ __device__ __forceinline__ float thr_xskip(float m, float scale, uint32_t steps,
 // boundary that no step holds is there, and much of a row can be, most of it at low
 // temperatures (64 lanes at one LDS address go one after the other: fp16 verify of 16
 // rows, V = 131,072, T = 0.1, top-k 20 97 us with it, 74 without).
-// `steps` is past every element (ALL) where a top-k's range holds them and T does not
-// press them together: the comparison costs such a pass 2%.
+// `steps` is past every element (ALL) with both filters, where the range holds them and
+// T does not press them together: the comparison costs such a pass 2%.
 template <int DIV, bool MASS, bool CNT, bool ALL = false>
 __device__ __forceinline__ void thr_hist_one(float x, bool ok, float T, float rT, float m,
                                              float scale, uint32_t steps, uint64_t* mass,
@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(TH_NT) thr_hist_kernel(ThrArgs a) {
   const float low = thr_xskip(m, scale, steps, T);
   thr_hist_kind(a, div, [&](auto DIV, auto MASS, auto CNT) {
     auto one = [&](int64_t, float xv, bool ok) {
-      thr_hist_one<DIV.value, MASS.value, CNT.value, CNT.value && !SKIP>(
+      thr_hist_one<DIV.value, MASS.value, CNT.value, MASS.value && CNT.value && !SKIP>(
           xv, ok, T, rT, m, scale, steps, L.mass, L.cnt, zlo, zhi);
     };
     thr_stream<E, 4, SKIP>(x, a.V, part, a.nparts, a.plen, one, [] {}, low);
@@ -891,7 +891,7 @@ __device__ __forceinline__ void thr_bin_add(bool in, uint32_t bits, uint32_t hi,
   }
 }
 
-constexpr int kThrCount = 2 * TH_NT;  // lists up to here are sorted by counting
+constexpr int kThrCount = 2 * TH_NT;  // lists up to here are sorted by TH_NT threads, by counting
 template <int NT>
 struct ThrResLds {
   uint64_t e[kThrList];  // the list; the refinement's masses
@@ -901,7 +901,7 @@ struct ThrResLds {
   ThrPickLds pick;
   uint32_t n, idcut;
   union {
-    uint64_t t[kThrCount];  // a list of up to kThrCount entries, sorted
+    uint64_t t[NT > TH_NT ? kThrList : kThrCount];  // a list sorted by counting
     ThrQueue<4> q[NT / kWave];
   };
 };
@@ -1088,8 +1088,9 @@ __device__ __forceinline__ bool thr_refine(const ThrArgs& a, ThrResLds<NT>& L, c
   }
 }
 
-// One workgroup per row. Only a refinement uses more than the first TH_NT threads; the
-// others end at once otherwise. NT 1,024 where every row has a CU of its own (a row of
+// One workgroup per row. Only a refinement and lists of more than kThrCount entries use
+// more than the first TH_NT threads (a list of 2,048 by counting with 1,024 threads, 15
+// us less than a bitonic sort with 256); the others end at once otherwise. NT 1,024 where every row has a CU of its own (a row of
 // 131,072 equal logits, T = 0.7, top_p 0.9, top-k 50 231 us against 546 with 256), 256
 // for more rows (fp16 to_probs of 576 rows of 32,000 85 us, 89 with 1,024).
 template <class E, int NT>
@@ -1110,7 +1111,7 @@ __global__ void __launch_bounds__(NT) thr_resolve_kernel(ThrArgs a) {
   sp.use_k = c->use_k != 0;
   sp.use_p = c->use_p != 0;
   float phi = c->phi;
-  if (NT > TH_NT && n <= (uint32_t)kThrList && tid >= TH_NT) return;  // whole waves
+  if (NT > TH_NT && n <= (uint32_t)kThrCount && tid >= TH_NT) return;  // whole waves
   const float xg = gid >= 0 && gid < a.V ? thr_f(x[gid]) : 0.0f;
   sp.above = wave_sum_u64(pm);
   sp.nabove = wave_sum_u32(pc);
@@ -1123,18 +1124,25 @@ __global__ void __launch_bounds__(NT) thr_resolve_kernel(ThrArgs a) {
     sp.hi = __float_as_uint(fminf(phi, 1.0f));
     done = thr_refine<E, NT>(a, L, x, c, sp, r);
     phi = __uint_as_float(sp.hi);
-    if (tid >= TH_NT) return;  // whole waves
   } else if (!done) {
     const uint64_t* const list = reinterpret_cast<const uint64_t*>(c + 1);
-    for (uint32_t i = tid; i < n; i += TH_NT) L.e[i] = list[i];
+    for (uint32_t i = tid; i < n; i += n > (uint32_t)kThrCount ? NT : TH_NT) L.e[i] = list[i];
   }
   if (!done) {  // uniform
-    uint32_t S = kThrCount;
-    while (S < sp.n) S <<= 1;
-    for (uint32_t i = sp.n + tid; i < S; i += TH_NT) L.e[i] = ~0ull;
-    __syncthreads();
-    r = thr_walk<TH_NT>(a, thr_sort<TH_NT, kThrCount>(L.e, L.t, sp.n), sp.n, sp.use_k, sp.use_p,
-                        sp.above, sp.nabove, phi, L.w, L.s64);
+    auto walk = [&](auto nt, auto count) {
+      uint32_t S = kThrCount;
+      while (S < sp.n) S <<= 1;
+      for (uint32_t i = sp.n + tid; i < S; i += nt.value) L.e[i] = ~0ull;
+      __syncthreads();
+      r = thr_walk<nt.value>(a, thr_sort<nt.value, count.value>(L.e, L.t, sp.n), sp.n, sp.use_k,
+                             sp.use_p, sp.above, sp.nabove, phi, L.w, L.s64);
+    };
+    if (NT > TH_NT && sp.n > (uint32_t)kThrCount) {  // uniform
+      walk(std::integral_constant<int, NT>{}, std::integral_constant<int, NT == TH_NT ? kThrCount : kThrList>{});
+    } else {
+      if (tid >= TH_NT) return;  // whole waves
+      walk(std::integral_constant<int, TH_NT>{}, std::integral_constant<int, kThrCount>{});
+    }
   }
   const bool nonfinite = __ballot(pnf != 0) != 0;
   if (tid == 0) a.stats[row] = thr_record(r, m, zf, c->xcut, gid, a.V, xg, T, nonfinite);
@@ -1784,15 +1792,19 @@ __global__ void __launch_bounds__(TH_NT) thr_draw_kernel(ThrDrawArgs a) {
 
 // ---------------------------------------------------------------- launches
 
-// How far below the maximum (in s) the boundary of a row can lie. Top-k: anywhere p is
-// above 0 (104 units). A nucleus ends where less than 1 - top_p of the mass is left,
+// How far below the maximum (in s) the steps reach. The k-th largest can be anywhere p is
+// above 0 (104 units); alone, in the thousands and at ordinary temperatures it is within
+// 32, and finite mask values do not widen the steps (where it is not, the last step is
+// refined: fp16 to_probs of 72 rows of 131,072, N(0, 1) with a -1e4 mask, T = 2, top-k
+// 5000 102 -> 86 us with the lists below). A nucleus ends where less than 1 - top_p of the mass is left,
 // and D units below the maximum that is at most V e^-D of it (of at least 1): within 15
 // units for V = 151,936 and top_p 0.95, so that a row's finite mask values do not widen
 // the steps; 32 units where top_p is so near 1 that its rounding counts. With a top-k
 // too, the nucleus bounds the range only at low temperatures (see thr_hist_one).
 constexpr float TH_LOWT = 0.25f;
 static float thr_dmax(const ThrArgs& a) {
-  const double most = a.use_k ? 104.0 : 32.0;
+  const bool near = !a.use_k || (!a.use_p && a.top_k > 1024 && a.T >= 0.7f);
+  const double most = near ? 32.0 : 104.0;
   const double rest = 1.0 - (double)a.top_p - 2e-6;  // the region's margin of 1e-6, and roundings
   if (!a.use_p || rest < 2e-6 || (a.use_k && a.T > TH_LOWT)) return (float)most;
   return (float)fmin(most, log((double)a.V) - log(rest) + 0.25);
